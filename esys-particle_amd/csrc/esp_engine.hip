@@ -269,7 +269,14 @@ struct esp_engine {
   int ring_size = 0;
   DBuf<int> halted, broken_list, dev_int;
   int broken_cap = 0;
-  DBuf<double> wall_part, wall_hist;
+  DBuf<double> wall_part;
+  PinBuf<double> batch_out;  // what the end of a batch reports: a BatchOut, then wall forces
+  // engines without bonded groups (contact_mode): the arrays a step writes, each
+  // particle's interactions as rows, the 64-particle groups with wall candidates
+  DBuf<double4> pos2, vel2, ang2;
+  DBuf<int> row_cnt, wall_mark, wall_list;
+  DBuf<int2> rows, contact_ent;
+  int row_stride = 0, row_width = 0;
 
   std::vector<DynGroup> dg;
   std::vector<BondGroup> bg;
@@ -316,6 +323,25 @@ struct esp_engine {
 };
 
 namespace {
+
+// Without bonded groups a step is one launch in which every particle evaluates
+// its own pairs (k_contact_step); with them the pair and bond laws run once per
+// interaction and a second launch gathers their shares (a bond's law is too
+// long to be evaluated from both ends).
+bool contact_mode(const esp_engine* e) { return e->bg.empty(); }
+
+// one NRotElastic group: a few lanes walk each particle's row (k_contact_step);
+// any other mix of groups: a block's pairs are packed first (k_contact_block)
+bool contact_rows(const esp_engine* e) { return e->dg.size() == 1 && e->dg[0].kind == 1; }
+
+// wall partials of one step
+int wall_blocks(const esp_engine* e)
+{
+  return contact_mode(e) ? contact_groups(e->n) : gather_blocks(e->n);
+}
+
+constexpr size_t kBatchHead = sizeof(BatchOut) / sizeof(double);
+static_assert(sizeof(BatchOut) % sizeof(double) == 0, "the wall forces follow the status");
 
 void sync(esp_engine* e) { HIPCHK(hipStreamSynchronize(e->stream)); }
 
@@ -761,14 +787,23 @@ void upload(esp_engine* e)
   e->xcnt.reserve(cap);
   e->flist.reserve(cap);
   zero(e, e->xcnt.p, cap);
-  const int nb = std::max(gather_blocks(n), 1);
+  if (contact_mode(e)) {
+    e->pos2.reserve(cap);
+    e->vel2.reserve(cap);
+    if (e->rot) e->ang2.reserve(cap);
+    e->row_cnt.reserve(cap);
+    e->wall_mark.reserve((size_t)contact_groups((int)cap));
+    e->wall_list.reserve((size_t)contact_groups((int)cap) + 1);
+    zero(e, e->wall_list.p, (size_t)contact_groups((int)cap) + 1);
+  }
+  const int nb = std::max(wall_blocks(e), 1);
   const int nwg = (int)e->wg.size();
   e->wall_part.reserve((size_t)(e->K + 1) * nb * std::max(nwg, 1) * 3);
   if (e->ss == 9) {
     e->sig.reserve((size_t)std::max(n, 1) * 9);
     zero(e, e->sig.p, (size_t)std::max(n, 1) * 9);
   }
-  e->wall_hist.reserve((size_t)(e->K + 1) * std::max(nwg, 1) * 3);
+  e->batch_out.reserve(kBatchHead + (size_t)(e->K + 1) * std::max(nwg, 1) * 3);
   sync(e);
   e->started = true;
 }
@@ -1340,10 +1375,15 @@ void rebuild_csr(esp_engine* e)
   for (int gi : e->dord)
     if (e->dg[gi].n >= (1 << 27)) throw EspError(ESP_ERR_CAPACITY, "more than 2^27 pairs in one group");
   e->nrec = (int)rec;
-  e->slot_of.reserve((size_t)std::max<long long>(rec, 1));
   zero(e, e->inc_cnt.p, e->n + 1);
   for (int gi : e->dord) launch_inc_count(e->stream, e->dg[gi].n, e->dg[gi].ij.p, e->inc_cnt.p);
   for (int gi : e->bord) launch_inc_count(e->stream, e->bg[gi].n, e->bg[gi].ij.p, e->inc_cnt.p);
+  int width = 0;  // longest run of a particle
+  if (contact_mode(e) && contact_rows(e)) {
+    zero(e, e->dev_int.p, 1);
+    launch_max_int(e->stream, e->n, e->inc_cnt.p, e->dev_int.p);
+    d2h(e, &width, e->dev_int.p, 1);
+  }
   const int total = scan_total(e, e->inc_cnt.p, e->inc_off.p, e->n);
   e->inc_ent.reserve(std::max(total, 1));
   e->inc_ent64.reserve(std::max(total, 1));
@@ -1362,6 +1402,28 @@ void rebuild_csr(esp_engine* e)
                     e->inc_fill.p, e->inc_ent64.p);
   }
   launch_inc_sort(e->stream, e->n, e->inc_off.p, e->inc_ent64.p, e->inc_ent.p);
+  if (contact_mode(e)) {
+    RecordLists rl;
+    memset(&rl, 0, sizeof rl);
+    for (int gi : e->dord) {
+      rl.rec_off[rl.count] = e->dg[gi].rec_off;
+      rl.ij[rl.count++] = e->dg[gi].ij.p;
+    }
+    if (contact_rows(e)) {
+      e->row_stride = (std::max(e->n, 1) + 63) & ~63;
+      e->row_width = width;
+      e->rows.reserve((size_t)std::max(width, 1) * e->row_stride);
+      launch_contact_rows(e->stream, e->n, e->row_stride, e->inc_off.p, e->inc_ent.p, rl,
+                          e->row_cnt.p, e->rows.p);
+    } else {
+      e->contact_ent.reserve(std::max(total, 1));
+      launch_contact_entries(e->stream, total, e->inc_ent.p, rl, e->contact_ent.p);
+    }
+    e->xbase = total;
+    HIPCHK(hipGetLastError());
+    return;
+  }
+  e->slot_of.reserve((size_t)std::max<long long>(rec, 1));
   launch_slot_of(e->stream, total, e->inc_ent.p, e->slot_of.p);
   // slots start at zero: a contact that is not touching keeps zero slots
   // without rewriting them every step
@@ -1493,15 +1555,103 @@ ScLaunch sc_launch(esp_engine* e, long long step)
   sl.nblocks = blk;
   return sl;
 }
+// walls, body forces, damping and the integrator of one step
+GatherParams gather_params(esp_engine* e, const StepCtl& ctl, bool last)
+{
+  GatherParams gp;
+  memset(&gp, 0, sizeof gp);
+  gp.inc_off = e->inc_off.p;
+  gp.xcnt = e->xcnt.p;
+  gp.xbase = e->xbase;
+  gp.grid = e->grid;
+  gp.slots = e->slots.p;
+  gp.sact = e->sact.p;
+  gp.dt = e->dt;
+  gp.rot = e->rot;
+  gp.do2d = e->do2d;
+  gp.nwg = (int)e->wg.size();
+  wall_params(e, gp.wall);
+  gp.ngrav = (int)e->gord.size();
+  for (size_t k = 0; k < e->gord.size(); k++)
+    for (int c = 0; c < 3; c++) gp.g[k][c] = e->grav[e->gord[k]].g[c];
+  gp.wall_part = e->wall_part.p + (size_t)(ctl.step_id - 1) * wall_blocks(e) * gp.nwg * 3;
+  gp.sig = e->ss == 9 ? e->sig.p : nullptr;
+  gp.n_app = e->dg.empty() ? nullptr : e->dg[e->dord[0]].napp.p;
+  gp.store_fm = last ? 1 : 0;
+  gp.ndamp = (int)e->damp.size();
+  for (int d = 0; d < gp.ndamp; d++) {
+    gp.damp_type[d] = e->damp[d].type;
+    gp.damp_visc[d] = e->damp[d].visc;
+    gp.damp_maxit[d] = e->damp[d].maxit;
+  }
+  gp.inert = e->inert.p;
+  gp.init = e->init.p;
+  return gp;
+}
+
+// a whole step of an engine without bonded groups
+void launch_contacts(esp_engine* e, const StepCtl& ctl, bool flip, bool last)
+{
+  PView p = e->view();
+  ContactLaunch cl;
+  memset(&cl, 0, sizeof cl);
+  cl.do2d = e->do2d;
+  cl.stride = e->row_stride;
+  cl.width = e->row_width;
+  cl.period = e->grid.period;
+  cl.dt = e->dt;
+  if (contact_rows(e)) {
+    cl.cnt = e->row_cnt.p;
+    cl.rows = e->rows.p;
+  }
+  cl.off = e->inc_off.p;
+  cl.ent = e->contact_ent.p;
+  cl.pos_o = e->pos2.p;
+  cl.vel_o = e->vel2.p;
+  cl.ang_o = e->ang2.p;
+  if (flip) {
+    std::swap(p.pos, cl.pos_o);
+    std::swap(p.vel, cl.vel_o);
+    std::swap(p.ang, cl.ang_o);
+  }
+  for (int gi : e->dord) {
+    DynGroup& G = e->dg[gi];
+    ContactSeg& s = cl.seg[cl.count++];
+    s.kind = G.kind == 1 ? ESP_SEG_NROT_ELASTIC : G.kind == 2 ? ESP_SEG_ROT_ELASTIC
+                                                              : ESP_SEG_ROT_FRICTION;
+    s.rec_off = G.rec_off;
+    if (G.kind == 3) {
+      s.ff = flip ? G.ff2.p : G.ff.p;
+      s.ff_out = flip ? G.ff.p : G.ff2.p;
+    }
+    s.k = G.k;
+    s.ks = G.ks;
+    s.mu_d = G.mu_d;
+    s.mu_s = G.mu_s;
+    s.rigid = G.rigid;
+    s.scaling = G.scaling;
+    s.meanR = G.meanR;
+  }
+  const GatherParams gp = gather_params(e, ctl, last);
+  const LaunchEvents t = launch_events(e);
+  note_launch(e, t, launch_contact_step(e->stream, ctl, p, cl, gp, t.a, t.b), ESP_KCLASS_GATHER,
+              ctl.step_id);
+  HIPCHK(hipGetLastError());
+}
+
 // last: the host may read the particles' total forces and moments after this
 // step (the last step of a queued batch, every host step); other steps keep
 // them in registers only
 void launch_step(esp_engine* e, const StepCtl& ctl, long long step, bool flip, bool last)
 {
+  if (contact_mode(e)) {
+    launch_contacts(e, ctl, flip, last);
+    return;
+  }
   PView p = e->view();
   const ForceLaunch fl = force_launch(e, step, flip);
   UpdParams up;
-  const bool dev_update = ctl.guarded && !e->bg.empty();
+  const bool dev_update = ctl.guarded;
   if (dev_update) {
     // bookkeeping of the previous step's bond breaks, on the device
     memset(&up, 0, sizeof up);
@@ -1547,34 +1697,7 @@ void launch_step(esp_engine* e, const StepCtl& ctl, long long step, bool flip, b
                 launch_forces(e->stream, ctl, p, fl, dev_update ? &up : nullptr, t.a, t.b, &ext),
                 ESP_KCLASS_FORCES, ctl.step_id);
   }
-  GatherParams gp;
-  memset(&gp, 0, sizeof gp);
-  gp.inc_off = e->inc_off.p;
-  gp.xcnt = e->xcnt.p;
-  gp.xbase = e->xbase;
-  gp.grid = e->grid;
-  gp.slots = e->slots.p;
-  gp.sact = e->sact.p;
-  gp.dt = e->dt;
-  gp.rot = e->rot;
-  gp.do2d = e->do2d;
-  gp.nwg = (int)e->wg.size();
-  wall_params(e, gp.wall);
-  gp.ngrav = (int)e->gord.size();
-  for (size_t k = 0; k < e->gord.size(); k++)
-    for (int c = 0; c < 3; c++) gp.g[k][c] = e->grav[e->gord[k]].g[c];
-  gp.wall_part = e->wall_part.p + (size_t)(ctl.step_id - 1) * gather_blocks(e->n) * gp.nwg * 3;
-  gp.sig = e->ss == 9 ? e->sig.p : nullptr;
-  gp.n_app = e->dg.empty() ? nullptr : e->dg[e->dord[0]].napp.p;
-  gp.store_fm = last ? 1 : 0;
-  gp.ndamp = (int)e->damp.size();
-  for (int d = 0; d < gp.ndamp; d++) {
-    gp.damp_type[d] = e->damp[d].type;
-    gp.damp_visc[d] = e->damp[d].visc;
-    gp.damp_maxit[d] = e->damp[d].maxit;
-  }
-  gp.inert = e->inert.p;
-  gp.init = e->init.p;
+  const GatherParams gp = gather_params(e, ctl, last);
   {
     const LaunchEvents t = launch_events(e);
     note_launch(e, t, launch_gather_integrate(e->stream, ctl, p, gp, t.a, t.b), ESP_KCLASS_GATHER,
@@ -1593,8 +1716,10 @@ unsigned long long thresh_bits(esp_engine* e)
   return b;
 }
 
-void record_walls(esp_engine* e, const std::vector<double>& h, int steps)
+// wall forces of the batch's completed steps, from e->batch_out
+void record_walls(esp_engine* e, int steps)
 {
+  const double* h = e->batch_out.p + kBatchHead;
   const int nwg = (int)e->wg.size();
   for (int s = 0; s < steps; s++)
     for (int w = 0; w < (int)e->walls.size(); w++) {
@@ -1644,10 +1769,40 @@ void sync_history_buffers(esp_engine* e)
   }
 }
 
-void swap_history_buffers(esp_engine* e)
+// after an odd number of steps: what they wrote becomes what the next step reads
+void swap_step_buffers(esp_engine* e)
 {
   for (auto& G : e->dg)
     if (G.kind == 3) G.ff.swap(G.ff2);
+  if (contact_mode(e)) {
+    e->pos.swap(e->pos2);
+    e->vel.swap(e->vel2);
+    e->ang.swap(e->ang2);
+  }
+}
+
+// the end of a batch of k steps from step0 on, reported into e->batch_out
+void launch_end(esp_engine* e, long long step0, int k)
+{
+  BatchEnd be;
+  memset(&be, 0, sizeof be);
+  be.part = e->wall_part.p;
+  be.nblocks = wall_blocks(e);
+  be.nwg = (int)e->wg.size();
+  be.nsteps = k;
+  if (contact_mode(e)) {
+    be.list = e->wall_list.p + 1;
+    be.list_n = e->wall_list.p;
+  }
+  be.ring = e->ring.p;
+  be.ring_size = e->ring_size;
+  be.step0 = step0;
+  be.halted = e->halted.p;
+  be.reason = &e->upd.p->halt_reason;
+  be.out = reinterpret_cast<BatchOut*>(e->batch_out.p);
+  be.walls = e->batch_out.p + kBatchHead;
+  launch_batch_end(e->stream, be);
+  HIPCHK(hipGetLastError());
 }
 
 // one step with host bookkeeping: the first step, a rebuild, or an
@@ -1694,34 +1849,33 @@ void host_step(esp_engine* e, int reason)
     if (!e->wg.empty()) {
       WallParam w[ESP_MAX_WALL_GROUPS];
       wall_params(e, w);
-      launch_wall_update(e->stream, e->view(), e->grid, (int)e->wg.size(), w);
+      const bool cm = contact_mode(e);
+      launch_wall_update(e->stream, e->view(), e->grid, (int)e->wg.size(), w,
+                         cm ? e->wall_mark.p : nullptr);
+      if (cm)
+        launch_wall_list(e->stream, contact_groups(e->n), e->wall_mark.p, e->wall_list.p + 1,
+                         e->wall_list.p);
       HIPCHK(hipGetLastError());
     }
     e->last_ns = e->timestamp;
   }
   rebuild_csr(e);
   sync_history_buffers(e);
-  launch_clear_status(e->stream, e->ring.p, e->ring_size, step, 1, e->halted.p);
   launch_step(e, make_ctl(e, step, 1, 0), step, false, true);
-  swap_history_buffers(e);
-  const int nwg = (int)e->wg.size();
-  launch_wall_finalize(e->stream, e->wall_part.p, gather_blocks(e->n), nwg, 1, e->wall_hist.p);
-  std::vector<double> h((size_t)nwg * 3);
-  if (nwg) d2h(e, h.data(), e->wall_hist.p, h.size());
+  swap_step_buffers(e);
+  launch_end(e, step, 1);
   sync(e);
   collect_timing(e, 1);
-  if (nwg) record_walls(e, h, 1);
+  if (!e->wg.empty()) record_walls(e, 1);
 }
 
 // up to K steps queued without host bookkeeping; returns steps completed
 int fast_batch(esp_engine* e, int k, int* reason)
 {
   const long long step0 = e->t + 1;
-  const int nwg = (int)e->wg.size();
   std::vector<double> before;
   for (auto& W : e->walls) before.insert(before.end(), W.o, W.o + 3);
   std::vector<std::vector<double>> wall_o;
-  launch_clear_status(e->stream, e->ring.p, e->ring_size, step0, k, e->halted.p);
   for (int s = 0; s < k; s++) {
     apply_wall_motion(e);  // pre-time-step runnables of this step
     std::vector<double> snap;
@@ -1730,24 +1884,19 @@ int fast_batch(esp_engine* e, int k, int* reason)
     const long long step = step0 + s;
     launch_step(e, make_ctl(e, step, s + 1, 1), step, (s & 1) != 0, s == k - 1);
   }
-  launch_wall_finalize(e->stream, e->wall_part.p, gather_blocks(e->n), nwg, k, e->wall_hist.p);
-  int halted = 0;
-  UpdState st;
-  d2h(e, &halted, e->halted.p, 1);
-  d2h(e, &st, e->upd.p, 1);
-  std::vector<double> h((size_t)k * nwg * 3);
-  if (nwg) d2h(e, h.data(), e->wall_hist.p, h.size());
+  launch_end(e, step0, k);
   sync(e);
-  const int done = halted ? halted - 1 : k;
-  *reason = halted ? st.halt_reason : 0;
+  const BatchOut& bo = *reinterpret_cast<const BatchOut*>(e->batch_out.p);
+  const int done = bo.halted ? bo.halted - 1 : k;
+  *reason = bo.halted ? bo.reason : 0;
   collect_timing(e, done);
   if (done < k) {  // walls stay where the last completed step left them
     const std::vector<double>& o = done > 0 ? wall_o[done - 1] : before;
     for (size_t w = 0; w < e->walls.size(); w++)
       for (int c = 0; c < 3; c++) e->walls[w].o[c] = o[3 * w + c];
   }
-  if (nwg) record_walls(e, h, done);
-  if (done & 1) swap_history_buffers(e);
+  if (!e->wg.empty()) record_walls(e, done);
+  if (done & 1) swap_step_buffers(e);
   e->t += done;
   e->pending_host = done < k;
   return done;
@@ -3488,12 +3637,26 @@ std::string check_state(esp_engine* e)
   d2h(e, xcnt.data(), e->xcnt.p, n);
   d2h(e, off.data(), e->inc_off.p, n + 1);
   d2h(e, &st, e->upd.p, 1);
+  const bool cm = contact_mode(e);  // rows instead of record slots
   std::vector<int2> so(std::max(e->nrec, 1));
-  d2h(e, so.data(), e->slot_of.p, e->nrec);
+  if (!cm) d2h(e, so.data(), e->slot_of.p, e->nrec);
+  const bool rm = cm && contact_rows(e);
+  const size_t nrow = rm ? (size_t)e->row_width * e->row_stride : cm && csr ? (size_t)e->xbase : 0;
+  std::vector<int2> rows(std::max<size_t>(nrow, 1));
+  std::vector<int> rcnt(std::max(n, 1));
+  if (cm && csr) {
+    d2h(e, rows.data(), rm ? e->rows.p : e->contact_ent.p, nrow);
+    if (rm) d2h(e, rcnt.data(), e->row_cnt.p, n);
+  }
   sync(e);
   for (int i = 0; i < n; i++)
     if (xcnt[i] < 0 || xcnt[i] > ESP_XSLOTS) {
       fail("appendix slot count " + std::to_string(xcnt[i]) + " at slot " + std::to_string(i));
+      break;
+    }
+  for (int i = 0; i < n && rm && csr; i++)
+    if (rcnt[i] != off[i + 1] - off[i] || rcnt[i] > e->row_width) {
+      fail("row count at slot " + std::to_string(i));
       break;
     }
   for (int i = 0; i < n && csr; i++)
@@ -3554,7 +3717,18 @@ std::string check_state(esp_engine* e)
       const int2 sl = !csr ? make_int2(0, 0)
                            : app ? so[G.app_rec_off + (c - G.n)] : so[G.rec_off + c];
       bool ok = q.x >= 0 && q.x < n && q.y >= 0 && q.y < n && q.x != q.y && key[c] == pkey(q.x, q.y);
-      if (ok && !app && csr) ok = in_run(sl.x, q.x) && in_run(sl.y, q.y);
+      if (ok && !app && csr && cm) {
+        // the pair is in the row of each of its particles
+        auto in_row = [&](int p, int other) {
+          for (int k = 0; k < off[p + 1] - off[p]; k++) {
+            const int2 v = rm ? rows[(size_t)k * e->row_stride + p] : rows[off[p] + k];
+            if (v.x == other && v.y == G.rec_off + c) return true;
+          }
+          return false;
+        };
+        ok = in_row(q.x, q.y) && in_row(q.y, q.x | (int)0x80000000u);
+      }
+      if (ok && !app && csr && !cm) ok = in_run(sl.x, q.x) && in_run(sl.y, q.y);
       if (ok && app && csr)
         ok = sl.x >= e->xbase + ESP_XSLOTS * q.x && sl.x < e->xbase + ESP_XSLOTS * (q.x + 1) &&
              sl.y >= e->xbase + ESP_XSLOTS * q.y && sl.y < e->xbase + ESP_XSLOTS * (q.y + 1) &&

@@ -287,11 +287,67 @@ void launch_bond_keys(hipStream_t s, int nb, const int2* ij, const int* id, long
 void launch_alive_flags(hipStream_t s, int nb, const int2* ij, int* keep);
 bool launch_gather_integrate(hipStream_t s, StepCtl ctl, PView p, const GatherParams& gp,
                              hipEvent_t ev_a = nullptr, hipEvent_t ev_b = nullptr);
-// wall forces [step][nwg][3] from the partials [step][block][nwg][3]
-void launch_wall_finalize(hipStream_t s, const double* part, int nblocks, int nwg, int nsteps,
-                          double* out);
-void launch_clear_status(hipStream_t s, StepStatus* ring, int ring_size, long long first_step,
-                         int count, int* halted);
+// the end of a batch of nsteps steps from step0 on: wall forces [step][nwg][3]
+// from the partials [step][block][nwg][3] and the queue's status, written to
+// page-locked host memory; the status ring and the halt mark are made ready
+// for the next batch
+struct BatchOut {
+  int halted;   // 0, or 1 + index of the first step that needs the host
+  int reason;   // why the queue halted
+  unsigned long long maxdisp2;  // status of the last completed step
+  int nbroken;
+  int pad;
+};
+struct BatchEnd {
+  const double* part;
+  int nblocks, nwg, nsteps;
+  const int* list;    // blocks the sums are taken over (list_n of them), or nullptr: all
+  const int* list_n;
+  StepStatus* ring;
+  int ring_size;
+  long long step0;
+  int* halted;
+  const int* reason;
+  BatchOut* out;   // host memory
+  double* walls;   // host memory
+};
+void launch_batch_end(hipStream_t s, const BatchEnd& be);
+// ---- engines without bonded groups: one launch per step ----
+struct ContactSeg {
+  int kind;      // ESP_SEG_* of a dynamic group
+  int rec_off;   // its first record
+  double4* ff;      // shear history read by this step (RotFriction)
+  double4* ff_out;  // shear history written by this step
+  double k, ks, mu_d, mu_s;
+  int scaling, meanR, rigid, pad;
+};
+struct ContactLaunch {
+  int count, do2d;
+  int stride, width;  // rows: [width][stride]
+  double period, dt;
+  const int* cnt;     // interactions per particle
+  const int2* rows;   // see k_contact_rows (one NRotElastic group), else nullptr
+  const int* off;     // CSR runs of ent, see k_contact_entries
+  const int2* ent;
+  double4 *pos_o, *vel_o, *ang_o;  // arrays the particles are stepped into
+  ContactSeg seg[ESP_MAX_FORCE_SEGS];
+};
+bool launch_contact_step(hipStream_t s, StepCtl ctl, PView p, const ContactLaunch& cl,
+                         const GatherParams& gp, hipEvent_t ev_a = nullptr,
+                         hipEvent_t ev_b = nullptr);
+int contact_groups(int n);  // 64-particle groups the wall partials are kept for
+// the pair lists behind the records (dynamic groups in record order)
+struct RecordLists {
+  int count;
+  int rec_off[ESP_MAX_FORCE_SEGS];
+  const int2* ij[ESP_MAX_FORCE_SEGS];
+};
+void launch_contact_rows(hipStream_t s, int n, int stride, const int* off, const int* ent,
+                         const RecordLists& rl, int* cnt, int2* rows);
+void launch_contact_entries(hipStream_t s, int total, const int* inc_ent, const RecordLists& rl,
+                            int2* ent);
+void launch_max_int(hipStream_t s, int n, const int* a, int* out);
+void launch_wall_list(hipStream_t s, int ng, const int* mark, int* list, int* list_n);
 int gather_blocks(int n);
 
 // ---- rebuild / update kernels ----
@@ -369,7 +425,9 @@ void launch_compact_bonds(hipStream_t s, int nb, const int* keep, const int* off
                           const int2* ij, const double4* k4, const double4* mx4,
                           const double4* D4, const int* rank, int2* ij2, double4* k42,
                           double4* mx42, double4* D42, int* rank2);
-void launch_wall_update(hipStream_t s, PView p, GridParams g, int nwg, const WallParam* walls);
+// mark (nullable): per 64-particle group, whether it holds wall candidates
+void launch_wall_update(hipStream_t s, PView p, GridParams g, int nwg, const WallParam* walls,
+                        int* mark = nullptr);
 void launch_inc_count(hipStream_t s, int nc, const int2* ij, int* inc_cnt);
 // rank: the interactions' positions in the group's reference order (nullptr:
 // storage order); grp: the group's position in the summation order (< 32)

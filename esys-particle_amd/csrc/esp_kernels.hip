@@ -31,6 +31,9 @@
 #include "esp_math.h"
 
 #define BS 256
+#ifndef ESP_G_EL
+#define ESP_G_EL 4
+#endif
 
 static inline int nblk(long long n, int bs = BS) { return (int)((n + bs - 1) / bs); }
 
@@ -449,9 +452,159 @@ __device__ __forceinline__ void stress_add(double (&sg)[3][3], dv3 f, dv3 rel)
     for (int j = 0; j < 3; j++) sg[i][j] -= fv[i] * rv[j];
 }
 
-// STRESS: records carry contact points and every applied force also updates
-// the particle's stress sum, in the order the forces are summed
-// EXTRA: damping groups or bonded walls exist (kept out of the plain kernel)
+// Wall interaction groups, name order (EWallInteraction.hpp:42-78), then body
+// forces, name order (BodyForceGroup.hpp:41-65): the force the particle's
+// interactions are added to.  In a bonded group the tagged candidates are
+// bonded instead.  flw: the particle's flags; i: its slot.
+// STRESS: every applied force also updates the particle's stress sum, in the
+// order the forces are summed.  EXTRA: damping groups, bonded or tagged walls
+// exist (kept out of the plain kernels).
+template <bool STRESS, bool EXTRA>
+__device__ __forceinline__ dv3 wall_body_force(const GatherParams& gp, int i, unsigned flw, dv3 x,
+                                               double r, double mass, double (&sg)[3][3])
+{
+  dv3 F = mk3(0.0, 0.0, 0.0);
+  const bool any = __ballot(((flw >> PF_WALL_SHIFT) & 0xFFu) != 0u) != 0ull;  // of the wave
+  for (int w = 0; any && w < gp.nwg; w++) {
+    if (!((flw >> (PF_WALL_SHIFT + w)) & 1u)) continue;
+    const WallParam& W = gp.wall[w];
+    if (EXTRA && W.tagged && !((flw >> (PF_BTAG_SHIFT + w)) & 1u)) continue;
+    if (EXTRA && W.bonded && ((flw >> (PF_BTAG_SHIFT + w)) & 1u)) {
+      const dv3 fb = bonded_wall_force(W, x, xyz(gp.init[i]), r, gp.do2d);
+      F = add3(F, fb);
+      if (STRESS) stress_add(sg, fb, sub3(x, x));
+      continue;
+    }
+    const dv3 n = mk3(W.nrm[0], W.nrm[1], W.nrm[2]);
+    const double dist = dot3(sub3(x, mk3(W.o[0], W.o[1], W.o[2])), n);
+    if (dist < r) {
+      double f = 1.0;
+      if (!gp.do2d) f *= 3.141592654 * r;
+      const dv3 force = mul3(n, (f * W.k) * (r - dist));
+      F = add3(F, force);
+      if (STRESS) stress_add(sg, force, sub3(sub3(x, mul3(n, dist)), x));
+    }
+  }
+  // applied at the centre
+  for (int g = 0; g < gp.ngrav; g++) {
+    const dv3 fg = mul3(mk3(gp.g[g][0], gp.g[g][1], gp.g[g][2]), mass);
+    F = add3(F, fg);
+    if (STRESS) stress_add(sg, fg, sub3(x, x));
+  }
+  return F;
+}
+
+// The wall force on an inner candidate of wall group w, as wall_body_force
+// applies it (the wall forces sum these; zero for every other particle)
+template <bool EXTRA>
+__device__ __forceinline__ dv3 wall_share(const GatherParams& gp, int w, int i, unsigned flw, dv3 x,
+                                          double r)
+{
+  if (!((flw >> (PF_WALL_SHIFT + w)) & 1u) || !((flw >> (PF_INNER_SHIFT + w)) & 1u))
+    return mk3(0.0, 0.0, 0.0);
+  const WallParam& W = gp.wall[w];
+  // untagged candidates of a tagged elastic wall: no interaction
+  if (EXTRA && W.tagged && !((flw >> (PF_BTAG_SHIFT + w)) & 1u)) return mk3(0.0, 0.0, 0.0);
+  // CWall::addForce(force) subtracts the bonded force: the particle's share
+  if (EXTRA && W.bonded && ((flw >> (PF_BTAG_SHIFT + w)) & 1u))
+    return bonded_wall_force(W, x, xyz(gp.init[i]), r, gp.do2d);
+  const dv3 n = mk3(W.nrm[0], W.nrm[1], W.nrm[2]);
+  const double dist = dot3(sub3(x, mk3(W.o[0], W.o[1], W.o[2])), n);
+  if (!(dist < r)) return mk3(0.0, 0.0, 0.0);
+  double f = 1.0;
+  if (!gp.do2d) f *= 3.141592654 * r;
+  return mul3(n, (f * W.k) * (r - dist));
+}
+
+// Damping groups, last (SubLattice.hpp:2143-2147), in their map order, then the
+// CParticle / CRotParticle update of particle i; writes its new state to po
+// (the arrays it is stepped into) and returns |x - x_old|^2.
+template <bool STRESS, bool EXTRA>
+__device__ __forceinline__ double damp_and_integrate(const PView& po, const GatherParams& gp, int i,
+                                                     unsigned fl, dv3 F, dv3 M, double4 P, double4 Vv,
+                                                     double4 O, double4 A, double4 Q,
+                                                     double (&sg)[3][3])
+{
+  dv3 x = xyz(P), v = xyz(Vv);
+  const double r = P.w, invm = Vv.w, mass = O.w;
+  const double dt = gp.dt;
+  for (int d = 0; EXTRA && d < gp.ndamp; d++) {
+    const int ty = gp.damp_type[d];
+    const double visc = gp.damp_visc[d];
+    if (ty == ESP_DAMPING || ty == ESP_ROT_DAMPING) {
+      const bool rd = ty == ESP_ROT_DAMPING;
+      const double mi = rd ? gp.inert[i] : mass;
+      const dv3 vr = esp_damping_vrel(rd ? xyz(A) : v, rd ? M : F, rd ? A.w : invm, mi, visc, dt,
+                                      gp.damp_maxit[d]);
+      const dv3 fd = mul3(mul3(vr, -1.0 * visc), mi);
+      if (rd) {
+        M = add3(M, fd);
+      } else {
+        F = add3(F, fd);
+        if (STRESS) stress_add(sg, fd, sub3(x, x));
+      }
+    } else {
+      const bool rd = ty == ESP_ROT_LOCAL_DAMPING;
+      const dv3 vv = rd ? xyz(A) : v, ff = rd ? M : F;
+      const dv3 fd = mul3(mk3(esp_local_damping_c(ff.x, vv.x), esp_local_damping_c(ff.y, vv.y),
+                              esp_local_damping_c(ff.z, vv.z)),
+                          -1.0 * visc);
+      if (rd) {
+        M = add3(M, fd);
+      } else {
+        F = add3(F, fd);
+        if (STRESS) stress_add(sg, fd, sub3(x, x));
+      }
+    }
+  }
+  if (gp.rot) {
+    dv3 w = xyz(A);
+    dquat q = dquat{Q.x, mk3(Q.y, Q.z, Q.w)};
+    if (fl & PF_ROT) {
+      if (gp.do2d) {
+        F = mk3(F.x, F.y, 0);
+        M = mk3(0, 0, M.z);
+      }
+      w = add3(w, mul3(M, dt * A.w));
+      const dquat dq = qmul4(dquat{0, w}, q);
+      const double h = dt / 2.0;
+      q.s += h * dq.s;
+      q.v = add3(q.v, mul3(dq.v, h));
+    } else {
+      w = mk3(0.0, 0.0, 0.0);
+    }
+    if (fl & PF_DYN) {
+      if (gp.do2d) F = mk3(F.x, F.y, 0);
+      v = add3(v, mul3(mul3(F, invm), dt));
+      x = add3(x, mul3(v, dt));
+    }
+    const double module = sqrt(q.s * q.s + q.v.x * q.v.x + q.v.y * q.v.y + q.v.z * q.v.z);
+    if (module != 0.0) {
+      const double inverse = 1.0 / module;
+      q.s = inverse * q.s;
+      q.v = mul3(q.v, inverse);
+    }
+    po.ang[i] = make_double4(w.x, w.y, w.z, A.w);
+    po.quat[i] = make_double4(q.s, q.v.x, q.v.y, q.v.z);
+    if (gp.store_fm) po.mom[i] = make_double4(M.x, M.y, M.z, 0.0);
+  } else if (fl & PF_DYN) {
+    if (gp.do2d) F = mk3(F.x, F.y, 0);
+    v = add3(v, mul3(mul3(F, invm), dt));
+    x = add3(x, mul3(v, dt));
+  }
+  po.pos[i] = make_double4(x.x, x.y, x.z, r);
+  po.vel[i] = make_double4(v.x, v.y, v.z, invm);
+  if (gp.store_fm) po.frc[i] = make_double4(F.x, F.y, F.z, 0.0);
+  if (STRESS) {
+    double* o = gp.sig + 9 * (size_t)i;
+    for (int a = 0; a < 3; a++)
+      for (int b = 0; b < 3; b++) o[3 * a + b] = sg[a][b];
+  }
+  const dv3 d = sub3(x, xyz(O));
+  return dot3(d, d);
+}
+
+// STRESS: records carry contact points
 template <bool STRESS, bool EXTRA>
 __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, GatherParams gp)
 {
@@ -485,9 +638,7 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
   }
   const int refresh = gp.nwg > 0 && ctl.guarded && ctl.prev->nbroken > 0;
   const dv3 x0 = xyz(P);
-  dv3 x = x0;
   const double r = P.w;
-  dv3 F = mk3(0.0, 0.0, 0.0), M = mk3(0.0, 0.0, 0.0);
   unsigned flw = fl;
   if (act && refresh) {
     // bonds broke in the previous step: the reference's updateInteractions
@@ -495,38 +646,10 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
     flw = wall_membership(gp.grid, gp.nwg, gp.wall, P, fl);
     p.flags[i] = flw;
   }
-  // wall interaction groups, name order (EWallInteraction.hpp:42-78); in a
-  // bonded group the tagged candidates are bonded instead
-  for (int w = 0; w < gp.nwg; w++) {
-    if (!act || !((flw >> (PF_WALL_SHIFT + w)) & 1u)) continue;
-    const WallParam& W = gp.wall[w];
-    if (EXTRA && W.tagged && !((flw >> (PF_BTAG_SHIFT + w)) & 1u)) continue;
-    if (EXTRA && W.bonded && ((flw >> (PF_BTAG_SHIFT + w)) & 1u)) {
-      const dv3 fb = bonded_wall_force(W, x, xyz(gp.init[i]), r, gp.do2d);
-      F = add3(F, fb);
-      if (STRESS) stress_add(sg, fb, sub3(x, x));
-      continue;
-    }
-    const dv3 n = mk3(W.nrm[0], W.nrm[1], W.nrm[2]);
-    const double dist = dot3(sub3(x, mk3(W.o[0], W.o[1], W.o[2])), n);
-    if (dist < r) {
-      double f = 1.0;
-      if (!gp.do2d) f *= 3.141592654 * r;
-      const dv3 force = mul3(n, (f * W.k) * (r - dist));
-      F = add3(F, force);
-      if (STRESS) stress_add(sg, force, sub3(sub3(x, mul3(n, dist)), x));
-    }
-  }
   unsigned long long md = 0;
   if (act) {
-    dv3 v = xyz(Vv);
-    const double invm = Vv.w, mass = O.w;
-    // body forces, name order (BodyForceGroup.hpp:41-65), applied at the centre
-    for (int g = 0; g < gp.ngrav; g++) {
-      const dv3 fg = mul3(mk3(gp.g[g][0], gp.g[g][1], gp.g[g][2]), mass);
-      F = add3(F, fg);
-      if (STRESS) stress_add(sg, fg, sub3(x, x));
-    }
+    dv3 F = wall_body_force<STRESS, EXTRA>(gp, i, flw, x0, r, O.w, sg);
+    dv3 M = mk3(0.0, 0.0, 0.0);
     // the particle's slots in summation order (its CSR run, then its appendix
     // slots), fetched GATHER_CHUNK at a time so their loads are in flight
     // together; the sum itself stays sequential.  Moments of laws without
@@ -614,82 +737,8 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
         M = add3(M, m[k]);
       }
     }
-    const double dt = gp.dt;
-    // damping groups, last (SubLattice.hpp:2143-2147), in their map order
-    for (int d = 0; EXTRA && d < gp.ndamp; d++) {
-      const int ty = gp.damp_type[d];
-      const double visc = gp.damp_visc[d];
-      if (ty == ESP_DAMPING || ty == ESP_ROT_DAMPING) {
-        const bool rd = ty == ESP_ROT_DAMPING;
-        const double mi = rd ? gp.inert[i] : mass;
-        const dv3 vr = esp_damping_vrel(rd ? xyz(A) : v, rd ? M : F, rd ? A.w : invm, mi, visc,
-                                        dt, gp.damp_maxit[d]);
-        const dv3 fd = mul3(mul3(vr, -1.0 * visc), mi);
-        if (rd) {
-          M = add3(M, fd);
-        } else {
-          F = add3(F, fd);
-          if (STRESS) stress_add(sg, fd, sub3(x, x));
-        }
-      } else {
-        const bool rd = ty == ESP_ROT_LOCAL_DAMPING;
-        const dv3 vv = rd ? xyz(A) : v, ff = rd ? M : F;
-        const dv3 fd = mul3(mk3(esp_local_damping_c(ff.x, vv.x), esp_local_damping_c(ff.y, vv.y),
-                                esp_local_damping_c(ff.z, vv.z)),
-                            -1.0 * visc);
-        if (rd) {
-          M = add3(M, fd);
-        } else {
-          F = add3(F, fd);
-          if (STRESS) stress_add(sg, fd, sub3(x, x));
-        }
-      }
-    }
-    if (gp.rot) {
-      dv3 w = xyz(A);
-      dquat q = dquat{Q.x, mk3(Q.y, Q.z, Q.w)};
-      if (fl & PF_ROT) {
-        if (gp.do2d) {
-          F = mk3(F.x, F.y, 0);
-          M = mk3(0, 0, M.z);
-        }
-        w = add3(w, mul3(M, dt * A.w));
-        const dquat dq = qmul4(dquat{0, w}, q);
-        const double h = dt / 2.0;
-        q.s += h * dq.s;
-        q.v = add3(q.v, mul3(dq.v, h));
-      } else {
-        w = mk3(0.0, 0.0, 0.0);
-      }
-      if (fl & PF_DYN) {
-        if (gp.do2d) F = mk3(F.x, F.y, 0);
-        v = add3(v, mul3(mul3(F, invm), dt));
-        x = add3(x, mul3(v, dt));
-      }
-      const double module = sqrt(q.s * q.s + q.v.x * q.v.x + q.v.y * q.v.y + q.v.z * q.v.z);
-      if (module != 0.0) {
-        const double inverse = 1.0 / module;
-        q.s = inverse * q.s;
-        q.v = mul3(q.v, inverse);
-      }
-      p.ang[i] = make_double4(w.x, w.y, w.z, A.w);
-      p.quat[i] = make_double4(q.s, q.v.x, q.v.y, q.v.z);
-      if (gp.store_fm) p.mom[i] = make_double4(M.x, M.y, M.z, 0.0);
-    } else if (fl & PF_DYN) {
-      if (gp.do2d) F = mk3(F.x, F.y, 0);
-      v = add3(v, mul3(mul3(F, invm), dt));
-      x = add3(x, mul3(v, dt));
-    }
-    p.pos[i] = make_double4(x.x, x.y, x.z, r);
-    p.vel[i] = make_double4(v.x, v.y, v.z, invm);
-    if (gp.store_fm) p.frc[i] = make_double4(F.x, F.y, F.z, 0.0);
-    if (STRESS) {
-      double* o = gp.sig + 9 * (size_t)i;
-      for (int a = 0; a < 3; a++)
-        for (int b = 0; b < 3; b++) o[3 * a + b] = sg[a][b];
-    }
-    const dv3 d = sub3(x, xyz(O));
-    md = (unsigned long long)__double_as_longlong(dot3(d, d));
+    md = (unsigned long long)__double_as_longlong(
+        damp_and_integrate<STRESS, EXTRA>(p, gp, i, fl, F, M, P, Vv, O, A, Q, sg));
   }
   // max displacement: wave, then block, then one atomic per block
   md = wave_max_u64(md);
@@ -714,24 +763,8 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
       }
       continue;
     }
-    double wx = 0.0, wy = 0.0, wz = 0.0;
-    if (act && ((flw >> (PF_WALL_SHIFT + w)) & 1u) && ((flw >> (PF_INNER_SHIFT + w)) & 1u)) {
-      const WallParam& W = gp.wall[w];
-      const dv3 n = mk3(W.nrm[0], W.nrm[1], W.nrm[2]);
-      const double dist = dot3(sub3(x0, mk3(W.o[0], W.o[1], W.o[2])), n);
-      if (EXTRA && W.tagged && !((flw >> (PF_BTAG_SHIFT + w)) & 1u)) {
-        // untagged candidates of a tagged elastic wall: no interaction
-      } else if (EXTRA && W.bonded && ((flw >> (PF_BTAG_SHIFT + w)) & 1u)) {
-        // CWall::addForce(force) subtracts the bonded force: the particle's share
-        const dv3 fb = bonded_wall_force(W, x0, xyz(gp.init[i]), r, gp.do2d);
-        wx = fb.x; wy = fb.y; wz = fb.z;
-      } else if (dist < r) {
-        double f = 1.0;
-        if (!gp.do2d) f *= 3.141592654 * r;
-        const dv3 force = mul3(n, (f * W.k) * (r - dist));
-        wx = force.x; wy = force.y; wz = force.z;
-      }
-    }
+    const dv3 sh = act ? wall_share<EXTRA>(gp, w, i, flw, x0, r) : mk3(0.0, 0.0, 0.0);
+    double wx = sh.x, wy = sh.y, wz = sh.z;
     block_sum3(wx, wy, wz, lds3);
     if (threadIdx.x == 0) {
       double* q = gp.wall_part + ((size_t)blockIdx.x * gp.nwg + w) * 3;
@@ -740,43 +773,529 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
   }
 }
 
-// Wall forces of a run of steps: block s sums step s's per-block partials in
-// block order.  Launched once per queued batch; slots of steps that were
-// skipped hold stale values and are not read by the host.
-__global__ __launch_bounds__(BS) void k_wall_finalize(const double* part, int nblocks, int nwg,
-                                                      double* out)
+// The end of a batch of steps, the one launch the host waits for.  Block s sums
+// step s's wall partials in a fixed order (LIST: the 64-particle groups named in
+// list, else every block's) straight into page-locked host memory, so no copy
+// follows; slots of steps that were skipped hold stale values the host does not
+// read.  Block 0 also reports why the queue halted and the last completed
+// step's status, and clears every other entry of the ring and the halt mark for
+// the next batch.  (Three copies into pageable memory, two launches around a
+// batch: 72 us a step for a batch of one step of 97 particles; this: see
+// k_contact_step and esp_engine.hip's fast_batch.)
+template <bool LIST>
+__global__ __launch_bounds__(BS) void k_batch_end(BatchEnd be)
 {
   __shared__ double lds3[3 * (BS / 64)];
-  const double* ps = part + (size_t)blockIdx.x * nblocks * nwg * 3;
-  for (int w = 0; w < nwg; w++) {
+  const int nb = LIST ? *be.list_n : be.nblocks;
+  const double* ps = be.part + (size_t)blockIdx.x * be.nblocks * be.nwg * 3;
+  for (int w = 0; w < be.nwg; w++) {
     double a = 0.0, b = 0.0, c = 0.0;
-    for (int k = threadIdx.x; k < nblocks; k += BS) {
-      const double* q = ps + ((size_t)k * nwg + w) * 3;
+    for (int k = threadIdx.x; k < nb; k += BS) {
+      const double* q = ps + ((size_t)(LIST ? be.list[k] : k) * be.nwg + w) * 3;
       a = a + q[0];
       b = b + q[1];
       c = c + q[2];
     }
     block_sum3(a, b, c, lds3);
     if (threadIdx.x == 0) {
-      double* o = out + ((size_t)blockIdx.x * nwg + w) * 3;
+      double* o = be.walls + ((size_t)blockIdx.x * be.nwg + w) * 3;
       o[0] = a;
       o[1] = b;
       o[2] = c;
     }
   }
+  if (blockIdx.x != 0) return;
+  const int halted = *be.halted;
+  __syncthreads();  // every thread has the mark before it is cleared
+  const int done = halted ? halted - 1 : be.nsteps;
+  const int last = (int)((be.step0 + done - 1) % be.ring_size);
+  for (int t = threadIdx.x; t < be.ring_size; t += BS) {
+    StepStatus& st = be.ring[t];
+    if (t == last) {
+      be.out->maxdisp2 = st.maxdisp2;
+      be.out->nbroken = st.nbroken;
+    } else {
+      st.maxdisp2 = 0ull;
+      st.nbroken = 0;
+      st.pad = 0;
+    }
+  }
+  if (threadIdx.x == 0) {
+    be.out->halted = halted;
+    be.out->reason = *be.reason;
+    *be.halted = 0;
+  }
 }
 
-__global__ void k_clear_status(StepStatus* ring, int ring_size, long long first_step, int count,
-                               int* halted)
+// ---------------------------------------------------------------------------
+// one whole step of an engine without bonded groups
+// ---------------------------------------------------------------------------
+// The value lane `q` of this lane's group of G (2 or 4) lanes holds
+template <int G>
+__device__ __forceinline__ double group_value(double v, int q)
 {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < count) {
-    StepStatus& s = ring[(first_step + t) % ring_size];
-    s.maxdisp2 = 0ull;
-    s.nbroken = 0;
-    s.pad = 0;
+  const long long b = __double_as_longlong(v);
+  int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
+#define ESP_DPP(ctrl)                                             \
+  {                                                               \
+    lo = __builtin_amdgcn_mov_dpp(lo, ctrl, 0xf, 0xf, true);      \
+    hi = __builtin_amdgcn_mov_dpp(hi, ctrl, 0xf, 0xf, true);      \
   }
-  if (t == 0) *halted = 0;
+  if (G == 4) {
+    if (q == 0) ESP_DPP(0x00)
+    else if (q == 1) ESP_DPP(0x55)
+    else if (q == 2) ESP_DPP(0xAA)
+    else ESP_DPP(0xFF)
+  } else if (G == 2) {
+    if (q == 0) ESP_DPP(0xA0)
+    else ESP_DPP(0xF5)
+  }
+#undef ESP_DPP
+  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+// A RotFriction pair apart, as its first particle sees it: history cleared; once
+// both buffers hold zero (flag bit 2) nothing is written.
+__device__ __forceinline__ void clear_history(const ContactSeg& g, int c)
+{
+  const double4 st = g.ff[c];
+  const int fw = (int)st.w;
+  if ((fw & 3) != 0 || st.x != 0.0 || st.y != 0.0 || st.z != 0.0) {
+    g.ff_out[c] = make_double4(0.0, 0.0, 0.0, 0.0);
+  } else if (!(fw & 4)) {
+    g.ff[c] = make_double4(0.0, 0.0, 0.0, 4.0);
+    g.ff_out[c] = make_double4(0.0, 0.0, 0.0, 4.0);
+  }
+}
+
+// the group of a record (KIND: the launch's only group, or 0)
+template <int KIND>
+__device__ __forceinline__ const ContactSeg& seg_of(const ContactLaunch& cl, int rec)
+{
+  int s = 0;
+  if (KIND == 0)
+    while (s + 1 < cl.count && rec >= cl.seg[s + 1].rec_off) s++;
+  return cl.seg[s];
+}
+
+// One pair as particle i sees it (row entry e): force and moment on it.  The law
+// is evaluated in the pair's own orientation (lower id first), so both particles
+// compute the same bits; the first one keeps the shear history.  KIND: the
+// launch's only group (ESP_SEG_*), or 0 for any mix of groups.
+template <int KIND>
+__device__ __forceinline__ void pair_share(const PView& p, const ContactLaunch& cl, int2 e,
+                                           const double4& Pi, const double4& Vi, const double4& Ai,
+                                           dv3& f, dv3& m)
+{
+  const bool second = e.x < 0;
+  const int j = e.x & 0x7fffffff;
+  const ContactSeg& g = seg_of<KIND>(cl, e.y);
+  const int kind = KIND ? KIND : g.kind;
+  const int c = e.y - g.rec_off;
+  const double4 Pj = p.pos[j];
+  const double4 P1 = second ? Pj : Pi, P2 = x_image(P1, second ? Pi : Pj, cl.period);
+  const dv3 D = sub3(xyz(P1), xyz(P2));
+  const double eq = P1.w + P2.w;
+  if (kind == ESP_SEG_NROT_ELASTIC) {  // ElasticInteraction.cpp:54-71
+    double dist = dot3(D, D);
+    if (!(dist < (eq * eq))) return;
+    const double kk = esp_elastic_k(g.k, g.scaling, P1.w, P2.w, cl.do2d);
+    dist = sqrt(dist);
+    const dv3 force = mul3(D, kk * (dist - eq) / dist);
+    f = second ? force : neg3(force);
+  } else if (kind == ESP_SEG_ROT_ELASTIC) {  // RotElasticInteraction.cpp:69-88
+    const double rbNorm = norm3(D);
+    if (!(rbNorm < eq)) return;
+    const dv3 delta_r = div3(mul3(D, rbNorm - eq), rbNorm);
+    const dv3 force = mul3(delta_r, esp_rotelastic_k(g.k, g.scaling, P1.w, P2.w, cl.do2d));
+    f = second ? force : neg3(force);
+  } else {  // RotFricInteraction.cpp:103-231
+    const double4 Vj = p.vel[j], Wj = p.ang[j], st = g.ff[c];
+    const double4 V1 = second ? Vj : Vi, V2 = second ? Vi : Vj;
+    const double4 W1 = second ? Wj : Ai, W2 = second ? Ai : Wj;
+    double kk, kks;
+    esp_friction_k(g.k, g.ks, g.scaling, g.meanR, P1.w, P2.w, cl.do2d, kk, kks);
+    dv3 ffr = mk3(st.x, st.y, st.z);
+    bool slipping = (((int)st.w) & 1) != 0;
+    dv3 f1, m1, m2;
+    if (KIND == 0 && g.rigid)
+      esp_rot_friction_rigid_law(xyz(P1), xyz(V1), xyz(W1), P1.w, xyz(P2), xyz(V2), xyz(W2), P2.w,
+                                 kk, kks, g.mu_d, g.mu_s, cl.dt, (((int)st.w) & 2) != 0, ffr,
+                                 slipping, f1, m1, m2);
+    else
+      esp_rot_friction_law(xyz(P1), xyz(V1), xyz(W1), P1.w, xyz(P2), xyz(V2), xyz(W2), P2.w, kk,
+                           kks, g.mu_d, g.mu_s, cl.dt, ffr, slipping, f1, m1, m2);
+    if (!second) g.ff_out[c] = make_double4(ffr.x, ffr.y, ffr.z, (double)((slipping ? 1 : 0) | 2));
+    f = second ? neg3(f1) : f1;
+    m = second ? m2 : m1;
+  }
+}
+
+// The end of a wave's step: whether a particle moved beyond verletDist/2, and the
+// wall forces on its 64 particles (flags fl, state before the step P) in a
+// fixed-order sum; waves without candidates are not in the list the sums are
+// taken over.
+template <bool EXTRA>
+__device__ __forceinline__ void step_tail(const StepCtl& ctl, const GatherParams& gp, int i, bool act,
+                                          unsigned fl, double4 P, unsigned long long md)
+{
+  const int lane = threadIdx.x & 63;
+  if (__ballot(md > ctl.thresh)) {
+    md = wave_max_u64(md);
+    if (lane == 0) atomicMax(&ctl.cur->maxdisp2, md);
+  }
+  if (gp.nwg > 0 && __ballot(act && ((fl >> PF_WALL_SHIFT) & 0xFFu) != 0u)) {
+    double* q = gp.wall_part + (size_t)(i >> 6) * gp.nwg * 3;
+    for (int w = 0; w < gp.nwg; w++) {
+      dv3 sh = act ? wall_share<EXTRA>(gp, w, i, fl, xyz(P), P.w) : mk3(0.0, 0.0, 0.0);
+      for (int o = 32; o > 0; o >>= 1) {
+        sh.x = sh.x + __shfl_xor(sh.x, o, 64);
+        sh.y = sh.y + __shfl_xor(sh.y, o, 64);
+        sh.z = sh.z + __shfl_xor(sh.z, o, 64);
+      }
+      if (lane == 0) put3(q + 3 * w, sh);
+    }
+  }
+}
+
+// Blocks go round-robin to the 8 XCDs: block b's place when each XCD takes a
+// contiguous range (a bijection on [0, nb)), so that neighbours' state is
+// fetched into one L2
+__device__ __forceinline__ int xcd_block(int b, int nb)
+{
+  const int d = b & 7, q8 = nb >> 3, r8 = nb & 7;
+  return d * q8 + min(d, r8) + (b >> 3);
+}
+
+// One whole step of an engine without bonded groups (their laws are two orders
+// of magnitude cheaper than a bond's): every particle evaluates its own pairs,
+// so each pair is evaluated twice and nothing is handed from particle to
+// particle through memory.  Against force slots written by one launch and
+// summed by a second, a touching friction pair saves two 48-byte slots written
+// and read, their two indices and activity bytes, and the step one launch.
+// Positions, velocities and angular velocities are stepped into a second set of
+// arrays (neighbours still read the old ones); the host swaps the sets.
+//
+// G lanes share a particle's pairs (row entries k = lane, lane + G, ...), their
+// shares are added in row order, then one lane per particle integrates.
+template <bool EXTRA, int G>
+__global__ __launch_bounds__(BS) void k_contact_step(StepCtl ctl, PView p, ContactLaunch cl,
+                                                     GatherParams gp)
+{
+  constexpr int PB = BS / G;  // particles per block
+  __shared__ double acc[3 * PB];
+  double none[3][3];
+  const int t = threadIdx.x;
+  const int p0 = xcd_block(blockIdx.x, gridDim.x) * PB;
+  const int i = p0 + t;  // the particle this lane integrates (t < PB)
+  const bool act = t < PB && i < p.n;
+  const int pi = p0 + t / G, sub = t % G;  // the particle whose pairs it evaluates
+  const int pc = pi < p.n ? pi : 0;
+  const int ii = act ? i : 0;
+  // loads that do not depend on others, together
+  const double4 Pi = p.pos[pc];
+  const unsigned fpi = p.flags[pc];
+  const int cnt = pi < p.n ? cl.cnt[pc] : 0;
+  const double mass = p.old[pc].w;
+  // row entries of this lane: the pair at hand, the next one and the one after
+  // it, so that the next neighbour's position is on its way during a law
+  int2 e0 = make_int2(0, 0), e1 = e0;
+  if (sub < cl.width) e0 = cl.rows[(size_t)sub * cl.stride + pc];
+  if (G + sub < cl.width) e1 = cl.rows[(size_t)(G + sub) * cl.stride + pc];
+  if (step_skip(ctl)) return;  // the same for the whole block
+  const ContactSeg& g = cl.seg[0];
+  dv3 F = wall_body_force<false, EXTRA>(gp, pc, fpi, xyz(Pi), Pi.w, mass, none);
+  double4 Pj = Pi;
+  if (sub < cnt) Pj = p.pos[e0.x & 0x7fffffff];
+#pragma unroll 1
+  for (int k = sub; k - sub < cnt; k += G) {  // as often for the G lanes of a particle
+    double4 Pn = Pj;
+    int2 e2 = e1;
+    if (k + G < cnt) Pn = p.pos[e1.x & 0x7fffffff];
+    if (k + 2 * G < cnt) e2 = cl.rows[(size_t)(k + 2 * G) * cl.stride + pc];
+    dv3 f = mk3(0.0, 0.0, 0.0);
+    if (k < cnt) {  // CElasticInteraction::calcForces (ElasticInteraction.cpp:54-71)
+      const bool second = e0.x < 0;
+      const double4 P1 = second ? Pj : Pi;
+      const double4 P2 = x_image(P1, second ? Pi : Pj, cl.period);
+      const dv3 D = sub3(xyz(P1), xyz(P2));
+      double dist = dot3(D, D);
+      const double eq = P1.w + P2.w;
+      if (dist < (eq * eq)) {
+        const double kk = esp_elastic_k(g.k, g.scaling, P1.w, P2.w, cl.do2d);
+        dist = sqrt(dist);
+        const dv3 force = mul3(D, kk * (dist - eq) / dist);
+        f = second ? force : neg3(force);
+      }
+    }
+    // adding the zero share of a pair apart changes no sum
+#pragma unroll
+    for (int q = 0; q < G; q++)
+      F = add3(F, mk3(group_value<G>(f.x, q), group_value<G>(f.y, q), group_value<G>(f.z, q)));
+    e0 = e1;
+    e1 = e2;
+    Pj = Pn;
+  }
+  if (sub == 0) put3(acc + 3 * (t / G), F);
+  // what the integrating lanes need, on its way meanwhile
+  double4 P = Pi, V = Pi, O = Pi, A = make_double4(0.0, 0.0, 0.0, 0.0), Q = A;
+  unsigned fl = 0u;
+  if (t < PB) {
+    P = p.pos[ii];
+    fl = p.flags[ii];
+    V = p.vel[ii];
+    O = p.old[ii];
+    if (gp.rot) {
+      A = p.ang[ii];
+      Q = p.quat[ii];
+    }
+  }
+  __syncthreads();
+  if (t >= PB) return;
+  unsigned long long md = 0;
+  if (act) {
+    PView po = p;
+    po.pos = cl.pos_o;
+    po.vel = cl.vel_o;
+    po.ang = cl.ang_o;
+    const dv3 F1 = mk3(acc[3 * t], acc[3 * t + 1], acc[3 * t + 2]), M1 = mk3(0.0, 0.0, 0.0);
+    md = (unsigned long long)__double_as_longlong(
+        damp_and_integrate<false, EXTRA>(po, gp, i, fl, F1, M1, P, V, O, A, Q, none));
+  }
+  step_tail<EXTRA>(ctl, gp, i, act, fl, P, md);
+}
+
+// The same step for laws with more work than an elastic contact: a block owns 64
+// particles and the run of CSR entries of their pairs.  All 256 threads test the
+// entries for contact; the touching ones are packed in entry order, so that the
+// law runs on full waves (of the 7.5 entries a particle has in a sheared bed
+// about 60 % touch, and a wave that walks its particles' runs waits for the
+// longest of 64), their shares go to LDS, and the first wave adds them in entry
+// order and integrates.
+template <bool EXTRA, int KIND>
+__global__ __launch_bounds__(BS, KIND ? 3 : 2) void k_contact_block(StepCtl ctl, PView p, ContactLaunch cl,
+                                                         GatherParams gp)
+{
+  constexpr int PB = 64;   // particles
+  constexpr int CH = 512;  // entries tested at a time
+  constexpr int SC = 320;  // touching entries whose laws are evaluated at a time
+  constexpr int U = CH / BS;
+  __shared__ double4 sP[PB], sV[PB], sO[PB], sA[PB], sQ[PB];
+  __shared__ int sOff[PB + 1];
+  __shared__ double slot[6 * SC];  // [component][touching entry]
+  __shared__ double sum[6 * PB];   // [component][particle]
+  __shared__ int2 sEnt[CH];
+  __shared__ unsigned char owner[CH];
+  __shared__ unsigned short queue[CH];  // touching entries of the chunk, in order
+  __shared__ unsigned long long touch_mask[CH / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int p0 = xcd_block(blockIdx.x, gridDim.x) * PB;
+  const int np = min(PB, p.n - p0);
+  const int i = p0 + lane;  // the particle this lane loads, and in wave 0 integrates
+  const int ic = lane < np ? i : p0;
+  unsigned fl = 0u;
+  if (wv == 0) {
+    sP[lane] = p.pos[ic];
+    fl = p.flags[ic];
+  } else if (wv == 1) {
+    sO[lane] = p.old[ic];
+    sOff[lane] = cl.off[min(i, p.n)];
+    if (lane == 0) sOff[PB] = cl.off[min(p0 + PB, p.n)];
+  } else if (wv == 2) {
+    sV[lane] = p.vel[ic];
+  } else if (gp.rot) {
+    sA[lane] = p.ang[ic];
+    sQ[lane] = p.quat[ic];
+  }
+  if (step_skip(ctl)) return;  // the same for the whole block
+  __syncthreads();
+  double none[3][3];
+  if (wv == 0) {  // the sums start from the walls' and body forces
+    const dv3 F = wall_body_force<false, EXTRA>(gp, ic, fl, xyz(sP[lane]), sP[lane].w, sO[lane].w, none);
+    sum[lane] = F.x;
+    sum[PB + lane] = F.y;
+    sum[2 * PB + lane] = F.z;
+    for (int c = 3; c < 6; c++) sum[c * PB + lane] = 0.0;
+  }
+  const int pl = t >> 2;  // the particle whose entries and sums this thread looks after
+  const int a0 = sOff[pl], a1 = sOff[pl + 1];
+  const int E0 = sOff[0], E1 = sOff[PB];
+  for (int cb = E0; cb < E1; cb += CH) {
+    int2 en[U];
+    double4 Pn[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = cb + u * BS + t;
+      en[u] = k < E1 ? cl.ent[k] : make_int2(0, 0);
+    }
+    // whose entries they are: 4 threads a particle
+    const int ca = max(a0, cb) - cb, ce = min(a1, cb + CH) - cb;
+    for (int k = ca + (t & 3); k < ce; k += 4) owner[k] = (unsigned char)pl;
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (cb + u * BS + t < E1) Pn[u] = p.pos[en[u].x & 0x7fffffff];
+    __syncthreads();
+    bool on[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      on[u] = false;
+      if (cb + u * BS + t < E1) {
+        sEnt[u * BS + t] = en[u];
+        const bool second = en[u].x < 0;
+        const double4 Pi = sP[owner[u * BS + t]];
+        const double4 P1 = second ? Pn[u] : Pi;
+        const double4 P2 = x_image(P1, second ? Pi : Pn[u], cl.period);
+        const dv3 D = sub3(xyz(P1), xyz(P2));
+        const double eq = P1.w + P2.w;
+        const ContactSeg& g = seg_of<KIND>(cl, en[u].y);
+        const int kind = KIND ? KIND : g.kind;
+        // (RotElastic tests |D| < eq; a pair that only rounding separates from
+        // that is left to its law)
+        on[u] = kind == ESP_SEG_ROT_ELASTIC ? dot3(D, D) <= (eq * eq) * 1.000001
+                                            : dot3(D, D) < (eq * eq);
+        if (!on[u] && !second && kind == ESP_SEG_ROT_FRICTION) clear_history(g, en[u].y - g.rec_off);
+      }
+      const unsigned long long m = __ballot(on[u]);
+      if (lane == 0) touch_mask[u * (BS / 64) + wv] = m;
+    }
+    __syncthreads();
+    // touching entries before entry x of the chunk: lane k of every wave holds
+    // those before the k-th 64 (every lane calls it)
+    int before = 0;
+    {
+      const int pc = lane < CH / 64 ? __popcll(touch_mask[lane]) : 0;
+      int inc = pc;
+#pragma unroll
+      for (int d = 1; d < 16; d <<= 1) {
+        const int v = __shfl_up(inc, d, 64);
+        if (lane >= d) inc += v;
+      }
+      before = inc - pc;
+    }
+    auto rank = [&](int x) {
+      const int w = x >> 6;
+      const unsigned long long m = w < CH / 64 ? touch_mask[w] : 0ull;
+      return __shfl(before, w, 64) + __popcll(m & ((1ull << (x & 63)) - 1ull));
+    };
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int q = rank(u * BS + t);
+      if (on[u]) queue[q] = (unsigned short)(u * BS + t);
+    }
+    const int nq = rank(CH);
+    const int qa = rank(min(ca, CH)), qe = rank(max(ce, 0));
+    __syncthreads();
+    for (int qb = 0; qb < nq; qb += SC) {
+      const int qn = min(nq - qb, SC);
+#pragma unroll 1
+      for (int q = t; q < qn; q += BS) {
+        const int x = queue[qb + q];
+        const int2 e = sEnt[x];
+        const int o = owner[x];
+        dv3 f = mk3(0.0, 0.0, 0.0), m = f;
+        pair_share<KIND>(p, cl, e, sP[o], sV[o], sA[o], f, m);
+        slot[q] = f.x;
+        slot[SC + q] = f.y;
+        slot[2 * SC + q] = f.z;
+        slot[3 * SC + q] = m.x;
+        slot[4 * SC + q] = m.y;
+        slot[5 * SC + q] = m.z;
+      }
+      __syncthreads();
+      // each particle's shares in entry order; its 4 threads take the components
+      // (force x, y, z and moment x; moment y, z)
+      {
+        const int u0 = max(qa, qb) - qb, u1 = min(qe, qb + SC) - qb;
+        const int c = t & 3;
+        if (u0 < u1) {
+          double s0 = sum[c * PB + pl], s1 = c < 2 ? sum[(c + 4) * PB + pl] : 0.0;
+          for (int q = u0; q < u1; q++) {
+            s0 = s0 + slot[c * SC + q];
+            if (c < 2) s1 = s1 + slot[(c + 4) * SC + q];
+          }
+          sum[c * PB + pl] = s0;
+          if (c < 2) sum[(c + 4) * PB + pl] = s1;
+        }
+      }
+      __syncthreads();
+    }
+  }
+  if (wv != 0) return;
+  const bool act = lane < np;
+  const double4 P = sP[lane];
+  unsigned long long md = 0;
+  if (act) {
+    PView po = p;
+    po.pos = cl.pos_o;
+    po.vel = cl.vel_o;
+    po.ang = cl.ang_o;
+    const dv3 F = mk3(sum[lane], sum[PB + lane], sum[2 * PB + lane]);
+    const dv3 M = mk3(sum[3 * PB + lane], sum[4 * PB + lane], sum[5 * PB + lane]);
+    md = (unsigned long long)__double_as_longlong(damp_and_integrate<false, EXTRA>(
+        po, gp, i, fl, F, M, P, sV[lane], sO[lane], sA[lane], sQ[lane], none));
+  }
+  step_tail<EXTRA>(ctl, gp, i, act, fl, P, md);
+}
+
+// rows[k * stride + i]: the k-th interaction of particle i in summation order:
+// the other particle (bit 31: i is the second of the pair) and the record
+__global__ void k_contact_rows(int n, int stride, const int* off, const int* ent, RecordLists rl,
+                               int* cnt, int2* rows)
+{
+  const int i = blockIdx.x * BS + threadIdx.x;
+  if (i >= n) return;
+  const int a = off[i], m = off[i + 1] - a;
+  cnt[i] = m;
+  for (int k = 0; k < m; k++) {
+    const int v = ent[a + k], rec = v >> 2;
+    int s = 0;
+    while (s + 1 < rl.count && rec >= rl.rec_off[s + 1]) s++;
+    const int2 e = rl.ij[s][rec - rl.rec_off[s]];
+    rows[(size_t)k * stride + i] =
+        (v & 1) ? make_int2(e.x | (int)0x80000000u, rec) : make_int2(e.y, rec);
+  }
+}
+
+// ent[off[i] + k]: the same entries in CSR order
+__global__ void k_contact_entries(int total, const int* inc_ent, RecordLists rl, int2* ent)
+{
+  const int t = blockIdx.x * BS + threadIdx.x;
+  if (t >= total) return;
+  const int v = inc_ent[t], rec = v >> 2;
+  int s = 0;
+  while (s + 1 < rl.count && rec >= rl.rec_off[s + 1]) s++;
+  const int2 e = rl.ij[s][rec - rl.rec_off[s]];
+  ent[t] = (v & 1) ? make_int2(e.x | (int)0x80000000u, rec) : make_int2(e.y, rec);
+}
+
+__global__ __launch_bounds__(BS) void k_max_int(int n, const int* a, int* out)
+{
+  const int i = blockIdx.x * BS + threadIdx.x;
+  int v = i < n ? a[i] : 0;
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  if ((threadIdx.x & 63) == 0 && v > 0) atomicMax(out, v);
+}
+
+// the 64-particle groups holding wall candidates, ascending (one block; marks
+// from k_wall_update)
+__global__ __launch_bounds__(1024) void k_wall_list(int ng, const int* mark, int* list, int* list_n)
+{
+  __shared__ int wsum[16], base_s;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  int base = 0;
+  for (int b0 = 0; b0 < ng; b0 += 1024) {
+    const bool on = b0 + t < ng && mark[b0 + t] != 0;
+    const unsigned long long bal = __ballot(on);
+    if (lane == 0) wsum[wv] = __popcll(bal);
+    __syncthreads();
+    int pre = base;
+    for (int w = 0; w < wv; w++) pre += wsum[w];
+    if (on) list[pre + __popcll(bal & ((1ull << lane) - 1ull))] = b0 + t;
+    if (t == 1023) base_s = pre + __popcll(bal);
+    __syncthreads();
+    base = base_s;
+  }
+  if (t == 0) *list_n = base;
 }
 
 // ---------------------------------------------------------------------------
@@ -1167,11 +1686,17 @@ __global__ void k_compact_bonds(int nb, const int* keep, const int* off, const i
 struct WallSet {
   WallParam w[ESP_MAX_WALL_GROUPS];
 };
-__global__ void k_wall_update(PView p, GridParams g, int nwg, WallSet ws)
+__global__ void k_wall_update(PView p, GridParams g, int nwg, WallSet ws, int* mark)
 {
   const int i = blockIdx.x * BS + threadIdx.x;
-  if (i >= p.n) return;
-  p.flags[i] = wall_membership(g, nwg, ws.w, p.pos[i], p.flags[i]);
+  unsigned fl = 0u;
+  if (i < p.n) {
+    fl = wall_membership(g, nwg, ws.w, p.pos[i], p.flags[i]);
+    p.flags[i] = fl;
+  }
+  // mark[group of 64 particles]: holds wall candidates
+  const unsigned long long any = __ballot(((fl >> PF_WALL_SHIFT) & 0xFFu) != 0u);
+  if (mark && (threadIdx.x & 63) == 0 && i < p.n) mark[i >> 6] = any ? 1 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1788,6 +2313,8 @@ void launch_alive_flags(hipStream_t s, int nb, const int2* ij, int* keep)
   hipLaunchKernelGGL(k_alive_flags, dim3(nblk(nb)), dim3(BS), 0, s, nb, ij, keep);
 }
 
+static bool extra_forces(const GatherParams& gp);
+
 template <bool STRESS, bool EXTRA>
 static void gather_launch(hipStream_t s, StepCtl ctl, PView p, const GatherParams& gp,
                           hipEvent_t ev_a, hipEvent_t ev_b)
@@ -1803,8 +2330,7 @@ bool launch_gather_integrate(hipStream_t s, StepCtl ctl, PView p, const GatherPa
                              hipEvent_t ev_a, hipEvent_t ev_b)
 {
   if (p.n <= 0) return false;
-  bool extra = gp.ndamp > 0;
-  for (int w = 0; w < gp.nwg; w++) extra |= gp.wall[w].bonded != 0 || gp.wall[w].tagged != 0;
+  const bool extra = extra_forces(gp);
   if (gp.sig) {
     if (extra) gather_launch<true, true>(s, ctl, p, gp, ev_a, ev_b);
     else gather_launch<true, false>(s, ctl, p, gp, ev_a, ev_b);
@@ -1842,19 +2368,81 @@ void launch_sc_break(hipStream_t s, StepCtl ctl, PView p, const ScLaunch& sl)
   hipLaunchKernelGGL(k_sc_break, dim3(sl.nblocks), dim3(BS), 0, s, ctl, p, sl);
 }
 
-void launch_wall_finalize(hipStream_t s, const double* part, int nblocks, int nwg, int nsteps,
-                          double* out)
+void launch_batch_end(hipStream_t s, const BatchEnd& be)
 {
-  if (nwg <= 0 || nsteps <= 0) return;
-  hipLaunchKernelGGL(k_wall_finalize, dim3(nsteps), dim3(BS), 0, s, part, nblocks, nwg, out);
+  const dim3 g(be.nwg > 0 ? be.nsteps : 1), b(BS);
+  if (be.list)
+    hipLaunchKernelGGL((k_batch_end<true>), g, b, 0, s, be);
+  else
+    hipLaunchKernelGGL((k_batch_end<false>), g, b, 0, s, be);
 }
 
-
-void launch_clear_status(hipStream_t s, StepStatus* ring, int ring_size, long long first_step,
-                         int count, int* halted)
+template <class K>
+static void contact_launch(K kern, dim3 g, hipStream_t s, StepCtl ctl, PView p,
+                           const ContactLaunch& cl, const GatherParams& gp, hipEvent_t ev_a,
+                           hipEvent_t ev_b)
 {
-  hipLaunchKernelGGL(k_clear_status, dim3(nblk(count > 0 ? count : 1)), dim3(BS), 0, s, ring,
-                     ring_size, first_step, count, halted);
+  if (ev_a && ev_b)
+    hipExtLaunchKernelGGL(kern, g, dim3(BS), 0, s, ev_a, ev_b, 0, ctl, p, cl, gp);
+  else
+    hipLaunchKernelGGL(kern, g, dim3(BS), 0, s, ctl, p, cl, gp);
+}
+
+static bool extra_forces(const GatherParams& gp)
+{
+  bool extra = gp.ndamp > 0;
+  for (int w = 0; w < gp.nwg; w++) extra |= gp.wall[w].bonded != 0 || gp.wall[w].tagged != 0;
+  return extra;
+}
+
+int contact_groups(int n) { return nblk(n, 64); }
+
+bool launch_contact_step(hipStream_t s, StepCtl ctl, PView p, const ContactLaunch& cl,
+                         const GatherParams& gp, hipEvent_t ev_a, hipEvent_t ev_b)
+{
+  if (p.n <= 0) return false;
+  const bool extra = extra_forces(gp);
+  if (cl.rows) {
+    constexpr int G = ESP_G_EL;
+    const dim3 g(nblk(p.n, BS / G));
+    if (extra) contact_launch(k_contact_step<true, G>, g, s, ctl, p, cl, gp, ev_a, ev_b);
+    else contact_launch(k_contact_step<false, G>, g, s, ctl, p, cl, gp, ev_a, ev_b);
+    return true;
+  }
+  const dim3 g(nblk(p.n, 64));
+  if (cl.count == 1 && cl.seg[0].kind == ESP_SEG_ROT_FRICTION && !cl.seg[0].rigid) {
+    if (extra) contact_launch(k_contact_block<true, ESP_SEG_ROT_FRICTION>, g, s, ctl, p, cl, gp, ev_a, ev_b);
+    else contact_launch(k_contact_block<false, ESP_SEG_ROT_FRICTION>, g, s, ctl, p, cl, gp, ev_a, ev_b);
+  } else {
+    if (extra) contact_launch(k_contact_block<true, 0>, g, s, ctl, p, cl, gp, ev_a, ev_b);
+    else contact_launch(k_contact_block<false, 0>, g, s, ctl, p, cl, gp, ev_a, ev_b);
+  }
+  return true;
+}
+
+void launch_contact_entries(hipStream_t s, int total, const int* inc_ent, const RecordLists& rl,
+                            int2* ent)
+{
+  if (total <= 0) return;
+  hipLaunchKernelGGL(k_contact_entries, dim3(nblk(total)), dim3(BS), 0, s, total, inc_ent, rl, ent);
+}
+
+void launch_contact_rows(hipStream_t s, int n, int stride, const int* off, const int* ent,
+                         const RecordLists& rl, int* cnt, int2* rows)
+{
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_contact_rows, dim3(nblk(n)), dim3(BS), 0, s, n, stride, off, ent, rl, cnt, rows);
+}
+
+void launch_max_int(hipStream_t s, int n, const int* a, int* out)
+{
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_max_int, dim3(nblk(n)), dim3(BS), 0, s, n, a, out);
+}
+
+void launch_wall_list(hipStream_t s, int ng, const int* mark, int* list, int* list_n)
+{
+  hipLaunchKernelGGL(k_wall_list, dim3(1), dim3(1024), 0, s, ng, mark, list, list_n);
 }
 
 void launch_cells_count(hipStream_t s, PView p, GridParams g, int* cell, int* cell_count,
@@ -2068,12 +2656,12 @@ void launch_compact_bonds(hipStream_t s, int nb, const int* keep, const int* off
 
 
 
-void launch_wall_update(hipStream_t s, PView p, GridParams g, int nwg, const WallParam* w)
+void launch_wall_update(hipStream_t s, PView p, GridParams g, int nwg, const WallParam* w, int* mark)
 {
   if (p.n <= 0) return;
   WallSet ws;
   for (int k = 0; k < ESP_MAX_WALL_GROUPS; k++) ws.w[k] = w[k];
-  hipLaunchKernelGGL(k_wall_update, dim3(nblk(p.n)), dim3(BS), 0, s, p, g, nwg, ws);
+  hipLaunchKernelGGL(k_wall_update, dim3(nblk(p.n)), dim3(BS), 0, s, p, g, nwg, ws, mark);
 }
 
 void launch_inc_count(hipStream_t s, int nc, const int2* ij, int* inc_cnt)
