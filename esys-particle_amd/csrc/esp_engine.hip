@@ -230,6 +230,12 @@ struct esp_engine {
   // staging buffers the candidates are packed into in that order
   DBuf<int> ord_slot;
   bool ord_valid = false;
+  // queries answer in id order: the slots by ascending id (host and device),
+  // laid out again after the slots change, and the device staging of a query
+  std::vector<int> id_slots;
+  bool id_slots_valid = false;
+  DBuf<int> id_slots_dev;
+  DBuf<double> query;
   DBuf<int> wc_mark, wc_off;
   DBuf<WallCand> wc_cand;
   PinBuf<WallCand> hw_cand;
@@ -271,6 +277,7 @@ struct esp_engine {
   int broken_cap = 0;
   DBuf<double> wall_part;
   PinBuf<double> batch_out;  // what the end of a batch reports: a BatchOut, then wall forces
+  size_t servo_at = 0;       // and the servo's sums (k_servo_sums)
   // engines without bonded groups (contact_mode): the arrays a step writes, each
   // particle's interactions as rows, the 64-particle groups with wall candidates
   DBuf<double4> pos2, vel2, ang2;
@@ -595,6 +602,7 @@ void spatial_order(esp_engine* e)
   permute(e->h_inert, 1);
   permute(e->h_order, 1);
   e->ord_valid = false;
+  e->id_slots_valid = false;
   e->id2slot.clear();
   for (int i = 0; i < n; i++) e->id2slot[e->h_id[i]] = i;
 }
@@ -803,7 +811,8 @@ void upload(esp_engine* e)
     e->sig.reserve((size_t)std::max(n, 1) * 9);
     zero(e, e->sig.p, (size_t)std::max(n, 1) * 9);
   }
-  e->batch_out.reserve(kBatchHead + (size_t)(e->K + 1) * std::max(nwg, 1) * 3);
+  e->servo_at = kBatchHead + (size_t)(e->K + 1) * std::max(nwg, 1) * 3;
+  e->batch_out.reserve(e->servo_at + 8 * ESP_SERVO_BLOCKS);
   sync(e);
   e->started = true;
 }
@@ -1005,6 +1014,7 @@ void erase_outside(esp_engine* e)
   compact_host(e->h_inert, hkeep, 1);
   compact_host(e->h_order, hkeep, 1);
   e->ord_valid = false;
+  e->id_slots_valid = false;
   e->id2slot.clear();
   for (int i = 0; i < nk; i++) e->id2slot[e->h_id[i]] = i;
   e->n = nk;
@@ -1941,12 +1951,45 @@ void run_steps(esp_engine* e, int nsteps)
 // ---------------------------------------------------------------------------
 // queries
 // ---------------------------------------------------------------------------
+// slots by ascending id: ids that fill most of their range are placed by
+// counting, others are sorted
 std::vector<int> id_order(esp_engine* e)
 {
   std::vector<int> order(e->n);
+  if (e->n == 0) return order;
+  const auto mm = std::minmax_element(e->h_id.begin(), e->h_id.begin() + e->n);
+  const long long lo = *mm.first, span = (long long)*mm.second - lo + 1;
+  if (span <= 4ll * e->n + 1024) {
+    std::vector<int> at((size_t)span, -1);
+    bool distinct = true;
+    for (int i = 0; i < e->n; i++) {
+      int& a = at[(size_t)(e->h_id[i] - lo)];
+      distinct &= a < 0;
+      a = i;
+    }
+    if (distinct) {
+      int k = 0;
+      for (int v : at)
+        if (v >= 0) order[k++] = v;
+      return order;
+    }
+  }
   for (int i = 0; i < e->n; i++) order[i] = i;
   std::sort(order.begin(), order.end(), [&](int a, int b) { return e->h_id[a] < e->h_id[b]; });
   return order;
+}
+
+// id_order of a running engine, kept (with its device copy) until slots change
+const std::vector<int>& kept_id_order(esp_engine* e)
+{
+  if (!e->id_slots_valid) {
+    e->id_slots = id_order(e);
+    e->id_slots_dev.reserve((size_t)std::max(e->n, 1));
+    h2d(e, e->id_slots_dev.p, e->id_slots.data(), e->id_slots.size());
+    sync(e);
+    e->id_slots_valid = true;
+  }
+  return e->id_slots;
 }
 
 // Read-only views for queries.  Dead bonds stay in storage and appended pairs
@@ -2628,6 +2671,7 @@ int esp_add_particles(esp_engine* e, int n, const int* id, const int* tag, const
     e->h_inert.push_back(0.0);
     e->h_order.push_back(e->next_order++);
     e->ord_valid = false;
+  e->id_slots_valid = false;
   }
   return ESP_OK;
   API_END
@@ -2956,8 +3000,60 @@ struct CandRange {
   const WallCand* end() const { return p + m; }
 };
 
+// BWallInteractionGroup::applyForce (BWallInteractionGroup.hpp:71-145) while no
+// untagged candidate touches the wall: the force is then linear in the wall's
+// displacement, so one pass over the candidates on the device gives what every
+// iteration needs.  Returns false, with nothing moved, when an untagged one could
+// touch during the iteration (the caller iterates over the candidates).  cap:
+// the most candidates the caller allows.
+bool servo_bonded(esp_engine* e, int k, const double Fa[3], long long cap)
+{
+  const WallGroup& G = e->wg[e->word[k]];
+  Wall& W = e->walls[G.wall];
+  if (!G.bonded || !e->started || e->n <= 0) return false;
+  HIPCHK(hipSetDevice(e->cfg.device));
+  WallParam wp[ESP_MAX_WALL_GROUPS];
+  wall_params(e, wp);
+  const bool cm = contact_mode(e);
+  double* out = e->batch_out.p + e->servo_at;
+  launch_servo_sums(e->stream, e->view(), wp[k], k, e->do2d, e->init.p,
+                    cm ? e->wall_list.p + 1 : nullptr, cm ? e->wall_list.p : nullptr, out);
+  HIPCHK(hipGetLastError());
+  sync(e);
+  double K = 0.0, cnt = 0.0, gap = 1e300;
+  dv3 S = mk3(0.0, 0.0, 0.0);
+  for (int b = 0; b < ESP_SERVO_BLOCKS; b++) {
+    const double* o = out + 8 * b;
+    K = K + o[0];
+    S = add3(S, mk3(o[1], o[2], o[3]));
+    gap = std::min(gap, o[4]);
+    cnt = cnt + o[5];
+  }
+  if (cnt > (double)cap || !(K > 0)) return false;  // the caller's path reports it
+  const dv3 F = mk3(Fa[0], Fa[1], Fa[2]);
+  const dv3 O_f = div3(F, norm3(F));
+  const double f0 = dot3(add3(F, S), O_f);
+  double d[10], moved = 0.0, far = 0.0;
+  int it = 0;
+  do {
+    d[it] = (f0 - K * moved) / K;
+    moved = moved + d[it];
+    far = std::max(far, std::fabs(moved));
+    it++;
+  } while ((it < 10) && (std::fabs(d[it - 1]) > 10e-6));
+  if (!(gap > far)) return false;
+  for (int t = 0; t < it; t++) {
+    const dv3 v = mul3(O_f, d[t]);
+    W.o[0] = W.o[0] + v.x;
+    W.o[1] = W.o[1] + v.y;
+    W.o[2] = W.o[2] + v.z;
+  }
+  return true;
+}
+
 void apply_force_to_wall(esp_engine* e, int k, const double Fa[3])
 {
+  if (servo_bonded(e, k, Fa, 1ll << 40)) return;
   const WallGroup& G = e->wg[e->word[k]];
   int m = 0;
   if (e->started && e->n > 0) {
@@ -3154,6 +3250,7 @@ int h_na_idx[ESP_NOALLOC_MAX_WALL_CANDIDATES];
 
 void apply_force_to_wall_noalloc(esp_engine* e, int k, const double Fa[3])
 {
+  if (servo_bonded(e, k, Fa, ESP_NOALLOC_MAX_WALL_CANDIDATES)) return;
   const WallGroup& G = e->wg[e->word[k]];
   int m = 0;
   if (e->started && e->n > 0) {
@@ -3276,7 +3373,8 @@ int esp_get_stats(esp_engine* e, esp_stats* o)
 int esp_get_particle_ids(esp_engine* e, int* out)
 {
   API_BEGIN
-  std::vector<int> order = id_order(e);
+  if (e->started) HIPCHK(hipSetDevice(e->cfg.device));
+  const std::vector<int> order = e->started ? kept_id_order(e) : id_order(e);
   for (int k = 0; k < e->n; k++) out[k] = e->h_id[order[k]];
   return ESP_OK;
   API_END
@@ -3286,8 +3384,8 @@ int esp_get_particle_data(esp_engine* e, int field, double* out)
 {
   API_BEGIN
   const int n = e->n;
-  std::vector<int> order = id_order(e);
   if (!e->started) {
+    const std::vector<int> order = id_order(e);
     for (int k = 0; k < n; k++) {
       const int i = order[k];
       const double r = e->h_rad[i];
@@ -3316,7 +3414,6 @@ int esp_get_particle_data(esp_engine* e, int field, double* out)
     return ESP_OK;
   }
   HIPCHK(hipSetDevice(e->cfg.device));
-  std::vector<double4> buf(std::max(n, 1));
   const double4* src = nullptr;
   int sel = 0;  // 0 xyz, 1 quat, 2 w
   switch (field) {
@@ -3331,22 +3428,18 @@ int esp_get_particle_data(esp_engine* e, int field, double* out)
     case ESP_FIELD_OLDPOS: src = e->old.p; break;
     default: throw EspError(ESP_ERR_ARG, "unknown field");
   }
-  if (src) {
-    d2h(e, buf.data(), src, n);
-    sync(e);
+  const int width = sel == 0 ? 3 : sel == 1 ? 4 : 1;
+  if (!src) {  // non-rotational particles
+    for (size_t k = 0; k < (size_t)width * n; k++) out[k] = (sel == 1 && k % 4 == 0) ? 1.0 : 0.0;
+    return ESP_OK;
   }
-  for (int k = 0; k < n; k++) {
-    const int i = order[k];
-    if (!src) {
-      if (sel == 1) { out[4 * k] = 1.0; out[4 * k + 1] = out[4 * k + 2] = out[4 * k + 3] = 0.0; }
-      else for (int c = 0; c < 3; c++) out[3 * k + c] = 0.0;
-      continue;
-    }
-    const double4 v = buf[i];
-    if (sel == 0) { out[3 * k] = v.x; out[3 * k + 1] = v.y; out[3 * k + 2] = v.z; }
-    else if (sel == 1) { out[4 * k] = v.x; out[4 * k + 1] = v.y; out[4 * k + 2] = v.z; out[4 * k + 3] = v.w; }
-    else out[k] = v.w;
-  }
+  // packed in id order on the device: what is copied is what the caller gets
+  kept_id_order(e);
+  e->query.reserve((size_t)4 * std::max(n, 1));
+  launch_pack_ordered(e->stream, n, e->id_slots_dev.p, src, width, e->query.p);
+  HIPCHK(hipGetLastError());
+  d2h(e, out, e->query.p, (size_t)width * n);
+  sync(e);
   return ESP_OK;
   API_END
 }

@@ -382,6 +382,13 @@ void launch_wall_mark_ordered(hipStream_t s, int no, const int* ord_slot, const 
                               int w, int* mark);
 void launch_wall_pack_ordered(hipStream_t s, int no, const int* ord_slot, const int* mark,
                               const int* off, PView p, const double4* init, WallCand* out);
+// the bonded servo's sums over wall group w (out: host memory, see k_servo_sums)
+#define ESP_SERVO_BLOCKS 128
+void launch_servo_sums(hipStream_t s, PView p, const WallParam& W, int w, int do2d,
+                       const double4* init, const int* list, const int* list_n, double* out);
+// a particle field packed in id order (order: slots by ascending id)
+void launch_pack_ordered(hipStream_t s, int n, const int* order, const double4* src, int width,
+                         double* out);
 // a[0..n) = v (a kernel, not a memset: safe under stream capture)
 void launch_fill_int(hipStream_t s, int n, int* a, int v);
 // erasure of particles outside the padded grid (NeighborTable::build):

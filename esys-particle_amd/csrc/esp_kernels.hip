@@ -1493,6 +1493,82 @@ __global__ void k_wall_cands(PView p, int w, const double4* init, int cap, int* 
   if (init) ipos[k] = init[i];
 }
 
+// What the bonded servo's iteration needs of wall group w's candidates, in one
+// pass: out[block][8] = (stiffness sum of the tagged inner ones, their force sum
+// at the wall displacement disp, the least gap of the untagged inner ones to the
+// wall, candidates), written to page-locked host memory and added up there in
+// block order.  Waves take the 64-particle groups of list (all groups: nullptr).
+__global__ __launch_bounds__(BS) void k_servo_sums(PView p, WallParam W, int w, int do2d, int ng,
+                                                   const double4* init, const int* list,
+                                                   const int* list_n, double* out)
+{
+  __shared__ double part[BS / 64][6];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int m = list ? *list_n : ng;
+  double K = 0.0, sx = 0.0, sy = 0.0, sz = 0.0, gap = 1e300, cnt = 0.0;
+  for (int t = blockIdx.x * (BS / 64) + wv; t < m; t += gridDim.x * (BS / 64)) {
+    const int i = (list ? list[t] : t) * 64 + lane;
+    if (i >= p.n) continue;
+    const unsigned fl = p.flags[i];
+    if (!((fl >> (PF_WALL_SHIFT + w)) & 1u)) continue;
+    cnt = cnt + 1.0;
+    if (!((fl >> (PF_INNER_SHIFT + w)) & 1u)) continue;
+    const double4 P = p.pos[i];
+    if ((fl >> (PF_BTAG_SHIFT + w)) & 1u) {
+      const double kb = W.k * (do2d ? 1.0 : 3.1415926536 * P.w);
+      const dv3 D = sub3(sub3(xyz(P), xyz(init[i])), mk3(W.disp[0], W.disp[1], W.disp[2]));
+      K = K + kb;
+      sx = sx + D.x * kb;
+      sy = sy + D.y * kb;
+      sz = sz + D.z * kb;
+    } else {
+      const double dist = dot3(sub3(xyz(P), mk3(W.o[0], W.o[1], W.o[2])),
+                               mk3(W.nrm[0], W.nrm[1], W.nrm[2]));
+      gap = fmin(gap, dist - P.w);
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    K = K + __shfl_xor(K, o, 64);
+    sx = sx + __shfl_xor(sx, o, 64);
+    sy = sy + __shfl_xor(sy, o, 64);
+    sz = sz + __shfl_xor(sz, o, 64);
+    cnt = cnt + __shfl_xor(cnt, o, 64);
+    gap = fmin(gap, __shfl_xor(gap, o, 64));
+  }
+  if (lane == 0) {
+    part[wv][0] = K;
+    part[wv][1] = sx;
+    part[wv][2] = sy;
+    part[wv][3] = sz;
+    part[wv][4] = gap;
+    part[wv][5] = cnt;
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    double a = part[0][threadIdx.x];
+    for (int k = 1; k < BS / 64; k++)
+      a = threadIdx.x == 4 ? fmin(a, part[k][4]) : a + part[k][threadIdx.x];
+    out[8 * blockIdx.x + threadIdx.x] = a;
+  }
+}
+
+// a field in id order, packed: 3 or 4 components, or (width 1) the fourth alone
+__global__ void k_pack_ordered(int n, const int* order, const double4* src, int width, double* out)
+{
+  const int k = blockIdx.x * BS + threadIdx.x;
+  if (k >= n) return;
+  const double4 v = src[order[k]];
+  if (width == 1) {
+    out[k] = v.w;
+    return;
+  }
+  double* o = out + (size_t)width * k;
+  o[0] = v.x;
+  o[1] = v.y;
+  o[2] = v.z;
+  if (width == 4) o[3] = v.w;
+}
+
 __global__ void k_wall_mark_ordered(int no, const int* ord_slot, const unsigned* flags, int w,
                                     int* mark)
 {
@@ -2545,6 +2621,20 @@ void launch_wall_mark_ordered(hipStream_t s, int no, const int* ord_slot, const 
   if (no <= 0) return;
   hipLaunchKernelGGL(k_wall_mark_ordered, dim3(nblk(no)), dim3(BS), 0, s, no, ord_slot, flags, w,
                      mark);
+}
+
+void launch_servo_sums(hipStream_t s, PView p, const WallParam& W, int w, int do2d,
+                       const double4* init, const int* list, const int* list_n, double* out)
+{
+  hipLaunchKernelGGL(k_servo_sums, dim3(ESP_SERVO_BLOCKS), dim3(BS), 0, s, p, W, w, do2d,
+                     contact_groups(p.n), init, list, list_n, out);
+}
+
+void launch_pack_ordered(hipStream_t s, int n, const int* order, const double4* src, int width,
+                         double* out)
+{
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_pack_ordered, dim3(nblk(n)), dim3(BS), 0, s, n, order, src, width, out);
 }
 
 void launch_wall_pack_ordered(hipStream_t s, int no, const int* ord_slot, const int* mark,
