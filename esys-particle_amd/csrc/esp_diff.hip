@@ -1094,13 +1094,13 @@ void rebuild(esp_diff* d, int step)
   launch_cells_fill(d->stream, n, d->cell.p, d->cell_start.p, d->cell_fill.p, d->cell_items.p);
   launch_cells_sort(d->stream, d->ncell, d->cell_start.p, d->cell_items.p);
   launch_pairs(d->stream, 0, 0, pv, d->grid, d->cfg.verlet_dist, d->cell.p, d->cell_start.p,
-               d->cell_items.p, d->ccnt.p, nullptr, nullptr, nullptr, nullptr);
+               d->cell_items.p, d->ccnt.p, nullptr, 0, nullptr, nullptr, nullptr);
   const int nc = dscan(d, d->ccnt.p, d->coff.p, n);
   d->cp.reserve(std::max(nc, 1));
   d->cq.reserve(std::max(nc, 1));
   d->ckey.reserve(std::max(nc, 1));
   launch_pairs(d->stream, 1, 0, pv, d->grid, d->cfg.verlet_dist, d->cell.p, d->cell_start.p,
-               d->cell_items.p, nullptr, d->coff.p, d->cp.p, d->cq.p, d->ckey.p);
+               d->cell_items.p, nullptr, d->coff.p, nc, d->cp.p, d->cq.p, d->ckey.p);
   DCHK(hipGetLastError());
   auto E = std::make_unique<Epoch>();
   E->start = step;

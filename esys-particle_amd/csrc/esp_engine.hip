@@ -259,7 +259,7 @@ struct esp_engine {
   DBuf<int2> tmp_ij, tmp_ij2;
   DBuf<long long> tmp_key, tmp_key2;
   DBuf<double4> tmp_ff, tmp_a, tmp_b, tmp_c;
-  DBuf<int> inc_cnt, inc_off, inc_fill, inc_ent, tmp_rank;
+  DBuf<int> inc_cnt, inc_off, inc_fill, tmp_rank;
   DBuf<unsigned long long> inc_ent64;
   DBuf<int> xcnt, flist;
   DBuf<int4> evt;
@@ -279,11 +279,10 @@ struct esp_engine {
   PinBuf<double> batch_out;  // what the end of a batch reports: a BatchOut, then wall forces
   size_t servo_at = 0;       // and the servo's sums (k_servo_sums)
   // engines without bonded groups (contact_mode): the arrays a step writes, each
-  // particle's interactions as rows, the 64-particle groups with wall candidates
+  // particle's interactions, the 64-particle groups with wall candidates
   DBuf<double4> pos2, vel2, ang2;
-  DBuf<int> row_cnt, wall_mark, wall_list;
-  DBuf<int2> rows, contact_ent;
-  int row_stride = 0, row_width = 0;
+  DBuf<int> wall_mark, wall_list;
+  DBuf<int2> contact_ent;
 
   std::vector<DynGroup> dg;
   std::vector<BondGroup> bg;
@@ -300,6 +299,7 @@ struct esp_engine {
 
   long long t = 0, timestamp = 0, last_ns = -1;
   bool first_time = true, pending_host = false;
+  bool erased_last = false;  // the last neighbour search erased particles
   int pending_reason = 0;
   long long num_host_phases = 0;
   std::vector<int> rebuild_steps;
@@ -336,10 +336,6 @@ namespace {
 // interaction and a second launch gathers their shares (a bond's law is too
 // long to be evaluated from both ends).
 bool contact_mode(const esp_engine* e) { return e->bg.empty(); }
-
-// one NRotElastic group: a few lanes walk each particle's row (k_contact_step);
-// any other mix of groups: a block's pairs are packed first (k_contact_block)
-bool contact_rows(const esp_engine* e) { return e->dg.size() == 1 && e->dg[0].kind == 1; }
 
 // wall partials of one step
 int wall_blocks(const esp_engine* e)
@@ -541,9 +537,10 @@ void reserve_group(DynGroup& G, size_t n_main, bool hist)
   if (hist) G.ff.reserve(c);
 }
 
+// stored pairs are looked up only when bonds break
 void rebuild_presence(esp_engine* e, DynGroup& G)
 {
-  if (G.kind != 3) return;
+  if (G.kind != 3 || contact_mode(e)) return;
   build_hash(e, G.hs, G.hs_mask, (size_t)G.n + ESP_APP_CAP, G.key.p, G.n);
 }
 
@@ -799,7 +796,6 @@ void upload(esp_engine* e)
     e->pos2.reserve(cap);
     e->vel2.reserve(cap);
     if (e->rot) e->ang2.reserve(cap);
-    e->row_cnt.reserve(cap);
     e->wall_mark.reserve((size_t)contact_groups((int)cap));
     e->wall_list.reserve((size_t)contact_groups((int)cap) + 1);
     zero(e, e->wall_list.p, (size_t)contact_groups((int)cap) + 1);
@@ -1047,6 +1043,7 @@ int rebuild_count(esp_engine* e)
 void rebuild_rest(esp_engine* e, long long step, int nout)
 {
   PView p = e->view();
+  e->erased_last = nout > 0;
   if (nout > 0) {
     erase_outside(e);
     p = e->view();
@@ -1061,13 +1058,13 @@ void rebuild_rest(esp_engine* e, long long step, int nout)
   launch_cells_sort(e->stream, e->ncell, e->cell_start.p, e->cell_items.p);
   // full candidate list (getFullList), sorted by (id1, id2)
   launch_pairs(e->stream, 0, 0, p, e->grid, e->alpha, e->cell.p, e->cell_start.p,
-               e->cell_items.p, e->cand_cnt.p, nullptr, nullptr, nullptr, nullptr);
+               e->cell_items.p, e->cand_cnt.p, nullptr, 0, nullptr, nullptr, nullptr);
   const int total = scan_total(e, e->cand_cnt.p, e->cand_off.p, e->n);
   e->cand_p.reserve(std::max(total, 1));
   e->cand_q.reserve(std::max(total, 1));
   e->cand_key.reserve(std::max(total, 1));
   launch_pairs(e->stream, 1, 0, p, e->grid, e->alpha, e->cell.p, e->cell_start.p,
-               e->cell_items.p, nullptr, e->cand_off.p, e->cand_p.p, e->cand_q.p, e->cand_key.p);
+               e->cell_items.p, nullptr, e->cand_off.p, total, e->cand_p.p, e->cand_q.p, e->cand_key.p);
   HIPCHK(hipGetLastError());
   e->ncand = total;
   e->timestamp++;
@@ -1081,13 +1078,13 @@ void new_pair_list(esp_engine* e)
 {
   PView p = e->view();
   launch_pairs(e->stream, 0, 1, p, e->grid, e->alpha, e->cell.p, e->cell_start.p,
-               e->cell_items.p, e->cand_cnt.p, nullptr, nullptr, nullptr, nullptr);
+               e->cell_items.p, e->cand_cnt.p, nullptr, 0, nullptr, nullptr, nullptr);
   const int total = scan_total(e, e->cand_cnt.p, e->cand_off.p, e->n);
   e->np_p.reserve(std::max(total, 1));
   e->np_q.reserve(std::max(total, 1));
   e->np_key.reserve(std::max(total, 1));
   launch_pairs(e->stream, 1, 1, p, e->grid, e->alpha, e->cell.p, e->cell_start.p,
-               e->cell_items.p, nullptr, e->cand_off.p, e->np_p.p, e->np_q.p, e->np_key.p);
+               e->cell_items.p, nullptr, e->cand_off.p, total, e->np_p.p, e->np_q.p, e->np_key.p);
   launch_clear_flag_bit(e->stream, p, e->upd.p);
   HIPCHK(hipGetLastError());
   e->nnew = total;
@@ -1309,7 +1306,7 @@ void dyn_update(esp_engine* e, DynGroup& G, bool& new_list_taken)
     e->tmp_key.reserve((size_t)total + ESP_APP_CAP);
     if (hist) e->tmp_ff.reserve((size_t)total + ESP_APP_CAP);
     launch_pair_emit(e->stream, nc, e->keep.p, e->keep_off.p, e->cand_p.p, e->cand_q.p,
-                     e->cand_key.p, hist ? e->src.p : nullptr, hist ? G.ff.p : nullptr,
+                     e->cand_key.p, hist ? e->src.p : nullptr, hist ? G.ff.p : nullptr, total,
                      e->tmp_ij.p, e->tmp_key.p, hist ? e->tmp_ff.p : nullptr);
     HIPCHK(hipGetLastError());
     G.ij.swap(e->tmp_ij);
@@ -1388,53 +1385,45 @@ void rebuild_csr(esp_engine* e)
   zero(e, e->inc_cnt.p, e->n + 1);
   for (int gi : e->dord) launch_inc_count(e->stream, e->dg[gi].n, e->dg[gi].ij.p, e->inc_cnt.p);
   for (int gi : e->bord) launch_inc_count(e->stream, e->bg[gi].n, e->bg[gi].ij.p, e->inc_cnt.p);
-  int width = 0;  // longest run of a particle
-  if (contact_mode(e) && contact_rows(e)) {
-    zero(e, e->dev_int.p, 1);
-    launch_max_int(e->stream, e->n, e->inc_cnt.p, e->dev_int.p);
-    d2h(e, &width, e->dev_int.p, 1);
-  }
-  const int total = scan_total(e, e->inc_cnt.p, e->inc_off.p, e->n);
-  e->inc_ent.reserve(std::max(total, 1));
+  // dead bonds were compacted out, so every stored interaction has two entries
+  long long pairs = 0;
+  for (auto& G : e->dg) pairs += G.n;
+  for (auto& G : e->bg) pairs += G.n;
+  const int total = (int)(2 * pairs);
+  e->scan_tmp.reserve(scan_tmp_size(e->n));
+  launch_exclusive_scan(e->stream, e->inc_cnt.p, e->inc_off.p, e->n, e->scan_tmp.p);
   e->inc_ent64.reserve(std::max(total, 1));
   zero(e, e->inc_fill.p, e->n + 1);
+  const bool cm = contact_mode(e);
+  if (cm) e->contact_ent.reserve(std::max(total, 1));
+  else e->slot_of.reserve((size_t)std::max<long long>(rec, 1));
   // summation order: dynamic groups by name (storage order), then bonded groups
   // by name (connection order)
-  int grp = 0;
-  for (int gi : e->dord) {
-    DynGroup& G = e->dg[gi];
-    launch_inc_fill(e->stream, G.n, G.ij.p, G.rec_off, G.kind == 3 ? 1 : 0, nullptr, grp++,
-                    e->inc_off.p, e->inc_fill.p, e->inc_ent64.p);
-  }
-  for (int gi : e->bord) {
-    BondGroup& G = e->bg[gi];
-    launch_inc_fill(e->stream, G.n, G.ij.p, G.rec_off, 1, G.rank.p, grp++, e->inc_off.p,
-                    e->inc_fill.p, e->inc_ent64.p);
-  }
-  launch_inc_sort(e->stream, e->n, e->inc_off.p, e->inc_ent64.p, e->inc_ent.p);
-  if (contact_mode(e)) {
-    RecordLists rl;
-    memset(&rl, 0, sizeof rl);
+  for (int pass = 0; pass < 2; pass++) {
+    int grp = 0;
+    auto place = [&](int n, const int2* ij, int rec_off, int has_m, const int* rank) {
+      if (pass == 0)
+        launch_inc_fill(e->stream, n, ij, rec_off, has_m, rank, grp, e->inc_off.p, e->inc_fill.p,
+                        e->inc_ent64.p);
+      else
+        launch_inc_rank(e->stream, n, ij, rec_off, has_m, rank, grp, e->inc_off.p, e->inc_ent64.p,
+                        e->slot_of.p, cm ? e->contact_ent.p : nullptr);
+      grp++;
+    };
     for (int gi : e->dord) {
-      rl.rec_off[rl.count] = e->dg[gi].rec_off;
-      rl.ij[rl.count++] = e->dg[gi].ij.p;
+      DynGroup& G = e->dg[gi];
+      place(G.n, G.ij.p, G.rec_off, G.kind == 3 ? 1 : 0, nullptr);
     }
-    if (contact_rows(e)) {
-      e->row_stride = (std::max(e->n, 1) + 63) & ~63;
-      e->row_width = width;
-      e->rows.reserve((size_t)std::max(width, 1) * e->row_stride);
-      launch_contact_rows(e->stream, e->n, e->row_stride, e->inc_off.p, e->inc_ent.p, rl,
-                          e->row_cnt.p, e->rows.p);
-    } else {
-      e->contact_ent.reserve(std::max(total, 1));
-      launch_contact_entries(e->stream, total, e->inc_ent.p, rl, e->contact_ent.p);
+    for (int gi : e->bord) {
+      BondGroup& G = e->bg[gi];
+      place(G.n, G.ij.p, G.rec_off, 1, G.rank.p);
     }
+  }
+  if (cm) {
     e->xbase = total;
     HIPCHK(hipGetLastError());
     return;
   }
-  e->slot_of.reserve((size_t)std::max<long long>(rec, 1));
-  launch_slot_of(e->stream, total, e->inc_ent.p, e->slot_of.p);
   // slots start at zero: a contact that is not touching keeps zero slots
   // without rewriting them every step
   e->xbase = total;
@@ -1606,14 +1595,8 @@ void launch_contacts(esp_engine* e, const StepCtl& ctl, bool flip, bool last)
   ContactLaunch cl;
   memset(&cl, 0, sizeof cl);
   cl.do2d = e->do2d;
-  cl.stride = e->row_stride;
-  cl.width = e->row_width;
   cl.period = e->grid.period;
   cl.dt = e->dt;
-  if (contact_rows(e)) {
-    cl.cnt = e->row_cnt.p;
-    cl.rows = e->rows.p;
-  }
   cl.off = e->inc_off.p;
   cl.ent = e->contact_ent.p;
   cl.pos_o = e->pos2.p;
@@ -1815,6 +1798,74 @@ void launch_end(esp_engine* e, long long step0, int k)
   HIPCHK(hipGetLastError());
 }
 
+// The neighbour search and the update of the only dynamic group of an engine
+// without bonded groups with one look at the host: everything is launched into
+// the room the last search left, each launch taking its sizes from the device,
+// and the host reads them at the end (a search of 10,000 particles took 0.5 ms
+// with a synchronisation for every size).  Returns false, with the group as it
+// was, when particles left the table or the room did not suffice; the caller
+// then searches step by step.
+bool quick_search(esp_engine* e, long long step)
+{
+  if (!contact_mode(e) || e->first_time || e->dg.size() != 1 || e->dg[0].track || e->erased_last)
+    return false;
+  DynGroup& G = e->dg[0];
+  const bool hist = G.kind == 3;
+  const int n = e->n;
+  const size_t room = std::min({e->cand_p.cap, e->cand_q.cap, e->cand_key.cap, (size_t)(1 << 30)});
+  if (n <= 0 || room == 0) return false;
+  const int cap = (int)room;
+  PView p = e->view();
+  if (e->grid.circ_x) launch_wrap_x(e->stream, p, e->grid.x0, e->grid.period, e->init.p);
+  zero(e, e->cell_count.p, e->ncell + 1);
+  zero(e, e->dev_int.p, 1);
+  launch_cells_count(e->stream, p, e->grid, e->cell.p, e->cell_count.p, e->dev_int.p);
+  e->scan_tmp.reserve(scan_tmp_size(std::max({e->ncell, n, cap})));
+  launch_exclusive_scan(e->stream, e->cell_count.p, e->cell_start.p, e->ncell, e->scan_tmp.p);
+  zero(e, e->cell_fill.p, e->ncell);
+  launch_cells_fill(e->stream, n, e->cell.p, e->cell_start.p, e->cell_fill.p, e->cell_items.p);
+  launch_cells_sort(e->stream, e->ncell, e->cell_start.p, e->cell_items.p);
+  for (int emit = 0; emit < 2; emit++) {
+    launch_pairs(e->stream, emit, 0, p, e->grid, e->alpha, e->cell.p, e->cell_start.p,
+                 e->cell_items.p, e->cand_cnt.p, e->cand_off.p, cap, e->cand_p.p, e->cand_q.p,
+                 e->cand_key.p);
+    if (!emit)
+      launch_exclusive_scan(e->stream, e->cand_cnt.p, e->cand_off.p, n, e->scan_tmp.p);
+  }
+  const int* nc = e->cand_off.p + n;
+  ExclSet ex = excl_set(e, G);
+  e->keep.reserve((size_t)cap + 1);
+  e->keep_off.reserve((size_t)cap + 1);
+  if (hist) {
+    e->src.reserve(cap);
+    launch_ed_mark(e->stream, cap, e->cand_p.p, e->cand_q.p, e->cand_key.p, ex, G.key.p, G.n,
+                   G.ij.p, p, e->grid.period, e->keep.p, e->src.p, nc);
+  } else {
+    launch_ne_mark(e->stream, cap, e->cand_p.p, e->cand_q.p, e->id.p, ex, e->keep.p, nc);
+  }
+  launch_exclusive_scan(e->stream, e->keep.p, e->keep_off.p, cap, e->scan_tmp.p);
+  e->tmp_ij.reserve((size_t)cap + ESP_APP_CAP);
+  e->tmp_key.reserve((size_t)cap + ESP_APP_CAP);
+  if (hist) e->tmp_ff.reserve((size_t)cap + ESP_APP_CAP);
+  launch_pair_emit(e->stream, cap, e->keep.p, e->keep_off.p, e->cand_p.p, e->cand_q.p,
+                   e->cand_key.p, hist ? e->src.p : nullptr, hist ? G.ff.p : nullptr, cap,
+                   e->tmp_ij.p, e->tmp_key.p, hist ? e->tmp_ff.p : nullptr);
+  int* size = reinterpret_cast<int*>(e->batch_out.p + e->servo_at);  // host memory
+  launch_report3(e->stream, e->dev_int.p, nc, e->keep_off.p + cap, size);
+  HIPCHK(hipGetLastError());
+  sync(e);
+  if (size[0] != 0 || size[1] > cap || size[2] > cap) return false;
+  G.ij.swap(e->tmp_ij);
+  G.key.swap(e->tmp_key);
+  if (hist) G.ff.swap(e->tmp_ff);
+  G.n = size[2];
+  e->ncand = size[1];
+  e->timestamp++;
+  G.update_ts = e->timestamp;
+  e->rebuild_steps.push_back((int)step);
+  return true;
+}
+
 // one step with host bookkeeping: the first step, a rebuild, or an
 // incremental update that did not fit the device appendix
 void host_step(esp_engine* e, int reason)
@@ -1823,9 +1874,13 @@ void host_step(esp_engine* e, int reason)
   const long long step = e->t + 1;
   StepStatus prev;
   memset(&prev, 0, sizeof prev);
-  if (!e->first_time) {
+  if (!e->first_time && e->forced_search) {  // a checkpoint's search may have erased breaks
     d2h(e, &prev, e->ring.p + ((step - 1) % e->ring_size), 1);
     sync(e);
+  } else if (!e->first_time) {  // as the last batch reported it
+    const BatchOut& bo = *reinterpret_cast<const BatchOut*>(e->batch_out.p);
+    prev.maxdisp2 = bo.maxdisp2;
+    prev.nbroken = bo.nbroken;
   }
   // forced search of the first runOneStep, or displacement past the threshold;
   // after a checkpoint's search displacements count from there
@@ -1833,7 +1888,8 @@ void host_step(esp_engine* e, int reason)
   // The reference searches first: particles that left the grid are erased with
   // their bonds before the bonds are tested.  The search's cell pass runs
   // first, so the break update knows whether any particle is outside.
-  const int nout = search ? rebuild_count(e) : 0;
+  const bool found = search && quick_search(e, step);
+  const int nout = search && !found ? rebuild_count(e) : 0;
   // PIS_EB::update for the previous step's breaks (already applied on the
   // device when the queue stopped in the incremental update); bonds of
   // particles the search erases are skipped
@@ -1843,8 +1899,8 @@ void host_step(esp_engine* e, int reason)
                        e->upd.p, e->flist.p, e->evt.p, step, nout > 0 ? &e->grid : nullptr);
     HIPCHK(hipGetLastError());
   }
-  fold(e);
-  if (search) rebuild_rest(e, step, nout);
+  if (!contact_mode(e)) fold(e);
+  if (search && !found) rebuild_rest(e, step, nout);
   e->first_time = false;
   e->forced_search = false;
   e->t = step;
@@ -1853,7 +1909,8 @@ void host_step(esp_engine* e, int reason)
   const bool need_update = prev.nbroken > 0;
   if (e->timestamp > e->last_ns || need_update) {
     bool new_list_taken = false;
-    for (int gi : e->dord) dyn_update(e, e->dg[gi], new_list_taken);
+    for (int gi : e->dord)
+      if (!found) dyn_update(e, e->dg[gi], new_list_taken);
     for (auto& G : e->dg)
       if (G.track) log_pair_diff(e, G, step);
     if (!e->wg.empty()) {
@@ -3730,26 +3787,16 @@ std::string check_state(esp_engine* e)
   d2h(e, xcnt.data(), e->xcnt.p, n);
   d2h(e, off.data(), e->inc_off.p, n + 1);
   d2h(e, &st, e->upd.p, 1);
-  const bool cm = contact_mode(e);  // rows instead of record slots
+  const bool cm = contact_mode(e);  // entries instead of record slots
   std::vector<int2> so(std::max(e->nrec, 1));
   if (!cm) d2h(e, so.data(), e->slot_of.p, e->nrec);
-  const bool rm = cm && contact_rows(e);
-  const size_t nrow = rm ? (size_t)e->row_width * e->row_stride : cm && csr ? (size_t)e->xbase : 0;
-  std::vector<int2> rows(std::max<size_t>(nrow, 1));
-  std::vector<int> rcnt(std::max(n, 1));
-  if (cm && csr) {
-    d2h(e, rows.data(), rm ? e->rows.p : e->contact_ent.p, nrow);
-    if (rm) d2h(e, rcnt.data(), e->row_cnt.p, n);
-  }
+  const size_t nent = cm && csr ? (size_t)e->xbase : 0;
+  std::vector<int2> ent(std::max<size_t>(nent, 1));
+  d2h(e, ent.data(), e->contact_ent.p, nent);
   sync(e);
   for (int i = 0; i < n; i++)
     if (xcnt[i] < 0 || xcnt[i] > ESP_XSLOTS) {
       fail("appendix slot count " + std::to_string(xcnt[i]) + " at slot " + std::to_string(i));
-      break;
-    }
-  for (int i = 0; i < n && rm && csr; i++)
-    if (rcnt[i] != off[i + 1] - off[i] || rcnt[i] > e->row_width) {
-      fail("row count at slot " + std::to_string(i));
       break;
     }
   for (int i = 0; i < n && csr; i++)
@@ -3811,15 +3858,15 @@ std::string check_state(esp_engine* e)
                            : app ? so[G.app_rec_off + (c - G.n)] : so[G.rec_off + c];
       bool ok = q.x >= 0 && q.x < n && q.y >= 0 && q.y < n && q.x != q.y && key[c] == pkey(q.x, q.y);
       if (ok && !app && csr && cm) {
-        // the pair is in the row of each of its particles
-        auto in_row = [&](int p, int other) {
+        // the pair is in the run of each of its particles
+        auto listed_in = [&](int p, int other) {
           for (int k = 0; k < off[p + 1] - off[p]; k++) {
-            const int2 v = rm ? rows[(size_t)k * e->row_stride + p] : rows[off[p] + k];
+            const int2 v = ent[off[p] + k];
             if (v.x == other && v.y == G.rec_off + c) return true;
           }
           return false;
         };
-        ok = in_row(q.x, q.y) && in_row(q.y, q.x | (int)0x80000000u);
+        ok = listed_in(q.x, q.y) && listed_in(q.y, q.x | (int)0x80000000u);
       }
       if (ok && !app && csr && !cm) ok = in_run(sl.x, q.x) && in_run(sl.y, q.y);
       if (ok && app && csr)

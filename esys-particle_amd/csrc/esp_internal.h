@@ -169,7 +169,8 @@ struct UpdState {
 // are stored after the key-sorted main list, with their force records in a
 // separate region and per-particle overflow slots in the CSR.
 #define ESP_APP_CAP 16384
-#define ESP_NEW_CAP 4096
+#define ESP_NEW_CAP 1024
+#define ESP_FLAG_CAP 512  // flagged particles a queued step takes care of itself
 #define ESP_XSLOTS 4
 struct DynAppend {
   int2* slot_of;     // record -> slots; appended records get appendix slots
@@ -323,11 +324,8 @@ struct ContactSeg {
 };
 struct ContactLaunch {
   int count, do2d;
-  int stride, width;  // rows: [width][stride]
   double period, dt;
-  const int* cnt;     // interactions per particle
-  const int2* rows;   // see k_contact_rows (one NRotElastic group), else nullptr
-  const int* off;     // CSR runs of ent, see k_contact_entries
+  const int* off;     // the particles' runs of ent, see k_inc_rank
   const int2* ent;
   double4 *pos_o, *vel_o, *ang_o;  // arrays the particles are stepped into
   ContactSeg seg[ESP_MAX_FORCE_SEGS];
@@ -336,17 +334,6 @@ bool launch_contact_step(hipStream_t s, StepCtl ctl, PView p, const ContactLaunc
                          const GatherParams& gp, hipEvent_t ev_a = nullptr,
                          hipEvent_t ev_b = nullptr);
 int contact_groups(int n);  // 64-particle groups the wall partials are kept for
-// the pair lists behind the records (dynamic groups in record order)
-struct RecordLists {
-  int count;
-  int rec_off[ESP_MAX_FORCE_SEGS];
-  const int2* ij[ESP_MAX_FORCE_SEGS];
-};
-void launch_contact_rows(hipStream_t s, int n, int stride, const int* off, const int* ent,
-                         const RecordLists& rl, int* cnt, int2* rows);
-void launch_contact_entries(hipStream_t s, int total, const int* inc_ent, const RecordLists& rl,
-                            int2* ent);
-void launch_max_int(hipStream_t s, int n, const int* a, int* out);
 void launch_wall_list(hipStream_t s, int ng, const int* mark, int* list, int* list_n);
 int gather_blocks(int n);
 
@@ -357,10 +344,11 @@ void launch_cells_fill(hipStream_t s, int n, const int* cell, const int* cell_st
                        int* cell_fill, int* cell_items);
 void launch_cells_sort(hipStream_t s, int ncell, const int* cell_start, int* cell_items);
 // candidate pairs from each particle in slot order, oriented (lower id, higher
-// id), keyed by the slot pair; flagged = getNewList
+// id), keyed by the slot pair; flagged = getNewList; cap: room of the output (pairs
+// beyond it are not written)
 void launch_pairs(hipStream_t s, int mode_emit, int flagged, PView p, GridParams g, double alpha,
                   const int* cell, const int* cell_start, const int* cell_items, int* cnt,
-                  const int* off, int* out_p, int* out_q, long long* out_key);
+                  const int* off, int cap, int* out_p, int* out_q, long long* out_key);
 void launch_clear_flag_bit(hipStream_t s, PView p, UpdState* st);
 // candidates of wall group w (any order): slots, flags, positions, initial
 // positions; *cnt counts all, the first cap are stored
@@ -389,6 +377,8 @@ void launch_servo_sums(hipStream_t s, PView p, const WallParam& W, int w, int do
 // a particle field packed in id order (order: slots by ascending id)
 void launch_pack_ordered(hipStream_t s, int n, const int* order, const double4* src, int width,
                          double* out);
+// out[0..3) = *a, *b, *c (out: host memory)
+void launch_report3(hipStream_t s, const int* a, const int* b, const int* c, int* out);
 // a[0..n) = v (a kernel, not a memset: safe under stream capture)
 void launch_fill_int(hipStream_t s, int n, int* a, int v);
 // erasure of particles outside the padded grid (NeighborTable::build):
@@ -411,15 +401,15 @@ void launch_pack_dyn(hipStream_t s, int nc, const int* keep, const int* off, con
                      const double4* ff, int2* oij, long long* okey, double4* off_);
 void launch_ed_mark(hipStream_t s, int nc, const int* cp, const int* cq, const long long* ckey,
                     ExclSet ex, const long long* okey, int nold, const int2* oij, PView p,
-                    double period, int* keep, int* src);
+                    double period, int* keep, int* src, const int* nc_dev = nullptr);
 // circular x: particles beyond an x end move to their image (position, old
 // position and, when kept, initial position)
 void launch_wrap_x(hipStream_t s, PView p, double x0, double period, double4* init);
 void launch_ne_mark(hipStream_t s, int nc, const int* cp, const int* cq, const int* id, ExclSet ex,
-                    int* keep);
+                    int* keep, const int* nc_dev = nullptr);
 void launch_pair_emit(hipStream_t s, int nc, const int* keep, const int* off, const int* cp,
                       const int* cq, const long long* ckey, const int* src, const double4* off_ff,
-                      int2* nij, long long* nkey, double4* nff);
+                      int cap, int2* nij, long long* nkey, double4* nff);
 void launch_filter_new(hipStream_t s, int nc, const int* cp, const int* cq, const int* id,
                        const long long* ckey, ExclSet ex, HashRef present, int check_present,
                        int* keep);
@@ -440,10 +430,10 @@ void launch_inc_count(hipStream_t s, int nc, const int2* ij, int* inc_cnt);
 // storage order); grp: the group's position in the summation order (< 32)
 void launch_inc_fill(hipStream_t s, int nc, const int2* ij, int rec_off, int has_m, const int* rank,
                      int grp, const int* inc_off, int* inc_fill, unsigned long long* ent64);
-void launch_inc_sort(hipStream_t s, int n, const int* inc_off, unsigned long long* ent64,
-                     int* inc_ent);
-// slot_of[record] = (CSR position on its first particle, on its second)
-void launch_slot_of(hipStream_t s, int total, const int* inc_ent, int2* slot_of);
+// the interactions' places in their particles' runs: slot_of (ent null) or ent
+void launch_inc_rank(hipStream_t s, int nc, const int2* ij, int rec_off, int has_m, const int* rank,
+                     int grp, const int* inc_off, const unsigned long long* ent64, int2* slot_of,
+                     int2* ent);
 
 // exclusive scan of n ints into out (out[n] = total); tmp sized by scan_tmp_size
 size_t scan_tmp_size(int n);

@@ -995,14 +995,15 @@ __global__ __launch_bounds__(BS) void k_contact_step(StepCtl ctl, PView p, Conta
   // loads that do not depend on others, together
   const double4 Pi = p.pos[pc];
   const unsigned fpi = p.flags[pc];
-  const int cnt = pi < p.n ? cl.cnt[pc] : 0;
   const double mass = p.old[pc].w;
-  // row entries of this lane: the pair at hand, the next one and the one after
-  // it, so that the next neighbour's position is on its way during a law
-  int2 e0 = make_int2(0, 0), e1 = e0;
-  if (sub < cl.width) e0 = cl.rows[(size_t)sub * cl.stride + pc];
-  if (G + sub < cl.width) e1 = cl.rows[(size_t)(G + sub) * cl.stride + pc];
+  const int a = cl.off[pc];
+  const int cnt = pi < p.n ? cl.off[pc + 1] - a : 0;
   if (step_skip(ctl)) return;  // the same for the whole block
+  // entries of this lane: the pair at hand, the next one and the one after it, so
+  // that the next neighbour's position is on its way during a law
+  int2 e0 = make_int2(0, 0), e1 = e0;
+  if (sub < cnt) e0 = cl.ent[a + sub];
+  if (G + sub < cnt) e1 = cl.ent[a + G + sub];
   const ContactSeg& g = cl.seg[0];
   dv3 F = wall_body_force<false, EXTRA>(gp, pc, fpi, xyz(Pi), Pi.w, mass, none);
   double4 Pj = Pi;
@@ -1012,7 +1013,7 @@ __global__ __launch_bounds__(BS) void k_contact_step(StepCtl ctl, PView p, Conta
     double4 Pn = Pj;
     int2 e2 = e1;
     if (k + G < cnt) Pn = p.pos[e1.x & 0x7fffffff];
-    if (k + 2 * G < cnt) e2 = cl.rows[(size_t)(k + 2 * G) * cl.stride + pc];
+    if (k + 2 * G < cnt) e2 = cl.ent[a + k + 2 * G];
     dv3 f = mk3(0.0, 0.0, 0.0);
     if (k < cnt) {  // CElasticInteraction::calcForces (ElasticInteraction.cpp:54-71)
       const bool second = e0.x < 0;
@@ -1237,45 +1238,6 @@ __global__ __launch_bounds__(BS, KIND ? 3 : 2) void k_contact_block(StepCtl ctl,
   step_tail<EXTRA>(ctl, gp, i, act, fl, P, md);
 }
 
-// rows[k * stride + i]: the k-th interaction of particle i in summation order:
-// the other particle (bit 31: i is the second of the pair) and the record
-__global__ void k_contact_rows(int n, int stride, const int* off, const int* ent, RecordLists rl,
-                               int* cnt, int2* rows)
-{
-  const int i = blockIdx.x * BS + threadIdx.x;
-  if (i >= n) return;
-  const int a = off[i], m = off[i + 1] - a;
-  cnt[i] = m;
-  for (int k = 0; k < m; k++) {
-    const int v = ent[a + k], rec = v >> 2;
-    int s = 0;
-    while (s + 1 < rl.count && rec >= rl.rec_off[s + 1]) s++;
-    const int2 e = rl.ij[s][rec - rl.rec_off[s]];
-    rows[(size_t)k * stride + i] =
-        (v & 1) ? make_int2(e.x | (int)0x80000000u, rec) : make_int2(e.y, rec);
-  }
-}
-
-// ent[off[i] + k]: the same entries in CSR order
-__global__ void k_contact_entries(int total, const int* inc_ent, RecordLists rl, int2* ent)
-{
-  const int t = blockIdx.x * BS + threadIdx.x;
-  if (t >= total) return;
-  const int v = inc_ent[t], rec = v >> 2;
-  int s = 0;
-  while (s + 1 < rl.count && rec >= rl.rec_off[s + 1]) s++;
-  const int2 e = rl.ij[s][rec - rl.rec_off[s]];
-  ent[t] = (v & 1) ? make_int2(e.x | (int)0x80000000u, rec) : make_int2(e.y, rec);
-}
-
-__global__ __launch_bounds__(BS) void k_max_int(int n, const int* a, int* out)
-{
-  const int i = blockIdx.x * BS + threadIdx.x;
-  int v = i < n ? a[i] : 0;
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  if ((threadIdx.x & 63) == 0 && v > 0) atomicMax(out, v);
-}
-
 // the 64-particle groups holding wall candidates, ascending (one block; marks
 // from k_wall_update)
 __global__ __launch_bounds__(1024) void k_wall_list(int ng, const int* mark, int* list, int* list_n)
@@ -1347,79 +1309,118 @@ __global__ void k_cells_sort(int ncell, const int* cell_start, int* items)
 }
 
 
-// Pairs of particle p (taken in ascending id order) with every particle q of
-// higher id in the 27 cells around p's cell: the full list keeps pairs with
-// |x_p - x_q|^2 <= (r_p + r_q + alpha)^2 (ntable.hpp:471-521); the flagged list
-// keeps pairs of two flagged particles without a distance test
-// (ntable.hpp:532-583).  The emit pass sorts each particle's run by the partner
-// id, so the whole list comes out sorted by (id1, id2).
-__global__ void k_pairs(int emit, int flagged, PView p, GridParams g, double alpha,
-                        const int* cell, const int* cell_start, const int* cell_items, int* cnt,
-                        const int* off, int* out_p, int* out_q, long long* out_key)
+// Pairs of particle p with every particle q of higher id in the 27 cells around
+// p's cell: the full list keeps pairs with |x_p - x_q|^2 <= (r_p + r_q + alpha)^2
+// (ntable.hpp:471-521); the flagged list keeps pairs of two flagged particles
+// without a distance test (ntable.hpp:532-583).  Two passes: the first counts,
+// the second writes each particle's run in the order of the partner's slot.
+//
+// 32 lanes search for one particle, a cell each (a single lane's chain of 27
+// cells took 57 us for 10,000 particles, all of it latency: 13 us so); the
+// second pass collects a particle's partners in LDS and places each by counting
+// the smaller ones.  Runs longer than PAIRS_CAP (wide size ranges with flagged
+// lists) are placed by a second look at the cells.
+#define PAIRS_CAP 192
+template <bool EMIT, bool FLAGGED>
+__global__ __launch_bounds__(BS) void k_pairs(PView p, GridParams g, double alpha, const int* cell,
+                                              const int* cell_start, const int* cell_items, int* cnt,
+                                              const int* off, int cap, int* out_p, int* out_q,
+                                              long long* out_key)
 {
-  const int k = blockIdx.x * BS + threadIdx.x;
-  if (k >= p.n) return;
-  const int pi = k;
-  if (flagged && !(p.flags[pi] & PF_FLAG)) {
-    if (!emit) cnt[k] = 0;
+  constexpr int L = 32, PPB = BS / L;
+  __shared__ int list[EMIT ? PPB * PAIRS_CAP : 1];
+  __shared__ int num[PPB];
+  const int grp = threadIdx.x / L, l = threadIdx.x % L;
+  const int pi = blockIdx.x * PPB + grp;
+  const bool on = pi < p.n && (!FLAGGED || (p.flags[pi] & PF_FLAG));
+  if (l == 0) num[grp] = 0;
+  __syncthreads();
+  int c2 = -1;  // this lane's cell
+  double4 P = make_double4(0.0, 0.0, 0.0, 0.0);
+  int idp = 0;
+  if (on && l < 27) {
+    const int c = cell[pi];
+    P = p.pos[pi];
+    idp = p.id[pi];
+    const int cx = c / (g.ny * g.nz);
+    const int rem = c - cx * (g.ny * g.nz);
+    const int cy = rem / g.nz;
+    int x = cx + l / 9 - 1;
+    const int y = cy + (l / 3) % 3 - 1, z = rem - cy * g.nz + l % 3 - 1;
+    // circular x: the stencil wraps (nx >= 3, so its cells are distinct)
+    if (g.circ_x) x = (x + g.nx) % g.nx;
+    if (x >= 0 && x < g.nx && y >= 0 && y < g.ny && z >= 0 && z < g.nz)
+      c2 = g.ny * g.nz * x + g.nz * y + z;
+  }
+  auto taken = [&](int q) {
+    if (p.id[q] <= idp) return false;
+    if (FLAGGED) return (p.flags[q] & PF_FLAG) != 0u;
+    const double4 Q = x_image(P, p.pos[q], g.period);
+    const dv3 d = sub3(xyz(P), xyz(Q));
+    const double dist2 = dot3(d, d);
+    const double dmax = P.w + Q.w + alpha;
+    return dist2 <= (dmax * dmax);
+  };
+  int count = 0;
+  if (c2 >= 0) {
+    const int t1 = cell_start[c2 + 1];
+    for (int t = cell_start[c2]; t < t1; t++) {
+      const int q = cell_items[t];
+      if (!taken(q)) continue;
+      if (EMIT) {
+        const int k = atomicAdd(&num[grp], 1);
+        if (k < PAIRS_CAP) list[grp * PAIRS_CAP + k] = q;
+      } else {
+        count++;
+      }
+    }
+  }
+  if (!EMIT) {
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) count += __shfl_xor(count, o, L);
+    if (l == 0 && pi < p.n) cnt[pi] = count;
     return;
   }
-  const int c = cell[pi];
-  const int cx = c / (g.ny * g.nz);
-  const int rem = c - cx * (g.ny * g.nz);
-  const int cy = rem / g.nz;
-  const int cz = rem - cy * g.nz;
-  const double4 P = p.pos[pi];
-  const int idp = p.id[pi];
-  const int base = emit ? off[k] : 0;
-  int count = 0;
-  // circular x: the stencil wraps (nx >= 3, so its cells are distinct)
-  const int x0 = g.circ_x ? cx - 1 : (cx > 0 ? cx - 1 : cx);
-  const int x1 = g.circ_x ? cx + 1 : (cx < g.nx - 1 ? cx + 1 : cx);
-  const int y0 = cy > 0 ? cy - 1 : cy, y1 = cy < g.ny - 1 ? cy + 1 : cy;
-  const int z0 = cz > 0 ? cz - 1 : cz, z1 = cz < g.nz - 1 ? cz + 1 : cz;
-  for (int xx = x0; xx <= x1; xx++)
-    for (int y = y0; y <= y1; y++)
-      for (int z = z0; z <= z1; z++) {
-        const int x = g.circ_x ? (xx + g.nx) % g.nx : xx;
-        const int c2 = g.ny * g.nz * x + g.nz * y + z;
-        const int t1 = cell_start[c2 + 1];
-        for (int t = cell_start[c2]; t < t1; t++) {
-          const int q = cell_items[t];
-          const int idq = p.id[q];
-          if (idq <= idp) continue;
-          if (flagged) {
-            if (!(p.flags[q] & PF_FLAG)) continue;
-          } else {
-            const double4 Q = x_image(P, p.pos[q], g.period);
-            const dv3 d = sub3(xyz(P), xyz(Q));
-            const double dist2 = dot3(d, d);
-            const double dmax = P.w + Q.w + alpha;
-            if (!(dist2 <= (dmax * dmax))) continue;
-          }
-          if (emit) {
-            out_p[base + count] = pi;
-            out_q[base + count] = q;
-            out_key[base + count] = pair_key(pi, q);
-          }
-          count++;
+  __syncthreads();
+  const int m = num[grp];
+  if (!on || m == 0) return;
+  const int base = off[pi];
+  auto put = [&](int q, int r) {
+    if (base + r >= cap) return;  // the caller sees the total and comes back with room
+    out_p[base + r] = pi;
+    out_q[base + r] = q;
+    out_key[base + r] = pair_key(pi, q);
+  };
+  const int* mine = list + grp * PAIRS_CAP;
+  if (m <= PAIRS_CAP) {
+    for (int e = l; e < m; e += L) {
+      const int q = mine[e];
+      int r = 0;
+      for (int k = 0; k < m; k++) r += mine[k] < q ? 1 : 0;
+      put(q, r);
+    }
+  } else if (c2 >= 0) {
+    // each of this lane's partners against those of every cell
+    const int t1 = cell_start[c2 + 1];
+    const int c = cell[pi];
+    const int cx = c / (g.ny * g.nz), cy = (c / g.nz) % g.ny, cz = c % g.nz;
+    for (int t = cell_start[c2]; t < t1; t++) {
+      const int q = cell_items[t];
+      if (!taken(q)) continue;
+      int r = 0;
+      for (int k = 0; k < 27; k++) {
+        int x = cx + k / 9 - 1;
+        const int y = cy + (k / 3) % 3 - 1, z = cz + k % 3 - 1;
+        if (g.circ_x) x = (x + g.nx) % g.nx;
+        if (x < 0 || x >= g.nx || y < 0 || y >= g.ny || z < 0 || z >= g.nz) continue;
+        const int c3 = g.ny * g.nz * x + g.nz * y + z;
+        for (int u = cell_start[c3]; u < cell_start[c3 + 1]; u++) {
+          const int o = cell_items[u];
+          if (o < q && taken(o)) r++;
         }
       }
-  if (!emit) {
-    cnt[k] = count;
-    return;
-  }
-  for (int i = base + 1; i < base + count; i++) {
-    const long long kv = out_key[i];
-    const int qv = out_q[i];
-    int j = i - 1;
-    while (j >= base && out_key[j] > kv) {
-      out_key[j + 1] = out_key[j];
-      out_q[j + 1] = out_q[j];
-      j--;
+      put(q, r);
     }
-    out_key[j + 1] = kv;
-    out_q[j + 1] = qv;
   }
 }
 
@@ -1638,12 +1639,18 @@ __device__ __forceinline__ int upper_bound_key(const long long* a, int n, long l
 // PIS_ED::update on a rebuilt table (pi_storage_ed.hpp:97-136): a candidate is
 // kept unless excluded; it inherits the history of the stored interaction with
 // the same key if that one is persistent (RotFricInteraction.cpp:345-351).
-__global__ void k_ed_mark(int nc, const int* cp, const int* cq, const long long* ckey, ExclSet ex,
+// nc_dev (nullable): the candidates there are, when only the device knows; nc is
+// then the room they have, and marks beyond them are zero
+__global__ void k_ed_mark(int nc, const int* nc_dev, const int* cp, const int* cq, const long long* ckey, ExclSet ex,
                           const long long* okey, int nold, const int2* oij, PView p, double period,
                           int* keep, int* src)
 {
   const int c = blockIdx.x * BS + threadIdx.x;
   if (c >= nc) return;
+  if (nc_dev && c >= *nc_dev) {
+    keep[c] = 0;
+    return;
+  }
   const long long key = ckey[c];
   if (rejected(ex, pair_key(p.id[cp[c]], p.id[cq[c]]), cp[c], cq[c])) {
     keep[c] = 0;
@@ -1664,19 +1671,23 @@ __global__ void k_ed_mark(int nc, const int* cp, const int* cq, const long long*
   src[c] = s;
 }
 
-__global__ void k_ne_mark(int nc, const int* cp, const int* cq, const int* id, ExclSet ex, int* keep)
+__global__ void k_ne_mark(int nc, const int* nc_dev, const int* cp, const int* cq, const int* id,
+                          ExclSet ex, int* keep)
 {
   const int c = blockIdx.x * BS + threadIdx.x;
-  if (c < nc) keep[c] = rejected(ex, pair_key(id[cp[c]], id[cq[c]]), cp[c], cq[c]) ? 0 : 1;
+  if (c >= nc) return;
+  if (nc_dev && c >= *nc_dev) keep[c] = 0;
+  else keep[c] = rejected(ex, pair_key(id[cp[c]], id[cq[c]]), cp[c], cq[c]) ? 0 : 1;
 }
 
 __global__ void k_pair_emit(int nc, const int* keep, const int* off, const int* cp, const int* cq,
-                            const long long* ckey, const int* src, const double4* off_ff,
+                            const long long* ckey, const int* src, const double4* off_ff, int cap,
                             int2* nij, long long* nkey, double4* nff)
 {
   const int c = blockIdx.x * BS + threadIdx.x;
   if (c >= nc || !keep[c]) return;
   const int w = off[c];
+  if (w >= cap) return;  // the caller sees the total and comes back with room
   nij[w] = make_int2(cp[c], cq[c]);
   nkey[w] = ckey[c];
   if (nff) {
@@ -1909,6 +1920,15 @@ __device__ void incremental_update(const StepCtl& ctl, const PView& p, const Upd
   }
   __syncthreads();
   const int nf = up.st->fcount;
+  // a cascade: four waves would take milliseconds over the flagged particles
+  // while the whole chip waits, the host path takes one
+  if (nf > ESP_FLAG_CAP) {
+    if (tid == 0) {
+      *ctl.reason = 2;
+      *ctl.halted = ctl.step_id;
+    }
+    return;
+  }
   // one wave per flagged particle; lane l scans half (l / 27) of the items of
   // neighbour cell l % 27, so the dependent loads of a cell scan run in parallel
   const int lane = tid & 63;
@@ -2190,59 +2210,32 @@ __global__ void k_inc_fill(int nc, const int2* ij, int rec_off, int has_m, const
   ent[off[e.y] + atomicAdd(&fill[e.y], 1)] = hi | v | 1u;
 }
 
-// Sorts each particle's run of CSR entries into summation order and keeps the
-// record references.  Runs of consecutive particles are contiguous, so a block
-// stages its 256 runs in LDS when they fit and each thread insertion-sorts its
-// own run there.
-#define INC_LDS 6144
-__global__ __launch_bounds__(BS) void k_inc_sort(int n, const int* off, unsigned long long* ent64,
-                                                 int* ent)
-{
-  __shared__ unsigned long long buf[INC_LDS];
-  const int p0 = blockIdx.x * BS;
-  const int p1 = min(p0 + BS, n);
-  const int base = off[p0], end = off[p1];
-  const int i = p0 + threadIdx.x;
-  if (end - base <= INC_LDS) {
-    for (int t = base + threadIdx.x; t < end; t += BS) buf[t - base] = ent64[t];
-    __syncthreads();
-    if (i < n) {
-      const int a = off[i] - base, b = off[i + 1] - base;
-      for (int s = a + 1; s < b; s++) {
-        const unsigned long long v = buf[s];
-        int j = s - 1;
-        while (j >= a && buf[j] > v) {
-          buf[j + 1] = buf[j];
-          j--;
-        }
-        buf[j + 1] = v;
-      }
-    }
-    __syncthreads();
-    for (int t = base + threadIdx.x; t < end; t += BS) ent[t] = (int)(unsigned)buf[t - base];
-    return;
-  }
-  if (i >= n) return;
-  const int a = off[i], b = off[i + 1];
-  for (int s = a + 1; s < b; s++) {
-    const unsigned long long v = ent64[s];
-    int j = s - 1;
-    while (j >= a && ent64[j] > v) {
-      ent64[j + 1] = ent64[j];
-      j--;
-    }
-    ent64[j + 1] = v;
-  }
-  for (int s = a; s < b; s++) ent[s] = (int)(unsigned)ent64[s];
-}
-
-__global__ void k_slot_of(int total, const int* ent, int2* slot_of)
+// Each interaction's place in its two particles' runs, in summation order: the
+// number of smaller entries of the run (the runs are short and shared by
+// neighbouring threads, so the reads stay in L1; sorting a run in one thread took
+// 0.8 ms where flagged pairs made runs of 200).  slot_of[record] = the two places;
+// with ent given, the places are filled instead: ent[place] = (the other
+// particle, bit 31: this one is the second; record).
+__global__ void k_inc_rank(int nc, const int2* ij, int rec_off, int has_m, const int* rank,
+                           unsigned long long grp, const int* off, const unsigned long long* ent64,
+                           int2* slot_of, int2* ent)
 {
   const int t = blockIdx.x * BS + threadIdx.x;
-  if (t >= total) return;
-  const int v = ent[t];
-  int* so = reinterpret_cast<int*>(slot_of + (v >> 2));
-  so[v & 1] = t;
+  const int c = t >> 1, side = t & 1;
+  if (c >= nc) return;
+  const int2 e = ij[c];
+  if (e.x < 0) return;
+  const unsigned v = ((unsigned)(rec_off + c) << 2) | ((unsigned)has_m << 1) | (unsigned)side;
+  const unsigned long long mine =
+      (grp << 59) | ((unsigned long long)(rank ? rank[c] : c) << 32) | v;
+  const int p = side ? e.y : e.x;
+  const int a = off[p], b = off[p + 1];
+  int r = a;
+  for (int k = a; k < b; k++) r += ent64[k] < mine ? 1 : 0;
+  if (ent)
+    ent[r] = make_int2(side ? (e.x | (int)0x80000000u) : e.y, rec_off + c);
+  else
+    reinterpret_cast<int*>(slot_of + rec_off + c)[side] = r;
 }
 
 // ---------------------------------------------------------------------------
@@ -2276,6 +2269,46 @@ __global__ __launch_bounds__(BS) void k_scan_local(const int* in, int nvalid, in
   if (bsum && threadIdx.x == BS - 1) bsum[blockIdx.x] = s[BS - 1];
 }
 
+// Short arrays in one block and one launch (three launches of 3.6 us each took
+// 13 us for 20,000 cells; this 5 us): tiles of 8 values a thread, the sums of a
+// wave by shuffles, the waves' and the tiles' through LDS.
+#define SCAN_ONE 32768
+__global__ __launch_bounds__(1024) void k_scan_one(const int* in, int nvalid, int* out, int m)
+{
+  constexpr int V = 8;
+  __shared__ int wsum[16];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  int carry = 0;
+  for (int b0 = 0; b0 < m; b0 += 1024 * V) {
+    const int base = b0 + t * V;
+    int v[V], acc = 0;
+#pragma unroll
+    for (int k = 0; k < V; k++) v[k] = base + k < nvalid ? in[base + k] : 0;
+#pragma unroll
+    for (int k = 0; k < V; k++) acc += v[k];
+    int inc = acc;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(inc, d, 64);
+      if (lane >= d) inc += u;
+    }
+    if (lane == 63) wsum[wv] = inc;
+    __syncthreads();
+    int run = carry + inc - acc, tile = 0;
+    for (int w = 0; w < 16; w++) {
+      if (w < wv) run += wsum[w];
+      tile += wsum[w];
+    }
+#pragma unroll
+    for (int k = 0; k < V; k++) {
+      if (base + k < m) out[base + k] = run;
+      run += v[k];
+    }
+    carry += tile;
+    __syncthreads();
+  }
+}
+
 __global__ void k_scan_add(int* out, int m, const int* boff)
 {
   const int idx = blockIdx.x * 4 * BS + threadIdx.x * 4;
@@ -2295,6 +2328,10 @@ size_t scan_tmp_size(int n) { return scan_tmp_rec((long long)n + 1) + 16; }
 
 static void scan_rec(hipStream_t s, const int* in, int nvalid, int* out, int m, int* tmp)
 {
+  if (m <= SCAN_ONE) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, in, nvalid, out, m);
+    return;
+  }
   const int nb = (m + 4 * BS - 1) / (4 * BS);
   int* bsum = nb > 1 ? tmp : nullptr;
   hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(BS), 0, s, in, nvalid, out, m, bsum);
@@ -2478,7 +2515,7 @@ bool launch_contact_step(hipStream_t s, StepCtl ctl, PView p, const ContactLaunc
 {
   if (p.n <= 0) return false;
   const bool extra = extra_forces(gp);
-  if (cl.rows) {
+  if (cl.count == 1 && cl.seg[0].kind == ESP_SEG_NROT_ELASTIC) {
     constexpr int G = ESP_G_EL;
     const dim3 g(nblk(p.n, BS / G));
     if (extra) contact_launch(k_contact_step<true, G>, g, s, ctl, p, cl, gp, ev_a, ev_b);
@@ -2494,26 +2531,6 @@ bool launch_contact_step(hipStream_t s, StepCtl ctl, PView p, const ContactLaunc
     else contact_launch(k_contact_block<false, 0>, g, s, ctl, p, cl, gp, ev_a, ev_b);
   }
   return true;
-}
-
-void launch_contact_entries(hipStream_t s, int total, const int* inc_ent, const RecordLists& rl,
-                            int2* ent)
-{
-  if (total <= 0) return;
-  hipLaunchKernelGGL(k_contact_entries, dim3(nblk(total)), dim3(BS), 0, s, total, inc_ent, rl, ent);
-}
-
-void launch_contact_rows(hipStream_t s, int n, int stride, const int* off, const int* ent,
-                         const RecordLists& rl, int* cnt, int2* rows)
-{
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_contact_rows, dim3(nblk(n)), dim3(BS), 0, s, n, stride, off, ent, rl, cnt, rows);
-}
-
-void launch_max_int(hipStream_t s, int n, const int* a, int* out)
-{
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_max_int, dim3(nblk(n)), dim3(BS), 0, s, n, a, out);
 }
 
 void launch_wall_list(hipStream_t s, int ng, const int* mark, int* list, int* list_n)
@@ -2544,11 +2561,21 @@ void launch_cells_sort(hipStream_t s, int ncell, const int* cell_start, int* cel
 
 void launch_pairs(hipStream_t s, int mode_emit, int flagged, PView p, GridParams g, double alpha,
                   const int* cell, const int* cell_start, const int* cell_items, int* cnt,
-                  const int* off, int* out_p, int* out_q, long long* out_key)
+                  const int* off, int cap, int* out_p, int* out_q, long long* out_key)
 {
   if (p.n <= 0) return;
-  hipLaunchKernelGGL(k_pairs, dim3(nblk(p.n)), dim3(BS), 0, s, mode_emit, flagged, p, g, alpha,
-                     cell, cell_start, cell_items, cnt, off, out_p, out_q, out_key);
+  const dim3 gr(nblk(p.n, BS / 32)), bl(BS);
+#define ESP_PAIRS(E, F)                                                                         \
+  hipLaunchKernelGGL((k_pairs<E, F>), gr, bl, 0, s, p, g, alpha, cell, cell_start, cell_items, \
+                     cnt, off, cap, out_p, out_q, out_key)
+  if (mode_emit) {
+    if (flagged) ESP_PAIRS(true, true);
+    else ESP_PAIRS(true, false);
+  } else {
+    if (flagged) ESP_PAIRS(false, true);
+    else ESP_PAIRS(false, false);
+  }
+#undef ESP_PAIRS
 }
 
 void launch_keep_cells(hipStream_t s, int n, const int* cell, int* keep)
@@ -2645,6 +2672,16 @@ void launch_wall_pack_ordered(hipStream_t s, int no, const int* ord_slot, const 
                      p, init, out);
 }
 
+__global__ void k_report3(const int* a, const int* b, const int* c, int* out)
+{
+  if (threadIdx.x < 3) out[threadIdx.x] = *(threadIdx.x == 0 ? a : threadIdx.x == 1 ? b : c);
+}
+
+void launch_report3(hipStream_t s, const int* a, const int* b, const int* c, int* out)
+{
+  hipLaunchKernelGGL(k_report3, dim3(1), dim3(64), 0, s, a, b, c, out);
+}
+
 void launch_fill_int(hipStream_t s, int n, int* a, int v)
 {
   if (n <= 0) return;
@@ -2658,10 +2695,10 @@ void launch_clear_flag_bit(hipStream_t s, PView p, UpdState* st)
 
 void launch_ed_mark(hipStream_t s, int nc, const int* cp, const int* cq, const long long* ckey,
                     ExclSet ex, const long long* okey, int nold, const int2* oij, PView p,
-                    double period, int* keep, int* src)
+                    double period, int* keep, int* src, const int* nc_dev)
 {
   if (nc <= 0) return;
-  hipLaunchKernelGGL(k_ed_mark, dim3(nblk(nc)), dim3(BS), 0, s, nc, cp, cq, ckey, ex, okey, nold,
+  hipLaunchKernelGGL(k_ed_mark, dim3(nblk(nc)), dim3(BS), 0, s, nc, nc_dev, cp, cq, ckey, ex, okey, nold,
                      oij, p, period, keep, src);
 }
 
@@ -2693,19 +2730,19 @@ void launch_wrap_x(hipStream_t s, PView p, double x0, double period, double4* in
 }
 
 void launch_ne_mark(hipStream_t s, int nc, const int* cp, const int* cq, const int* id, ExclSet ex,
-                    int* keep)
+                    int* keep, const int* nc_dev)
 {
   if (nc <= 0) return;
-  hipLaunchKernelGGL(k_ne_mark, dim3(nblk(nc)), dim3(BS), 0, s, nc, cp, cq, id, ex, keep);
+  hipLaunchKernelGGL(k_ne_mark, dim3(nblk(nc)), dim3(BS), 0, s, nc, nc_dev, cp, cq, id, ex, keep);
 }
 
 void launch_pair_emit(hipStream_t s, int nc, const int* keep, const int* off, const int* cp,
                       const int* cq, const long long* ckey, const int* src, const double4* off_ff,
-                      int2* nij, long long* nkey, double4* nff)
+                      int cap, int2* nij, long long* nkey, double4* nff)
 {
   if (nc <= 0) return;
   hipLaunchKernelGGL(k_pair_emit, dim3(nblk(nc)), dim3(BS), 0, s, nc, keep, off, cp, cq, ckey, src,
-                     off_ff, nij, nkey, nff);
+                     off_ff, cap, nij, nkey, nff);
 }
 
 void launch_filter_new(hipStream_t s, int nc, const int* cp, const int* cq, const int* id,
@@ -2768,15 +2805,11 @@ void launch_inc_fill(hipStream_t s, int nc, const int2* ij, int rec_off, int has
                      (unsigned long long)grp, inc_off, inc_fill, ent64);
 }
 
-void launch_slot_of(hipStream_t s, int total, const int* inc_ent, int2* slot_of)
+void launch_inc_rank(hipStream_t s, int nc, const int2* ij, int rec_off, int has_m, const int* rank,
+                     int grp, const int* inc_off, const unsigned long long* ent64, int2* slot_of,
+                     int2* ent)
 {
-  if (total <= 0) return;
-  hipLaunchKernelGGL(k_slot_of, dim3(nblk(total)), dim3(BS), 0, s, total, inc_ent, slot_of);
-}
-
-void launch_inc_sort(hipStream_t s, int n, const int* inc_off, unsigned long long* ent64,
-                     int* inc_ent)
-{
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_inc_sort, dim3(nblk(n)), dim3(BS), 0, s, n, inc_off, ent64, inc_ent);
+  if (nc <= 0) return;
+  hipLaunchKernelGGL(k_inc_rank, dim3(nblk(2ll * nc)), dim3(BS), 0, s, nc, ij, rec_off, has_m, rank,
+                     (unsigned long long)grp, inc_off, ent64, slot_of, ent);
 }
