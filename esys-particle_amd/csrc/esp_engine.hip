@@ -340,7 +340,7 @@ bool contact_mode(const esp_engine* e) { return e->bg.empty(); }
 // wall partials of one step
 int wall_blocks(const esp_engine* e)
 {
-  return contact_mode(e) ? contact_groups(e->n) : gather_blocks(e->n);
+  return e->ss == 9 ? gather_blocks(e->n) : contact_groups(e->n);
 }
 
 constexpr size_t kBatchHead = sizeof(BatchOut) / sizeof(double);

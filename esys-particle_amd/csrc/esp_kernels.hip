@@ -7,7 +7,7 @@
 //       into both particles' slots.  In a queued step block 0 meanwhile applies
 //       the previous step's bond breaks and appends the new pairs of the
 //       flagged particles (and computes their forces)
-//   k_gather_integrate
+//   k_gather_integrate (k_gather_stress where particle stresses are kept)
 //       one thread per particle: wall and body forces, then the records of its
 //       interactions in a fixed order (CSR), then the CParticle/CRotParticle
 //       first-order update and the max-displacement reduction; per-block
@@ -418,16 +418,40 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
   return v;
 }
 
-// Fixed-order sum of (a, b, c) over the block, valid in thread 0: xor butterfly
-// inside each wave (every lane ends with the same value; a + b == b + a), then
-// the waves in index order.  Every thread of the block must call it.
+// Sum over the wave in a fixed order, the same value in every lane: pairs within
+// the rows of 16 lanes by DPP (a few cycles a step where a shuffle through LDS
+// takes a hundred), then the four rows.  Every lane of the wave must be active.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
+{
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffll), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+__device__ __forceinline__ double wave_sum(double v)
+{
+  v = v + dpp_move<0xB1>(v);   // lanes 1,0,3,2 of every four
+  v = v + dpp_move<0x4E>(v);   // lanes 2,3,0,1
+  v = v + dpp_move<0x141>(v);  // mirrored within 8 lanes
+  v = v + dpp_move<0x140>(v);  // mirrored within 16 lanes
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
+}
+
+// Fixed-order sum of (a, b, c) over the block, valid in thread 0: within each
+// wave, then the waves in index order.  Every thread of the block must call it.
 __device__ __forceinline__ void block_sum3(double& a, double& b, double& c, double* lds)
 {
-  for (int o = 32; o > 0; o >>= 1) {
-    a = a + __shfl_xor(a, o, 64);
-    b = b + __shfl_xor(b, o, 64);
-    c = c + __shfl_xor(c, o, 64);
-  }
+  a = wave_sum(a);
+  b = wave_sum(b);
+  c = wave_sum(c);
   __syncthreads();  // lds free from the previous call
   if ((threadIdx.x & 63) == 0) {
     const int w = threadIdx.x >> 6;
@@ -604,14 +628,12 @@ __device__ __forceinline__ double damp_and_integrate(const PView& po, const Gath
   return dot3(d, d);
 }
 
-// STRESS: records carry contact points
-template <bool STRESS, bool EXTRA>
-__global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, GatherParams gp)
+// The gather of an engine that accumulates particle stresses: slots carry contact
+// points (9 doubles)
+template <bool EXTRA>
+__global__ __launch_bounds__(BS) void k_gather_stress(StepCtl ctl, PView p, GatherParams gp)
 {
-  constexpr int GATHER_CHUNK = STRESS ? 2 : 4;
-  constexpr int GATHER_CHUNK6 = 8;  // active slots fetched together (6-double slots)
-  constexpr int GATHER_WIN = 28;    // slots per activity-mask window (8 words with any offset)
-  static_assert(GATHER_WIN < 32 && GATHER_WIN % 4 == 0, "a window's mask fits 32 bits");
+  constexpr int GATHER_CHUNK = 2;
   double sg[3][3];
   for (int i = 0; i < 3; i++)
     for (int j = 0; j < 3; j++) sg[i][j] = 0.0;
@@ -648,7 +670,7 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
   }
   unsigned long long md = 0;
   if (act) {
-    dv3 F = wall_body_force<STRESS, EXTRA>(gp, i, flw, x0, r, O.w, sg);
+    dv3 F = wall_body_force<true, EXTRA>(gp, i, flw, x0, r, O.w, sg);
     dv3 M = mk3(0.0, 0.0, 0.0);
     // the particle's slots in summation order (its CSR run, then its appendix
     // slots), fetched GATHER_CHUNK at a time so their loads are in flight
@@ -657,88 +679,27 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
     // adding them changes nothing.
     const int nmain = e1 - e0;
     const int cnt = nmain + xcnt;
-    const int ss = STRESS ? 9 : 6;
-    if (!STRESS) {
-      // A zero slot (a contact apart) is skipped: adding +0 changes no sum.
-      // The activity bytes (0 or 1) of up to GATHER_WIN slots of the run come
-      // in as aligned 32-bit words in one round of loads and become a bit
-      // mask; the active slots then load GATHER_CHUNK6 at a time, in run order.
-      // 6-double slots are 16-byte aligned: three 16-byte loads each.
-      const unsigned* sw = reinterpret_cast<const unsigned*>(gp.sact);
-      for (int wb = 0; wb < cnt; wb += GATHER_WIN) {
-        unsigned mask = 0;
-        int base = 0;  // slot index of mask bit 0
-        if (wb < nmain) {
-          const int s0 = e0 + wb, nw = min(GATHER_WIN, nmain - wb), sh = s0 & 3;
-          unsigned wv[GATHER_WIN / 4 + 1];
-#pragma unroll
-          for (int k = 0; k <= GATHER_WIN / 4; k++) wv[k] = 4 * k < sh + nw ? sw[(s0 >> 2) + k] : 0u;
-          unsigned long long m = 0;
-#pragma unroll
-          for (int k = 0; k <= GATHER_WIN / 4; k++) {
-            const unsigned v = wv[k];
-            const unsigned long long m4 = (v & 1u) | ((v >> 7) & 2u) | ((v >> 14) & 4u) | ((v >> 21) & 8u);
-            m |= m4 << (4 * k);
-          }
-          mask = (unsigned)(m >> sh) & ((1u << nw) - 1u);  // nw <= GATHER_WIN < 32
-          base = s0;
-        } else {
-          // the appendix slots follow the run (at most ESP_XSLOTS of them)
-          for (int t = 0; t < xcnt; t++)
-            if (gp.sact[gp.xbase + ESP_XSLOTS * i + t]) mask |= 1u << t;
-          base = gp.xbase + ESP_XSLOTS * i;
-        }
-        while (mask) {
-          double2 qa[GATHER_CHUNK6], qb[GATHER_CHUNK6], qc[GATHER_CHUNK6];
-          int sl[GATHER_CHUNK6];
-          bool on[GATHER_CHUNK6];
-#pragma unroll
-          for (int k = 0; k < GATHER_CHUNK6; k++) {
-            on[k] = mask != 0;
-            sl[k] = base + (on[k] ? __builtin_ctz(mask) : 0);
-            mask &= mask - 1u;
-          }
-#pragma unroll
-          for (int k = 0; k < GATHER_CHUNK6; k++) {
-            if (on[k]) {
-              const double2* q = reinterpret_cast<const double2*>(gp.slots + 6 * (size_t)sl[k]);
-              qa[k] = q[0];
-              qb[k] = q[1];
-              qc[k] = q[2];
-            }
-          }
-#pragma unroll
-          for (int k = 0; k < GATHER_CHUNK6; k++) {
-            if (!on[k]) continue;
-            F = add3(F, mk3(qa[k].x, qa[k].y, qb[k].x));
-            M = add3(M, mk3(qb[k].y, qc[k].x, qc[k].y));
-          }
-        }
-        // the appendix starts its own window right after the run
-        if (wb < nmain && wb + GATHER_WIN >= nmain) wb = nmain - GATHER_WIN;
-      }
-    }
-    for (int b = 0; STRESS && b < cnt; b += GATHER_CHUNK) {
+    for (int b = 0; b < cnt; b += GATHER_CHUNK) {
       dv3 f[GATHER_CHUNK], m[GATHER_CHUNK], rl[GATHER_CHUNK];
 #pragma unroll
       for (int k = 0; k < GATHER_CHUNK; k++) {
         const int t = b + k;
         const int slot = t >= cnt ? 0 : t < nmain ? e0 + t : gp.xbase + ESP_XSLOTS * i + (t - nmain);
-        const double* q = gp.slots + (size_t)ss * slot;
+        const double* q = gp.slots + (size_t)9 * slot;
         f[k] = mk3(q[0], q[1], q[2]);
         m[k] = mk3(q[3], q[4], q[5]);
-        if (STRESS) rl[k] = mk3(q[6], q[7], q[8]);
+        rl[k] = mk3(q[6], q[7], q[8]);
       }
 #pragma unroll
       for (int k = 0; k < GATHER_CHUNK; k++) {
         if (b + k >= cnt) break;
         F = add3(F, f[k]);
-        if (STRESS) stress_add(sg, f[k], rl[k]);
+        stress_add(sg, f[k], rl[k]);
         M = add3(M, m[k]);
       }
     }
     md = (unsigned long long)__double_as_longlong(
-        damp_and_integrate<STRESS, EXTRA>(p, gp, i, fl, F, M, P, Vv, O, A, Q, sg));
+        damp_and_integrate<true, EXTRA>(p, gp, i, fl, F, M, P, Vv, O, A, Q, sg));
   }
   // max displacement: wave, then block, then one atomic per block
   md = wave_max_u64(md);
@@ -854,6 +815,17 @@ __device__ __forceinline__ double group_value(double v, int q)
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+// bits of the four lanes of a group of 4
+__device__ __forceinline__ unsigned long long group_or(unsigned long long v)
+{
+  int lo = (int)(v & 0xffffffffull), hi = (int)(v >> 32);
+  lo |= __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xf, 0xf, true);  // lanes 1,0,3,2
+  hi |= __builtin_amdgcn_mov_dpp(hi, 0xB1, 0xf, 0xf, true);
+  lo |= __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xf, 0xf, true);  // lanes 2,3,0,1
+  hi |= __builtin_amdgcn_mov_dpp(hi, 0x4E, 0xf, 0xf, true);
+  return ((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo;
+}
+
 // A RotFriction pair apart, as its first particle sees it: history cleared; once
 // both buffers hold zero (flag bit 2) nothing is written.
 __device__ __forceinline__ void clear_history(const ContactSeg& g, int c)
@@ -934,26 +906,27 @@ __device__ __forceinline__ void pair_share(const PView& p, const ContactLaunch& 
 // The end of a wave's step: whether a particle moved beyond verletDist/2, and the
 // wall forces on its 64 particles (flags fl, state before the step P) in a
 // fixed-order sum; waves without candidates are not in the list the sums are
-// taken over.
+// taken over (all: there is no list, they leave zeros).
 template <bool EXTRA>
 __device__ __forceinline__ void step_tail(const StepCtl& ctl, const GatherParams& gp, int i, bool act,
-                                          unsigned fl, double4 P, unsigned long long md)
+                                          unsigned fl, double4 P, unsigned long long md,
+                                          bool all = false)
 {
   const int lane = threadIdx.x & 63;
   if (__ballot(md > ctl.thresh)) {
     md = wave_max_u64(md);
     if (lane == 0) atomicMax(&ctl.cur->maxdisp2, md);
   }
-  if (gp.nwg > 0 && __ballot(act && ((fl >> PF_WALL_SHIFT) & 0xFFu) != 0u)) {
+  if (gp.nwg > 0 && __ballot(act)) {
     double* q = gp.wall_part + (size_t)(i >> 6) * gp.nwg * 3;
+    if (!__ballot(act && ((fl >> PF_WALL_SHIFT) & 0xFFu) != 0u)) {
+      if (all && lane < 3 * gp.nwg) q[lane] = 0.0;
+      return;
+    }
     for (int w = 0; w < gp.nwg; w++) {
-      dv3 sh = act ? wall_share<EXTRA>(gp, w, i, fl, xyz(P), P.w) : mk3(0.0, 0.0, 0.0);
-      for (int o = 32; o > 0; o >>= 1) {
-        sh.x = sh.x + __shfl_xor(sh.x, o, 64);
-        sh.y = sh.y + __shfl_xor(sh.y, o, 64);
-        sh.z = sh.z + __shfl_xor(sh.z, o, 64);
-      }
-      if (lane == 0) put3(q + 3 * w, sh);
+      const dv3 sh = act ? wall_share<EXTRA>(gp, w, i, fl, xyz(P), P.w) : mk3(0.0, 0.0, 0.0);
+      const dv3 tot = mk3(wave_sum(sh.x), wave_sum(sh.y), wave_sum(sh.z));
+      if (lane == 0) put3(q + 3 * w, tot);
     }
   }
 }
@@ -1236,6 +1209,224 @@ __global__ __launch_bounds__(BS, KIND ? 3 : 2) void k_contact_block(StepCtl ctl,
         po, gp, i, fl, F, M, P, sV[lane], sO[lane], sA[lane], sQ[lane], none));
   }
   step_tail<EXTRA>(ctl, gp, i, act, fl, P, md);
+}
+
+// The gather for 6-double slots: four lanes share a particle's slots.  A
+// block is 64 particles.  The activity bytes of a run come in as aligned words,
+// one a lane, 64 slots at a time, and become one bit mask that all four lanes
+// hold; each lane then loads every fourth active slot, and the shares are added
+// in slot order.  One lane for each of the particles (the first wave) integrates;
+// its state is on its way meanwhile.
+// With one lane a particle the run's words, then up to eight slots of 48 bytes,
+// were a chain in every lane: 9.0 us for 2,000 particles (13 us where flagged
+// pairs make runs of 200 slots), 15.4 us for 100,000.
+template <bool EXTRA>
+__global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, GatherParams gp)
+{
+  constexpr int G = 4, PB = BS / G;
+  __shared__ double sum[6 * PB];
+  double none[3][3];
+  const int t = threadIdx.x;
+  const int p0 = xcd_block(blockIdx.x, gridDim.x) * PB;
+  const int pi = p0 + t / G, sub = t % G;  // the particle whose slots it adds
+  const int pc = pi < p.n ? pi : 0;
+  const int i = p0 + t;  // the particle it integrates (t < PB)
+  const bool act = t < PB && i < p.n;
+  const int ii = act ? i : 0;
+  const int e0 = gp.inc_off[pc], e1 = gp.inc_off[pc + 1], xcnt = gp.xcnt[pc];
+  double4 P = make_double4(0.0, 0.0, 0.0, 0.0), V = P, O = P, A = P, Q = P;
+  unsigned fl = 0u;
+  if (t < PB) {
+    P = p.pos[ii];
+    fl = p.flags[ii];
+    V = p.vel[ii];
+    O = p.old[ii];
+    if (gp.rot) {
+      A = p.ang[ii];
+      Q = p.quat[ii];
+    }
+  }
+  const unsigned* sw = reinterpret_cast<const unsigned*>(gp.sact);
+  const int nmain = pi < p.n ? e1 - e0 : 0;
+  const int nx = pi < p.n ? xcnt : 0;
+  const int w0 = e0 >> 2, sh = e0 & 3;  // the run starts sh bytes into word w0
+  // words of the first 64 slots, and the appendix's activity
+  unsigned wd[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) wd[r] = 16 * r + 4 * sub < sh + nmain ? sw[w0 + 4 * r + sub] : 0u;
+  const unsigned ax = sub < nx ? gp.sact[gp.xbase + ESP_XSLOTS * pc + sub] : 0u;
+  if (step_skip(ctl)) return;  // the same for the whole block
+  // pairs appended by this step's incremental update are covered by the force
+  // blocks from the next step on
+  if (gp.n_app && blockIdx.x == 0 && t == 0) gp.n_app[1] = gp.n_app[0];
+  if (t < PB) {
+    if (act && gp.nwg > 0 && ctl.guarded && ctl.prev->nbroken > 0) {
+      // bonds broke in the previous step: the reference's updateInteractions
+      // re-Updates the wall groups (EWallInteractionGroup.hpp:57-82) before forces
+      fl = wall_membership(gp.grid, gp.nwg, gp.wall, P, fl);
+      p.flags[i] = fl;
+    }
+    const dv3 F = wall_body_force<false, EXTRA>(gp, ii, act ? fl : 0u, xyz(P), P.w, O.w, none);
+    put3(sum + 6 * t, F);
+  }
+  __syncthreads();
+  const double* s0 = sum + 6 * (t / G);
+  dv3 F = mk3(s0[0], s0[1], s0[2]), M = mk3(0.0, 0.0, 0.0);
+  auto add_active = [&](unsigned long long m, size_t base) {
+    for (int k = 0; k < sub; k++) m &= m - 1ull;  // this lane's first
+    while (__ballot(m != 0ull)) {
+      double2 qa = make_double2(0.0, 0.0), qb = qa, qc = qa;
+      if (m) {
+        const double2* q =
+            reinterpret_cast<const double2*>(gp.slots + 6 * (base + __builtin_ctzll(m)));
+        qa = q[0];
+        qb = q[1];
+        qc = q[2];
+        for (int k = 0; k < G; k++) m &= m - 1ull;
+      }
+#pragma unroll
+      for (int k = 0; k < G; k++) {
+        F = add3(F, mk3(group_value<G>(qa.x, k), group_value<G>(qa.y, k), group_value<G>(qb.x, k)));
+        M = add3(M, mk3(group_value<G>(qb.y, k), group_value<G>(qc.x, k), group_value<G>(qc.y, k)));
+      }
+    }
+  };
+  // 64 bytes of activity a turn, from the run's first aligned word
+  for (int b = 0; __ballot(b < sh + nmain); b += 64) {
+    unsigned long long m = 0ull;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const unsigned v = wd[r];
+      const unsigned m4 = (v & 1u) | ((v >> 7) & 2u) | ((v >> 14) & 4u) | ((v >> 21) & 8u);
+      m |= (unsigned long long)m4 << (16 * r + 4 * sub);
+      const int nb = b + 64 + 16 * r + 4 * sub;
+      wd[r] = nb < sh + nmain ? sw[w0 + (nb >> 2)] : 0u;
+    }
+    m = group_or(m);
+    const int lo = b == 0 ? sh : 0, hi = min(64, sh + nmain - b);
+    if (hi <= lo) m = 0ull;
+    else m &= (hi == 64 ? ~0ull : ((1ull << hi) - 1ull)) & (~0ull << lo);
+    add_active(m, (size_t)(4ll * w0 + b));
+  }
+  if (__ballot(nx > 0)) {
+    const unsigned long long m = group_or((unsigned long long)(ax ? 1u : 0u) << sub);
+    add_active(m, (size_t)gp.xbase + (size_t)ESP_XSLOTS * pc);
+  }
+  __syncthreads();  // the walls' forces have been read
+  if (sub == 0) {
+    double* o = sum + 6 * (t / G);
+    put3(o, F);
+    put3(o + 3, M);
+  }
+  __syncthreads();
+  if (t >= PB) return;
+  unsigned long long md = 0;
+  if (act) {
+    const double* o = sum + 6 * t;
+    md = (unsigned long long)__double_as_longlong(
+        damp_and_integrate<false, EXTRA>(p, gp, i, fl, mk3(o[0], o[1], o[2]), mk3(o[3], o[4], o[5]), P,
+                                         V, O, A, Q, none));
+  }
+  step_tail<EXTRA>(ctl, gp, i, act, fl, P, md, true);
+}
+
+// The same with one lane a particle, for particle counts that fill the chip by
+// themselves (four lanes then only add waves: 66 us against 80 us for 600,000
+// particles, equal at 100,000).  A run's activity bytes become a bit mask in one
+// round of loads, GATHER_WIN slots at a time, and the active slots load
+// GATHER_CHUNK together.
+template <bool EXTRA>
+__global__ __launch_bounds__(BS) void k_gather_wide(StepCtl ctl, PView p, GatherParams gp)
+{
+  constexpr int GATHER_CHUNK = 8;  // active slots fetched together
+  constexpr int GATHER_WIN = 28;   // slots per activity-mask window (8 words with any offset)
+  static_assert(GATHER_WIN < 32 && GATHER_WIN % 4 == 0, "a window's mask fits 32 bits");
+  double none[3][3];
+  if (step_skip(ctl)) return;
+  if (gp.n_app && blockIdx.x == 0 && threadIdx.x == 0) gp.n_app[1] = gp.n_app[0];
+  const int i = blockIdx.x * BS + threadIdx.x;
+  const bool act = i < p.n;
+  const int ii = act ? i : 0;
+  // every load that does not depend on another is issued here, together
+  const double4 P = p.pos[ii];
+  unsigned fl = p.flags[ii];
+  const double4 V = p.vel[ii];
+  const double4 O = p.old[ii];
+  const int e0 = gp.inc_off[ii], e1 = gp.inc_off[ii + 1];
+  const int xcnt = gp.xcnt[ii];
+  double4 A = make_double4(0.0, 0.0, 0.0, 0.0), Q = A;
+  if (gp.rot) {
+    A = p.ang[ii];
+    Q = p.quat[ii];
+  }
+  if (act && gp.nwg > 0 && ctl.guarded && ctl.prev->nbroken > 0) {
+    // as in k_gather_integrate
+    fl = wall_membership(gp.grid, gp.nwg, gp.wall, P, fl);
+    p.flags[i] = fl;
+  }
+  unsigned long long md = 0;
+  if (act) {
+    dv3 F = wall_body_force<false, EXTRA>(gp, i, fl, xyz(P), P.w, O.w, none);
+    dv3 M = mk3(0.0, 0.0, 0.0);
+    const int nmain = e1 - e0;
+    const int cnt = nmain + xcnt;
+    const unsigned* sw = reinterpret_cast<const unsigned*>(gp.sact);
+    for (int wb = 0; wb < cnt; wb += GATHER_WIN) {
+      unsigned mask = 0;
+      int base = 0;  // slot index of mask bit 0
+      if (wb < nmain) {
+        const int s0 = e0 + wb, nw = min(GATHER_WIN, nmain - wb), sh = s0 & 3;
+        unsigned wv[GATHER_WIN / 4 + 1];
+#pragma unroll
+        for (int k = 0; k <= GATHER_WIN / 4; k++) wv[k] = 4 * k < sh + nw ? sw[(s0 >> 2) + k] : 0u;
+        unsigned long long m = 0;
+#pragma unroll
+        for (int k = 0; k <= GATHER_WIN / 4; k++) {
+          const unsigned v = wv[k];
+          const unsigned long long m4 = (v & 1u) | ((v >> 7) & 2u) | ((v >> 14) & 4u) | ((v >> 21) & 8u);
+          m |= m4 << (4 * k);
+        }
+        mask = (unsigned)(m >> sh) & ((1u << nw) - 1u);  // nw <= GATHER_WIN < 32
+        base = s0;
+      } else {
+        // the appendix slots follow the run (at most ESP_XSLOTS of them)
+        for (int t = 0; t < xcnt; t++)
+          if (gp.sact[gp.xbase + ESP_XSLOTS * i + t]) mask |= 1u << t;
+        base = gp.xbase + ESP_XSLOTS * i;
+      }
+      while (mask) {
+        double2 qa[GATHER_CHUNK], qb[GATHER_CHUNK], qc[GATHER_CHUNK];
+        int sl[GATHER_CHUNK];
+        bool on[GATHER_CHUNK];
+#pragma unroll
+        for (int k = 0; k < GATHER_CHUNK; k++) {
+          on[k] = mask != 0;
+          sl[k] = base + (on[k] ? __builtin_ctz(mask) : 0);
+          mask &= mask - 1u;
+        }
+#pragma unroll
+        for (int k = 0; k < GATHER_CHUNK; k++) {
+          if (on[k]) {
+            const double2* q = reinterpret_cast<const double2*>(gp.slots + 6 * (size_t)sl[k]);
+            qa[k] = q[0];
+            qb[k] = q[1];
+            qc[k] = q[2];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < GATHER_CHUNK; k++) {
+          if (!on[k]) continue;
+          F = add3(F, mk3(qa[k].x, qa[k].y, qb[k].x));
+          M = add3(M, mk3(qb[k].y, qc[k].x, qc[k].y));
+        }
+      }
+      // the appendix starts its own window right after the run
+      if (wb < nmain && wb + GATHER_WIN >= nmain) wb = nmain - GATHER_WIN;
+    }
+    md = (unsigned long long)__double_as_longlong(
+        damp_and_integrate<false, EXTRA>(p, gp, i, fl, F, M, P, V, O, A, Q, none));
+  }
+  step_tail<EXTRA>(ctl, gp, i, act, fl, P, md, true);
 }
 
 // the 64-particle groups holding wall candidates, ascending (one block; marks
@@ -1528,14 +1719,12 @@ __global__ __launch_bounds__(BS) void k_servo_sums(PView p, WallParam W, int w, 
       gap = fmin(gap, dist - P.w);
     }
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    K = K + __shfl_xor(K, o, 64);
-    sx = sx + __shfl_xor(sx, o, 64);
-    sy = sy + __shfl_xor(sy, o, 64);
-    sz = sz + __shfl_xor(sz, o, 64);
-    cnt = cnt + __shfl_xor(cnt, o, 64);
-    gap = fmin(gap, __shfl_xor(gap, o, 64));
-  }
+  K = wave_sum(K);
+  sx = wave_sum(sx);
+  sy = wave_sum(sy);
+  sz = wave_sum(sz);
+  cnt = wave_sum(cnt);
+  for (int o = 32; o > 0; o >>= 1) gap = fmin(gap, __shfl_xor(gap, o, 64));
   if (lane == 0) {
     part[wv][0] = K;
     part[wv][1] = sx;
@@ -2269,43 +2458,35 @@ __global__ __launch_bounds__(BS) void k_scan_local(const int* in, int nvalid, in
   if (bsum && threadIdx.x == BS - 1) bsum[blockIdx.x] = s[BS - 1];
 }
 
-// Short arrays in one block and one launch (three launches of 3.6 us each took
-// 13 us for 20,000 cells; this 5 us): tiles of 8 values a thread, the sums of a
-// wave by shuffles, the waves' and the tiles' through LDS.
+// Short arrays in one block and one launch: V values a thread, all loaded at
+// once, the sums of a wave by shuffles, the waves' through LDS
 #define SCAN_ONE 32768
+template <int V>
 __global__ __launch_bounds__(1024) void k_scan_one(const int* in, int nvalid, int* out, int m)
 {
-  constexpr int V = 8;
   __shared__ int wsum[16];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  int carry = 0;
-  for (int b0 = 0; b0 < m; b0 += 1024 * V) {
-    const int base = b0 + t * V;
-    int v[V], acc = 0;
+  const int base = t * V;
+  int v[V], acc = 0;
 #pragma unroll
-    for (int k = 0; k < V; k++) v[k] = base + k < nvalid ? in[base + k] : 0;
+  for (int k = 0; k < V; k++) v[k] = base + k < nvalid ? in[base + k] : 0;
 #pragma unroll
-    for (int k = 0; k < V; k++) acc += v[k];
-    int inc = acc;
+  for (int k = 0; k < V; k++) acc += v[k];
+  int inc = acc;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int u = __shfl_up(inc, d, 64);
-      if (lane >= d) inc += u;
-    }
-    if (lane == 63) wsum[wv] = inc;
-    __syncthreads();
-    int run = carry + inc - acc, tile = 0;
-    for (int w = 0; w < 16; w++) {
-      if (w < wv) run += wsum[w];
-      tile += wsum[w];
-    }
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(inc, d, 64);
+    if (lane >= d) inc += u;
+  }
+  if (lane == 63) wsum[wv] = inc;
+  __syncthreads();
+  int run = inc - acc;
 #pragma unroll
-    for (int k = 0; k < V; k++) {
-      if (base + k < m) out[base + k] = run;
-      run += v[k];
-    }
-    carry += tile;
-    __syncthreads();
+  for (int w = 0; w < 16; w++) run += w < wv ? wsum[w] : 0;
+#pragma unroll
+  for (int k = 0; k < V; k++) {
+    if (base + k < m) out[base + k] = run;
+    run += v[k];
   }
 }
 
@@ -2329,7 +2510,10 @@ size_t scan_tmp_size(int n) { return scan_tmp_rec((long long)n + 1) + 16; }
 static void scan_rec(hipStream_t s, const int* in, int nvalid, int* out, int m, int* tmp)
 {
   if (m <= SCAN_ONE) {
-    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, in, nvalid, out, m);
+    if (m <= SCAN_ONE / 4)
+      hipLaunchKernelGGL(k_scan_one<8>, dim3(1), dim3(1024), 0, s, in, nvalid, out, m);
+    else
+      hipLaunchKernelGGL(k_scan_one<32>, dim3(1), dim3(1024), 0, s, in, nvalid, out, m);
     return;
   }
   const int nb = (m + 4 * BS - 1) / (4 * BS);
@@ -2426,30 +2610,41 @@ void launch_alive_flags(hipStream_t s, int nb, const int2* ij, int* keep)
   hipLaunchKernelGGL(k_alive_flags, dim3(nblk(nb)), dim3(BS), 0, s, nb, ij, keep);
 }
 
-static bool extra_forces(const GatherParams& gp);
-
-template <bool STRESS, bool EXTRA>
-static void gather_launch(hipStream_t s, StepCtl ctl, PView p, const GatherParams& gp,
-                          hipEvent_t ev_a, hipEvent_t ev_b)
+static bool extra_forces(const GatherParams& gp)
 {
-  const dim3 g(nblk(p.n)), b(BS);
-  if (ev_a && ev_b)
-    hipExtLaunchKernelGGL((k_gather_integrate<STRESS, EXTRA>), g, b, 0, s, ev_a, ev_b, 0, ctl, p, gp);
-  else
-    hipLaunchKernelGGL((k_gather_integrate<STRESS, EXTRA>), g, b, 0, s, ctl, p, gp);
+  bool extra = gp.ndamp > 0;
+  for (int w = 0; w < gp.nwg; w++) extra |= gp.wall[w].bonded != 0 || gp.wall[w].tagged != 0;
+  return extra;
 }
 
+template <class K>
+static void gather_launch(K kern, int blocks, hipStream_t s, StepCtl ctl, PView p,
+                          const GatherParams& gp, hipEvent_t ev_a, hipEvent_t ev_b)
+{
+  if (ev_a && ev_b)
+    hipExtLaunchKernelGGL(kern, dim3(blocks), dim3(BS), 0, s, ev_a, ev_b, 0, ctl, p, gp);
+  else
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(BS), 0, s, ctl, p, gp);
+}
+
+// above this many particles one lane a particle: both forms take the same time
+// at 100,000 (15.9 and 15.4 us); at 64,000 particles one lane each is one wave
+// for every SIMD of the chip
+#define GATHER_WIDE 65536
 bool launch_gather_integrate(hipStream_t s, StepCtl ctl, PView p, const GatherParams& gp,
                              hipEvent_t ev_a, hipEvent_t ev_b)
 {
   if (p.n <= 0) return false;
   const bool extra = extra_forces(gp);
   if (gp.sig) {
-    if (extra) gather_launch<true, true>(s, ctl, p, gp, ev_a, ev_b);
-    else gather_launch<true, false>(s, ctl, p, gp, ev_a, ev_b);
+    if (extra) gather_launch(k_gather_stress<true>, nblk(p.n), s, ctl, p, gp, ev_a, ev_b);
+    else gather_launch(k_gather_stress<false>, nblk(p.n), s, ctl, p, gp, ev_a, ev_b);
+  } else if (p.n > GATHER_WIDE) {
+    if (extra) gather_launch(k_gather_wide<true>, nblk(p.n), s, ctl, p, gp, ev_a, ev_b);
+    else gather_launch(k_gather_wide<false>, nblk(p.n), s, ctl, p, gp, ev_a, ev_b);
   } else {
-    if (extra) gather_launch<false, true>(s, ctl, p, gp, ev_a, ev_b);
-    else gather_launch<false, false>(s, ctl, p, gp, ev_a, ev_b);
+    if (extra) gather_launch(k_gather_integrate<true>, nblk(p.n, 64), s, ctl, p, gp, ev_a, ev_b);
+    else gather_launch(k_gather_integrate<false>, nblk(p.n, 64), s, ctl, p, gp, ev_a, ev_b);
   }
   return true;
 }
@@ -2499,13 +2694,6 @@ static void contact_launch(K kern, dim3 g, hipStream_t s, StepCtl ctl, PView p,
     hipExtLaunchKernelGGL(kern, g, dim3(BS), 0, s, ev_a, ev_b, 0, ctl, p, cl, gp);
   else
     hipLaunchKernelGGL(kern, g, dim3(BS), 0, s, ctl, p, cl, gp);
-}
-
-static bool extra_forces(const GatherParams& gp)
-{
-  bool extra = gp.ndamp > 0;
-  for (int w = 0; w < gp.nwg; w++) extra |= gp.wall[w].bonded != 0 || gp.wall[w].tagged != 0;
-  return extra;
 }
 
 int contact_groups(int n) { return nblk(n, 64); }
