@@ -3,33 +3,35 @@
 // Forward: the reference's time step for the calibration model class over one
 // particle set holding any number of specimens (per-specimen parameters),
 // with the main engine's neighbour-search kernels (cell binning, 27-cell pair
-// search) and three step kernels:
-//   k_bond_fwd    per bond: ARotBondedInteraction::calcForces + the break test
-//                 (the bond leaves at the next step)
-//   k_fric_fwd    per neighbour pair: RotFriction unless a live bond excludes
-//                 it; shear history read from one buffer, written to the other
+// search) and two launches a step:
+//   k_bond_fwd_pairs  per bond: ARotBondedInteraction::calcForces + the break
+//                 test (the bond leaves at the next step); per neighbour pair:
+//                 RotFriction unless a live bond excludes it, shear history read
+//                 from one buffer, written to the other
 //   k_gather_fwd  per particle: walls, gravity, then its interactions in a
 //                 fixed order (pairs by key, then bonds), the CParticle /
 //                 CRotParticle update, the rebuild test
 // plus a per-specimen, fixed-order sum of the measured wall's force at sample
-// steps.  Checkpoints every K steps keep the state, the shear histories and
-// the bond break steps; the neighbour lists ("epochs", one per rebuild) are
-// immutable and kept for the whole run.
+// steps.  The neighbour lists ("epochs", one per rebuild) are immutable and kept
+// for the whole run.
 //
-// Backward: segments in reverse order; each is recomputed forward from its
-// checkpoint (recorded epochs, no search) storing the state of every step,
-// then swept backwards:
-//   k_adj_particle  the integrator's adjoint (symplectic Euler, quaternion
-//                   step and normalisation), the walls' and the loss's terms
+// Every step writes its state next to the one before, so a run whose states and
+// shear histories fit kTapeBytes is its own tape.  A longer run keeps a checkpoint
+// every K steps (state, shear histories), and the reverse sweep recomputes one
+// segment's tape at a time (recorded epochs, no search).
+//
+// Backward, per step, three launches:
 //   k_adj_bond      vector-Jacobian product of the bond law (16 inputs), by
 //                   its hand-written reverse mode
 //   k_adj_fric      vector-Jacobian product of the friction law (24 inputs,
 //                   the history among them, on the recorded slip branch), by
 //                   its hand-written reverse mode
-//   k_adj_gather    per particle, the interactions' adjoints in a fixed order,
-//                   and the parameter gradients credited to the first particle
-// The laws' Jacobian columns come from their dual-number evaluation
-// (esp_difflaw.h); every reduction has a fixed order (no atomics on doubles).
+//   k_adj_step      per particle, the interactions' adjoints in a fixed order
+//                   and the parameter gradients credited to the first particle,
+//                   then the integrator's adjoint (symplectic Euler, quaternion
+//                   step and normalisation), the walls' and the loss's terms of
+//                   the step before
+// Every reduction has a fixed order (no atomics on doubles).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -46,12 +48,17 @@
 #include "esp_difflaw.h"
 #include "esp_internal.h"
 #include "esp_math.h"
+#include "esp_wave.h"
 
 namespace {
 
 struct DiffError : std::runtime_error {
   int code;
   DiffError(int c, const std::string& m) : std::runtime_error(m), code(c) {}
+};
+
+struct DiffMemory : DiffError {
+  explicit DiffMemory(const std::string& m) : DiffError(ESP_ERR_DEVICE, m) {}
 };
 
 #define DCHK(expr)                                                                       \
@@ -81,8 +88,20 @@ struct DevBuf {
     }
     p = nullptr;
     const size_t c = std::max<size_t>(n, 16);
-    DCHK(hipMalloc(&p, c * sizeof(T)));
+    cap = 0;
+    if (hipError_t e = hipMalloc(&p, c * sizeof(T)); e != hipSuccess) {
+      p = nullptr;
+      if (e != hipErrorOutOfMemory) DCHK(e);
+      (void)hipGetLastError();
+      throw DiffMemory(std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     cap = c;
+  }
+  void release()
+  {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    cap = 0;
   }
   void swap(DevBuf& o)
   {
@@ -141,31 +160,19 @@ struct DStep {
   double g[3];
   double dt;
   int step;
-  const double* wo;  // wall origins per step [step][wall][3] (forward), or wall[].o
 };
 
-__device__ __forceinline__ dv3 wall_origin(const DStep& sp, int k, int step)
-{
-  if (sp.wo) {
-    const double* o = sp.wo + ((size_t)step * sp.nw + k) * 3;
-    return mk3(o[0], o[1], o[2]);
-  }
-  return mk3(sp.wall[k].o[0], sp.wall[k].o[1], sp.wall[k].o[2]);
-}
-
-// Device-driven stepping: the kernels of a forward step read the step they
-// belong to from `step`; a step whose displacement test asks for a neighbour
-// search records itself in `halt`, and every later step of the queue (or of a
-// replayed graph) returns at once; steps past `end` return too.
+// Steps are queued without host decisions: a step whose displacement test asks
+// for a neighbour search records itself in `halt`, and every later step of the
+// queue returns at once.
 struct DRun {
-  int step, halt, end, pad;
+  int halt, pad;
 };
 
-__device__ __forceinline__ bool run_skip(const DRun* R, int& step)
+__device__ __forceinline__ bool run_skip(const DRun* R, int step)
 {
-  step = R->step;
   const int h = R->halt;
-  return step > R->end || (h != 0 && h < step);
+  return h != 0 && h < step;
 }
 
 // Largest block of the per-step kernels.  The law kernels declare it as their
@@ -173,21 +180,9 @@ __device__ __forceinline__ bool run_skip(const DRun* R, int& step)
 // threads caps them at 128, and the bond law then spills to scratch memory).
 #define DIFF_MAX_BS 512
 
-__global__ void k_set_run(DRun* R, int step, int halt, int end)
+__global__ void k_clear_run(DRun* R)
 {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    R->step = step;
-    R->halt = halt;
-    R->end = end;
-  }
-}
-
-// the last launch of a step
-__global__ void k_advance(DRun* R)
-{
-  int step;
-  if (blockIdx.x != 0 || threadIdx.x != 0 || run_skip(R, step)) return;
-  R->step = step + 1;
+  if (blockIdx.x == 0 && threadIdx.x == 0) R->halt = 0;
 }
 
 struct DBonds {
@@ -230,9 +225,8 @@ __device__ __forceinline__ tquat<esp_dual> ddq(double4 a, double4 t)
 }
 
 __global__ __launch_bounds__(DIFF_MAX_BS) void k_bond_tan(DState S, DTan T, DBonds B, const double4* theta, const double4* dtheta,
-                           const DRun* run, double* bt)
+                           const DRun* run, int step, double* bt)
 {
-  int step;
   if (run_skip(run, step)) return;
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= B.nb) return;
@@ -262,9 +256,8 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_bond_tan(DState S, DTan T, DBon
 
 __global__ __launch_bounds__(DIFF_MAX_BS) void k_fric_tan(DState S, DTan T, DCands C, const int* bstep, const double4* theta,
                            const double4* dtheta, const double4* H0, const double4* H1,
-                           double4* TH0, double4* TH1, const DRun* run, double dt, double* ct)
+                           double4* TH0, double4* TH1, const DRun* run, int step, double dt, double* ct)
 {
-  int step;
   if (run_skip(run, step)) return;
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= C.nc) return;
@@ -301,11 +294,9 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_fric_tan(DState S, DTan T, DCan
 // ---------------------------------------------------------------------------
 // forward kernels
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(DIFF_MAX_BS) void k_bond_fwd(DState S, DBonds B, const double4* theta, const DRun* run, double* bout)
+__device__ __forceinline__ void bond_fwd_item(const DState& S, const DBonds& B, const double4* theta,
+                                              int step, int b, double* bout)
 {
-  int step;
-  if (run_skip(run, step)) return;
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= B.nb) return;
   double* o = bout + 9 * (size_t)b;
   const int bs = B.bstep[b];
@@ -344,14 +335,14 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_bond_fwd(DState S, DBonds B, co
 // History flag bits (w of a history): 1 slipping, 2 touching, 4 zero in both
 // buffers (the pair has been apart for at least the last step, so neither
 // buffer needs writing until it touches).  act[c]: the record of pair c holds
-// this step's (nonzero) force; the gathers read only such records.
-__global__ void k_fric_fwd(DState S, DCands C, const int* bstep, const double4* theta,
-                           double4* H0, double4* H1, const DRun* run, double dt, double* cout,
-                           unsigned char* act, unsigned long long* dig_base)
+// this step's (nonzero) force; the gathers read only such records.  htape
+// (nullable): the histories touching pairs read, kept for the reverse sweep.
+__device__ __forceinline__ void fric_fwd_item(const DState& S, const DCands& C, const int* bstep,
+                                              const double4* theta, double4* H0, double4* H1,
+                                              double4* htape, int step, double dt, int c,
+                                              double* cout, unsigned char* act,
+                                              unsigned long long* dig_base)
 {
-  int step;
-  if (run_skip(run, step)) return;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= C.nc) return;
   // step s reads the histories of buffer s & 1 and writes the other
   double4* hin = (step & 1) ? H1 : H0;
@@ -359,11 +350,10 @@ __global__ void k_fric_fwd(DState S, DCands C, const int* bstep, const double4* 
   unsigned long long* dig = dig_base ? dig_base + step : nullptr;
   const int bb = C.bond[c];
   if (bb >= 0 && bstep[bb] >= step) {
-    // excluded while the bond lives: no record, and no history is read until
-    // the step after its break, which reads the zero history written here at
-    // the break step
+    // excluded while the bond lives (a break found by this launch's bonds sets
+    // bstep to step: excluded still): no record.  Its history is the zero it
+    // starts with, in both buffers.
     act[c] = 0;
-    if (bstep[bb] == step) hout[c] = make_double4(0.0, 0.0, 0.0, 0.0);
     return;
   }
   const int2 e = C.ij[c];
@@ -401,6 +391,7 @@ __global__ void k_fric_fwd(DState S, DCands C, const int* bstep, const double4* 
     return;
   }
   double* o = cout + 9 * (size_t)c;
+  if (htape) htape[c] = h;
   hout[c] = make_double4(ffr.x, ffr.y, ffr.z, (double)((slipping ? 1 : 0) | 2));
   o[0] = f1.x; o[1] = f1.y; o[2] = f1.z;
   o[3] = m1.x; o[4] = m1.y; o[5] = m1.z;
@@ -408,116 +399,159 @@ __global__ void k_fric_fwd(DState S, DCands C, const int* bstep, const double4* 
   act[c] = 1;
 }
 
-// per particle: the measured wall's normal force on it (sample steps), walls,
-// gravity, interactions in CSR order, then the update (integrate = 1) or only
-// the total force and moment (integrate = 0 writes fm)
-__global__ void k_gather_fwd(DState S, const double4* mass_old, const int* inc_off,
-                             const int* inc_ent, int ncand, const double* cout, const double* bout,
-                             const unsigned char* cact, const int* bstep, DStep sp, int every,
-                             double* wfn_s, DRun* run, unsigned long long thresh,
-                             unsigned long long* dig_base, DTan T, const double* ct,
-                             const double* bt, double* wft_s)
+// The force laws of one step: blocks [0, nbb) take the bonds, the others the
+// candidate pairs, so the two laws' latencies overlap in one launch.
+__global__ __launch_bounds__(DIFF_MAX_BS) void k_bond_fwd_pairs(DState S, DBonds B, DCands C,
+                                                            const double4* theta, double4* H0,
+                                                            double4* H1, double4* htape,
+                                                            const DRun* run, int step, double dt,
+                                                            int nbb, double* bout, double* cout,
+                                                            unsigned char* act,
+                                                            unsigned long long* dig_base)
 {
-  int step;
   if (run_skip(run, step)) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= S.n) return;
-  const bool sample = every > 0 && step % every == 0;
-  double* wfn = sample ? wfn_s : nullptr;
-  double* wft = sample ? wft_s : nullptr;
+  if ((int)blockIdx.x < nbb)
+    bond_fwd_item(S, B, theta, step, blockIdx.x * blockDim.x + threadIdx.x, bout);
+  else
+    fric_fwd_item(S, C, B.bstep, theta, H0, H1, htape, step, dt,
+                  ((int)blockIdx.x - nbb) * (int)blockDim.x + (int)threadIdx.x, cout, act, dig_base);
+}
+
+// per particle: the measured wall's normal force on it (sample steps), walls,
+// gravity, interactions in CSR order, then the update from S into So (the same
+// arrays, or the next step's of a tape).
+// Bound by the chain entry -> activity -> record over a particle's run.  Four
+// lanes share a particle: each takes every fourth entry, two at a time, and the
+// shares are added in entry order by all of them; the block's first threads, one
+// for each of its particles, integrate.  Against one lane a particle (us a step):
+// 2,000 particles 22.0 -> 11.0, 20,000 26.6 -> 12.4, 24 specimens together
+// (230,000) 55.0 -> 49.1, so there is no size to go back to one lane.  TAN: the
+// state's tangent is carried along.
+template <bool TAN>
+__global__ __launch_bounds__(DIFF_MAX_BS) void k_gather_fwd(
+    DState S, DState So, const double4* mass_old, const int* inc_off, const int* inc_ent, int ncand,
+    const double* cout, const double* bout, const unsigned char* cact, const int* bstep, DStep sp,
+    double* wfn, DRun* run, unsigned long long thresh, unsigned long long* dig_base, DTan T,
+    const double* ct, const double* bt, double* wft)
+{
+  constexpr int NS = TAN ? 12 : 6;
+  constexpr int G = 4;
+  constexpr int R = 2;  // entries a lane has in flight
+  __shared__ double sum[NS * (DIFF_MAX_BS / G)];  // [particle][component]
+  const int step = sp.step;
+  const int t = threadIdx.x;
+  const int PB = blockDim.x / G;  // particles per block
+  const int p0 = blockIdx.x * PB;
+  const int pi = p0 + t / G, sub = t % G;  // the particle whose entries it adds
+  const int pc = pi < S.n ? pi : 0;
+  const int i = p0 + t;  // the particle it integrates (t < PB)
+  const bool own = t < PB && i < S.n;
+  const int e0 = inc_off[pc];
+  const int e1 = pi < S.n ? inc_off[pc + 1] : e0;
+  if (run_skip(run, step)) return;  // the same for the whole block
   unsigned long long* dig = dig_base ? dig_base + step : nullptr;
-  const double4 P = S.x[i];
-  const dv3 x0 = mk3(P.x, P.y, P.z);
-  const double r = P.w;
-  dv3 F = mk3(0.0, 0.0, 0.0), M = mk3(0.0, 0.0, 0.0);
-  dv3 tF = mk3(0.0, 0.0, 0.0), tM = mk3(0.0, 0.0, 0.0);  // tangents (T.x set)
-  double wn = 0.0, twn = 0.0;
-  for (int k = 0; k < sp.nw; k++) {  // CElasticWallInteraction::calcForces
-    const DWall& W = sp.wall[k];
-    const dv3 n = mk3(W.n[0], W.n[1], W.n[2]);
-    const double dist = dot3(sub3(x0, wall_origin(sp, k, step)), n);
-    if (dig) wave_digest(dig, ((unsigned long long)(i & ~63) << 3) | (unsigned long long)(k + 1),
-                         __ballot(dist < r), 0ull);
-    if (dist < r) {
-      double f = 1.0;
-      f *= 3.141592654 * r;
-      const dv3 force = mul3(n, (f * W.k) * (r - dist));
-      F = add3(F, force);
-      if (W.measure) wn = dot3(force, n);
-      if (T.x) {  // d force = -k' n (n . dx)
-        const double4 Tx = T.x[i];
-        const dv3 tf = mul3(n, -((f * W.k) * dot3(n, mk3(Tx.x, Tx.y, Tx.z))));
-        tF = add3(tF, tf);
-        if (W.measure) twn = dot3(tf, n);
-      }
-    }
-  }
-  if (wfn) wfn[i] = wn;
-  if (wft) wft[i] = twn;
-  const double4 Om = mass_old[i];
-  if (sp.has_g) F = add3(F, mul3(mk3(sp.g[0], sp.g[1], sp.g[2]), Om.w));
-  // The interactions in CSR order.  Up to GATHER_FWD_RUN entries of the run
-  // load their record references together, then their activity together, then
-  // the records of each chunk of GATHER_FWD_CH entries that holds an active one
-  // (bonds, which are nearly all active, sit at the end of a particle's run);
-  // the sums stay sequential.  A record with no force this step (a pair apart
-  // or excluded by its bond, a bond broken in an earlier step) is skipped: it
-  // would add zeros, and a sum that starts at +0 is not changed by a zero.
-  constexpr int GATHER_FWD_RUN = 8, GATHER_FWD_CH = 4;
-  const int e0 = inc_off[i], e1 = inc_off[i + 1];
-  for (int r0 = e0; r0 < e1; r0 += GATHER_FWD_RUN) {
-    int ent[GATHER_FWD_RUN];
-#pragma unroll
-    for (int k = 0; k < GATHER_FWD_RUN; k++) ent[k] = r0 + k < e1 ? inc_ent[r0 + k] : -1;
-    unsigned act = 0;
-#pragma unroll
-    for (int k = 0; k < GATHER_FWD_RUN; k++) {
-      const int rec = ent[k] >> 1;
-      const bool on =
-          ent[k] >= 0 && (rec < ncand ? cact[rec] != 0 : bstep[rec - ncand] >= step);
-      act |= (on ? 1u : 0u) << k;
-    }
-#pragma unroll
-    for (int c0 = 0; c0 < GATHER_FWD_RUN; c0 += GATHER_FWD_CH) {
-      if (!((act >> c0) & ((1u << GATHER_FWD_CH) - 1u))) continue;
-      dv3 f[GATHER_FWD_CH], m[GATHER_FWD_CH];
-#pragma unroll
-      for (int k = 0; k < GATHER_FWD_CH; k++) {
-        if (!((act >> (c0 + k)) & 1u)) continue;
-        const int rec = ent[c0 + k] >> 1, side = ent[c0 + k] & 1;
-        const double* q = rec < ncand ? cout + 9 * (size_t)rec : bout + 9 * (size_t)(rec - ncand);
-        f[k] = mk3(q[0], q[1], q[2]);
-        m[k] = side == 0 ? mk3(q[3], q[4], q[5]) : mk3(q[6], q[7], q[8]);
-      }
-#pragma unroll
-      for (int k = 0; k < GATHER_FWD_CH; k++) {
-        if (!((act >> (c0 + k)) & 1u)) continue;
-        if ((ent[c0 + k] & 1) == 0) F = add3(F, f[k]);
-        else F = add3(F, mk3(-f[k].x, -f[k].y, -f[k].z));
-        M = add3(M, m[k]);
-      }
-      if (T.x) {
-#pragma unroll
-        for (int k = 0; k < GATHER_FWD_CH; k++) {
-          if (!((act >> (c0 + k)) & 1u)) continue;
-          const int rec = ent[c0 + k] >> 1, side = ent[c0 + k] & 1;
-          const double* u = rec < ncand ? ct + 9 * (size_t)rec : bt + 9 * (size_t)(rec - ncand);
-          if (side == 0) {
-            tF = add3(tF, mk3(u[0], u[1], u[2]));
-            tM = add3(tM, mk3(u[3], u[4], u[5]));
-          } else {
-            tF = sub3(tF, mk3(u[0], u[1], u[2]));
-            tM = add3(tM, mk3(u[6], u[7], u[8]));
-          }
+  double4 P = make_double4(0.0, 0.0, 0.0, 0.0), Om = P, Vv = P, A = P, Q = P;
+  if (own) {
+    P = S.x[i];
+    Om = mass_old[i];
+    Vv = S.v[i];
+    A = S.w[i];
+    Q = S.q[i];
+    const dv3 x0 = mk3(P.x, P.y, P.z);
+    const double r = P.w;
+    dv3 F = mk3(0.0, 0.0, 0.0), tF = F;
+    double wn = 0.0, twn = 0.0;
+    for (int k = 0; k < sp.nw; k++) {  // CElasticWallInteraction::calcForces
+      const DWall& W = sp.wall[k];
+      const dv3 n = mk3(W.n[0], W.n[1], W.n[2]);
+      const double dist = dot3(sub3(x0, mk3(W.o[0], W.o[1], W.o[2])), n);
+      if (dig) wave_digest(dig, ((unsigned long long)(i - (t & 63)) << 3) | (unsigned long long)(k + 1),
+                           __ballot(dist < r), 0ull);
+      if (dist < r) {
+        double f = 1.0;
+        f *= 3.141592654 * r;
+        const dv3 force = mul3(n, (f * W.k) * (r - dist));
+        F = add3(F, force);
+        if (W.measure) wn = dot3(force, n);
+        if (TAN) {  // d force = -k' n (n . dx)
+          const double4 Tx = T.x[i];
+          const dv3 tf = mul3(n, -((f * W.k) * dot3(n, mk3(Tx.x, Tx.y, Tx.z))));
+          tF = add3(tF, tf);
+          if (W.measure) twn = dot3(tf, n);
         }
       }
     }
+    if (wfn) wfn[i] = wn;
+    if (TAN && wft) wft[i] = twn;
+    if (sp.has_g) F = add3(F, mul3(mk3(sp.g[0], sp.g[1], sp.g[2]), Om.w));
+    double* o = sum + NS * t;
+    o[0] = F.x; o[1] = F.y; o[2] = F.z;
+    if (TAN) {
+      o[6] = tF.x; o[7] = tF.y; o[8] = tF.z;
+    }
   }
+  __syncthreads();
+  double acc[NS];
+  {
+    const double* o = sum + NS * (t / G);
+    for (int c = 0; c < NS; c++) acc[c] = (c < 3 || (c >= 6 && c < 9)) ? o[c] : 0.0;
+  }
+  // The interactions in CSR order.  A record with no force this step (a pair
+  // apart or excluded by its bond, a bond broken in an earlier step) adds zeros:
+  // a sum that starts at +0 is not changed by a zero.
+  int ent[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) ent[r] = e0 + r * G + sub < e1 ? inc_ent[e0 + r * G + sub] : -1;
+  for (int b = e0; b < e1; b += R * G) {  // as often for the G lanes of a particle
+    bool on[R];
+    double v[R][NS];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int rec = ent[r] >> 1;
+      on[r] = ent[r] >= 0 && (rec < ncand ? cact[rec] != 0 : bstep[rec - ncand] >= step);
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      for (int c = 0; c < NS; c++) v[r][c] = 0.0;
+      if (!on[r]) continue;
+      const int rec = ent[r] >> 1, side = ent[r] & 1;
+      const size_t at = 9 * (size_t)(rec < ncand ? rec : rec - ncand);
+      const double* q = (rec < ncand ? cout : bout) + at;
+      const double* qm = q + 3 + 3 * side;
+      const double sg = side ? -1.0 : 1.0;  // the second particle's force is the opposite
+      v[r][0] = sg * q[0]; v[r][1] = sg * q[1]; v[r][2] = sg * q[2];
+      v[r][3] = qm[0]; v[r][4] = qm[1]; v[r][5] = qm[2];
+      if (TAN) {
+        const double* u = (rec < ncand ? ct : bt) + at;
+        const double* um = u + 3 + 3 * side;
+        v[r][6] = sg * u[0]; v[r][7] = sg * u[1]; v[r][8] = sg * u[2];
+        v[r][9] = um[0]; v[r][10] = um[1]; v[r][11] = um[2];
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int nx = b + (R + r) * G + sub;
+      ent[r] = nx < e1 ? inc_ent[nx] : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int k = 0; k < G; k++)
+        for (int c = 0; c < NS; c++)
+          acc[c] = acc[c] + group_value<G>(v[r][c], k);
+    }
+  }
+  __syncthreads();  // the walls' forces have been read
+  if (sub == 0)
+    for (int c = 0; c < NS; c++) sum[NS * (t / G) + c] = acc[c];
+  __syncthreads();
+  if (!own) return;
+  for (int c = 0; c < NS; c++) acc[c] = sum[NS * t + c];
+  const dv3 F = mk3(acc[0], acc[1], acc[2]), M = mk3(acc[3], acc[4], acc[5]);
   // CRotParticle::integrate + rescale, CParticle::integrate (RotParticle.cpp:
-  // 277-321, Particle.cpp:257-274), the expression order of k_gather_integrate
+  // 277-321, Particle.cpp:257-274), the expression order of the plain engine
   const double dt = sp.dt;
-  const double4 Vv = S.v[i], A = S.w[i], Q = S.q[i];
-  dv3 v = mk3(Vv.x, Vv.y, Vv.z), x = x0;
+  dv3 v = mk3(Vv.x, Vv.y, Vv.z), x = mk3(P.x, P.y, P.z);
   dv3 w = mk3(A.x, A.y, A.z);
   dquat qq = dquat{Q.x, mk3(Q.y, Q.z, Q.w)};
   w = add3(w, mul3(M, dt * A.w));
@@ -533,7 +567,8 @@ __global__ void k_gather_fwd(DState S, const double4* mass_old, const int* inc_o
     qq.s = inverse * qq.s;
     qq.v = mul3(qq.v, inverse);
   }
-  if (T.x) {
+  if (TAN) {
+    const dv3 tF = mk3(acc[6], acc[7], acc[8]), tM = mk3(acc[9], acc[10], acc[11]);
     // tangents of w1 = w + M dt/I, qt = q + h (0, w1) q, q1 = qt/|qt|,
     // v1 = v + F dt/m, x1 = x + v1 dt (q0, w: the state before the step)
     const double4 Tx = T.x[i], Tv = T.v[i], Tw = T.w[i], Tq = T.q[i];
@@ -553,35 +588,36 @@ __global__ void k_gather_fwd(DState S, const double4* mass_old, const int* inc_o
     T.w[i] = make_double4(tw1.x, tw1.y, tw1.z, 0.0);
     T.q[i] = make_double4(tq1.s, tq1.v.x, tq1.v.y, tq1.v.z);
   }
-  S.x[i] = make_double4(x.x, x.y, x.z, r);
-  S.v[i] = make_double4(v.x, v.y, v.z, Vv.w);
-  S.w[i] = make_double4(w.x, w.y, w.z, A.w);
-  S.q[i] = make_double4(qq.s, qq.v.x, qq.v.y, qq.v.z);
+  So.x[i] = make_double4(x.x, x.y, x.z, P.w);
+  So.v[i] = make_double4(v.x, v.y, v.z, Vv.w);
+  So.w[i] = make_double4(w.x, w.y, w.z, A.w);
+  So.q[i] = make_double4(qq.s, qq.v.x, qq.v.y, qq.v.z);
   const dv3 d = sub3(x, mk3(Om.x, Om.y, Om.z));
   const unsigned long long m = (unsigned long long)__double_as_longlong(dot3(d, d));
   if (m > thresh) atomicMax(&run->halt, step);  // a neighbour search before the next step
 }
 
-// per specimen: fixed-order sum of its particles' measured wall forces, at the
-// sample steps (the sum of sample k goes to out_base[k * nspec + s])
-__global__ void k_spec_sum(const DRun* run, int every, const double* val, const int* spec_start,
-                           int nspec, double* out_base)
+// per specimen: fixed-order sum of its particles' measured wall forces
+__global__ __launch_bounds__(256) void k_spec_sum(const DRun* run, int step, const double* val,
+                                                  const int* spec_start, double* out)
 {
-  __shared__ double red[1024];
-  int step;
-  if (run_skip(run, step) || every <= 0 || step % every != 0) return;
-  double* out = out_base + (size_t)(step / every - 1) * nspec;
+  __shared__ double red[4];
+  if (run_skip(run, step)) return;
   const int s = blockIdx.x;
   const int a = spec_start[s], b = spec_start[s + 1];
   double acc = 0.0;
-  for (int i = a + (int)threadIdx.x; i < b; i += blockDim.x) acc = acc + val[i];
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = 0.0;
-    for (int k = 0; k < (int)blockDim.x; k++) t = t + red[k];
-    out[s] = t;
+  // eight loads in flight a thread (20,000 particles: 20 us with one)
+  for (int i = a + (int)threadIdx.x; i < b; i += 256 * 8) {
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = i + 256 * k < b ? val[i + 256 * k] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc = acc + v[k];
   }
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) out[s] = ((red[0] + red[1]) + red[2]) + red[3];
 }
 
 // ---------------------------------------------------------------------------
@@ -661,16 +697,15 @@ __global__ void k_inc_sort2(int n, const int* off, int* ent)
 // ---------------------------------------------------------------------------
 // adjoint kernels
 // ---------------------------------------------------------------------------
-// lam: per particle 4 double4 (x, v, w, q) holding the adjoint of the state
-// after the step on entry and the partial adjoint of the state before it on
-// exit; lfm: per particle (lambda_F, lambda_M) for the interaction adjoints.
-// coef[s]: d loss_s / d stress_s / area_s at a sample step (else 0).
-__global__ void k_adj_particle(DState Sn, DState Sn1, double4* lam, double* lfm, DStep sp,
-                               const double* coef)
+// The adjoint of one particle's update in the step whose state before is Sn and
+// after Sn1: L holds the adjoint of the state after the step (x, v, w, q) on
+// entry and the partial adjoint of the state before it on exit; o: (lambda_F,
+// lambda_M) for the interaction adjoints.  cf: d loss / d stress / area of the
+// particle's specimen at a sample step (else 0).
+__device__ __forceinline__ void adj_particle_item(const DState& Sn, const DState& Sn1, int i,
+                                                  double4 (&L)[4], double* o, const DStep& sp,
+                                                  double cf)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= Sn.n) return;
-  double4* L = lam + 4 * (size_t)i;
   const double4 Lx = L[0], Lv1 = L[1], Lw1 = L[2], Lq1 = L[3];
   const double dt = sp.dt, h = dt / 2.0;
   const double4 Vv = Sn.v[i], A = Sn.w[i], Q = Sn.q[i];
@@ -700,7 +735,6 @@ __global__ void k_adj_particle(DState Sn, DState Sn1, double4* lam, double* lfm,
   // force also enters the stress
   const double4 P = Sn.x[i];
   const double r = P.w;
-  const double cf = coef ? coef[Sn.spec[i]] : 0.0;
   for (int k = 0; k < sp.nw; k++) {
     const DWall& W = sp.wall[k];
     const dv3 n = mk3(W.n[0], W.n[1], W.n[2]);
@@ -717,7 +751,6 @@ __global__ void k_adj_particle(DState Sn, DState Sn1, double4* lam, double* lfm,
   L[1] = make_double4(lv1.x, lv1.y, lv1.z, 0.0);
   L[2] = make_double4(lw1.x, lw1.y, lw1.z, 0.0);
   L[3] = make_double4(lq.s, lq.v.x, lq.v.y, lq.v.z);
-  double* o = lfm + 6 * (size_t)i;
   o[0] = lF.x; o[1] = lF.y; o[2] = lF.z;
   o[3] = lM.x; o[4] = lM.y; o[5] = lM.z;
 }
@@ -736,7 +769,7 @@ __global__ __launch_bounds__(ADJ_BOND_BS) void k_adj_bond(DState S, DBonds B,
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= B.nb) return;
   double* c = ab + NB_TAN * (size_t)b;
-  if (B.bstep[b] < step) return;  // broken earlier: no record (k_adj_gather skips it)
+  if (B.bstep[b] < step) return;  // broken earlier: no record (k_adj_step skips it)
   const int2 e = B.ij[b];
   const double4 P1 = S.x[e.x], P2 = S.x[e.y], Q1 = S.q[e.x], Q2 = S.q[e.y];
   const double4 D = B.D0[b];
@@ -827,87 +860,111 @@ __global__ void k_adj_fric(DState S, DCands C, const int* bstep, const double4* 
   lh_prev[c] = make_double4(g[6].x, g[6].y, g[6].z, 0.0);
 }
 
-// per particle: add the interactions' adjoints (CSR order) to the state
-// adjoint; parameter gradients of the interactions whose first particle this
-// is go to gth (kn, ks, -, mu).  Entries go ADJ_GATHER_CH at a time with their
-// loads in flight together; records without a Jacobian this step (pairs apart
-// or excluded, bonds broken earlier) are skipped: they would add zeros.
-__global__ void k_adj_gather(int n, const int* inc_off, const int* inc_ent, int ncand,
-                             const double* ac, const double* ab, const unsigned char* cact,
-                             const int* bstep, int step, double4* lam, double4* gth)
+// Per particle: the interactions' adjoints of step `step` are added to the state
+// adjoint lam in CSR order (GATHER; parameter gradients of the interactions whose
+// first particle this is go to gth: kn, ks, -, mu), then the particle's own update
+// in the step before, sp.step, is taken back (PART: states Sn, Sn1, adjoints for
+// its interactions to lfm).  One launch between two steps' laws instead of two,
+// and lam passes through memory once.
+// Four lanes share a particle, each with one of lam's vectors: lane 0 adds the
+// position adjoints of every entry, 1 the velocities, 2 the angular velocities (of
+// a bond: the parameters), 3 the quaternions (of a pair: the parameters), so a
+// record's 96 bytes for one side are read by neighbouring lanes.  With the two parts
+// as launches of one lane a particle (us a step): 2,000 particles 20.4 + 5.0 -> 21.0,
+// 20,000 24.9 + 5.9 -> 28.6.  Records without a Jacobian this step (pairs apart or excluded, bonds broken earlier) are skipped.
+template <bool GATHER, bool PART>
+__global__ __launch_bounds__(DIFF_MAX_BS) void k_adj_step(
+    int n, const int* inc_off, const int* inc_ent, int ncand, const double* ac, const double* ab,
+    const unsigned char* cact, const int* bstep, int step, double4* lam, double4* gth, DState Sn,
+    DState Sn1, double* lfm, DStep sp, const double* coef)
 {
-  constexpr int ADJ_GATHER_RUN = 12, ADJ_GATHER_CH = 2;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double4* L = lam + 4 * (size_t)i;
-  double4 lx = L[0], lv = L[1], lw = L[2], lq = L[3];
-  double4 g = gth[i];
-  const int e0 = inc_off[i], e1 = inc_off[i + 1];
-  for (int r0 = e0; r0 < e1; r0 += ADJ_GATHER_RUN) {
-    int ent[ADJ_GATHER_RUN];
+  constexpr int G = 4, R = 4;
+  __shared__ double4 sl[PART ? DIFF_MAX_BS : 1];
+  const int t = threadIdx.x;
+  const int PB = blockDim.x / G;
+  const int p0 = blockIdx.x * PB;
+  const int pi = p0 + t / G, sub = t % G;
+  const int pc = pi < n ? pi : 0;
+  double4 L = lam[4 * (size_t)pc + sub];
+  if (GATHER) {
+    const int e0 = inc_off[pc], e1 = pi < n ? inc_off[pc + 1] : e0;
+    double ga[3] = {0.0, 0.0, 0.0};
+    int ent[R];
 #pragma unroll
-    for (int k = 0; k < ADJ_GATHER_RUN; k++) ent[k] = r0 + k < e1 ? inc_ent[r0 + k] : -1;
-    unsigned act = 0;
+    for (int r = 0; r < R; r++) ent[r] = e0 + r < e1 ? inc_ent[e0 + r] : -1;
+    for (int b = e0; b < e1; b += R) {
+      bool on[R];
+      double a[R][4];
 #pragma unroll
-    for (int k = 0; k < ADJ_GATHER_RUN; k++) {
-      const int rec = ent[k] >> 1;
-      const bool on =
-          ent[k] >= 0 && (rec < ncand ? cact[rec] != 0 : bstep[rec - ncand] >= step);
-      act |= (on ? 1u : 0u) << k;
+      for (int r = 0; r < R; r++) {
+        const int rec = ent[r] >> 1;
+        on[r] = ent[r] >= 0 && (rec < ncand ? cact[rec] != 0 : bstep[rec - ncand] >= step);
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        a[r][0] = a[r][1] = a[r][2] = a[r][3] = 0.0;
+        const int rec = ent[r] >> 1, side = ent[r] & 1;
+        const bool pair = rec < ncand;
+        // a pair: x, v, w at 0, 6, 12 (+3 for the second), parameters at 21; a
+        // bond: x at 0, q at 6 (+4 for the second), parameters at 14
+        const int at = pair ? (sub == 3 ? 21 : 6 * sub + 3 * side)
+                            : (sub == 0 ? 3 * side : sub == 3 ? 6 + 4 * side : 14);
+        const bool use = on[r] && (pair ? (sub < 3 || side == 0)
+                                        : (sub == 0 || sub == 3 || (sub == 2 && side == 0)));
+        if (!use) continue;
+        const double* c = pair ? ac + NF_TAN * (size_t)rec + at : ab + NB_TAN * (size_t)(rec - ncand) + at;
+        a[r][0] = c[0];
+        a[r][1] = c[1];
+        if (pair || sub != 2) a[r][2] = c[2];
+        if (!pair && sub == 3) a[r][3] = c[3];
+      }
+      bool par[R];  // this lane's terms of the entry are parameter gradients
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        par[r] = (ent[r] >> 1) < ncand ? sub == 3 : sub == 2;
+        const int nx = b + R + r;
+        ent[r] = nx < e1 ? inc_ent[nx] : -1;
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        if (par[r]) {
+          ga[0] += a[r][0];
+          ga[1] += a[r][1];
+          ga[2] += a[r][2];
+        } else {
+          L.x += a[r][0];
+          L.y += a[r][1];
+          L.z += a[r][2];
+          L.w += a[r][3];
+        }
+      }
     }
-#pragma unroll
-    for (int c0 = 0; c0 < ADJ_GATHER_RUN; c0 += ADJ_GATHER_CH) {
-      if (!((act >> c0) & ((1u << ADJ_GATHER_CH) - 1u))) continue;
-      // per entry: x (3), v or q (4), w (3), parameter terms (3)
-      double a[ADJ_GATHER_CH][13];
-#pragma unroll
-      for (int k = 0; k < ADJ_GATHER_CH; k++) {
-        if (!((act >> (c0 + k)) & 1u)) continue;
-        const int rec = ent[c0 + k] >> 1, side = ent[c0 + k] & 1;
-        if (rec < ncand) {
-          const double* c = ac + NF_TAN * (size_t)rec;
-          const int xo = side ? 3 : 0, vo = side ? 9 : 6, wo = side ? 15 : 12;
-          a[k][0] = c[xo]; a[k][1] = c[xo + 1]; a[k][2] = c[xo + 2];
-          a[k][3] = c[vo]; a[k][4] = c[vo + 1]; a[k][5] = c[vo + 2]; a[k][6] = 0.0;
-          a[k][7] = c[wo]; a[k][8] = c[wo + 1]; a[k][9] = c[wo + 2];
-          if (!side) {
-            a[k][10] = c[21]; a[k][11] = c[22]; a[k][12] = c[23];
-          }
-        } else {
-          const double* c = ab + NB_TAN * (size_t)(rec - ncand);
-          const int xo = side ? 3 : 0, qo = side ? 10 : 6;
-          a[k][0] = c[xo]; a[k][1] = c[xo + 1]; a[k][2] = c[xo + 2];
-          a[k][3] = c[qo]; a[k][4] = c[qo + 1]; a[k][5] = c[qo + 2]; a[k][6] = c[qo + 3];
-          if (!side) {
-            a[k][10] = c[14]; a[k][11] = c[15];
-          }
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < ADJ_GATHER_CH; k++) {
-        if (!((act >> (c0 + k)) & 1u)) continue;
-        const int rec = ent[c0 + k] >> 1, side = ent[c0 + k] & 1;
-        lx.x += a[k][0]; lx.y += a[k][1]; lx.z += a[k][2];
-        if (rec < ncand) {
-          lv.x += a[k][3]; lv.y += a[k][4]; lv.z += a[k][5];
-          lw.x += a[k][7]; lw.y += a[k][8]; lw.z += a[k][9];
-          if (!side) {
-            g.x += a[k][10];
-            g.y += a[k][11];
-            g.w += a[k][12];
-          }
-        } else {
-          lq.x += a[k][3]; lq.y += a[k][4]; lq.z += a[k][5]; lq.w += a[k][6];
-          if (!side) {
-            g.x += a[k][10];
-            g.y += a[k][11];
-          }
-        }
-      }
+    // (kn, ks) of the bonds in lane 2, (kn, ks, mu) of the pairs in lane 3
+    const double g0 = group_value<G>(ga[0], 3) + group_value<G>(ga[0], 2);
+    const double g1 = group_value<G>(ga[1], 3) + group_value<G>(ga[1], 2);
+    const double g3 = group_value<G>(ga[2], 3);
+    if (sub == 0 && pi < n) {
+      double4 g = gth[pi];
+      g.x += g0;
+      g.y += g1;
+      g.w += g3;
+      gth[pi] = g;
     }
   }
-  L[0] = lx; L[1] = lv; L[2] = lw; L[3] = lq;
-  gth[i] = g;
+  if (!PART) {
+    if (pi < n) lam[4 * (size_t)pi + sub] = L;
+    return;
+  }
+  sl[t] = L;
+  __syncthreads();
+  const int i = p0 + t;
+  if (t < PB && i < n) {
+    double4 l4[4] = {sl[4 * t], sl[4 * t + 1], sl[4 * t + 2], sl[4 * t + 3]};
+    adj_particle_item(Sn, Sn1, i, l4, lfm + 6 * (size_t)i, sp, coef ? coef[Sn.spec[i]] : 0.0);
+    for (int k = 0; k < 4; k++) sl[4 * t + k] = l4[k];
+  }
+  __syncthreads();
+  if (pi < n) lam[4 * (size_t)pi + sub] = sl[t];
 }
 
 // adjoint of the history read at the first step of an epoch, to the pairs of
@@ -920,21 +977,22 @@ __global__ void k_map_lh(int nc, const int* src, const double4* lnew, double4* l
   if (s >= 0) lold[s] = lnew[c];
 }
 
-__global__ void k_spec_sum4(const double4* val, const int* spec_start, double4* out)
+__global__ __launch_bounds__(256) void k_spec_sum4(const double4* val, const int* spec_start, double4* out)
 {
-  __shared__ double4 red[1024];
+  __shared__ double4 red[4];
   const int s = blockIdx.x;
   const int a = spec_start[s], b = spec_start[s + 1];
   double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
-  for (int i = a + (int)threadIdx.x; i < b; i += blockDim.x) {
+  for (int i = a + (int)threadIdx.x; i < b; i += 256) {
     const double4 v = val[i];
     acc.x = acc.x + v.x; acc.y = acc.y + v.y; acc.z = acc.z + v.z; acc.w = acc.w + v.w;
   }
-  red[threadIdx.x] = acc;
+  acc = make_double4(wave_sum(acc.x), wave_sum(acc.y), wave_sum(acc.z), wave_sum(acc.w));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
   if (threadIdx.x == 0) {
-    double4 t = make_double4(0.0, 0.0, 0.0, 0.0);
-    for (int k = 0; k < (int)blockDim.x; k++) {
+    double4 t = red[0];
+    for (int k = 1; k < 4; k++) {
       t.x = t.x + red[k].x; t.y = t.y + red[k].y; t.z = t.z + red[k].z; t.w = t.w + red[k].w;
     }
     out[s] = t;
@@ -957,8 +1015,7 @@ struct Epoch {
 struct Checkpoint {
   int step = 0;
   int epoch = 0;
-  DevBuf<double4> x, v, w, q, o, hist;
-  DevBuf<int> bstep;
+  DevBuf<double4> x, v, w, q, hist;
 };
 
 }  // namespace
@@ -1001,12 +1058,20 @@ struct esp_diff {
   std::vector<int> rebuild_steps;
   DevBuf<double4> H[2];  // shear histories: step s reads H[s & 1], writes the other
   DevBuf<DRun> run;
-  DevBuf<double> wo;     // wall origins per step of the run [step][wall][3]
-  // the forward steps of one epoch captured as a graph (device-driven steps)
-  hipGraphExec_t gexec = nullptr;
-  int g_epoch = -1, g_len = 0;
-  bool use_graph = true;
-  int graph_steps = 16;
+  std::vector<double> wo;  // wall origins per step of the run [step][wall][3]
+  // The states of the last forward run, step by step ([step][x, v, w, q][n]), and
+  // the histories touching pairs read in each: kept by runs whose tape fits
+  // kTapeBytes, so that the adjoint sweeps them without recomputing its segments.
+  // Longer runs keep checkpoints, and the sweep one segment's tape at a time.
+  bool full_tape = false;
+  DevBuf<double4> tape;
+  std::vector<std::unique_ptr<DevBuf<double4>>> hchunk;  // room the histories are laid out in
+  std::vector<double4*> htape;                           // [step]
+  // the reverse sweep's arrays
+  DevBuf<double4> lam, gth, lh, lh2;
+  DevBuf<double> lfm, ab, ac;
+  DevBuf<unsigned char> aact;  // per pair: its record holds a Jacobian this step
+  std::vector<std::unique_ptr<DevBuf<double4>>> hseg;
   DevBuf<double> bout, cout, wfn, stress_dev;
   DevBuf<unsigned char> cact;  // per pair of the epoch: its record holds this step's force
   DevBuf<double4> theta;
@@ -1016,10 +1081,8 @@ struct esp_diff {
   // branch digests are computed only when asked for (esp_diff_track_branches):
   // every wave of the contact and gather kernels adds to one counter per step
   bool track_digest = false;
-  // the state and break steps at the end of the last forward run: the backward
-  // sweep recomputes earlier states in the same arrays and puts these back
-  DevBuf<double4> fx, fv, fw, fq;
-  DevBuf<int> fbstep;
+  DState fin = {};  // the state at the end of the last forward run
+  DevBuf<double4> x0, v0, w0, q0;  // the initial state
   // tangent-linear run (forward with a parameter direction)
   bool tan_on = false;
   DevBuf<double4> tx, tv, tw, tq, TH[2], dtheta;
@@ -1036,6 +1099,12 @@ struct esp_diff {
   {
     return DState{x.p, v.p, w.p, q.p, spec.p, n};
   }
+  // a state of a tape laid out as [x][v][w][q]
+  DState tape_state(double4* t)
+  {
+    const size_t c = (size_t)n;
+    return DState{t, t + c, t + 2 * c, t + 3 * c, spec.p, n};
+  }
   // wall origins of a step: moved by their step before every step (the
   // pre-time-step moveWallBy of the main engine's setWallStepMotion)
   DStep step_params(int step)
@@ -1045,8 +1114,7 @@ struct esp_diff {
     s.nw = nw;
     for (int k = 0; k < nw; k++) {
       s.wall[k] = wall0[k];
-      for (int t = 0; t < step; t++)
-        for (int c = 0; c < 3; c++) s.wall[k].o[c] = s.wall[k].o[c] + wstep[k][c];
+      for (int c = 0; c < 3; c++) s.wall[k].o[c] = wo[((size_t)step * nw + k) * 3 + c];
     }
     s.has_g = has_g;
     for (int c = 0; c < 3; c++) s.g[c] = g[c];
@@ -1057,6 +1125,12 @@ struct esp_diff {
 };
 
 namespace {
+
+// a run's tape (states and histories of every step) is kept up to this size
+// (24 specimens of 2,000 to 30,000 particles take 70 MB a step); recomputing the
+// segments and copying their states cost a third of a forward and backward pass
+// (2,000 particles, 100 steps: 12.7 -> 5.8 ms with the launches below)
+constexpr size_t kTapeBytes = (size_t)24 << 30;
 
 void dsync(esp_diff* d) { DCHK(hipStreamSynchronize(d->stream)); }
 
@@ -1072,12 +1146,12 @@ int dscan(esp_diff* d, const int* in, int* out, int cnt)
 }
 
 // neighbour search (NeighborTable::build + getFullList) -> a new epoch
-void rebuild(esp_diff* d, int step)
+void rebuild(esp_diff* d, const DState& S, int step)
 {
   const int n = d->n;
   PView pv;
   memset(&pv, 0, sizeof pv);
-  pv.pos = d->x.p; pv.vel = d->v.p; pv.ang = d->w.p; pv.quat = d->q.p; pv.old = d->o.p;
+  pv.pos = S.x; pv.vel = S.v; pv.ang = S.w; pv.quat = S.q; pv.old = d->o.p;
   pv.flags = d->flags.p; pv.id = d->id.p; pv.n = n;
   DCHK(hipMemsetAsync(d->cell_count.p, 0, sizeof(int) * (d->ncell + 1), d->stream));
   DCHK(hipMemsetAsync(d->md.p, 0, sizeof(unsigned long long) * 2, d->stream));
@@ -1187,27 +1261,29 @@ void d2d(esp_diff* d, T* dst, const T* src, size_t cnt)
   if (cnt) DCHK(hipMemcpyAsync(dst, src, cnt * sizeof(T), hipMemcpyDeviceToDevice, d->stream));
 }
 
-void save_checkpoint(esp_diff* d, int step)
+void save_checkpoint(esp_diff* d, int step, const DState& S)
 {
   auto C = std::make_unique<Checkpoint>();
   C->step = step;
   C->epoch = (int)d->epochs.size() - 1;
   const size_t n = std::max(d->n, 1);
-  C->x.reserve(n); C->v.reserve(n); C->w.reserve(n); C->q.reserve(n); C->o.reserve(n);
-  d2d(d, C->x.p, d->x.p, d->n); d2d(d, C->v.p, d->v.p, d->n); d2d(d, C->w.p, d->w.p, d->n);
-  d2d(d, C->q.p, d->q.p, d->n); d2d(d, C->o.p, d->o.p, d->n);
+  C->x.reserve(n); C->v.reserve(n); C->w.reserve(n); C->q.reserve(n);
+  d2d(d, C->x.p, S.x, d->n); d2d(d, C->v.p, S.v, d->n); d2d(d, C->w.p, S.w, d->n);
+  d2d(d, C->q.p, S.q, d->n);
   const int nc = d->epochs.back()->nc;
   C->hist.reserve(std::max(nc, 1));
   d2d(d, C->hist.p, d->H[step & 1].p, nc);
-  C->bstep.reserve(std::max(d->nb, 1));
-  d2d(d, C->bstep.p, d->bstep.p, d->nb);
   d->ckpts.push_back(std::move(C));
 }
 
-void restore_checkpoint(esp_diff* d, const Checkpoint& C)
+// a checkpoint's state into the tape at T, its histories into the arrays a segment
+// is recomputed with (the run's break steps hold for every step of it: a bond lives
+// up to the step it breaks in)
+void restore_checkpoint(esp_diff* d, const Checkpoint& C, double4* T)
 {
-  d2d(d, d->x.p, C.x.p, d->n); d2d(d, d->v.p, C.v.p, d->n); d2d(d, d->w.p, C.w.p, d->n);
-  d2d(d, d->q.p, C.q.p, d->n); d2d(d, d->o.p, C.o.p, d->n);
+  const DState S = d->tape_state(T);
+  d2d(d, S.x, C.x.p, d->n); d2d(d, S.v, C.v.p, d->n); d2d(d, S.w, C.w.p, d->n);
+  d2d(d, S.q, C.q.p, d->n);
   const int nc = d->epochs[C.epoch]->nc;
   d->H[0].reserve(std::max(nc, 1));
   d->H[1].reserve(std::max(nc, 1));
@@ -1215,47 +1291,16 @@ void restore_checkpoint(esp_diff* d, const Checkpoint& C)
   // "zero in both buffers" writes neither)
   d2d(d, d->H[0].p, C.hist.p, nc);
   d2d(d, d->H[1].p, C.hist.p, nc);
-  d2d(d, d->bstep.p, C.bstep.p, d->nb);
 }
 
-void upload_initial(esp_diff* d)
-{
-  const int n = d->n;
-  std::vector<double4> X(n), V(n), W(n), Q(n), O(n);
-  for (int i = 0; i < n; i++) {
-    const double m = d->h_mass[i], r = d->h_rad[i];
-    X[i] = make_double4(d->h_pos[3 * i], d->h_pos[3 * i + 1], d->h_pos[3 * i + 2], r);
-    V[i] = make_double4(d->h_vel[3 * i], d->h_vel[3 * i + 1], d->h_vel[3 * i + 2],
-                        m != 0.0 ? 1.0 / m : 0.0);
-    const double I = 0.4 * m * r * r;  // CRotParticle, 3-D (RotParticle.cpp:80-124)
-    W[i] = make_double4(0.0, 0.0, 0.0, 1.0 / I);
-    Q[i] = make_double4(1.0, 0.0, 0.0, 0.0);
-    O[i] = make_double4(X[i].x, X[i].y, X[i].z, m);
-  }
-  const size_t c = std::max(n, 1);
-  d->x.reserve(c); d->v.reserve(c); d->w.reserve(c); d->q.reserve(c); d->o.reserve(c);
-  DCHK(hipMemcpyAsync(d->x.p, X.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
-  DCHK(hipMemcpyAsync(d->v.p, V.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
-  DCHK(hipMemcpyAsync(d->w.p, W.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
-  DCHK(hipMemcpyAsync(d->q.p, Q.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
-  DCHK(hipMemcpyAsync(d->o.p, O.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
-  std::vector<int> bs(std::max(d->nb, 1), INT_MAX);
-  DCHK(hipMemcpyAsync(d->bstep.p, bs.data(), sizeof(int) * d->nb, hipMemcpyHostToDevice,
-                      d->stream));
-  dsync(d);
-}
-
-// one forward step (no search): forces, update, sample
-// The launches of one forward step (no search): tangents (tangent runs),
-// forces, update and sampling; the step index comes from d->run on the device
-// (k_advance ends the step), so the same launches serve every step and can be
-// captured in a graph.  record: branch digests into d->digest (forward runs);
-// halting: the displacement test may stop the queue (not while recomputing a
-// recorded segment).
-void fwd_step(esp_diff* d, const Epoch& E, bool record, bool halting)
+// The launches of one forward step (no search) from S into So: tangents (tangent
+// runs), the force laws, the update.  htape: where touching pairs leave the histories they read, or nullptr; record: branch digests
+// and samples (forward runs); halting: the displacement test may stop the queue
+// (not while recomputing a recorded segment).
+void fwd_step(esp_diff* d, const Epoch& E, int step, const DState& S, const DState& So,
+              double4* htape, bool record, bool halting)
 {
   const int bs = d->bs;
-  DState S = d->state();
   DBonds B{d->nb, d->bij.p, d->bD0.p, d->brel.p, d->bstep.p, d->tkb.p};
   DCands C{E.nc, E.ij.p, E.bond.p};
   DRun* R = d->run.p;
@@ -1263,88 +1308,140 @@ void fwd_step(esp_diff* d, const Epoch& E, bool record, bool halting)
   if (d->tan_on) {  // tangents from the state before the step (before the forward kernels)
     if (d->nb > 0)
       hipLaunchKernelGGL(k_bond_tan, dim3(nblocks(d->nb, bs)), dim3(bs), 0, d->stream, S, T, B,
-                         d->theta.p, d->dtheta.p, R, d->bt.p);
+                         d->theta.p, d->dtheta.p, R, step, d->bt.p);
     if (E.nc > 0)
       hipLaunchKernelGGL(k_fric_tan, dim3(nblocks(E.nc, bs)), dim3(bs), 0, d->stream, S, T, C,
                          d->bstep.p, d->theta.p, d->dtheta.p, d->H[0].p, d->H[1].p, d->TH[0].p,
-                         d->TH[1].p, R, d->cfg.dt, d->ct.p);
+                         d->TH[1].p, R, step, d->cfg.dt, d->ct.p);
   }
-  if (d->nb > 0)
-    hipLaunchKernelGGL(k_bond_fwd, dim3(nblocks(d->nb, bs)), dim3(bs), 0, d->stream, S, B,
-                       d->theta.p, R, d->bout.p);
-  if (E.nc > 0)
-    hipLaunchKernelGGL(k_fric_fwd, dim3(nblocks(E.nc, bs)), dim3(bs), 0, d->stream, S, C, d->bstep.p,
-                       d->theta.p, d->H[0].p, d->H[1].p, R, d->cfg.dt, d->cout.p, d->cact.p,
-                       record && d->track_digest ? d->digest.p : nullptr);
+  unsigned long long* dig = record && d->track_digest ? d->digest.p : nullptr;
+  const int nbb = d->nb > 0 ? nblocks(d->nb, bs) : 0, ncb = E.nc > 0 ? nblocks(E.nc, bs) : 0;
+  if (nbb + ncb > 0)
+    hipLaunchKernelGGL(k_bond_fwd_pairs, dim3(nbb + ncb), dim3(bs), 0, d->stream, S, B, C, d->theta.p,
+                       d->H[0].p, d->H[1].p, htape, R, step, d->cfg.dt, nbb, d->bout.p, d->cout.p,
+                       d->cact.p, dig);
   unsigned long long thresh = ~0ull;
   if (halting) {
     const double a = 0.5 * d->cfg.verlet_dist;
     const double sr = a * a;
     memcpy(&thresh, &sr, 8);
   }
-  DStep sp = d->step_params(0);
-  sp.wo = d->wo.p;
-  hipLaunchKernelGGL(k_gather_fwd, dim3(nblocks(d->n, bs)), dim3(bs), 0, d->stream, S, d->o.p,
-                     E.inc_off.p, E.inc_ent.p, E.nc, d->cout.p, d->bout.p, d->cact.p, d->bstep.p,
-                     sp, d->every, d->wfn.p,
-                     R, thresh, record && d->track_digest ? d->digest.p : nullptr, T, d->ct.p,
-                     d->bt.p,
-                     d->tan_on ? d->wft.p : nullptr);
-  if (record) {
-    hipLaunchKernelGGL(k_spec_sum, dim3(d->nspec), dim3(256), 0, d->stream, R, d->every, d->wfn.p,
-                       d->spec_start.p, d->nspec, d->stress_dev.p);
+  const DStep sp = d->step_params(step);
+  const bool sample = record && step % d->every == 0;
+  hipLaunchKernelGGL(d->tan_on ? k_gather_fwd<true> : k_gather_fwd<false>,
+                     dim3(nblocks(4ll * d->n, bs)), dim3(bs), 0, d->stream, S, So, d->o.p,
+                     E.inc_off.p, E.inc_ent.p, E.nc, d->cout.p, d->bout.p, d->cact.p, d->bstep.p, sp,
+                     sample ? d->wfn.p : nullptr, R, thresh, dig, T, d->ct.p, d->bt.p,
+                     sample && d->tan_on ? d->wft.p : nullptr);
+  if (sample) {
+    const size_t at = (size_t)(step / d->every - 1) * d->nspec;
+    hipLaunchKernelGGL(k_spec_sum, dim3(d->nspec), dim3(256), 0, d->stream, R, step, d->wfn.p,
+                       d->spec_start.p, d->stress_dev.p + at);
     if (d->tan_on)
-      hipLaunchKernelGGL(k_spec_sum, dim3(d->nspec), dim3(256), 0, d->stream, R, d->every,
-                         d->wft.p, d->spec_start.p, d->nspec, d->stress_t.p);
+      hipLaunchKernelGGL(k_spec_sum, dim3(d->nspec), dim3(256), 0, d->stream, R, step, d->wft.p,
+                         d->spec_start.p, d->stress_t.p + at);
   }
-  hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, d->stream, R);
   DCHK(hipGetLastError());
 }
 
-void set_run(esp_diff* d, int step, int end)
+void clear_run(esp_diff* d)
 {
-  hipLaunchKernelGGL(k_set_run, dim3(1), dim3(64), 0, d->stream, d->run.p, step, 0, end);
+  hipLaunchKernelGGL(k_clear_run, dim3(1), dim3(64), 0, d->stream, d->run.p);
   DCHK(hipGetLastError());
 }
 
-void drop_graph(esp_diff* d)
-{
-  if (d->gexec) {
-    (void)hipStreamSynchronize(d->stream);
-    (void)hipGraphExecDestroy(d->gexec);
+// where a step's touching pairs leave their histories: laid out one after the
+// other in chunks that are kept for later runs
+struct HistoryRoom {
+  esp_diff* d;
+  size_t chunk, at;
+  double4* take(size_t n, int steps_left)
+  {
+    while (chunk < d->hchunk.size() && at + n > d->hchunk[chunk]->cap) {
+      chunk++;
+      at = 0;
+    }
+    if (chunk == d->hchunk.size()) {
+      d->hchunk.push_back(std::make_unique<DevBuf<double4>>());
+      const size_t most = (size_t)1 << 25;  // 1 GiB
+      d->hchunk.back()->reserve(std::max(n, std::min(most, n * (size_t)std::max(steps_left, 1))));
+      at = 0;
+    }
+    double4* p = d->hchunk[chunk]->p + at;
+    at += n;
+    return p;
   }
-  d->gexec = nullptr;
-  d->g_epoch = -1;
-}
-
-// forward steps d->run.step .. end on the current epoch (the run record is
-// set): graph_steps forward steps captured once per epoch and replayed, or
-// plain launches
-void run_chunk(esp_diff* d, int from, int end)
-{
-  const Epoch& E = *d->epochs.back();
-  const int G = std::max(1, d->graph_steps);
-  if (!d->use_graph) {
-    for (int s = from; s <= end; s++) fwd_step(d, E, true, true);
-    return;
-  }
-  const int ep = (int)d->epochs.size() - 1;
-  if (d->g_epoch != ep || d->g_len != G) {
-    drop_graph(d);
-    hipGraph_t g = nullptr;
-    DCHK(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < G; k++) fwd_step(d, E, true, true);
-    DCHK(hipStreamEndCapture(d->stream, &g));
-    const hipError_t rc = hipGraphInstantiate(&d->gexec, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    DCHK(rc);
-    d->g_epoch = ep;
-    d->g_len = G;
-  }
-  for (int s = from; s <= end; s += G) DCHK(hipGraphLaunch(d->gexec, d->stream));
-}
+};
 
 int nsamples(const esp_diff* d) { return d->nsteps / d->every; }
+
+// the steps of a forward run; tape: keep every step's state if that fits kTapeBytes
+void run_forward(esp_diff* d, bool tape)
+{
+  d->epochs.clear();
+  d->ckpts.clear();
+  d->rebuild_steps.clear();
+  d->full_tape = false;
+  DCHK(hipMemsetAsync(d->digest.p, 0, sizeof(unsigned long long) * (d->nsteps + 1), d->stream));
+  if (d->nb > 0) launch_fill_int(d->stream, d->nb, d->bstep.p, INT_MAX);
+  // chunks of steps between checkpoints queued without host decisions; a step
+  // whose displacement asks for a neighbour search halts the queue, the host
+  // rebuilds the table before the next step and continues
+  const int K = std::max(1, d->cfg.checkpoint_every);
+  const size_t c4 = 4 * (size_t)d->n;
+  DState S0{d->x0.p, d->v0.p, d->w0.p, d->q0.p, d->spec.p, d->n};
+  rebuild(d, S0, 1);
+  d->full_tape = tape && !d->tan_on &&
+                 (size_t)d->nsteps * (32 * c4 + 32 * (size_t)d->epochs[0]->nc) <= kTapeBytes;
+  DState cur;
+  if (d->full_tape) {
+    d->tape.reserve(((size_t)d->nsteps + 1) * c4);
+    cur = d->tape_state(d->tape.p);
+    d->htape.assign((size_t)d->nsteps + 1, nullptr);
+  } else {
+    const size_t c = std::max(d->n, 1);
+    d->x.reserve(c); d->v.reserve(c); d->w.reserve(c); d->q.reserve(c);
+    cur = d->state();
+  }
+  d2d(d, cur.x, S0.x, d->n); d2d(d, cur.v, S0.v, d->n); d2d(d, cur.w, S0.w, d->n);
+  d2d(d, cur.q, S0.q, d->n);
+  HistoryRoom room{d, 0, 0};
+  bool need = false;
+  int step = 1;
+  std::vector<HistoryRoom> mark;
+  while (step <= d->nsteps) {
+    if (need) {
+      rebuild(d, d->full_tape ? d->tape_state(d->tape.p + (size_t)(step - 1) * c4) : cur, step);
+      need = false;
+    }
+    if (!d->full_tape && (step - 1) % K == 0) save_checkpoint(d, step, cur);
+    const int end = std::min(d->nsteps, d->full_tape ? step + 63 : ((step - 1) / K + 1) * K);
+    const Epoch& E = *d->epochs.back();
+    clear_run(d);
+    mark.clear();
+    for (int s = step; s <= end; s++) {
+      if (d->full_tape) {
+        mark.push_back(room);
+        d->htape[s] = room.take(std::max(E.nc, 1), d->nsteps - s + 1);
+        fwd_step(d, E, s, d->tape_state(d->tape.p + (size_t)(s - 1) * c4),
+                 d->tape_state(d->tape.p + (size_t)s * c4), d->htape[s], true, true);
+      } else {
+        fwd_step(d, E, s, cur, cur, nullptr, true, true);
+      }
+    }
+    DRun r;
+    DCHK(hipMemcpyAsync(&r, d->run.p, sizeof r, hipMemcpyDeviceToHost, d->stream));
+    dsync(d);
+    if (r.halt != 0) {
+      need = true;
+      if (d->full_tape && r.halt < end) room = mark[r.halt + 1 - step];  // the rest did nothing
+      step = r.halt + 1;
+    } else {
+      step = end + 1;
+    }
+  }
+  d->fin = d->full_tape ? d->tape_state(d->tape.p + (size_t)d->nsteps * c4) : cur;
+}
 
 // dtheta (nullable): a parameter direction per specimen; the run then also
 // carries the state's tangent along it and dloss gets d loss / d epsilon at
@@ -1368,10 +1465,8 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
                       d->stream));
   d->stress_dev.reserve((size_t)std::max(ns, 1) * d->nspec);
   d->digest.reserve((size_t)d->nsteps + 1);
-  DCHK(hipMemsetAsync(d->digest.p, 0, sizeof(unsigned long long) * (d->nsteps + 1), d->stream));
-  d->epochs.clear();
-  d->ckpts.clear();
-  d->rebuild_steps.clear();
+  d->have_forward = false;
+  d->fin = DState{};
   d->tan_on = dtheta != nullptr;
   if (d->tan_on) {
     const size_t c = std::max(d->n, 1);
@@ -1389,12 +1484,12 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
                         d->stream));
     dsync(d);  // the copy reads dt4, which ends with this block
   }
-  upload_initial(d);
   // wall origins of every step: moved by their step before every step (the
   // pre-time-step moveWallBy of the main engine's setWallStepMotion)
   {
     const int nw = std::max(d->nw, 1);
-    std::vector<double> wo((size_t)(d->nsteps + 2) * nw * 3, 0.0);
+    std::vector<double>& wo = d->wo;
+    wo.assign((size_t)(d->nsteps + 2) * nw * 3, 0.0);
     double o[DIFF_MAX_WALLS][3];
     for (int k = 0; k < d->nw; k++)
       for (int c = 0; c < 3; c++) o[k][c] = d->wall0[k].o[c];
@@ -1404,48 +1499,18 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
       for (int k = 0; k < d->nw; k++)
         for (int c = 0; c < 3; c++) o[k][c] = o[k][c] + d->wstep[k][c];
     }
-    d->wo.reserve(wo.size());
-    DCHK(hipMemcpyAsync(d->wo.p, wo.data(), sizeof(double) * wo.size(), hipMemcpyHostToDevice,
-                        d->stream));
-    dsync(d);  // the copy reads wo, which ends with this block
   }
   d->run.reserve(1);
   d->wfn.reserve(std::max(d->n, 1));
-  drop_graph(d);
-  // chunks of steps between checkpoints queued without host decisions; a step
-  // whose displacement asks for a neighbour search halts the queue, the host
-  // rebuilds the table before the next step and continues
-  const int K = std::max(1, d->cfg.checkpoint_every);
-  bool need = true;
-  int step = 1;
-  while (step <= d->nsteps) {
-    if (need) {
-      drop_graph(d);
-      rebuild(d, step);
-      need = false;
-    }
-    if ((step - 1) % K == 0) save_checkpoint(d, step);
-    const int end = std::min(d->nsteps, ((step - 1) / K + 1) * K);
-    set_run(d, step, end);
-    run_chunk(d, step, end);
-    DRun r;
-    DCHK(hipMemcpyAsync(&r, d->run.p, sizeof r, hipMemcpyDeviceToHost, d->stream));
+  try {
+    run_forward(d, true);
+  } catch (const DiffMemory&) {
+    // no room for the run's tape: again with checkpoints
+    if (!d->full_tape) throw;
     dsync(d);
-    if (r.halt != 0) {
-      need = true;
-      step = r.halt + 1;
-    } else {
-      step = end + 1;
-    }
-  }
-  drop_graph(d);
-  {
-    const size_t c = std::max(d->n, 1);
-    d->fx.reserve(c); d->fv.reserve(c); d->fw.reserve(c); d->fq.reserve(c);
-    d->fbstep.reserve(std::max(d->nb, 1));
-    d2d(d, d->fx.p, d->x.p, d->n); d2d(d, d->fv.p, d->v.p, d->n);
-    d2d(d, d->fw.p, d->w.p, d->n); d2d(d, d->fq.p, d->q.p, d->n);
-    d2d(d, d->fbstep.p, d->bstep.p, d->nb);
+    d->tape.release();
+    d->hchunk.clear();
+    run_forward(d, false);
   }
   d->h_stress.assign((size_t)ns * d->nspec, 0.0);
   DCHK(hipMemcpyAsync(d->h_stress.data(), d->stress_dev.p, sizeof(double) * ns * d->nspec,
@@ -1507,19 +1572,19 @@ void backward(esp_diff* d, double* grad)
   coef_d.reserve(coef.size());
   DCHK(hipMemcpyAsync(coef_d.p, coef.data(), sizeof(double) * coef.size(), hipMemcpyHostToDevice,
                       d->stream));
-  DevBuf<double4> lam, gth, lh, lh2;
-  DevBuf<double> lfm, ab, ac;
-  DevBuf<unsigned char> aact;  // per pair: its record holds a Jacobian this step
+  auto &lam = d->lam, &gth = d->gth, &lh = d->lh, &lh2 = d->lh2;
+  auto &lfm = d->lfm, &ab = d->ab, &ac = d->ac;
+  auto& aact = d->aact;
   lam.reserve(4 * c);
   gth.reserve(c);
   lfm.reserve(6 * c);
   ab.reserve((size_t)std::max(d->nb, 1) * NB_TAN);
   DCHK(hipMemsetAsync(lam.p, 0, sizeof(double4) * 4 * c, d->stream));
   DCHK(hipMemsetAsync(gth.p, 0, sizeof(double4) * c, d->stream));
-  // tape of one segment: states of steps s0..s1, histories read at s0..s1-1
-  DevBuf<double4> tape;
-  tape.reserve((size_t)(K + 1) * 4 * c);
-  std::vector<std::unique_ptr<DevBuf<double4>>> htape;
+  const size_t c4 = 4 * (size_t)n;
+  // without the run's tape: that of one segment, the states of steps s0..s1 and
+  // the histories read at s0..s1-1
+  if (!d->full_tape) d->tape.reserve((size_t)(K + 1) * c4);
   int lh_epoch = -1;  // epoch whose pairs lh is indexed by
   DBonds B{d->nb, d->bij.p, d->bD0.p, d->brel.p, d->bstep.p, d->tkb.p};
   auto epoch_of = [&](int step) {
@@ -1527,96 +1592,94 @@ void backward(esp_diff* d, double* grad)
     while (e + 1 < (int)d->epochs.size() && d->epochs[e + 1]->start <= step) e++;
     return e;
   };
-  for (int seg = (int)d->ckpts.size() - 1; seg >= 0; seg--) {
-    const Checkpoint& C = *d->ckpts[seg];
-    const int s0 = C.step, s1 = std::min(s0 + K, d->nsteps + 1);
-    restore_checkpoint(d, C);
-    // recompute the segment forward, recording the states and histories
-    if ((int)htape.size() < K) htape.resize(K);
-    int cur = C.epoch;
-    set_run(d, s0, s1 - 1);
-    for (int step = s0; step < s1; step++) {
-      const int e = epoch_of(step);
-      if (e != cur) {  // the rebuild of this step: histories carried by key
-        const Epoch& E = *d->epochs[e];
-        DevBuf<double4> hn;
-        hn.reserve(std::max(E.nc, 1));
-        if (E.nc > 0)
-          hipLaunchKernelGGL(k_carry_hist, dim3(nblocks(E.nc, bs)), dim3(bs), 0, d->stream, E.nc,
-                             E.src.p, d->H[step & 1].p, hn.p);
-        d->H[step & 1].swap(hn);
-        d->H[(step + 1) & 1].reserve(std::max(E.nc, 1));
-        d2d(d, d->H[(step + 1) & 1].p, d->H[step & 1].p, E.nc);
-        d->cout.reserve((size_t)std::max(E.nc, 1) * 9);
-        d->cact.reserve((size_t)std::max(E.nc, 1));
-        cur = e;
+  clear_run(d);
+  const int nseg = d->full_tape ? 1 : (int)d->ckpts.size();
+  for (int seg = nseg - 1; seg >= 0; seg--) {
+    const int s0 = d->full_tape ? 1 : d->ckpts[seg]->step;
+    const int s1 = d->full_tape ? d->nsteps + 1 : std::min(s0 + K, d->nsteps + 1);
+    auto state_before = [&](int step) { return d->tape_state(d->tape.p + (size_t)(step - s0) * c4); };
+    if (!d->full_tape) {
+      const Checkpoint& C = *d->ckpts[seg];
+      restore_checkpoint(d, C, d->tape.p);
+      // recompute the segment forward, recording the states and histories
+      if ((int)d->hseg.size() < K) d->hseg.resize(K);
+      int cur = C.epoch;
+      for (int step = s0; step < s1; step++) {
+        const int e = epoch_of(step);
+        if (e != cur) {  // the rebuild of this step: histories carried by key
+          const Epoch& E = *d->epochs[e];
+          DevBuf<double4> hn;
+          hn.reserve(std::max(E.nc, 1));
+          if (E.nc > 0)
+            hipLaunchKernelGGL(k_carry_hist, dim3(nblocks(E.nc, bs)), dim3(bs), 0, d->stream, E.nc,
+                               E.src.p, d->H[step & 1].p, hn.p);
+          d->H[step & 1].swap(hn);
+          d->H[(step + 1) & 1].reserve(std::max(E.nc, 1));
+          d2d(d, d->H[(step + 1) & 1].p, d->H[step & 1].p, E.nc);
+          d->cout.reserve((size_t)std::max(E.nc, 1) * 9);
+          d->cact.reserve((size_t)std::max(E.nc, 1));
+          dsync(d);  // hn now holds the old histories, freed with this block
+          cur = e;
+        }
+        const int t = step - s0;
+        if (!d->hseg[t]) d->hseg[t] = std::make_unique<DevBuf<double4>>();
+        d->hseg[t]->reserve(std::max(d->epochs[cur]->nc, 1));
+        fwd_step(d, *d->epochs[cur], step, state_before(step), state_before(step + 1),
+                 d->hseg[t]->p, false, false);
       }
-      const int t = step - s0;
-      double4* T = tape.p + (size_t)t * 4 * c;
-      d2d(d, T, d->x.p, n); d2d(d, T + c, d->v.p, n); d2d(d, T + 2 * c, d->w.p, n);
-      d2d(d, T + 3 * c, d->q.p, n);
-      const int nc = d->epochs[cur]->nc;
-      if (!htape[t]) htape[t] = std::make_unique<DevBuf<double4>>();
-      htape[t]->reserve(std::max(nc, 1));
-      d2d(d, htape[t]->p, d->H[step & 1].p, nc);
-      fwd_step(d, *d->epochs[cur], false, false);
     }
-    {
-      double4* T = tape.p + (size_t)(s1 - s0) * 4 * c;
-      d2d(d, T, d->x.p, n); d2d(d, T + c, d->v.p, n); d2d(d, T + 2 * c, d->w.p, n);
-      d2d(d, T + 3 * c, d->q.p, n);
-    }
-    // reverse sweep
+    // reverse sweep: a step's particle updates, its laws, then its gather with
+    // the particle updates of the step before it
+    auto coef_of = [&](int step) {
+      return step % d->every == 0 ? coef_d.p + (size_t)(step / d->every - 1) * d->nspec : nullptr;
+    };
+    const dim3 g4(nblocks(4ll * n, bs));
+    hipLaunchKernelGGL((k_adj_step<false, true>), g4, dim3(bs), 0, d->stream, n, nullptr, nullptr, 0,
+                       nullptr, nullptr, nullptr, nullptr, 0, lam.p, gth.p, state_before(s1 - 1),
+                       state_before(s1), lfm.p, d->step_params(s1 - 1), coef_of(s1 - 1));
     for (int step = s1 - 1; step >= s0; step--) {
       const int e = epoch_of(step);
       const Epoch& E = *d->epochs[e];
       if (lh_epoch != e) {
         // the history adjoint of the next step's pairs, taken back to this
         // step's pairs (the next step started an epoch) or started at zero
-        DevBuf<double4> nl;
-        nl.reserve(std::max(E.nc, 1));
-        DCHK(hipMemsetAsync(nl.p, 0, sizeof(double4) * std::max(E.nc, 1), d->stream));
+        lh2.reserve(std::max(E.nc, 1));
+        DCHK(hipMemsetAsync(lh2.p, 0, sizeof(double4) * std::max(E.nc, 1), d->stream));
         if (lh_epoch >= 0) {
           const Epoch& N = *d->epochs[lh_epoch];
           if (N.nc > 0)
             hipLaunchKernelGGL(k_map_lh, dim3(nblocks(N.nc, bs)), dim3(bs), 0, d->stream, N.nc,
-                               N.src.p, lh.p, nl.p);
+                               N.src.p, lh.p, lh2.p);
         }
-        lh.swap(nl);
+        lh.swap(lh2);
         lh_epoch = e;
         lh2.reserve(std::max(E.nc, 1));
         ac.reserve((size_t)std::max(E.nc, 1) * NF_TAN);
         aact.reserve((size_t)std::max(E.nc, 1));
       }
-      const int t = step - s0;
-      double4* T0 = tape.p + (size_t)t * 4 * c;
-      double4* T1 = tape.p + (size_t)(t + 1) * 4 * c;
-      DState Sn{T0, T0 + c, T0 + 2 * c, T0 + 3 * c, d->spec.p, n};
-      DState Sn1{T1, T1 + c, T1 + 2 * c, T1 + 3 * c, d->spec.p, n};
-      const bool sample = step % d->every == 0;
-      const double* cf = sample ? coef_d.p + (size_t)(step / d->every - 1) * d->nspec : nullptr;
-      hipLaunchKernelGGL(k_adj_particle, dim3(nblocks(n, bs)), dim3(bs), 0, d->stream, Sn, Sn1,
-                         lam.p, lfm.p, d->step_params(step), cf);
+      const DState Sn = state_before(step);
       if (d->nb > 0)
         hipLaunchKernelGGL(k_adj_bond, dim3(nblocks(d->nb, ADJ_BOND_BS)), dim3(ADJ_BOND_BS), 0,
                            d->stream, Sn, B, d->theta.p, step, lfm.p, ab.p);
       DCands Cd{E.nc, E.ij.p, E.bond.p};
       if (E.nc > 0)
         hipLaunchKernelGGL(k_adj_fric, dim3(nblocks(E.nc, bs)), dim3(bs), 0, d->stream, Sn, Cd,
-                           d->bstep.p, d->theta.p, htape[t]->p, step, d->cfg.dt, lfm.p, lh.p, ac.p,
-                           aact.p, lh2.p);
-      hipLaunchKernelGGL(k_adj_gather, dim3(nblocks(n, bs)), dim3(bs), 0, d->stream, n,
-                         E.inc_off.p, E.inc_ent.p, E.nc, ac.p, ab.p, aact.p, d->bstep.p, step,
-                         lam.p, gth.p);
+                           d->bstep.p, d->theta.p, d->full_tape ? d->htape[step] : d->hseg[step - s0]->p,
+                           step, d->cfg.dt, lfm.p, lh.p, ac.p, aact.p, lh2.p);
+      if (step > s0)
+        hipLaunchKernelGGL((k_adj_step<true, true>), g4, dim3(bs), 0, d->stream, n, E.inc_off.p,
+                           E.inc_ent.p, E.nc, ac.p, ab.p, aact.p, d->bstep.p, step, lam.p, gth.p,
+                           state_before(step - 1), Sn, lfm.p, d->step_params(step - 1),
+                           coef_of(step - 1));
+      else
+        hipLaunchKernelGGL((k_adj_step<true, false>), g4, dim3(bs), 0, d->stream, n, E.inc_off.p,
+                           E.inc_ent.p, E.nc, ac.p, ab.p, aact.p, d->bstep.p, step, lam.p, gth.p, Sn,
+                           Sn, lfm.p, d->step_params(step), nullptr);
       DCHK(hipGetLastError());
       lh.swap(lh2);
     }
-    dsync(d);
+    if (!d->full_tape) dsync(d);
   }
-  // the forward run's final state and break steps, for later queries
-  d2d(d, d->x.p, d->fx.p, n); d2d(d, d->v.p, d->fv.p, n);
-  d2d(d, d->w.p, d->fw.p, n); d2d(d, d->q.p, d->fq.p, n);
-  d2d(d, d->bstep.p, d->fbstep.p, d->nb);
   DevBuf<double4> gs;
   gs.reserve(std::max(d->nspec, 1));
   hipLaunchKernelGGL(k_spec_sum4, dim3(d->nspec), dim3(256), 0, d->stream, gth.p, d->spec_start.p,
@@ -1740,7 +1803,6 @@ void esp_diff_destroy(esp_diff* d)
 {
   if (!d) return;
   if (d->stream) (void)hipStreamSynchronize(d->stream);
-  drop_graph(d);
   d->epochs.clear();
   d->ckpts.clear();
   hipStream_t s = d->stream;
@@ -1779,6 +1841,23 @@ int esp_diff_set_particles(esp_diff* d, int n, int nspec, const int* spec, const
   d->ccnt.reserve(n + 1);
   d->coff.reserve(n + 1);
   d->wfn.reserve(n);
+  std::vector<double4> X(n), V(n), W(n), Q(n), O(n);
+  for (int i = 0; i < n; i++) {
+    const double m = d->h_mass[i], r = d->h_rad[i];
+    X[i] = make_double4(d->h_pos[3 * i], d->h_pos[3 * i + 1], d->h_pos[3 * i + 2], r);
+    V[i] = make_double4(d->h_vel[3 * i], d->h_vel[3 * i + 1], d->h_vel[3 * i + 2],
+                        m != 0.0 ? 1.0 / m : 0.0);
+    const double I = 0.4 * m * r * r;  // CRotParticle, 3-D (RotParticle.cpp:80-124)
+    W[i] = make_double4(0.0, 0.0, 0.0, 1.0 / I);
+    Q[i] = make_double4(1.0, 0.0, 0.0, 0.0);
+    O[i] = make_double4(X[i].x, X[i].y, X[i].z, m);
+  }
+  d->x0.reserve(n); d->v0.reserve(n); d->w0.reserve(n); d->q0.reserve(n); d->o.reserve(n);
+  DCHK(hipMemcpyAsync(d->x0.p, X.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
+  DCHK(hipMemcpyAsync(d->v0.p, V.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
+  DCHK(hipMemcpyAsync(d->w0.p, W.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
+  DCHK(hipMemcpyAsync(d->q0.p, Q.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
+  DCHK(hipMemcpyAsync(d->o.p, O.data(), sizeof(double4) * n, hipMemcpyHostToDevice, d->stream));
   std::vector<int> ids(n);
   std::vector<unsigned> fl(n, PF_DYN | PF_ROT);
   for (int i = 0; i < n; i++) ids[i] = i;
@@ -1789,6 +1868,7 @@ int esp_diff_set_particles(esp_diff* d, int n, int nspec, const int* spec, const
   DCHK(hipMemcpyAsync(d->flags.p, fl.data(), sizeof(unsigned) * n, hipMemcpyHostToDevice,
                       d->stream));
   dsync(d);
+  d->fin = DState{};
   d->have_forward = false;
   return ESP_OK;
   DAPI_END
@@ -1925,8 +2005,9 @@ int esp_diff_get_particle_data(esp_diff* d, int field, double* out)
   DAPI_BEGIN
   const int n = d->n;
   std::vector<double4> a(n);
-  const double4* src = field == ESP_FIELD_POS ? d->x.p : field == ESP_FIELD_VEL ? d->v.p
-                     : field == ESP_FIELD_ANGVEL ? d->w.p : field == ESP_FIELD_QUAT ? d->q.p : nullptr;
+  const double4* src = field == ESP_FIELD_POS ? d->fin.x : field == ESP_FIELD_VEL ? d->fin.v
+                     : field == ESP_FIELD_ANGVEL ? d->fin.w : field == ESP_FIELD_QUAT ? d->fin.q
+                                                                                     : nullptr;
   if (!src) throw DiffError(ESP_ERR_ARG, "unknown field");
   DCHK(hipMemcpyAsync(a.data(), src, sizeof(double4) * n, hipMemcpyDeviceToHost, d->stream));
   dsync(d);

@@ -29,6 +29,7 @@
 
 #include "esp_internal.h"
 #include "esp_math.h"
+#include "esp_wave.h"
 
 #define BS 256
 #ifndef ESP_G_EL
@@ -418,33 +419,6 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
   return v;
 }
 
-// Sum over the wave in a fixed order, the same value in every lane: pairs within
-// the rows of 16 lanes by DPP (a few cycles a step where a shuffle through LDS
-// takes a hundred), then the four rows.  Every lane of the wave must be active.
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double v)
-{
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffll), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-__device__ __forceinline__ double lane_value(double v, int l)
-{
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), l);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-__device__ __forceinline__ double wave_sum(double v)
-{
-  v = v + dpp_move<0xB1>(v);   // lanes 1,0,3,2 of every four
-  v = v + dpp_move<0x4E>(v);   // lanes 2,3,0,1
-  v = v + dpp_move<0x141>(v);  // mirrored within 8 lanes
-  v = v + dpp_move<0x140>(v);  // mirrored within 16 lanes
-  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
-}
-
 // Fixed-order sum of (a, b, c) over the block, valid in thread 0: within each
 // wave, then the waves in index order.  Every thread of the block must call it.
 __device__ __forceinline__ void block_sum3(double& a, double& b, double& c, double* lds)
@@ -791,30 +765,6 @@ __global__ __launch_bounds__(BS) void k_batch_end(BatchEnd be)
 // ---------------------------------------------------------------------------
 // one whole step of an engine without bonded groups
 // ---------------------------------------------------------------------------
-// The value lane `q` of this lane's group of G (2 or 4) lanes holds
-template <int G>
-__device__ __forceinline__ double group_value(double v, int q)
-{
-  const long long b = __double_as_longlong(v);
-  int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
-#define ESP_DPP(ctrl)                                             \
-  {                                                               \
-    lo = __builtin_amdgcn_mov_dpp(lo, ctrl, 0xf, 0xf, true);      \
-    hi = __builtin_amdgcn_mov_dpp(hi, ctrl, 0xf, 0xf, true);      \
-  }
-  if (G == 4) {
-    if (q == 0) ESP_DPP(0x00)
-    else if (q == 1) ESP_DPP(0x55)
-    else if (q == 2) ESP_DPP(0xAA)
-    else ESP_DPP(0xFF)
-  } else if (G == 2) {
-    if (q == 0) ESP_DPP(0xA0)
-    else ESP_DPP(0xF5)
-  }
-#undef ESP_DPP
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-
 // bits of the four lanes of a group of 4
 __device__ __forceinline__ unsigned long long group_or(unsigned long long v)
 {

@@ -31,10 +31,11 @@
  *
  * Gradients: esp_diff_backward differentiates every specimen's loss with
  * respect to its theta exactly along the branch the forward run took (contact
- * topology, slip states and bond breaks as recorded): a reverse sweep over
- * checkpointed segments of `checkpoint_every` steps, each recomputed forward
- * before its adjoint; the laws' local Jacobians come from their dual-number
- * evaluation (esp_difflaw.h).  The break criterion depends on cohesion only
+ * topology, slip states and bond breaks as recorded): a reverse sweep over the
+ * states the forward run kept or, for a run whose states exceed 24 GiB (or one by
+ * esp_diff_forward_tangent), over checkpointed segments of `checkpoint_every`
+ * steps, each recomputed forward before its adjoint; the laws' vector-Jacobian
+ * products are their hand-written reverse mode (esp_difflaw.h).  The break criterion depends on cohesion only
  * through events, so d loss / d cohesion is zero on the branch.
  */
 #ifndef ESP_DIFF_H
