@@ -300,9 +300,12 @@ __device__ __forceinline__ void bond_fwd_item(const DState& S, const DBonds& B, 
   if (b >= B.nb) return;
   double* o = bout + 9 * (size_t)b;
   const int bs = B.bstep[b];
-  // removed after the step whose criterion broke it: no record (the gathers
-  // skip a bond whose break step is before theirs)
-  if (bs < step) return;
+  // removed after the step whose criterion broke it: the record is zero from then on
+  if (bs < step) {
+    if (bs == step - 1)
+      for (int k = 0; k < 9; k++) o[k] = 0.0;
+    return;
+  }
   const int2 e = B.ij[b];
   const double4 P1 = S.x[e.x], P2 = S.x[e.y], Q1 = S.q[e.x], Q2 = S.q[e.y];
   const double4 D = B.D0[b];
@@ -420,23 +423,21 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_bond_fwd_pairs(DState S, DBonds
 // per particle: the measured wall's normal force on it (sample steps), walls,
 // gravity, interactions in CSR order, then the update from S into So (the same
 // arrays, or the next step's of a tape).
-// Bound by the chain entry -> activity -> record over a particle's run.  Four
-// lanes share a particle: each takes every fourth entry, two at a time, and the
-// shares are added in entry order by all of them; the block's first threads, one
-// for each of its particles, integrate.  Against one lane a particle (us a step):
-// 2,000 particles 22.0 -> 11.0, 20,000 26.6 -> 12.4, 24 specimens together
-// (230,000) 55.0 -> 49.1, so there is no size to go back to one lane.  TAN: the
-// state's tangent is carried along.
-template <bool TAN>
+// Bound by the chain entry -> activity -> record over a particle's run.  G lanes (a
+// quad, or a row of 16) share a particle: each takes every G-th entry, with the next
+// one's activity and the entry after that under way, and the shares are added in
+// entry order by all of them; the block's first threads, one for each of its
+// particles, integrate.  One lane a particle -> this (us a step): 2,000 particles
+// 22.0 -> 6.9, 20,000 26.6 -> 11.1, 254,000 55.0 -> 41.4.  TAN: the state's tangent
+// is carried along.
+template <int G, bool TAN>
 __global__ __launch_bounds__(DIFF_MAX_BS) void k_gather_fwd(
     DState S, DState So, const double4* mass_old, const int* inc_off, const int* inc_ent, int ncand,
-    const double* cout, const double* bout, const unsigned char* cact, const int* bstep, DStep sp,
+    const double* cout, const double* bout, const unsigned char* cact, DStep sp,
     double* wfn, DRun* run, unsigned long long thresh, unsigned long long* dig_base, DTan T,
     const double* ct, const double* bt, double* wft)
 {
   constexpr int NS = TAN ? 12 : 6;
-  constexpr int G = 4;
-  constexpr int R = 2;  // entries a lane has in flight
   __shared__ double sum[NS * (DIFF_MAX_BS / G)];  // [particle][component]
   const int step = sp.step;
   const int t = threadIdx.x;
@@ -497,49 +498,34 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_gather_fwd(
     for (int c = 0; c < NS; c++) acc[c] = (c < 3 || (c >= 6 && c < 9)) ? o[c] : 0.0;
   }
   // The interactions in CSR order.  A record with no force this step (a pair
-  // apart or excluded by its bond, a bond broken in an earlier step) adds zeros:
-  // a sum that starts at +0 is not changed by a zero.
-  int ent[R];
-#pragma unroll
-  for (int r = 0; r < R; r++) ent[r] = e0 + r * G + sub < e1 ? inc_ent[e0 + r * G + sub] : -1;
-  for (int b = e0; b < e1; b += R * G) {  // as often for the G lanes of a particle
-    bool on[R];
-    double v[R][NS];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int rec = ent[r] >> 1;
-      on[r] = ent[r] >= 0 && (rec < ncand ? cact[rec] != 0 : bstep[rec - ncand] >= step);
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      for (int c = 0; c < NS; c++) v[r][c] = 0.0;
-      if (!on[r]) continue;
-      const int rec = ent[r] >> 1, side = ent[r] & 1;
+  // apart or excluded by its bond) adds zeros: a sum that starts at +0 is not
+  // changed by a zero.
+  auto entry = [&](int at) { return at < e1 ? inc_ent[at] : -1; };
+  auto active = [&](int e) { return e >= 0 && ((e >> 1) >= ncand || cact[e >> 1] != 0); };
+  int ent = entry(e0 + sub), nxt = entry(e0 + G + sub);
+  bool on = active(ent);
+  for (int b = e0; b < e1; b += G) {  // as often for the G lanes of a particle
+    double v[NS];
+    for (int c = 0; c < NS; c++) v[c] = 0.0;
+    if (on) {
+      const int rec = ent >> 1, side = ent & 1;
       const size_t at = 9 * (size_t)(rec < ncand ? rec : rec - ncand);
       const double* q = (rec < ncand ? cout : bout) + at;
       const double* qm = q + 3 + 3 * side;
       const double sg = side ? -1.0 : 1.0;  // the second particle's force is the opposite
-      v[r][0] = sg * q[0]; v[r][1] = sg * q[1]; v[r][2] = sg * q[2];
-      v[r][3] = qm[0]; v[r][4] = qm[1]; v[r][5] = qm[2];
+      v[0] = sg * q[0]; v[1] = sg * q[1]; v[2] = sg * q[2];
+      v[3] = qm[0]; v[4] = qm[1]; v[5] = qm[2];
       if (TAN) {
         const double* u = (rec < ncand ? ct : bt) + at;
         const double* um = u + 3 + 3 * side;
-        v[r][6] = sg * u[0]; v[r][7] = sg * u[1]; v[r][8] = sg * u[2];
-        v[r][9] = um[0]; v[r][10] = um[1]; v[r][11] = um[2];
+        v[6] = sg * u[0]; v[7] = sg * u[1]; v[8] = sg * u[2];
+        v[9] = um[0]; v[10] = um[1]; v[11] = um[2];
       }
     }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int nx = b + (R + r) * G + sub;
-      ent[r] = nx < e1 ? inc_ent[nx] : -1;
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-#pragma unroll
-      for (int k = 0; k < G; k++)
-        for (int c = 0; c < NS; c++)
-          acc[c] = acc[c] + group_value<G>(v[r][c], k);
-    }
+    ent = nxt;
+    on = active(ent);
+    nxt = entry(b + 2 * G + sub);
+    add_in_order<G>(acc, v);
   }
   __syncthreads();  // the walls' forces have been read
   if (sub == 0)
@@ -755,8 +741,12 @@ __device__ __forceinline__ void adj_particle_item(const DState& Sn, const DState
   o[3] = lM.x; o[4] = lM.y; o[5] = lM.z;
 }
 
-#define NB_TAN 16
-#define NF_TAN 24
+// Interaction adjoints, 32-byte vectors that one lane of k_adj_step loads whole:
+// of a bond (x1, kn), (x2, ks), q1, q2 (its particles are of one specimen); of a
+// pair (x1, kn), (x2, 0), (v1, mu), (v2, 0), (w1, ks), (w2, 0): the parameters, in
+// the fourth component, are credited to the first particle's specimen.
+#define NB_REC 4
+#define NF_REC 6
 
 // bond law VJP: c[k] = lambda_out . d out / d in_k over the inputs
 // (x1, x2, q1, q2, theta_kn, theta_ks), one thread per bond, by the law's
@@ -764,12 +754,14 @@ __device__ __forceinline__ void adj_particle_item(const DState& Sn, const DState
 #define ADJ_BOND_BS 256
 __global__ __launch_bounds__(ADJ_BOND_BS) void k_adj_bond(DState S, DBonds B,
                                                            const double4* theta, int step,
-                                                           const double* lfm, double* ab)
+                                                           const double* lfm, double4* ab)
 {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= B.nb) return;
-  double* c = ab + NB_TAN * (size_t)b;
-  if (B.bstep[b] < step) return;  // broken earlier: no record (k_adj_step skips it)
+  // broken earlier: the record is the zero the sweep, which goes back in time,
+  // started with
+  if (B.bstep[b] < step) return;
+  double4* c = ab + NB_REC * (size_t)b;
   const int2 e = B.ij[b];
   const double4 P1 = S.x[e.x], P2 = S.x[e.y], Q1 = S.q[e.x], Q2 = S.q[e.y];
   const double4 D = B.D0[b];
@@ -791,12 +783,10 @@ __global__ __launch_bounds__(ADJ_BOND_BS) void k_adj_bond(DState S, DBonds B,
                 tv3<double>{D.x, D.y, D.z}, tv3<double>{l1[0] - l2[0], l1[1] - l2[1], l1[2] - l2[2]},
                 tv3<double>{l1[3], l1[4], l1[5]}, tv3<double>{l2[3], l2[4], l2[5]}, g1, g2, gq1, gq2,
                 gkr, gks);
-  c[0] = g1.x; c[1] = g1.y; c[2] = g1.z;
-  c[3] = g2.x; c[4] = g2.y; c[5] = g2.z;
-  c[6] = gq1.s; c[7] = gq1.v.x; c[8] = gq1.v.y; c[9] = gq1.v.z;
-  c[10] = gq2.s; c[11] = gq2.v.x; c[12] = gq2.v.y; c[13] = gq2.v.z;
-  c[14] = gkr * dkr;
-  c[15] = gks * dks;
+  c[0] = make_double4(g1.x, g1.y, g1.z, gkr * dkr);
+  c[1] = make_double4(g2.x, g2.y, g2.z, gks * dks);
+  c[2] = make_double4(gq1.s, gq1.v.x, gq1.v.y, gq1.v.z);
+  c[3] = make_double4(gq2.s, gq2.v.x, gq2.v.y, gq2.v.z);
 }
 
 // friction law VJP over the inputs (x1, x2, v1, v2, w1, w2, history,
@@ -808,11 +798,10 @@ __global__ __launch_bounds__(ADJ_BOND_BS) void k_adj_bond(DState S, DBonds B,
 // gather reads only such records.
 __global__ void k_adj_fric(DState S, DCands C, const int* bstep, const double4* theta,
                            const double4* hin, int step, double dt, const double* lfm,
-                           const double4* lh, double* ac, unsigned char* act, double4* lh_prev)
+                           const double4* lh, double4* ac, unsigned char* act, double4* lh_prev)
 {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= C.nc) return;
-  double* o = ac + NF_TAN * (size_t)c;
   const int bb = C.bond[c];
   if (bb >= 0 && bstep[bb] >= step) {
     // excluded while bonded: zero Jacobian.  The history adjoint it would pass
@@ -849,14 +838,9 @@ __global__ void k_adj_fric(DState S, DCands C, const int* bstep, const double4* 
                     tv3<double>{l1[0] - l2[0], l1[1] - l2[1], l1[2] - l2[2]},
                     tv3<double>{l1[3], l1[4], l1[5]}, tv3<double>{l2[3], l2[4], l2[5]},
                     tv3<double>{lo.x, lo.y, lo.z}, g);
-  for (int t = 0; t < 7; t++) {
-    o[3 * t] = g[t].x;
-    o[3 * t + 1] = g[t].y;
-    o[3 * t + 2] = g[t].z;
-  }
-  o[21] = g[7].x * dk;
-  o[22] = g[7].y * dks;
-  o[23] = g[7].z;
+  double4* o = ac + NF_REC * (size_t)c;
+  const double par[6] = {g[7].x * dk, 0.0, g[7].z, 0.0, g[7].y * dks, 0.0};
+  for (int t = 0; t < 6; t++) o[t] = make_double4(g[t].x, g[t].y, g[t].z, par[t]);
   lh_prev[c] = make_double4(g[6].x, g[6].y, g[6].z, 0.0);
 }
 
@@ -866,96 +850,94 @@ __global__ void k_adj_fric(DState S, DCands C, const int* bstep, const double4* 
 // in the step before, sp.step, is taken back (PART: states Sn, Sn1, adjoints for
 // its interactions to lfm).  One launch between two steps' laws instead of two,
 // and lam passes through memory once.
-// Four lanes share a particle, each with one of lam's vectors: lane 0 adds the
-// position adjoints of every entry, 1 the velocities, 2 the angular velocities (of
-// a bond: the parameters), 3 the quaternions (of a pair: the parameters), so a
-// record's 96 bytes for one side are read by neighbouring lanes.  With the two parts
-// as launches of one lane a particle (us a step): 2,000 particles 20.4 + 5.0 -> 21.0,
-// 20,000 24.9 + 5.9 -> 28.6.  Records without a Jacobian this step (pairs apart or excluded, bonds broken earlier) are skipped.
-template <bool GATHER, bool PART>
+// The lanes of a quad take one of lam's vectors each (x, v, w, q) and load the
+// entry's record for that vector; the next entries' activity and the entries after
+// those are under way meanwhile.  G: one quad a particle, or four that take the
+// entries in turn and add them in entry order.  Records of pairs without a Jacobian
+// this step (apart or excluded) are skipped; those of bonds broken earlier are
+// zeros.  Two launches of one lane a particle, 13 components an entry -> this (us a
+// step): 2,000 particles 25.4 -> 8.2, 20,000 30.8 -> 13.2, 254,000 83.8 -> 72.6.
+template <bool GATHER, bool PART, int G>
 __global__ __launch_bounds__(DIFF_MAX_BS) void k_adj_step(
-    int n, const int* inc_off, const int* inc_ent, int ncand, const double* ac, const double* ab,
-    const unsigned char* cact, const int* bstep, int step, double4* lam, double4* gth, DState Sn,
-    DState Sn1, double* lfm, DStep sp, const double* coef)
+    int n, const int* inc_off, const int* inc_ent, int ncand, const double4* ac, const double4* ab,
+    const unsigned char* cact, double4* lam, double4* gth, DState Sn, DState Sn1, double* lfm,
+    DStep sp, const double* coef)
 {
-  constexpr int G = 4, R = 4;
-  __shared__ double4 sl[PART ? DIFF_MAX_BS : 1];
+  constexpr int NQ = G / 4;         // quads a particle
+  constexpr int R = G == 4 ? 4 : 2;  // entries a quad has in flight
+  __shared__ double4 sl[PART ? DIFF_MAX_BS / NQ : 1];
   const int t = threadIdx.x;
   const int PB = blockDim.x / G;
   const int p0 = blockIdx.x * PB;
-  const int pi = p0 + t / G, sub = t % G;
+  const int pi = p0 + t / G, sub = t % 4, quad = (t % G) / 4;
   const int pc = pi < n ? pi : 0;
   double4 L = lam[4 * (size_t)pc + sub];
   if (GATHER) {
     const int e0 = inc_off[pc], e1 = pi < n ? inc_off[pc + 1] : e0;
-    double ga[3] = {0.0, 0.0, 0.0};
-    int ent[R];
+    // the vector's adjoint; parameters: in the lanes of x, v, w kn, mu, the pairs'
+    // ks; the bonds' ks (in the first quad of a particle)
+    double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    auto entry = [&](int at) { return at < e1 ? inc_ent[at] : -1; };
+    auto active = [&](int ent) {
+      return ent >= 0 && ((ent >> 1) >= ncand || cact[ent >> 1] != 0);
+    };
+    int ent[R], nxt[R];
+    bool on[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) ent[r] = e0 + r < e1 ? inc_ent[e0 + r] : -1;
-    for (int b = e0; b < e1; b += R) {
-      bool on[R];
-      double a[R][4];
+    for (int r = 0; r < R; r++) ent[r] = entry(e0 + r * NQ + quad);
+#pragma unroll
+    for (int r = 0; r < R; r++) nxt[r] = entry(e0 + (R + r) * NQ + quad);
+#pragma unroll
+    for (int r = 0; r < R; r++) on[r] = active(ent[r]);
+    for (int b = e0; b < e1; b += R * NQ) {
+      double4 a[R];
+      int side[R];
 #pragma unroll
       for (int r = 0; r < R; r++) {
+        a[r] = make_double4(0.0, 0.0, 0.0, 0.0);
         const int rec = ent[r] >> 1;
-        on[r] = ent[r] >= 0 && (rec < ncand ? cact[rec] != 0 : bstep[rec - ncand] >= step);
-      }
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        a[r][0] = a[r][1] = a[r][2] = a[r][3] = 0.0;
-        const int rec = ent[r] >> 1, side = ent[r] & 1;
-        const bool pair = rec < ncand;
-        // a pair: x, v, w at 0, 6, 12 (+3 for the second), parameters at 21; a
-        // bond: x at 0, q at 6 (+4 for the second), parameters at 14
-        const int at = pair ? (sub == 3 ? 21 : 6 * sub + 3 * side)
-                            : (sub == 0 ? 3 * side : sub == 3 ? 6 + 4 * side : 14);
-        const bool use = on[r] && (pair ? (sub < 3 || side == 0)
-                                        : (sub == 0 || sub == 3 || (sub == 2 && side == 0)));
-        if (!use) continue;
-        const double* c = pair ? ac + NF_TAN * (size_t)rec + at : ab + NB_TAN * (size_t)(rec - ncand) + at;
-        a[r][0] = c[0];
-        a[r][1] = c[1];
-        if (pair || sub != 2) a[r][2] = c[2];
-        if (!pair && sub == 3) a[r][3] = c[3];
-      }
-      bool par[R];  // this lane's terms of the entry are parameter gradients
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        par[r] = (ent[r] >> 1) < ncand ? sub == 3 : sub == 2;
-        const int nx = b + R + r;
-        ent[r] = nx < e1 ? inc_ent[nx] : -1;
-      }
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        if (par[r]) {
-          ga[0] += a[r][0];
-          ga[1] += a[r][1];
-          ga[2] += a[r][2];
-        } else {
-          L.x += a[r][0];
-          L.y += a[r][1];
-          L.z += a[r][2];
-          L.w += a[r][3];
+        side[r] = ent[r] & 1;
+        if (!on[r]) continue;
+        if (rec < ncand) {
+          if (sub < 3) a[r] = ac[NF_REC * (size_t)rec + 2 * sub + side[r]];
+        } else if (sub == 0 || sub == 3) {
+          a[r] = ab[NB_REC * (size_t)(rec - ncand) + (sub ? 2 : 0) + side[r]];
         }
       }
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        ent[r] = nxt[r];
+        on[r] = active(ent[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < R; r++) nxt[r] = entry(b + (2 * R + r) * NQ + quad);
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const bool p = sub != 3, s2 = side[r] != 0;
+        const double v[6] = {a[r].x, a[r].y, a[r].z, p ? 0.0 : a[r].w, p && !s2 ? a[r].w : 0.0,
+                             p && s2 ? a[r].w : 0.0};
+        add_quads<NQ>(acc, v);
+      }
     }
-    // (kn, ks) of the bonds in lane 2, (kn, ks, mu) of the pairs in lane 3
-    const double g0 = group_value<G>(ga[0], 3) + group_value<G>(ga[0], 2);
-    const double g1 = group_value<G>(ga[1], 3) + group_value<G>(ga[1], 2);
-    const double g3 = group_value<G>(ga[2], 3);
-    if (sub == 0 && pi < n) {
+    L.x += acc[0];
+    L.y += acc[1];
+    L.z += acc[2];
+    L.w += acc[3];
+    const double g0 = acc[4], g1 = acc[5];
+    const double gmu = group_value<4>(g0, 1), gks = group_value<4>(g0, 2);
+    if (t % G == 0 && pi < n) {
       double4 g = gth[pi];
       g.x += g0;
-      g.y += g1;
-      g.w += g3;
+      g.y += g1 + gks;
+      g.w += gmu;
       gth[pi] = g;
     }
   }
   if (!PART) {
-    if (pi < n) lam[4 * (size_t)pi + sub] = L;
+    if (quad == 0 && pi < n) lam[4 * (size_t)pi + sub] = L;
     return;
   }
-  sl[t] = L;
+  if (quad == 0) sl[4 * (t / G) + sub] = L;
   __syncthreads();
   const int i = p0 + t;
   if (t < PB && i < n) {
@@ -964,7 +946,7 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_adj_step(
     for (int k = 0; k < 4; k++) sl[4 * t + k] = l4[k];
   }
   __syncthreads();
-  if (pi < n) lam[4 * (size_t)pi + sub] = sl[t];
+  if (quad == 0 && pi < n) lam[4 * (size_t)pi + sub] = sl[4 * (t / G) + sub];
 }
 
 // adjoint of the history read at the first step of an epoch, to the pairs of
@@ -1069,7 +1051,8 @@ struct esp_diff {
   std::vector<double4*> htape;                           // [step]
   // the reverse sweep's arrays
   DevBuf<double4> lam, gth, lh, lh2;
-  DevBuf<double> lfm, ab, ac;
+  DevBuf<double> lfm;
+  DevBuf<double4> ab, ac;
   DevBuf<unsigned char> aact;  // per pair: its record holds a Jacobian this step
   std::vector<std::unique_ptr<DevBuf<double4>>> hseg;
   DevBuf<double> bout, cout, wfn, stress_dev;
@@ -1131,6 +1114,12 @@ namespace {
 // segments and copying their states cost a third of a forward and backward pass
 // (2,000 particles, 100 steps: 12.7 -> 5.8 ms with the launches below)
 constexpr size_t kTapeBytes = (size_t)24 << 30;
+// A row of 16 lanes a particle up to this many particles, a quad above (the sums
+// are the same, bit by bit): the longest run of interactions sets the time while
+// the chip is not full.  Quad / row, us a step: forward gather 2,000 particles
+// 9.7 / 6.9, 20,000 11.1 / 12.1, 50,000 12.2 / 15.9; adjoint 2,000 14.5 / 8.2,
+// 20,000 17.0 / 13.2, 254,000 72.6 / 108.2.
+constexpr int kGatherRow = 8192, kAdjointRow = 32768;
 
 void dsync(esp_diff* d) { DCHK(hipStreamSynchronize(d->stream)); }
 
@@ -1328,9 +1317,13 @@ void fwd_step(esp_diff* d, const Epoch& E, int step, const DState& S, const DSta
   }
   const DStep sp = d->step_params(step);
   const bool sample = record && step % d->every == 0;
-  hipLaunchKernelGGL(d->tan_on ? k_gather_fwd<true> : k_gather_fwd<false>,
-                     dim3(nblocks(4ll * d->n, bs)), dim3(bs), 0, d->stream, S, So, d->o.p,
-                     E.inc_off.p, E.inc_ent.p, E.nc, d->cout.p, d->bout.p, d->cact.p, d->bstep.p, sp,
+  const bool wide = d->n <= kGatherRow;
+  const auto gather = d->tan_on ? k_gather_fwd<4, true>
+                      : wide    ? k_gather_fwd<16, false>
+                                : k_gather_fwd<4, false>;
+  hipLaunchKernelGGL(gather,
+                     dim3(nblocks((wide && !d->tan_on ? 16ll : 4ll) * d->n, bs)), dim3(bs), 0, d->stream, S, So, d->o.p,
+                     E.inc_off.p, E.inc_ent.p, E.nc, d->cout.p, d->bout.p, d->cact.p, sp,
                      sample ? d->wfn.p : nullptr, R, thresh, dig, T, d->ct.p, d->bt.p,
                      sample && d->tan_on ? d->wft.p : nullptr);
   if (sample) {
@@ -1573,12 +1566,14 @@ void backward(esp_diff* d, double* grad)
   DCHK(hipMemcpyAsync(coef_d.p, coef.data(), sizeof(double) * coef.size(), hipMemcpyHostToDevice,
                       d->stream));
   auto &lam = d->lam, &gth = d->gth, &lh = d->lh, &lh2 = d->lh2;
-  auto &lfm = d->lfm, &ab = d->ab, &ac = d->ac;
+  auto& lfm = d->lfm;
+  auto &ab = d->ab, &ac = d->ac;
   auto& aact = d->aact;
   lam.reserve(4 * c);
   gth.reserve(c);
   lfm.reserve(6 * c);
-  ab.reserve((size_t)std::max(d->nb, 1) * NB_TAN);
+  ab.reserve((size_t)std::max(d->nb, 1) * NB_REC);
+  DCHK(hipMemsetAsync(ab.p, 0, sizeof(double4) * NB_REC * std::max(d->nb, 1), d->stream));
   DCHK(hipMemsetAsync(lam.p, 0, sizeof(double4) * 4 * c, d->stream));
   DCHK(hipMemsetAsync(gth.p, 0, sizeof(double4) * c, d->stream));
   const size_t c4 = 4 * (size_t)n;
@@ -1633,10 +1628,15 @@ void backward(esp_diff* d, double* grad)
     auto coef_of = [&](int step) {
       return step % d->every == 0 ? coef_d.p + (size_t)(step / d->every - 1) * d->nspec : nullptr;
     };
-    const dim3 g4(nblocks(4ll * n, bs));
-    hipLaunchKernelGGL((k_adj_step<false, true>), g4, dim3(bs), 0, d->stream, n, nullptr, nullptr, 0,
-                       nullptr, nullptr, nullptr, nullptr, 0, lam.p, gth.p, state_before(s1 - 1),
-                       state_before(s1), lfm.p, d->step_params(s1 - 1), coef_of(s1 - 1));
+    const bool wide = n <= kAdjointRow;
+    auto adj_step = [&](auto kern, const Epoch* E, const DState& Sn, const DState& Sn1, int part) {
+      hipLaunchKernelGGL(kern, dim3(nblocks((wide ? 16ll : 4ll) * n, bs)), dim3(bs), 0, d->stream, n,
+                         E ? E->inc_off.p : nullptr, E ? E->inc_ent.p : nullptr, E ? E->nc : 0, ac.p,
+                         ab.p, aact.p, lam.p, gth.p, Sn, Sn1, lfm.p,
+                         d->step_params(part), part > 0 ? coef_of(part) : nullptr);
+    };
+    adj_step(wide ? k_adj_step<false, true, 16> : k_adj_step<false, true, 4>, nullptr,
+             state_before(s1 - 1), state_before(s1), s1 - 1);
     for (int step = s1 - 1; step >= s0; step--) {
       const int e = epoch_of(step);
       const Epoch& E = *d->epochs[e];
@@ -1654,7 +1654,7 @@ void backward(esp_diff* d, double* grad)
         lh.swap(lh2);
         lh_epoch = e;
         lh2.reserve(std::max(E.nc, 1));
-        ac.reserve((size_t)std::max(E.nc, 1) * NF_TAN);
+        ac.reserve((size_t)std::max(E.nc, 1) * NF_REC);
         aact.reserve((size_t)std::max(E.nc, 1));
       }
       const DState Sn = state_before(step);
@@ -1667,14 +1667,10 @@ void backward(esp_diff* d, double* grad)
                            d->bstep.p, d->theta.p, d->full_tape ? d->htape[step] : d->hseg[step - s0]->p,
                            step, d->cfg.dt, lfm.p, lh.p, ac.p, aact.p, lh2.p);
       if (step > s0)
-        hipLaunchKernelGGL((k_adj_step<true, true>), g4, dim3(bs), 0, d->stream, n, E.inc_off.p,
-                           E.inc_ent.p, E.nc, ac.p, ab.p, aact.p, d->bstep.p, step, lam.p, gth.p,
-                           state_before(step - 1), Sn, lfm.p, d->step_params(step - 1),
-                           coef_of(step - 1));
+        adj_step(wide ? k_adj_step<true, true, 16> : k_adj_step<true, true, 4>, &E,
+                 state_before(step - 1), Sn, step - 1);
       else
-        hipLaunchKernelGGL((k_adj_step<true, false>), g4, dim3(bs), 0, d->stream, n, E.inc_off.p,
-                           E.inc_ent.p, E.nc, ac.p, ab.p, aact.p, d->bstep.p, step, lam.p, gth.p, Sn,
-                           Sn, lfm.p, d->step_params(step), nullptr);
+        adj_step(wide ? k_adj_step<true, false, 16> : k_adj_step<true, false, 4>, &E, Sn, Sn, 0);
       DCHK(hipGetLastError());
       lh.swap(lh2);
     }

@@ -55,3 +55,31 @@ __device__ __forceinline__ double group_value(double v, int q)
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
+// acc[c] += the value v[c] of lane 0, 1, ... G - 1 of this lane's group (4 or 16
+// lanes), one after the other
+template <int G, int NS, int K = 0>
+__device__ __forceinline__ void add_in_order(double (&acc)[NS], const double (&v)[NS])
+{
+  static_assert(G == 4 || G == 16, "a quad or a row");
+  if constexpr (K < G) {
+#pragma unroll
+    for (int c = 0; c < NS; c++)
+      acc[c] = acc[c] + dpp_move<G == 4 ? 0x55 * K : 0x150 + K>(v[c]);
+    add_in_order<G, NS, K + 1>(acc, v);
+  }
+}
+
+// In the first quad of a row (one quad: NQ = 1): acc[c] += v[c] of the same lane of
+// quad 0, 1, ... NQ - 1, one after the other; the other quads' sums mean nothing
+template <int NQ, int NS, int K = 0>
+__device__ __forceinline__ void add_quads(double (&acc)[NS], const double (&v)[NS])
+{
+  if constexpr (K < NQ) {
+#pragma unroll
+    for (int c = 0; c < NS; c++) {
+      if constexpr (K == 0) acc[c] = acc[c] + v[c];
+      else acc[c] = acc[c] + dpp_move<0x100 + 4 * K>(v[c]);  // the lane 4 K above
+    }
+    add_quads<NQ, NS, K + 1>(acc, v);
+  }
+}
