@@ -1,0 +1,225 @@
+"""The launches that take a size or a form of their own: the fused step of engines
+without bonded groups, its two contact kernels, the pair search's and the summation
+runs' group sizes, the queries' order, the servo's two ways to its force sum, and
+the calibration engine's gathers and tapes.  Sizes are the edges of waves, of the
+64-particle groups, of the runs a group of lanes holds and of the dispatch rules.
+
+Tolerances: events and lists bit-exact; a step's arithmetic is the oracle's up to
+the order of a particle's sum, so positions after the few dozen steps here agree to
+1e-9 of a radius (sums of up to 500 forces at 2^-53 each, grown by the contacts)."""
+import importlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-9
+
+
+@pytest.fixture(scope="module")
+def spm(pkg):
+    return importlib.import_module("esys_particle_amd.specimens")
+
+
+def follow(pkg, orc, spm, spec, steps, names, batch=32, extra=None, lists=True):
+    g = pkg.LsmMpi(stepsPerBatch=batch)
+    o = orc.oracle_lsm_class(pkg)()
+    for sim in (g, o):
+        spm.apply(sim, spec)
+        if extra:
+            extra(sim)
+    print("case: n=%d steps=%d batch=%d" % (len(spec["ids"]), steps, batch), flush=True)
+    g.runTimeSteps(steps)
+    o.runTimeSteps(steps)
+    assert g.engine.rebuild_steps().tolist() == o.engine.rebuild_steps().tolist()
+    if lists:
+        np.testing.assert_array_equal(g.engine.neighbour_pairs(), o.engine.neighbour_pairs())
+        for name in names:
+            np.testing.assert_array_equal(g.getInteractionPairs(name), o.getInteractionPairs(name))
+    r = float(np.mean(spec["rad"]))
+    po = o.getParticleData("pos")
+    assert np.max(np.abs(g.getParticleData("pos") - po)) <= TOL * r
+    vo = o.getParticleData("vel")
+    assert np.max(np.abs(g.getParticleData("vel") - vo)) <= TOL * max(np.abs(vo).max(), 1e-300)
+    return g, o
+
+
+def cloud(spm, n, seed=5):
+    """n particles packed in a box with some moving into each other."""
+    L = max(1.6, (n * 0.9) ** (1.0 / 3.0))
+    spec = spm.gravity_settling(n=n, seed=seed, box=(L, 2.0 * L, L), dt=2e-3, k=100.0, wall_k=100.0)
+    spec["vel"] = np.random.default_rng(seed).normal(0.0, 2.0, (n, 3))
+    return spec
+
+
+def hub(n_small=420, seed=3):
+    """One large particle under a shell of small ones that overlap it: a run of
+    more than 400 touching pairs in one group."""
+    rng = np.random.default_rng(seed)
+    k = np.arange(n_small) + 0.5
+    phi, th = np.arccos(1.0 - 2.0 * k / n_small), np.pi * (1.0 + 5.0 ** 0.5) * k
+    d = np.stack([np.cos(th) * np.sin(phi), np.sin(th) * np.sin(phi), np.cos(phi)], 1)
+    R, r = 3.0, 0.12
+    pos = np.concatenate([np.zeros((1, 3)), d * (R + 0.97 * r)]) + 5.0
+    rad = np.concatenate([[R], np.full(n_small, r)])
+    n = len(rad)
+    return {"ptype": "RotSphere", "grid": 2 * R + 0.1, "alpha": 0.1, "dt": 1e-4,
+            "domain": ((-3.0, -3.0, -3.0), (13.0, 13.0, 13.0)),
+            "ids": np.arange(n, dtype=np.int32), "pos": pos, "rad": rad, "density": 1.0,
+            "vel": rng.normal(0.0, 0.5, (n, 3)), "walls": []}
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 257])
+def test_elastic_step_sizes(pkg, orc, spm, n):
+    g, o = follow(pkg, orc, spm, cloud(spm, n), 80, ["elastic"])
+    np.testing.assert_allclose(g.engine.wall_force_history("bottom", 80),
+                               o.engine.wall_force_history("bottom", 80), rtol=TOL, atol=1e-9)
+
+
+def test_elastic_step_searches_and_queue_depth(pkg, orc, spm):
+    """Several searches within a queue, with the same bits step by step."""
+    spec = cloud(spm, 300)
+    g, o = follow(pkg, orc, spm, spec, 200, ["elastic"], batch=64)
+    assert len(o.engine.rebuild_steps()) >= 4
+    s = pkg.LsmMpi(stepsPerBatch=1)
+    spm.apply(s, spec)
+    s.runTimeSteps(200)
+    for f in ("pos", "vel"):
+        assert s.getParticleData(f).tobytes() == g.getParticleData(f).tobytes()
+
+
+def add_groups(pkg, form):
+    def add(sim):
+        if form in ("friction", "mixed"):
+            sim.createInteractionGroup(pkg.RotFrictionPrms("fr", 200.0, 0.4, 0.4, 100.0))
+        if form == "rigid":
+            sim.createInteractionGroup(pkg.RotFrictionPrms("fr", 200.0, 0.4, 0.4, 100.0, rigid=True))
+        if form in ("rotelastic", "mixed"):
+            sim.createInteractionGroup(pkg.RotElasticPrms("el", 50.0))
+        if form == "two":
+            sim.createInteractionGroup(pkg.NRotElasticPrms("el", 50.0))
+            sim.createInteractionGroup(pkg.NRotElasticPrms("fr", 25.0))
+        if form == "nrot":
+            sim.createInteractionGroup(pkg.NRotElasticPrms("el", 50.0))
+    return add
+
+
+NAMES = {"friction": ["fr"], "rigid": ["fr"], "rotelastic": ["el"], "mixed": ["fr", "el"],
+         "two": ["el", "fr"], "nrot": ["el"]}
+
+
+@pytest.mark.parametrize("form", ["friction", "rigid", "rotelastic", "mixed", "two"])
+@pytest.mark.parametrize("n", [63, 65, 300])
+def test_contact_block_forms(pkg, orc, spm, form, n):
+    spec = cloud(spm, n, seed=n)
+    spec["ptype"] = "RotSphere"
+    spec["elastic"] = []
+    g, o = follow(pkg, orc, spm, spec, 80, NAMES[form], extra=add_groups(pkg, form))
+    assert np.max(np.abs(g.getParticleData("angvel") - o.getParticleData("angvel"))) <= \
+        TOL * max(np.abs(o.getParticleData("angvel")).max(), 1e-300)
+    if "fr" in NAMES[form] and form != "two":
+        np.testing.assert_array_equal(g.engine.friction_state("fr")[1],
+                                      o.engine.friction_state("fr")[1])
+
+
+@pytest.mark.parametrize("form", ["nrot", "friction", "mixed"])
+def test_long_runs(pkg, orc, spm, form):
+    """More pairs of one particle than a search run (192) or a block's packed
+    entries (320 touching, 512) hold."""
+    g, o = follow(pkg, orc, spm, hub(), 20, NAMES[form], extra=add_groups(pkg, form))
+    assert len(o.engine.neighbour_pairs()) > 400
+
+
+@pytest.mark.parametrize("tagged", [False, True])
+def test_long_search_runs_with_large_skin(pkg, orc, spm, tagged):
+    """A search cutoff that gives every particle hundreds of neighbours, with and
+    without a tag mask on the group."""
+    spec = cloud(spm, 500)
+    spec["alpha"], spec["grid"] = 6.0, 7.0
+    spec["elastic"] = [] if tagged else spec["elastic"]
+    spec["tags"] = (np.arange(500) % 2).astype(np.int32)
+
+    def add(sim):
+        if tagged:
+            sim.createInteractionGroupTagged(pkg.NRotElasticPrms("elastic", 100.0), 1, 1, 0, 1)
+    follow(pkg, orc, spm, spec, 30, ["elastic"], extra=add)
+
+
+@pytest.mark.parametrize("n", [8191, 8193, 33000])
+def test_search_at_scan_sizes(pkg, orc, spm, n):
+    spec = spm.gravity_settling(n=n, seed=n, box=(30.0, 90.0, 30.0))
+    follow(pkg, orc, spm, spec, 3, ["elastic"])
+
+
+def test_queries_with_sparse_ids(pkg, orc, spm):
+    spec = cloud(spm, 130)
+    rng = np.random.default_rng(4)
+    spec["ids"] = np.sort(rng.choice(10 ** 6, 130, replace=False)).astype(np.int32)[
+        rng.permutation(130)]
+    g, o = follow(pkg, orc, spm, spec, 40, ["elastic"])
+    np.testing.assert_array_equal(g.getParticleData("rad"), o.getParticleData("rad"))
+
+
+def test_servo_with_untagged_particle_at_the_wall(pkg, orc, spm):
+    """A wall's untagged particles are not bonded to it but may touch it: the servo
+    then iterates over the candidates instead of one pass of sums."""
+    spec = spm.shear_cell(n=600, seed=3, phi=0.35, dt=5e-4, wall_speed=10.0)
+    spec["vel"] = np.random.default_rng(3).normal(0.0, 2.0, (600, 3))
+    tags = np.array(spec["tags"])
+    tag = spec["bonded_walls"][1][4]
+    mine = np.flatnonzero(tags == tag)
+    assert len(mine) > 4
+    tags[mine[::2]] = 1
+    spec["tags"] = tags
+    g, o = follow(pkg, orc, spm, spec, 60, ["friction"])
+    np.testing.assert_allclose(list(g.getWallPosition("top")), list(o.getWallPosition("top")),
+                               rtol=1e-12, atol=1e-12)
+
+
+# ---- the calibration engine ----
+@pytest.fixture(scope="module")
+def cal(pkg):
+    return importlib.import_module("esys_particle_amd.calibration")
+
+
+@pytest.fixture(scope="module")
+def weak(spm):
+    return spm.dense_bonded_compression(n=1500, seed=9, coh_mean=2.0, coh_sd=0.2, wall_speed=20.0)
+
+
+THETA = np.array([1e5, 3e4, 2.0, 0.3])
+
+
+@pytest.mark.parametrize("K", [1, 37, 100])
+def test_tape_equals_checkpoints(cal, weak, K):
+    """A plain run keeps every state, a tangent run checkpoints: the sweeps over
+    both give the same bits, over neighbour searches and broken bonds."""
+    # the small skin makes the run search for neighbours again and again
+    m = cal.DiffModel.from_specimens([weak], 200, 20, checkpoint_every=K, alpha=0.02)
+    target = np.full((1, m.nsamples), 5.0)
+    st, loss = m.forward(THETA, target)
+    g = m.backward()
+    pos = m.particle_data("pos")
+    assert len(m.bond_breaks()) > 100 and len(m.rebuild_steps()) > 1
+    st2, loss2, _ = m.forward_tangent(THETA, np.ones((1, 4)), target)
+    np.testing.assert_array_equal(st2, st)
+    np.testing.assert_array_equal(m.particle_data("pos"), pos)
+    np.testing.assert_array_equal(m.backward(), g)
+    np.testing.assert_array_equal(m.particle_data("pos"), pos)
+
+
+@pytest.mark.parametrize("copies", [7, 25])
+def test_wide_batch_equals_single(cal, weak, copies):
+    """Past the sizes where a particle's row of lanes becomes a quad (8,192 in the
+    forward gather, 32,768 in the adjoint) a specimen keeps its bits."""
+    mb = cal.DiffModel.from_specimens([weak] * copies, 40, 10)
+    th = np.tile(THETA, (copies, 1))
+    target = np.full((copies, mb.nsamples), 3.0)
+    _, lb = mb.forward(th, target)
+    gb = mb.backward()
+    for s in (0, copies - 1):
+        ms = cal.DiffModel.from_specimens([weak], 40, 10, x_start=mb.starts[s])
+        _, ls = ms.forward(THETA, target[:1])
+        assert lb[s] == ls[0]
+        np.testing.assert_array_equal(gb[s], ms.backward()[0])
