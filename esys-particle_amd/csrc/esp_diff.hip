@@ -748,14 +748,21 @@ __device__ __forceinline__ void adj_particle_item(const DState& Sn, const DState
 #define NB_REC 4
 #define NF_REC 6
 
-// bond law VJP: c[k] = lambda_out . d out / d in_k over the inputs
-// (x1, x2, q1, q2, theta_kn, theta_ks), one thread per bond, by the law's
-// hand-written reverse mode (tbond_law_vjp) on the branch the forward step took
+// bond law VJP, one thread per bond, by the law's hand-written reverse mode
+// (tbond_law_vjp) on the branch the forward step took: about 2,300 FP64
+// instructions, 66 divisions among them, so a wave alone on its SIMD leaves the
+// memory phases of its gathers and stores uncovered.  The law takes its two halves
+// one after the other and parks what is used only at the ends in LDS: 223 VGPRs
+// instead of 326, two waves a SIMD, 478,000 bonds 79.2 -> 52.9 us a step (2,000
+// particles 9.8, one wave's time either way).
 #define ADJ_BOND_BS 256
-__global__ __launch_bounds__(ADJ_BOND_BS) void k_adj_bond(DState S, DBonds B,
+__global__ __launch_bounds__(ADJ_BOND_BS, 2) void k_adj_bond(DState S, DBonds B,
                                                            const double4* theta, int step,
                                                            const double* lfm, double4* ab)
 {
+  // volatile: the compiler would keep the values in registers instead
+  typedef __attribute__((address_space(3))) volatile double* lds_park;
+  __shared__ double park[BOND_VJP_PARK * ADJ_BOND_BS];
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= B.nb) return;
   // broken earlier: the record is the zero the sweep, which goes back in time,
@@ -782,7 +789,7 @@ __global__ __launch_bounds__(ADJ_BOND_BS) void k_adj_bond(DState S, DBonds B,
                 tquat<double>{Q2.x, {Q2.y, Q2.z, Q2.w}}, P2.w, kr, ks, kt, kb,
                 tv3<double>{D.x, D.y, D.z}, tv3<double>{l1[0] - l2[0], l1[1] - l2[1], l1[2] - l2[2]},
                 tv3<double>{l1[3], l1[4], l1[5]}, tv3<double>{l2[3], l2[4], l2[5]}, g1, g2, gq1, gq2,
-                gkr, gks);
+                gkr, gks, (lds_park)(park + threadIdx.x), ADJ_BOND_BS);
   c[0] = make_double4(g1.x, g1.y, g1.z, gkr * dkr);
   c[1] = make_double4(g2.x, g2.y, g2.z, gks * dks);
   c[2] = make_double4(gq1.s, gq1.v.x, gq1.v.y, gq1.v.z);
