@@ -1372,7 +1372,7 @@ void wall_params(esp_engine* e, WallParam* out)
 // force records: main lists of the dynamic groups (name order), bonded groups
 // (name order), then one appendix region per dynamic group; the CSR covers the
 // first two, the per-particle overflow slots the appendices
-void rebuild_csr(esp_engine* e)
+void rebuild_csr(esp_engine* e, bool cleared)
 {
   long long rec = 0;
   for (int gi : e->dord) { e->dg[gi].rec_off = (int)rec; rec += e->dg[gi].n; }
@@ -1382,7 +1382,7 @@ void rebuild_csr(esp_engine* e)
   for (int gi : e->dord)
     if (e->dg[gi].n >= (1 << 27)) throw EspError(ESP_ERR_CAPACITY, "more than 2^27 pairs in one group");
   e->nrec = (int)rec;
-  zero(e, e->inc_cnt.p, e->n + 1);
+  if (!cleared) zero(e, e->inc_cnt.p, e->n + 1);
   for (int gi : e->dord) launch_inc_count(e->stream, e->dg[gi].n, e->dg[gi].ij.p, e->inc_cnt.p);
   for (int gi : e->bord) launch_inc_count(e->stream, e->bg[gi].n, e->bg[gi].ij.p, e->inc_cnt.p);
   // dead bonds were compacted out, so every stored interaction has two entries
@@ -1393,7 +1393,7 @@ void rebuild_csr(esp_engine* e)
   e->scan_tmp.reserve(scan_tmp_size(e->n));
   launch_exclusive_scan(e->stream, e->inc_cnt.p, e->inc_off.p, e->n, e->scan_tmp.p);
   e->inc_ent64.reserve(std::max(total, 1));
-  zero(e, e->inc_fill.p, e->n + 1);
+  if (!cleared) zero(e, e->inc_fill.p, e->n + 1);
   const bool cm = contact_mode(e);
   if (cm) e->contact_ent.reserve(std::max(total, 1));
   else e->slot_of.reserve((size_t)std::max<long long>(rec, 1));
@@ -1817,12 +1817,19 @@ bool quick_search(esp_engine* e, long long step)
   const int cap = (int)room;
   PView p = e->view();
   if (e->grid.circ_x) launch_wrap_x(e->stream, p, e->grid.x0, e->grid.period, e->init.p);
-  zero(e, e->cell_count.p, e->ncell + 1);
-  zero(e, e->dev_int.p, 1);
+  // with the counters of rebuild_csr, which follows: five fills of 2.5 us and their
+  // gaps are one launch
+  ClearSet cs;
+  cs.p[0] = e->cell_count.p; cs.n[0] = e->ncell + 1;
+  cs.p[1] = e->cell_fill.p; cs.n[1] = e->ncell;
+  cs.p[2] = e->inc_cnt.p; cs.n[2] = n + 1;
+  cs.p[3] = e->inc_fill.p; cs.n[3] = n + 1;
+  cs.p[4] = e->dev_int.p; cs.n[4] = 1;
+  cs.count = 5;
+  launch_clear(e->stream, cs);
   launch_cells_count(e->stream, p, e->grid, e->cell.p, e->cell_count.p, e->dev_int.p);
   e->scan_tmp.reserve(scan_tmp_size(std::max({e->ncell, n, cap})));
   launch_exclusive_scan(e->stream, e->cell_count.p, e->cell_start.p, e->ncell, e->scan_tmp.p);
-  zero(e, e->cell_fill.p, e->ncell);
   launch_cells_fill(e->stream, n, e->cell.p, e->cell_start.p, e->cell_fill.p, e->cell_items.p);
   launch_cells_sort(e->stream, e->ncell, e->cell_start.p, e->cell_items.p);
   for (int emit = 0; emit < 2; emit++) {
@@ -1926,7 +1933,7 @@ void host_step(esp_engine* e, int reason)
     }
     e->last_ns = e->timestamp;
   }
-  rebuild_csr(e);
+  rebuild_csr(e, found);
   sync_history_buffers(e);
   launch_step(e, make_ctl(e, step, 1, 0), step, false, true);
   swap_step_buffers(e);

@@ -381,6 +381,12 @@ void launch_pack_ordered(hipStream_t s, int n, const int* order, const double4* 
 void launch_report3(hipStream_t s, const int* a, const int* b, const int* c, int* out);
 // a[0..n) = v (a kernel, not a memset: safe under stream capture)
 void launch_fill_int(hipStream_t s, int n, int* a, int v);
+struct ClearSet {
+  int* p[5];
+  int n[5];
+  int count;
+};
+void launch_clear(hipStream_t s, const ClearSet& c);
 // erasure of particles outside the padded grid (NeighborTable::build):
 // keep[i] = cell[i] >= 0; nslot[i] = new slot or -1; stable compaction of a
 // per-particle field of `width` elements; interaction pairs remapped to the new

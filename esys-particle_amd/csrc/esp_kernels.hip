@@ -7,13 +7,18 @@
 //       into both particles' slots.  In a queued step block 0 meanwhile applies
 //       the previous step's bond breaks and appends the new pairs of the
 //       flagged particles (and computes their forces)
-//   k_gather_integrate (k_gather_stress where particle stresses are kept)
-//       one thread per particle: wall and body forces, then the records of its
+//   k_gather_integrate (k_gather_wide for many particles, k_gather_stress where
+//       particle stresses are kept)
+//       per particle: wall and body forces, then the records of its
 //       interactions in a fixed order (CSR), then the CParticle/CRotParticle
-//       first-order update and the max-displacement reduction; per-block
-//       partials of the wall forces
-//   k_wall_finalize (once per queued batch)
-//       fixed-order sums of the wall-force partials of every step of the batch
+//       first-order update and the max-displacement reduction; wall-force
+//       partials of every 64 particles
+//   k_contact_step, k_contact_block
+//       instead of these two where no group is bonded: each particle evaluates
+//       its side of its interactions and integrates
+//   k_batch_end (once per queued batch)
+//       fixed-order sums of the wall-force partials of every step of the batch,
+//       written with the batch's status to page-locked host memory
 // Every per-step kernel first evaluates the previous step's status; if that
 // step displaced a particle by more than verletDist/2 or broke a bond, the host
 // must do bookkeeping first, so the kernel records the halt and returns, and
@@ -32,10 +37,6 @@
 #include "esp_wave.h"
 
 #define BS 256
-#ifndef ESP_G_EL
-#define ESP_G_EL 4
-#endif
-
 static inline int nblk(long long n, int bs = BS) { return (int)((n + bs - 1) / bs); }
 
 __device__ __forceinline__ dv3 xyz(double4 a) { return mk3(a.x, a.y, a.z); }
@@ -714,9 +715,8 @@ __global__ __launch_bounds__(BS) void k_gather_stress(StepCtl ctl, PView p, Gath
 // follows; slots of steps that were skipped hold stale values the host does not
 // read.  Block 0 also reports why the queue halted and the last completed
 // step's status, and clears every other entry of the ring and the halt mark for
-// the next batch.  (Three copies into pageable memory, two launches around a
-// batch: 72 us a step for a batch of one step of 97 particles; this: see
-// k_contact_step and esp_engine.hip's fast_batch.)
+// the next batch.  With three copies into pageable memory and two launches around a
+// batch a batch of one step of 97 particles took 72 us; with this 38.
 template <bool LIST>
 __global__ __launch_bounds__(BS) void k_batch_end(BatchEnd be)
 {
@@ -900,7 +900,9 @@ __device__ __forceinline__ int xcd_block(int b, int nb)
 // arrays (neighbours still read the old ones); the host swaps the sets.
 //
 // G lanes share a particle's pairs (row entries k = lane, lane + G, ...), their
-// shares are added in row order, then one lane per particle integrates.
+// shares are added in row order, then one lane per particle integrates.  Bound by
+// the chain row -> entry -> neighbour's position while the chip is not full: 10,000
+// settling spheres 14.1 us (4.7 + 9.4 in two launches) -> 4.3.
 template <bool EXTRA, int G>
 __global__ __launch_bounds__(BS) void k_contact_step(StepCtl ctl, PView p, ContactLaunch cl,
                                                      GatherParams gp)
@@ -995,7 +997,10 @@ __global__ __launch_bounds__(BS) void k_contact_step(StepCtl ctl, PView p, Conta
 // law runs on full waves (of the 7.5 entries a particle has in a sheared bed
 // about 60 % touch, and a wave that walks its particles' runs waits for the
 // longest of 64), their shares go to LDS, and the first wave adds them in entry
-// order and integrates.
+// order and integrates.  Bound by the gathers of the touching neighbours (160 bytes
+// each, twice a pair) at the three waves a SIMD its registers allow.  Sheared bed,
+// us a step: 30,000 particles 17.2 (7.1 + 10.0 in two launches) -> 14.2, 1,000,000
+// 266 -> 242; four lanes walking a particle's run took 20 and 252.
 template <bool EXTRA, int KIND>
 __global__ __launch_bounds__(BS, KIND ? 3 : 2) void k_contact_block(StepCtl ctl, PView p, ContactLaunch cl,
                                                          GatherParams gp)
@@ -1169,8 +1174,12 @@ __global__ __launch_bounds__(BS, KIND ? 3 : 2) void k_contact_block(StepCtl ctl,
 // its state is on its way meanwhile.
 // With one lane a particle the run's words, then up to eight slots of 48 bytes,
 // were a chain in every lane: 9.0 us for 2,000 particles (13 us where flagged
-// pairs make runs of 200 slots), 15.4 us for 100,000.
-template <bool EXTRA>
+// pairs make runs of 200 slots), 15.4 us for 100,000.  RQ: active slots a lane has
+// in flight, as a turn of the sum waits for memory once.  One / three: 7.1 / 6.8 us
+// for 2,000 particles, 9.1 / 7.9 for 5,000 with flagged pairs, 8.4 / 8.1 for 30,000,
+// but 11.1 / 12.7 for 60,000, where the registers of three cost a wave a SIMD:
+// three up to GATHER_DEEP.
+template <bool EXTRA, int RQ>
 __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, GatherParams gp)
 {
   constexpr int G = 4, PB = BS / G;
@@ -1225,20 +1234,30 @@ __global__ __launch_bounds__(BS) void k_gather_integrate(StepCtl ctl, PView p, G
   auto add_active = [&](unsigned long long m, size_t base) {
     for (int k = 0; k < sub; k++) m &= m - 1ull;  // this lane's first
     while (__ballot(m != 0ull)) {
-      double2 qa = make_double2(0.0, 0.0), qb = qa, qc = qa;
-      if (m) {
-        const double2* q =
-            reinterpret_cast<const double2*>(gp.slots + 6 * (base + __builtin_ctzll(m)));
-        qa = q[0];
-        qb = q[1];
-        qc = q[2];
-        for (int k = 0; k < G; k++) m &= m - 1ull;
+      double v[RQ][6];
+#pragma unroll
+      for (int r = 0; r < RQ; r++) {
+        double2 qa = make_double2(0.0, 0.0), qb = qa, qc = qa;
+        if (m) {
+          const double2* q =
+              reinterpret_cast<const double2*>(gp.slots + 6 * (base + __builtin_ctzll(m)));
+          qa = q[0];
+          qb = q[1];
+          qc = q[2];
+          for (int k = 0; k < G; k++) m &= m - 1ull;
+        }
+        v[r][0] = qa.x; v[r][1] = qa.y; v[r][2] = qb.x;
+        v[r][3] = qb.y; v[r][4] = qc.x; v[r][5] = qc.y;
       }
 #pragma unroll
-      for (int k = 0; k < G; k++) {
-        F = add3(F, mk3(group_value<G>(qa.x, k), group_value<G>(qa.y, k), group_value<G>(qb.x, k)));
-        M = add3(M, mk3(group_value<G>(qb.y, k), group_value<G>(qc.x, k), group_value<G>(qc.y, k)));
-      }
+      for (int r = 0; r < RQ; r++)
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+          F = add3(F, mk3(group_value<G>(v[r][0], k), group_value<G>(v[r][1], k),
+                          group_value<G>(v[r][2], k)));
+          M = add3(M, mk3(group_value<G>(v[r][3], k), group_value<G>(v[r][4], k),
+                          group_value<G>(v[r][5], k)));
+        }
     }
   };
   // 64 bytes of activity a turn, from the run's first aligned word
@@ -2409,17 +2428,29 @@ __global__ __launch_bounds__(BS) void k_scan_local(const int* in, int nvalid, in
 }
 
 // Short arrays in one block and one launch: V values a thread, all loaded at
-// once, the sums of a wave by shuffles, the waves' through LDS
+// once, the sums of a wave by shuffles, the waves' through LDS.  A thread's values
+// are consecutive, so every load of a wave touches 64 lines: bound by the line
+// look-ups of one CU, which 16-byte loads and stores (`vec`: both arrays are so
+// aligned) cut to a quarter.  15,000 values 16.3 -> 4.0 us.
 #define SCAN_ONE 32768
 template <int V>
-__global__ __launch_bounds__(1024) void k_scan_one(const int* in, int nvalid, int* out, int m)
+__global__ __launch_bounds__(1024) void k_scan_one(const int* in, int nvalid, int* out, int m,
+                                                   int vec)
 {
   __shared__ int wsum[16];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int base = t * V;
   int v[V], acc = 0;
+  if (vec && base + V <= nvalid) {
 #pragma unroll
-  for (int k = 0; k < V; k++) v[k] = base + k < nvalid ? in[base + k] : 0;
+    for (int k = 0; k < V; k += 4) {
+      const int4 q = *reinterpret_cast<const int4*>(in + base + k);
+      v[k] = q.x; v[k + 1] = q.y; v[k + 2] = q.z; v[k + 3] = q.w;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < V; k++) v[k] = base + k < nvalid ? in[base + k] : 0;
+  }
 #pragma unroll
   for (int k = 0; k < V; k++) acc += v[k];
   int inc = acc;
@@ -2433,10 +2464,22 @@ __global__ __launch_bounds__(1024) void k_scan_one(const int* in, int nvalid, in
   int run = inc - acc;
 #pragma unroll
   for (int w = 0; w < 16; w++) run += w < wv ? wsum[w] : 0;
+  if (vec && base + V <= m) {
 #pragma unroll
-  for (int k = 0; k < V; k++) {
-    if (base + k < m) out[base + k] = run;
-    run += v[k];
+    for (int k = 0; k < V; k += 4) {
+      int4 q;
+      q.x = run; run += v[k];
+      q.y = run; run += v[k + 1];
+      q.z = run; run += v[k + 2];
+      q.w = run; run += v[k + 3];
+      *reinterpret_cast<int4*>(out + base + k) = q;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < V; k++) {
+      if (base + k < m) out[base + k] = run;
+      run += v[k];
+    }
   }
 }
 
@@ -2460,10 +2503,11 @@ size_t scan_tmp_size(int n) { return scan_tmp_rec((long long)n + 1) + 16; }
 static void scan_rec(hipStream_t s, const int* in, int nvalid, int* out, int m, int* tmp)
 {
   if (m <= SCAN_ONE) {
-    if (m <= SCAN_ONE / 4)
-      hipLaunchKernelGGL(k_scan_one<8>, dim3(1), dim3(1024), 0, s, in, nvalid, out, m);
-    else
-      hipLaunchKernelGGL(k_scan_one<32>, dim3(1), dim3(1024), 0, s, in, nvalid, out, m);
+    const int vec = (((uintptr_t)in | (uintptr_t)out) & 15) == 0;
+    const auto scan = m <= SCAN_ONE / 4   ? k_scan_one<8>
+                      : m <= SCAN_ONE / 2 ? k_scan_one<16>
+                                          : k_scan_one<32>;
+    hipLaunchKernelGGL(scan, dim3(1), dim3(1024), 0, s, in, nvalid, out, m, vec);
     return;
   }
   const int nb = (m + 4 * BS - 1) / (4 * BS);
@@ -2581,6 +2625,8 @@ static void gather_launch(K kern, int blocks, hipStream_t s, StepCtl ctl, PView 
 // at 100,000 (15.9 and 15.4 us); at 64,000 particles one lane each is one wave
 // for every SIMD of the chip
 #define GATHER_WIDE 65536
+// three active slots a lane in flight up to this many, see k_gather_integrate
+#define GATHER_DEEP 32768
 bool launch_gather_integrate(hipStream_t s, StepCtl ctl, PView p, const GatherParams& gp,
                              hipEvent_t ev_a, hipEvent_t ev_b)
 {
@@ -2593,8 +2639,9 @@ bool launch_gather_integrate(hipStream_t s, StepCtl ctl, PView p, const GatherPa
     if (extra) gather_launch(k_gather_wide<true>, nblk(p.n), s, ctl, p, gp, ev_a, ev_b);
     else gather_launch(k_gather_wide<false>, nblk(p.n), s, ctl, p, gp, ev_a, ev_b);
   } else {
-    if (extra) gather_launch(k_gather_integrate<true>, nblk(p.n, 64), s, ctl, p, gp, ev_a, ev_b);
-    else gather_launch(k_gather_integrate<false>, nblk(p.n, 64), s, ctl, p, gp, ev_a, ev_b);
+    const auto deep = extra ? k_gather_integrate<true, 3> : k_gather_integrate<false, 3>;
+    const auto flat = extra ? k_gather_integrate<true, 1> : k_gather_integrate<false, 1>;
+    gather_launch(p.n <= GATHER_DEEP ? deep : flat, nblk(p.n, 64), s, ctl, p, gp, ev_a, ev_b);
   }
   return true;
 }
@@ -2654,7 +2701,7 @@ bool launch_contact_step(hipStream_t s, StepCtl ctl, PView p, const ContactLaunc
   if (p.n <= 0) return false;
   const bool extra = extra_forces(gp);
   if (cl.count == 1 && cl.seg[0].kind == ESP_SEG_NROT_ELASTIC) {
-    constexpr int G = ESP_G_EL;
+    constexpr int G = 4;  // lanes a particle: its 7 or so pairs in two rounds
     const dim3 g(nblk(p.n, BS / G));
     if (extra) contact_launch(k_contact_step<true, G>, g, s, ctl, p, cl, gp, ev_a, ev_b);
     else contact_launch(k_contact_step<false, G>, g, s, ctl, p, cl, gp, ev_a, ev_b);
@@ -2818,6 +2865,20 @@ __global__ void k_report3(const int* a, const int* b, const int* c, int* out)
 void launch_report3(hipStream_t s, const int* a, const int* b, const int* c, int* out)
 {
   hipLaunchKernelGGL(k_report3, dim3(1), dim3(64), 0, s, a, b, c, out);
+}
+
+// several arrays to zero in one launch
+__global__ void k_clear(ClearSet c)
+{
+  for (int k = 0; k < c.count; k++)
+    for (int i = blockIdx.x * BS + threadIdx.x; i < c.n[k]; i += gridDim.x * BS) c.p[k][i] = 0;
+}
+
+void launch_clear(hipStream_t s, const ClearSet& c)
+{
+  int most = 0;
+  for (int k = 0; k < c.count; k++) most = max(most, c.n[k]);
+  if (most > 0) hipLaunchKernelGGL(k_clear, dim3(min(nblk(most), 1024)), dim3(BS), 0, s, c);
 }
 
 void launch_fill_int(hipStream_t s, int n, int* a, int v)

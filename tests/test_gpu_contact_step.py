@@ -146,7 +146,7 @@ def test_long_search_runs_with_large_skin(pkg, orc, spm, tagged):
     follow(pkg, orc, spm, spec, 30, ["elastic"], extra=add)
 
 
-@pytest.mark.parametrize("n", [8191, 8193, 33000])
+@pytest.mark.parametrize("n", [8191, 8193, 16385, 33000])
 def test_search_at_scan_sizes(pkg, orc, spm, n):
     spec = spm.gravity_settling(n=n, seed=n, box=(30.0, 90.0, 30.0))
     follow(pkg, orc, spm, spec, 3, ["elastic"])
@@ -223,3 +223,12 @@ def test_wide_batch_equals_single(cal, weak, copies):
         _, ls = ms.forward(THETA, target[:1])
         assert lb[s] == ls[0]
         np.testing.assert_array_equal(gb[s], ms.backward()[0])
+
+
+@pytest.mark.parametrize("nx", [31, 33])
+def test_bonded_gather_sizes(pkg, orc, spm, nx):
+    """Below and past 32,768 particles the bonded gather keeps three active slots of
+    a particle in flight a lane, or one."""
+    spec = spm.lattice_block(nx=nx, ny=32, nz=32, dt=1e-4, vel_sd=0.05)
+    g, o = follow(pkg, orc, spm, spec, 12, ["bonded", "friction"], lists=False)
+    np.testing.assert_array_equal(g.getBondBreaks(), o.getBondBreaks())
