@@ -1048,6 +1048,7 @@ struct esp_diff {
   DevBuf<double4> H[2];  // shear histories: step s reads H[s & 1], writes the other
   DevBuf<DRun> run;
   std::vector<double> wo;  // wall origins per step of the run [step][wall][3]
+  int run_nw = 0;          // its walls
   // The states of the last forward run, step by step ([step][x, v, w, q][n]), and
   // the histories touching pairs read in each: kept by runs whose tape fits
   // kTapeBytes, so that the adjoint sweeps them without recomputing its segments.
@@ -1101,10 +1102,10 @@ struct esp_diff {
   {
     DStep s;
     memset(&s, 0, sizeof s);
-    s.nw = nw;
-    for (int k = 0; k < nw; k++) {
+    s.nw = run_nw;
+    for (int k = 0; k < run_nw; k++) {
       s.wall[k] = wall0[k];
-      for (int c = 0; c < 3; c++) s.wall[k].o[c] = wo[((size_t)step * nw + k) * 3 + c];
+      for (int c = 0; c < 3; c++) s.wall[k].o[c] = wo[((size_t)step * run_nw + k) * 3 + c];
     }
     s.has_g = has_g;
     for (int c = 0; c < 3; c++) s.g[c] = g[c];
@@ -1287,6 +1288,9 @@ void restore_checkpoint(esp_diff* d, const Checkpoint& C, double4* T)
   // "zero in both buffers" writes neither)
   d2d(d, d->H[0].p, C.hist.p, nc);
   d2d(d, d->H[1].p, C.hist.p, nc);
+  // bonds broken before the segment have zero records; what a sweep before this
+  // one left is of other steps
+  if (d->nb > 0) DCHK(hipMemsetAsync(d->bout.p, 0, sizeof(double) * 9 * (size_t)d->nb, d->stream));
 }
 
 // The launches of one forward step (no search) from S into So: tangents (tangent
@@ -1487,7 +1491,7 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
   // wall origins of every step: moved by their step before every step (the
   // pre-time-step moveWallBy of the main engine's setWallStepMotion)
   {
-    const int nw = std::max(d->nw, 1);
+    const int nw = d->run_nw = d->nw;
     std::vector<double>& wo = d->wo;
     wo.assign((size_t)(d->nsteps + 2) * nw * 3, 0.0);
     double o[DIFF_MAX_WALLS][3];
@@ -1586,7 +1590,7 @@ void backward(esp_diff* d, double* grad)
   const size_t c4 = 4 * (size_t)n;
   // without the run's tape: that of one segment, the states of steps s0..s1 and
   // the histories read at s0..s1-1
-  if (!d->full_tape) d->tape.reserve((size_t)(K + 1) * c4);
+  if (!d->full_tape) d->tape.reserve((size_t)(std::min(K, d->nsteps) + 1) * c4);
   int lh_epoch = -1;  // epoch whose pairs lh is indexed by
   DBonds B{d->nb, d->bij.p, d->bD0.p, d->brel.p, d->bstep.p, d->tkb.p};
   auto epoch_of = [&](int step) {
@@ -1966,6 +1970,7 @@ int esp_diff_set_run(esp_diff* d, int nsteps, int sample_every)
 {
   DAPI_BEGIN
   if (nsteps <= 0 || sample_every <= 0) throw DiffError(ESP_ERR_ARG, "bad run");
+  if (nsteps != d->nsteps || sample_every != d->every) d->have_forward = false;
   d->nsteps = nsteps;
   d->every = sample_every;
   return ESP_OK;

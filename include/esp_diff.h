@@ -54,7 +54,8 @@ typedef struct esp_diff_config {
   double domain_max[3];
   double dt;
   int device;
-  int checkpoint_every;  /* steps per checkpointed segment of the adjoint (>= 1) */
+  int checkpoint_every;  /* steps per recomputed segment of the adjoint (>= 1), for runs
+                            whose states are not all kept */
   int block;             /* threads per block of the per-step kernels (64..512, multiple of 64) */
 } esp_diff_config;
 
@@ -87,7 +88,8 @@ int esp_diff_set_run(esp_diff* d, int nsteps, int sample_every);
 
 /* One forward run from the initial state with theta [4 nspec] against the
  * target stresses [nspec * nsamples]: the sampled stresses (may be NULL) and
- * the loss per specimen.  Keeps the checkpoints for esp_diff_backward. */
+ * the loss per specimen.  Keeps the states (or checkpoints) for esp_diff_backward,
+ * until the next forward run or a change by esp_diff_set_run. */
 int esp_diff_forward(esp_diff* d, const double* theta, const double* target, double* stress,
                      double* loss);
 /* d loss_s / d theta_s [4 nspec] of the last forward run. */

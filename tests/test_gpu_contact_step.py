@@ -205,8 +205,9 @@ def test_tape_equals_checkpoints(cal, weak, K):
     st2, loss2, _ = m.forward_tangent(THETA, np.ones((1, 4)), target)
     np.testing.assert_array_equal(st2, st)
     np.testing.assert_array_equal(m.particle_data("pos"), pos)
-    np.testing.assert_array_equal(m.backward(), g)
-    np.testing.assert_array_equal(m.particle_data("pos"), pos)
+    for _ in range(2):  # the second sweep starts from what the first left
+        np.testing.assert_array_equal(m.backward(), g)
+        np.testing.assert_array_equal(m.particle_data("pos"), pos)
 
 
 @pytest.mark.parametrize("copies", [7, 25])
