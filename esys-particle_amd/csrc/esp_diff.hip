@@ -112,11 +112,6 @@ struct DevBuf {
 
 thread_local std::string g_diff_create_err;
 
-__device__ __forceinline__ long long dpair_key(int a, int b)
-{
-  return (long long)(((unsigned long long)(unsigned)a << 32) | (unsigned long long)(unsigned)b);
-}
-
 // Branch digest of a step: each wave hashes (its first index, its lanes'
 // branch bits) and adds the hash into the step's word; the sum is independent
 // of the order the waves finish in.  Two runs with equal digests took the same

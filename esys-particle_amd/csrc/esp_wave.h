@@ -4,9 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
-// Sum over the wave in a fixed order, the same value in every lane: pairs within
-// the rows of 16 lanes by DPP (a few cycles a step where a shuffle through LDS
-// takes a hundred), then the four rows.  Every lane of the wave must be active.
+// v of the lane that the DPP control CTRL names (zero past the row's ends), and v of
+// lane l of the wave
 template <int CTRL>
 __device__ __forceinline__ double dpp_move(double v)
 {
@@ -22,6 +21,10 @@ __device__ __forceinline__ double lane_value(double v, int l)
   const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
+
+// Sum over the wave in a fixed order, the same value in every lane: pairs within
+// the rows of 16 lanes by DPP (a few cycles a step where a shuffle through LDS
+// takes a hundred), then the four rows.  Every lane of the wave must be active.
 __device__ __forceinline__ double wave_sum(double v)
 {
   v = v + dpp_move<0xB1>(v);   // lanes 1,0,3,2 of every four
@@ -31,28 +34,15 @@ __device__ __forceinline__ double wave_sum(double v)
   return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
-// The value lane `q` of this lane's group of G (2 or 4) lanes holds
+// The value lane `q` of this lane's group of four holds
 template <int G>
 __device__ __forceinline__ double group_value(double v, int q)
 {
-  const long long b = __double_as_longlong(v);
-  int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
-#define ESP_DPP(ctrl)                                             \
-  {                                                               \
-    lo = __builtin_amdgcn_mov_dpp(lo, ctrl, 0xf, 0xf, true);      \
-    hi = __builtin_amdgcn_mov_dpp(hi, ctrl, 0xf, 0xf, true);      \
-  }
-  if (G == 4) {
-    if (q == 0) ESP_DPP(0x00)
-    else if (q == 1) ESP_DPP(0x55)
-    else if (q == 2) ESP_DPP(0xAA)
-    else ESP_DPP(0xFF)
-  } else if (G == 2) {
-    if (q == 0) ESP_DPP(0xA0)
-    else ESP_DPP(0xF5)
-  }
-#undef ESP_DPP
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+  static_assert(G == 4, "a quad");
+  return q == 0   ? dpp_move<0x00>(v)
+         : q == 1 ? dpp_move<0x55>(v)
+         : q == 2 ? dpp_move<0xAA>(v)
+                  : dpp_move<0xFF>(v);
 }
 
 // acc[c] += the value v[c] of lane 0, 1, ... G - 1 of this lane's group (4 or 16
