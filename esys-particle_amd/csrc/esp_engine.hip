@@ -282,6 +282,7 @@ struct esp_engine {
   // particle's interactions, the 64-particle groups with wall candidates
   DBuf<double4> pos2, vel2, ang2;
   DBuf<int> wall_mark, wall_list;
+  bool wall_list_valid = false;  // false once slots moved under it, until the next host step
   DBuf<int2> contact_ent;
 
   std::vector<DynGroup> dg;
@@ -1011,6 +1012,7 @@ void erase_outside(esp_engine* e)
   compact_host(e->h_order, hkeep, 1);
   e->ord_valid = false;
   e->id_slots_valid = false;
+  e->wall_list_valid = false;
   e->id2slot.clear();
   for (int i = 0; i < nk; i++) e->id2slot[e->h_id[i]] = i;
   e->n = nk;
@@ -1926,9 +1928,11 @@ void host_step(esp_engine* e, int reason)
       const bool cm = contact_mode(e);
       launch_wall_update(e->stream, e->view(), e->grid, (int)e->wg.size(), w,
                          cm ? e->wall_mark.p : nullptr);
-      if (cm)
+      if (cm) {
         launch_wall_list(e->stream, contact_groups(e->n), e->wall_mark.p, e->wall_list.p + 1,
                          e->wall_list.p);
+        e->wall_list_valid = true;
+      }
       HIPCHK(hipGetLastError());
     }
     e->last_ns = e->timestamp;
@@ -2735,7 +2739,7 @@ int esp_add_particles(esp_engine* e, int n, const int* id, const int* tag, const
     e->h_inert.push_back(0.0);
     e->h_order.push_back(e->next_order++);
     e->ord_valid = false;
-  e->id_slots_valid = false;
+    e->id_slots_valid = false;
   }
   return ESP_OK;
   API_END
@@ -3078,10 +3082,12 @@ bool servo_bonded(esp_engine* e, int k, const double Fa[3], long long cap)
   HIPCHK(hipSetDevice(e->cfg.device));
   WallParam wp[ESP_MAX_WALL_GROUPS];
   wall_params(e, wp);
-  const bool cm = contact_mode(e);
+  // a checkpoint's search may have erased particles and moved the slots of the
+  // others since the list was made: then every group is looked at
+  const bool listed = contact_mode(e) && e->wall_list_valid;
   double* out = e->batch_out.p + e->servo_at;
   launch_servo_sums(e->stream, e->view(), wp[k], k, e->do2d, e->init.p,
-                    cm ? e->wall_list.p + 1 : nullptr, cm ? e->wall_list.p : nullptr, out);
+                    listed ? e->wall_list.p + 1 : nullptr, listed ? e->wall_list.p : nullptr, out);
   HIPCHK(hipGetLastError());
   sync(e);
   double K = 0.0, cnt = 0.0, gap = 1e300;
@@ -3823,6 +3829,21 @@ std::string check_state(esp_engine* e)
     for (int v : fl)
       if (v < 0 || v >= n) {
         fail("flagged particle slot " + std::to_string(v));
+        break;
+      }
+  }
+  if (cm && e->wall_list_valid) {  // every wall candidate is in a listed group
+    const int ng = contact_groups(n);
+    std::vector<int> wl(ng + 1), listed(std::max(ng, 1), 0);
+    std::vector<unsigned> fl(std::max(n, 1));
+    d2h(e, wl.data(), e->wall_list.p, ng + 1);
+    d2h(e, fl.data(), e->flags.p, n);
+    sync(e);
+    for (int k = 0; k < wl[0] && k < ng; k++)
+      if (wl[k + 1] >= 0 && wl[k + 1] < ng) listed[wl[k + 1]] = 1;
+    for (int i = 0; i < n; i++)
+      if (((fl[i] >> PF_WALL_SHIFT) & 0xFFu) && !listed[i >> 6]) {
+        fail("wall candidate at slot " + std::to_string(i) + " in no listed group");
         break;
       }
   }

@@ -177,6 +177,61 @@ def test_servo_with_untagged_particle_at_the_wall(pkg, orc, spm):
                                rtol=1e-12, atol=1e-12)
 
 
+def column(spm, flyers=40):
+    """4 x 40 x 4 spheres apart from each other between two bonded walls, most
+    64-particle groups away from both; some of the middle ones fly out of the domain
+    in the first step."""
+    k = np.stack(np.meshgrid(np.arange(4), np.arange(40), np.arange(4), indexing="ij"), -1)
+    pos = 1.2 * k.reshape(-1, 3) + 0.6
+    n = len(pos)
+    tags = np.ones(n, np.int32)
+    tags[pos[:, 1] < 2.0] = 2
+    tags[pos[:, 1] > 46.0] = 3
+    mid = np.flatnonzero(np.abs(pos[:, 1] - 20.0) < 5.0)[:flyers]
+    vel = np.random.default_rng(8).normal(0.0, 0.5, (n, 3))
+    vel[mid, 2] = 4e4  # 20 diameters a step
+    v = 1e-3
+    return {"ptype": "RotSphere", "grid": 1.4, "alpha": 0.2, "dt": 5e-4,
+            "domain": ((-1.0, -2.0, -1.0), (6.0, 50.0, 6.0)),
+            "ids": np.random.default_rng(9).permutation(n).astype(np.int32), "pos": pos,
+            "rad": np.full(n, 0.5), "tags": tags, "vel": vel, "density": 1.0,
+            "friction": ("friction", 1e3, 0.5, 0.5, 1e3), "walls": [],
+            "bonded_walls": [("bottom", (0.0, 0.0, 0.0), (0.0, 1.0, 0.0), 1e3, 2, (v, 0.0, 0.0)),
+                             ("top", (0.0, 48.0, 0.0), (0.0, -1.0, 0.0), 1e3, 3, (0.0, 0.0, 0.0))]}
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_servo_after_checkpoint_that_erased_particles(pkg, orc, spm, tmp_path, noalloc):
+    """A checkpoint's search erases the particles outside the domain and moves the
+    slots of those behind them; a servo call before the next step still sums over
+    every candidate of its wall."""
+    spec = column(spm)
+    n = len(spec["ids"])
+    g, o = pkg.LsmMpi(stepsPerBatch=32), orc.oracle_lsm_class(pkg)()
+    for sim in (g, o):
+        spm.apply(sim, spec)
+        sim.runTimeSteps(1)
+    # (the oracle erases them at its next step's search: no wall candidate is among them)
+    g.engine.save_checkpoint(str(tmp_path / "cp"), 0, 12)
+    assert g.getNumParticles() == n - 40
+    force = [0.0, -30.0, 4.0]
+    print("case: servo after a checkpoint, n=%d, noalloc=%d" % (n, noalloc), flush=True)
+    g.engine.check_state()
+    for _ in range(3):  # before the step after the checkpoint, and between later steps
+        if noalloc:
+            g.engine.apply_force_to_wall_noalloc("top_bonds", force)
+        else:
+            g.applyForceToWall("top_bonds", force)
+        o.applyForceToWall("top_bonds", force)
+        np.testing.assert_allclose(list(g.getWallPosition("top")), list(o.getWallPosition("top")),
+                                   rtol=1e-12, atol=1e-12)
+        for sim in (g, o):
+            sim.runTimeSteps(4)
+        g.engine.check_state()
+    r = 0.5
+    assert np.max(np.abs(g.getParticleData("pos") - o.getParticleData("pos"))) <= TOL * r
+
+
 # ---- the calibration engine ----
 @pytest.fixture(scope="module")
 def cal(pkg):
