@@ -1067,7 +1067,7 @@ struct esp_diff {
   // branch digests are computed only when asked for (esp_diff_track_branches):
   // every wave of the contact and gather kernels adds to one counter per step
   bool track_digest = false;
-  DState fin = {};  // the state at the end of the last forward run
+  DState fin = {};  // the state the last forward run ended with, or had reached when it failed
   DevBuf<double4> x0, v0, w0, q0;  // the initial state
   // tangent-linear run (forward with a parameter direction)
   bool tan_on = false;
@@ -1389,6 +1389,7 @@ void run_forward(esp_diff* d, bool tape)
   const int K = std::max(1, d->cfg.checkpoint_every);
   const size_t c4 = 4 * (size_t)d->n;
   DState S0{d->x0.p, d->v0.p, d->w0.p, d->q0.p, d->spec.p, d->n};
+  d->fin = S0;
   rebuild(d, S0, 1);
   d->full_tape = tape && !d->tan_on &&
                  (size_t)d->nsteps * (32 * c4 + 32 * (size_t)d->epochs[0]->nc) <= kTapeBytes;
@@ -1404,13 +1405,14 @@ void run_forward(esp_diff* d, bool tape)
   }
   d2d(d, cur.x, S0.x, d->n); d2d(d, cur.v, S0.v, d->n); d2d(d, cur.w, S0.w, d->n);
   d2d(d, cur.q, S0.q, d->n);
+  d->fin = cur;
   HistoryRoom room{d, 0, 0};
   bool need = false;
   int step = 1;
   std::vector<HistoryRoom> mark;
   while (step <= d->nsteps) {
     if (need) {
-      rebuild(d, d->full_tape ? d->tape_state(d->tape.p + (size_t)(step - 1) * c4) : cur, step);
+      rebuild(d, d->fin, step);
       need = false;
     }
     if (!d->full_tape && (step - 1) % K == 0) save_checkpoint(d, step, cur);
@@ -1438,8 +1440,8 @@ void run_forward(esp_diff* d, bool tape)
     } else {
       step = end + 1;
     }
+    if (d->full_tape) d->fin = d->tape_state(d->tape.p + (size_t)(step - 1) * c4);
   }
-  d->fin = d->full_tape ? d->tape_state(d->tape.p + (size_t)d->nsteps * c4) : cur;
 }
 
 // dtheta (nullable): a parameter direction per specimen; the run then also
@@ -1465,7 +1467,6 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
   d->stress_dev.reserve((size_t)std::max(ns, 1) * d->nspec);
   d->digest.reserve((size_t)d->nsteps + 1);
   d->have_forward = false;
-  d->fin = DState{};
   d->tan_on = dtheta != nullptr;
   if (d->tan_on) {
     const size_t c = std::max(d->n, 1);
@@ -1827,6 +1828,8 @@ int esp_diff_set_particles(esp_diff* d, int n, int nspec, const int* spec, const
   for (int s = 0; s < nspec; s++) start[s + 1] += start[s];
   d->n = n;
   d->nspec = nspec;
+  d->fin = DState{};
+  d->have_forward = false;
   d->h_spec.assign(spec, spec + n);
   d->h_spec_start = start;
   d->h_pos.assign(pos, pos + 3 * n);
@@ -1870,8 +1873,6 @@ int esp_diff_set_particles(esp_diff* d, int n, int nspec, const int* spec, const
   DCHK(hipMemcpyAsync(d->flags.p, fl.data(), sizeof(unsigned) * n, hipMemcpyHostToDevice,
                       d->stream));
   dsync(d);
-  d->fin = DState{};
-  d->have_forward = false;
   return ESP_OK;
   DAPI_END
 }

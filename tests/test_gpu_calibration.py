@@ -208,3 +208,23 @@ def test_queries_after_adjoint_and_digest_opt_in(cal, spm):
     np.testing.assert_array_equal(st2, st)
     np.testing.assert_array_equal(loss2, loss)
     np.testing.assert_array_equal(m.backward(), g)
+
+
+def test_state_of_a_run_that_lost_particles(cal):
+    """A run whose particles leave the domain fails; a query then gives the state it
+    had reached."""
+    n, dt = 3, 1e-3
+    pos = np.array([[1.0, 1.0, 1.0], [4.0, 1.0, 1.0], [7.0, 1.0, 1.0]])
+    vel = np.array([[0.0, 0.0, 0.0], [0.0, 100.0, 0.0], [0.0, 0.0, 2.0]])
+    m = cal.DiffModel(1.4, 0.4, dt, ((0.0, 0.0, 0.0), (8.0, 8.0, 8.0)), 200, 20)
+    m.set_particles(np.zeros(n), pos, np.full(n, 0.5), np.ones(n), vel)
+    m.set_bonds([], [], np.zeros((0, 4)), [1.0], [1.0])
+    m.add_wall((0.0, 0.0, 0.0), (1.0, 0.0, 0.0), 1e3, (0.0, 0.0, 0.0), True, [1.0])
+    with pytest.raises(RuntimeError, match="left the neighbour-table domain"):
+        m.forward(THETA0, np.zeros((1, m.nsamples)))
+    # straight flights, up to the search that did not find the second one
+    x = m.particle_data("pos")
+    steps = (x[1, 1] - pos[1, 1]) / (vel[1, 1] * dt)
+    assert x[1, 1] > 8.0 and abs(steps - round(steps)) < 1e-9
+    np.testing.assert_allclose(x, pos + vel * dt * round(steps), rtol=1e-12)
+    np.testing.assert_array_equal(m.particle_data("vel"), vel)
