@@ -415,6 +415,25 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_bond_fwd_pairs(DState S, DBonds
                   ((int)blockIdx.x - nbb) * (int)blockDim.x + (int)threadIdx.x, cout, act, dig_base);
 }
 
+// The wall contacts' part of a step's branch digest (tracked runs), of the state
+// before it: one launch of its own, since what a wave of the gather integrates
+// depends on the launch's shape and the digest must not.
+__global__ void k_wall_digest(DState S, DStep sp, const DRun* run, unsigned long long* dig_base)
+{
+  if (run_skip(run, sp.step)) return;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= S.n) return;
+  const double4 P = S.x[i];
+  for (int k = 0; k < sp.nw; k++) {
+    const DWall& W = sp.wall[k];
+    const double dist = dot3(sub3(mk3(P.x, P.y, P.z), mk3(W.o[0], W.o[1], W.o[2])),
+                             mk3(W.n[0], W.n[1], W.n[2]));
+    wave_digest(dig_base + sp.step,
+                ((unsigned long long)(i & ~63) << 3) | (unsigned long long)(k + 1),
+                __ballot(dist < P.w), 0ull);
+  }
+}
+
 // per particle: the measured wall's normal force on it (sample steps), walls,
 // gravity, interactions in CSR order, then the update from S into So (the same
 // arrays, or the next step's of a tape).
@@ -429,8 +448,8 @@ template <int G, bool TAN>
 __global__ __launch_bounds__(DIFF_MAX_BS) void k_gather_fwd(
     DState S, DState So, const double4* mass_old, const int* inc_off, const int* inc_ent, int ncand,
     const double* cout, const double* bout, const unsigned char* cact, DStep sp,
-    double* wfn, DRun* run, unsigned long long thresh, unsigned long long* dig_base, DTan T,
-    const double* ct, const double* bt, double* wft)
+    double* wfn, DRun* run, unsigned long long thresh, DTan T, const double* ct, const double* bt,
+    double* wft)
 {
   constexpr int NS = TAN ? 12 : 6;
   __shared__ double sum[NS * (DIFF_MAX_BS / G)];  // [particle][component]
@@ -445,7 +464,6 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_gather_fwd(
   const int e0 = inc_off[pc];
   const int e1 = pi < S.n ? inc_off[pc + 1] : e0;
   if (run_skip(run, step)) return;  // the same for the whole block
-  unsigned long long* dig = dig_base ? dig_base + step : nullptr;
   double4 P = make_double4(0.0, 0.0, 0.0, 0.0), Om = P, Vv = P, A = P, Q = P;
   if (own) {
     P = S.x[i];
@@ -461,8 +479,6 @@ __global__ __launch_bounds__(DIFF_MAX_BS) void k_gather_fwd(
       const DWall& W = sp.wall[k];
       const dv3 n = mk3(W.n[0], W.n[1], W.n[2]);
       const double dist = dot3(sub3(x0, mk3(W.o[0], W.o[1], W.o[2])), n);
-      if (dig) wave_digest(dig, ((unsigned long long)(i - (t & 63)) << 3) | (unsigned long long)(k + 1),
-                           __ballot(dist < r), 0ull);
       if (dist < r) {
         double f = 1.0;
         f *= 3.141592654 * r;
@@ -1322,6 +1338,8 @@ void fwd_step(esp_diff* d, const Epoch& E, int step, const DState& S, const DSta
     memcpy(&thresh, &sr, 8);
   }
   const DStep sp = d->step_params(step);
+  if (dig && sp.nw > 0)
+    hipLaunchKernelGGL(k_wall_digest, dim3(nblocks(d->n, bs)), dim3(bs), 0, d->stream, S, sp, R, dig);
   const bool sample = record && step % d->every == 0;
   const bool wide = d->n <= kGatherRow;
   const auto gather = d->tan_on ? k_gather_fwd<4, true>
@@ -1330,7 +1348,7 @@ void fwd_step(esp_diff* d, const Epoch& E, int step, const DState& S, const DSta
   hipLaunchKernelGGL(gather,
                      dim3(nblocks((wide && !d->tan_on ? 16ll : 4ll) * d->n, bs)), dim3(bs), 0, d->stream, S, So, d->o.p,
                      E.inc_off.p, E.inc_ent.p, E.nc, d->cout.p, d->bout.p, d->cact.p, sp,
-                     sample ? d->wfn.p : nullptr, R, thresh, dig, T, d->ct.p, d->bt.p,
+                     sample ? d->wfn.p : nullptr, R, thresh, T, d->ct.p, d->bt.p,
                      sample && d->tan_on ? d->wft.p : nullptr);
   if (sample) {
     const size_t at = (size_t)(step / d->every - 1) * d->nspec;

@@ -210,6 +210,27 @@ def test_queries_after_adjoint_and_digest_opt_in(cal, spm):
     np.testing.assert_array_equal(m.backward(), g)
 
 
+def test_branch_digest_is_of_the_branch_alone(cal, spm):
+    """The digest names the contacts, slips and wall contacts of a step, whatever
+    the launches' shapes: a plain run, a tangent run (another gather) and runs in
+    blocks of 64 to 512 threads that take the same branch give the same digests."""
+    spec = spm.dense_bonded_compression(n=500, seed=5, height=12.0)
+    theta = THETA0[None]
+    ref = None
+    for block in (64, 256, 512):
+        m = cal.DiffModel.from_specimens([spec], 60, EVERY, block=block)
+        m.track_branches()
+        target = np.zeros((1, m.nsamples))
+        st, _ = m.forward(theta, target)
+        dig = m.branch_digest()
+        assert np.any(st != 0.0)  # the walls press
+        if ref is None:
+            ref = dig
+        np.testing.assert_array_equal(dig, ref)
+        m.forward_tangent(theta, np.ones((1, 4)), target)
+        np.testing.assert_array_equal(m.branch_digest(), ref)
+
+
 def test_state_of_a_run_that_lost_particles(cal):
     """A run whose particles leave the domain fails; a query then gives the state it
     had reached."""
