@@ -55,6 +55,8 @@ _SIGS = {
                                          ctypes.c_int, _pd]),
     "esp_diff_set_gravity": (ctypes.c_int, [ctypes.c_void_p, _pd]),
     "esp_diff_set_run": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_int]),
+    "esp_diff_set_tape_limit": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_ulonglong]),
+    "esp_diff_get_tape_bytes": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_ulonglong)]),
     "esp_diff_forward": (ctypes.c_int, [ctypes.c_void_p, _pd, _pd, _pd, _pd]),
     "esp_diff_backward": (ctypes.c_int, [ctypes.c_void_p, _pd]),
     "esp_diff_forward_tangent": (ctypes.c_int, [ctypes.c_void_p, _pd, _pd, _pd, _pd, _pd, _pd]),
@@ -161,6 +163,17 @@ class DiffModel:
         self._check(self.lib.esp_diff_add_wall(self.h, _dp(o), _dp(nn), float(k), _dp(st),
                                                int(bool(measure)), None if a is None else _dp(a)),
                     "add_wall")
+
+    def set_tape_limit(self, nbytes):
+        """Device memory a run may keep for its gradient, every step's state
+        (default 24 GiB); 0: checkpoints every ``checkpoint_every`` steps."""
+        self._check(self.lib.esp_diff_set_tape_limit(self.h, int(nbytes)), "set_tape_limit")
+
+    def tape_bytes(self):
+        """Device memory of the last run's tape; 0 if it kept checkpoints."""
+        b = ctypes.c_ulonglong()
+        self._check(self.lib.esp_diff_get_tape_bytes(self.h, ctypes.byref(b)), "tape_bytes")
+        return b.value
 
     # ---- runs ----
     def forward(self, theta, target):

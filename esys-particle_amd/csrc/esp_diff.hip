@@ -16,7 +16,7 @@
 // for the whole run.
 //
 // Every step writes its state next to the one before, so a run whose states and
-// shear histories fit kTapeBytes is its own tape.  A longer run keeps a checkpoint
+// shear histories fit the tape limit is its own tape.  A longer run keeps a checkpoint
 // every K steps (state, shear histories), and the reverse sweep recomputes one
 // segment's tape at a time (recorded epochs, no search).
 //
@@ -1062,9 +1062,10 @@ struct esp_diff {
   int run_nw = 0;          // its walls
   // The states of the last forward run, step by step ([step][x, v, w, q][n]), and
   // the histories touching pairs read in each: kept by runs whose tape fits
-  // kTapeBytes, so that the adjoint sweeps them without recomputing its segments.
+  // tape_limit, so that the adjoint sweeps them without recomputing its segments.
   // Longer runs keep checkpoints, and the sweep one segment's tape at a time.
   bool full_tape = false;
+  size_t tape_limit;
   DevBuf<double4> tape;
   std::vector<std::unique_ptr<DevBuf<double4>>> hchunk;  // room the histories are laid out in
   std::vector<double4*> htape;                           // [step]
@@ -1128,11 +1129,12 @@ struct esp_diff {
 
 namespace {
 
-// a run's tape (states and histories of every step) is kept up to this size
+// a run's tape (states and histories of every step) is kept up to this size unless
+// the caller sets another
 // (24 specimens of 2,000 to 30,000 particles take 70 MB a step); recomputing the
 // segments and copying their states cost a third of a forward and backward pass
 // (2,000 particles, 100 steps: 12.7 -> 5.8 ms with the launches below)
-constexpr size_t kTapeBytes = (size_t)24 << 30;
+constexpr size_t kTapeLimit = (size_t)24 << 30;
 // A row of 16 lanes a particle up to this many particles, a quad above (the sums
 // are the same, bit by bit): the longest run of interactions sets the time while
 // the chip is not full.  Quad / row, us a step: forward gather 2,000 particles
@@ -1305,9 +1307,10 @@ void restore_checkpoint(esp_diff* d, const Checkpoint& C, double4* T)
 }
 
 // The launches of one forward step (no search) from S into So: tangents (tangent
-// runs), the force laws, the update.  htape: where touching pairs leave the histories they read, or nullptr; record: branch digests
-// and samples (forward runs); halting: the displacement test may stop the queue
-// (not while recomputing a recorded segment).
+// runs), the force laws, the update.  htape: where touching pairs leave the
+// histories they read, or nullptr; record: branch digests and samples (forward
+// runs); halting: the displacement test may stop the queue (not while recomputing
+// a recorded segment).
 void fwd_step(esp_diff* d, const Epoch& E, int step, const DState& S, const DState& So,
               double4* htape, bool record, bool halting)
 {
@@ -1367,8 +1370,47 @@ void clear_run(esp_diff* d)
   DCHK(hipGetLastError());
 }
 
+// device bytes kept for tapes
+size_t tape_bytes(const esp_diff* d)
+{
+  size_t c = d->tape.cap;
+  for (const auto& h : d->hchunk) c += h->cap;
+  return c * sizeof(double4);
+}
+
+// Gives the tape back.  Queries keep their answer; a sweep of the run that was on
+// it runs it again first.
+void release_tape(esp_diff* d)
+{
+  const size_t n = d->n, b = n * sizeof(double4);
+  // the state queries answer with moves by way of the host: there may be no room for
+  // it beside the tape
+  std::vector<double4> h;
+  if (d->tape.p && d->fin.x >= d->tape.p && d->fin.x < d->tape.p + d->tape.cap) {
+    h.resize(4 * n);
+    const double4* src[4] = {d->fin.x, d->fin.v, d->fin.w, d->fin.q};
+    for (int k = 0; k < 4; k++)
+      DCHK(hipMemcpyAsync(h.data() + k * n, src[k], b, hipMemcpyDeviceToHost, d->stream));
+    d->fin = DState{};
+  }
+  dsync(d);
+  d->tape.release();
+  d->hchunk.clear();
+  d->htape.clear();
+  d->full_tape = false;
+  if (h.empty()) return;
+  d->x.reserve(n); d->v.reserve(n); d->w.reserve(n); d->q.reserve(n);
+  const DState S = d->state();
+  double4* dst[4] = {S.x, S.v, S.w, S.q};
+  for (int k = 0; k < 4; k++)
+    DCHK(hipMemcpyAsync(dst[k], h.data() + k * n, b, hipMemcpyHostToDevice, d->stream));
+  dsync(d);
+  d->fin = S;
+}
+
 // where a step's touching pairs leave their histories: laid out one after the
-// other in chunks that are kept for later runs
+// other in chunks that are kept for later runs; past the tape limit (searches may
+// list more pairs than the first one did) the run keeps checkpoints instead
 struct HistoryRoom {
   esp_diff* d;
   size_t chunk, at;
@@ -1379,8 +1421,11 @@ struct HistoryRoom {
       at = 0;
     }
     if (chunk == d->hchunk.size()) {
+      const size_t kept = tape_bytes(d);
+      const size_t left = d->tape_limit > kept ? (d->tape_limit - kept) / sizeof(double4) : 0;
+      if (n > left) throw DiffMemory("the run's tape is past its limit");
       d->hchunk.push_back(std::make_unique<DevBuf<double4>>());
-      const size_t most = (size_t)1 << 25;  // 1 GiB
+      const size_t most = std::min(left, (size_t)1 << 25);  // 1 GiB
       d->hchunk.back()->reserve(std::max(n, std::min(most, n * (size_t)std::max(steps_left, 1))));
       at = 0;
     }
@@ -1392,9 +1437,12 @@ struct HistoryRoom {
 
 int nsamples(const esp_diff* d) { return d->nsteps / d->every; }
 
-// the steps of a forward run; tape: keep every step's state if that fits kTapeBytes
+// the steps of a forward run; tape: keep every step's state if that fits the limit
 void run_forward(esp_diff* d, bool tape)
 {
+  if (d->tan_on)  // the start state is fixed
+    for (DevBuf<double4>* b : {&d->tx, &d->tv, &d->tw, &d->tq})
+      DCHK(hipMemsetAsync(b->p, 0, sizeof(double4) * std::max(d->n, 1), d->stream));
   d->epochs.clear();
   d->ckpts.clear();
   d->rebuild_steps.clear();
@@ -1409,11 +1457,20 @@ void run_forward(esp_diff* d, bool tape)
   DState S0{d->x0.p, d->v0.p, d->w0.p, d->q0.p, d->spec.p, d->n};
   d->fin = S0;
   rebuild(d, S0, 1);
-  d->full_tape = tape && !d->tan_on &&
-                 (size_t)d->nsteps * (32 * c4 + 32 * (size_t)d->epochs[0]->nc) <= kTapeBytes;
+  const size_t states = ((size_t)d->nsteps + 1) * c4;
+  const size_t hists = (size_t)d->nsteps * std::max(d->epochs[0]->nc, 1);
+  const size_t room_for = d->tape_limit / sizeof(double4);
+  const bool fits = tape && !d->tan_on && states + hists <= room_for;
+  // an earlier run's tape that this one cannot use within the limit is given back, as
+  // is one beside a run of checkpoints (but for the room of a segment's states)
+  const size_t kept = tape_bytes(d) / sizeof(double4) - d->tape.cap;
+  if (fits ? std::max(d->tape.cap, states) + std::max(kept, hists) > room_for
+           : !d->tan_on && (kept > 0 || d->tape.cap > ((size_t)std::min(K, d->nsteps) + 1) * c4))
+    release_tape(d);
+  d->full_tape = fits;
   DState cur;
   if (d->full_tape) {
-    d->tape.reserve(((size_t)d->nsteps + 1) * c4);
+    d->tape.reserve(states);
     cur = d->tape_state(d->tape.p);
     d->htape.assign((size_t)d->nsteps + 1, nullptr);
   } else {
@@ -1489,8 +1546,6 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
   if (d->tan_on) {
     const size_t c = std::max(d->n, 1);
     d->tx.reserve(c); d->tv.reserve(c); d->tw.reserve(c); d->tq.reserve(c);
-    for (DevBuf<double4>* b : {&d->tx, &d->tv, &d->tw, &d->tq})
-      DCHK(hipMemsetAsync(b->p, 0, sizeof(double4) * c, d->stream));  // the start state is fixed
     d->wft.reserve(c);
     d->bt.reserve((size_t)std::max(d->nb, 1) * 9);
     d->stress_t.reserve((size_t)std::max(ns, 1) * d->nspec);
@@ -1523,11 +1578,9 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
   try {
     run_forward(d, true);
   } catch (const DiffMemory&) {
-    // no room for the run's tape: again with checkpoints
-    if (!d->full_tape) throw;
-    dsync(d);
-    d->tape.release();
-    d->hchunk.clear();
+    // no room for the run's tape, or beside one kept: again with checkpoints
+    if (tape_bytes(d) == 0 && !d->full_tape) throw;
+    release_tape(d);
     run_forward(d, false);
   }
   d->h_stress.assign((size_t)ns * d->nspec, 0.0);
@@ -1568,13 +1621,9 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
   d->have_forward = true;
 }
 
-void backward(esp_diff* d, double* grad)
+// the reverse sweep over the last forward run; done is recorded at its end
+void sweep(esp_diff* d, double* grad, hipEvent_t done)
 {
-  if (!d->have_forward) throw DiffError(ESP_ERR_STATE, "backward needs a forward run first");
-  hipEvent_t e0, e1;
-  DCHK(hipEventCreate(&e0));
-  DCHK(hipEventCreate(&e1));
-  DCHK(hipEventRecord(e0, d->stream));
   const int n = d->n, bs = d->bs, ns = nsamples(d);
   const int K = std::max(1, d->cfg.checkpoint_every);
   const size_t c = std::max(n, 1);
@@ -1708,19 +1757,46 @@ void backward(esp_diff* d, double* grad)
   std::vector<double4> hg(d->nspec);
   DCHK(hipMemcpyAsync(hg.data(), gs.p, sizeof(double4) * d->nspec, hipMemcpyDeviceToHost,
                       d->stream));
-  DCHK(hipEventRecord(e1, d->stream));
+  DCHK(hipEventRecord(done, d->stream));
   dsync(d);
-  float ms = 0;
-  DCHK(hipEventElapsedTime(&ms, e0, e1));
-  d->t_bwd = ms;
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
   for (int s = 0; s < d->nspec; s++) {
     grad[4 * s] = hg[s].x;
     grad[4 * s + 1] = hg[s].y;
     grad[4 * s + 2] = 0.0;  // cohesion moves only the break events
     grad[4 * s + 3] = hg[s].w;
   }
+}
+
+// the last run again, with checkpoints: every step gives the bits it gave
+void rerun(esp_diff* d)
+{
+  d->have_forward = false;
+  run_forward(d, false);
+  d->have_forward = true;
+}
+
+void backward(esp_diff* d, double* grad)
+{
+  if (!d->have_forward) throw DiffError(ESP_ERR_STATE, "backward needs a forward run first");
+  hipEvent_t e0, e1;
+  DCHK(hipEventCreate(&e0));
+  DCHK(hipEventCreate(&e1));
+  DCHK(hipEventRecord(e0, d->stream));
+  if (!d->full_tape && d->ckpts.empty()) rerun(d);  // its tape was given back
+  try {
+    sweep(d, grad, e1);
+  } catch (const DiffMemory&) {
+    // no room for the adjoint beside the tape
+    if (!d->full_tape) throw;
+    release_tape(d);
+    rerun(d);
+    sweep(d, grad, e1);
+  }
+  float ms = 0;
+  DCHK(hipEventElapsedTime(&ms, e0, e1));
+  d->t_bwd = ms;
+  (void)hipEventDestroy(e0);
+  (void)hipEventDestroy(e1);
 }
 
 }  // namespace
@@ -1794,6 +1870,7 @@ int esp_diff_create(const esp_diff_config* cfg, esp_diff** out)
   }
   esp_diff* d = new esp_diff();
   d->cfg = *cfg;
+  d->tape_limit = kTapeLimit;
   d->bs = bsz;
   memset(&d->grid, 0, sizeof d->grid);
   d->grid.x0 = nmin[0]; d->grid.y0 = nmin[1]; d->grid.z0 = nmin[2];
@@ -1987,6 +2064,24 @@ int esp_diff_set_run(esp_diff* d, int nsteps, int sample_every)
   if (nsteps != d->nsteps || sample_every != d->every) d->have_forward = false;
   d->nsteps = nsteps;
   d->every = sample_every;
+  return ESP_OK;
+  DAPI_END
+}
+
+int esp_diff_set_tape_limit(esp_diff* d, unsigned long long bytes)
+{
+  DAPI_BEGIN
+  d->tape_limit = (size_t)bytes;
+  if (tape_bytes(d) > d->tape_limit) release_tape(d);
+  return ESP_OK;
+  DAPI_END
+}
+
+int esp_diff_get_tape_bytes(esp_diff* d, unsigned long long* out)
+{
+  DAPI_BEGIN
+  if (!out) throw DiffError(ESP_ERR_ARG, "null argument");
+  *out = d->full_tape ? tape_bytes(d) : 0;
   return ESP_OK;
   DAPI_END
 }

@@ -32,11 +32,13 @@
  * Gradients: esp_diff_backward differentiates every specimen's loss with
  * respect to its theta exactly along the branch the forward run took (contact
  * topology, slip states and bond breaks as recorded): a reverse sweep over the
- * states the forward run kept or, for a run whose states exceed 24 GiB (or one by
- * esp_diff_forward_tangent), over checkpointed segments of `checkpoint_every`
- * steps, each recomputed forward before its adjoint; the laws' vector-Jacobian
- * products are their hand-written reverse mode (esp_difflaw.h).  The break criterion depends on cohesion only
- * through events, so d loss / d cohesion is zero on the branch.
+ * states the forward run kept (its tape) or, for a run whose tape exceeds the limit
+ * (24 GiB unless esp_diff_set_tape_limit sets another) and for one by
+ * esp_diff_forward_tangent, over checkpointed segments of `checkpoint_every` steps,
+ * each recomputed forward before its adjoint; the gradients are the same, bit by
+ * bit.  The laws' vector-Jacobian products are their hand-written reverse mode
+ * (esp_difflaw.h).  The break criterion depends on cohesion only through events,
+ * so d loss / d cohesion is zero on the branch.
  */
 #ifndef ESP_DIFF_H
 #define ESP_DIFF_H
@@ -85,6 +87,14 @@ int esp_diff_add_wall(esp_diff* d, const double origin[3], const double normal[3
 int esp_diff_set_gravity(esp_diff* d, const double g[3]);
 /* Steps of one run and the sampling interval of the stress. */
 int esp_diff_set_run(esp_diff* d, int nsteps, int sample_every);
+/* Device memory that a run may keep as its tape (every step's state and the shear
+ * histories read in it), in bytes.  0: runs keep checkpoints every
+ * `checkpoint_every` steps, and their memory is bounded by that interval.  A tape
+ * larger than the limit is given back at once (its run's gradient then runs the
+ * steps again), as is one the device has no room beside. */
+int esp_diff_set_tape_limit(esp_diff* d, unsigned long long bytes);
+/* Device memory of the last run's tape; 0 if it kept checkpoints. */
+int esp_diff_get_tape_bytes(esp_diff* d, unsigned long long* bytes);
 
 /* One forward run from the initial state with theta [4 nspec] against the
  * target stresses [nspec * nsamples]: the sampled stresses (may be NULL) and

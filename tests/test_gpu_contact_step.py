@@ -265,6 +265,59 @@ def test_tape_equals_checkpoints(cal, weak, K):
         np.testing.assert_array_equal(m.particle_data("pos"), pos)
 
 
+def pairs_within(spec, alpha):
+    """Neighbour pairs a search of the specimen lists."""
+    spatial = pytest.importorskip("scipy.spatial")
+    pos, rad = np.asarray(spec["pos"]), np.asarray(spec["rad"])
+    a, b = spatial.cKDTree(pos).query_pairs(2 * rad.max() + alpha, output_type="ndarray").T
+    return int(np.sum(np.linalg.norm(pos[a] - pos[b], axis=1) <= rad[a] + rad[b] + alpha))
+
+
+def test_tape_limit(cal, weak):
+    """Past its limit a tape is given back, before the run, in the middle of it (a
+    later search lists more pairs than the first) or between a run and its gradient;
+    losses, gradients and the final state keep their bits."""
+    steps, n = 200, len(weak["rad"])
+    target = np.full((1, 10), 5.0)
+    states = 32 * 4 * n * (steps + 1)
+    first = 32 * steps * pairs_within(weak, 0.02)
+    ref = None
+    for limit, kept in ((24 << 30, True), (states + first, False), (states, False), (0, False)):
+        m = cal.DiffModel.from_specimens([weak], steps, 20, checkpoint_every=37, alpha=0.02)
+        m.set_tape_limit(limit)
+        for rep in range(2):
+            out = m.forward(THETA, target) + (m.backward(), m.particle_data("pos"))
+            assert (m.tape_bytes() > 0) == kept and m.tape_bytes() <= limit
+            ref = out if ref is None else ref
+            for a, b in zip(out, ref):
+                np.testing.assert_array_equal(a, b)
+        if kept:
+            assert m.tape_bytes() > states + first  # the searches do list more pairs
+    m = cal.DiffModel.from_specimens([weak], steps, 20, checkpoint_every=37, alpha=0.02)
+    m.forward(THETA, target)
+    m.set_tape_limit(states)
+    assert m.tape_bytes() == 0
+    for _ in range(2):
+        np.testing.assert_array_equal(m.particle_data("pos"), ref[3])
+        np.testing.assert_array_equal(m.backward(), ref[2])
+
+
+@pytest.mark.parametrize("copies", [1, 25])
+def test_checkpointed_batch_equals_tape(cal, weak, copies):
+    """Forward runs stepped in place and segments recomputed for the sweep, in a row
+    of lanes a particle and (37,500 particles) in quads, against the tape; segments
+    shorter and longer than the run."""
+    th = np.tile(THETA, (copies, 1))
+    ref = None
+    for K, limit in ((9, 24 << 30), (9, 0), (64, 0)):
+        m = cal.DiffModel.from_specimens([weak] * copies, 40, 10, checkpoint_every=K, alpha=0.05)
+        m.set_tape_limit(limit)
+        out = m.forward(th, np.full((copies, 4), 3.0)) + (m.backward(), m.particle_data("quat"))
+        ref = out if ref is None else ref
+        for a, b in zip(out, ref):
+            np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("copies", [7, 25])
 def test_wide_batch_equals_single(cal, weak, copies):
     """Past the sizes where a particle's row of lanes becomes a quad (8,192 in the
