@@ -146,13 +146,17 @@ def test_adjoint_matches_tangent_linear_slipping(cal, spm):
 
 
 def test_checkpoint_interval_changes_nothing(cal, spec2k):
+    """Checkpoints every step, within and past the run's length, and the tape."""
     out = []
-    for K in (1, 37, 400):
+    for K, limit in ((100, None), (1, 0), (37, 0), (400, 0)):
         m = model_of(cal, [spec2k], K=K)
+        if limit is not None:
+            m.set_tape_limit(limit)
         target = np.full((1, m.nsamples), 5.0)
         _, loss = m.forward(THETA0, target)
+        assert (m.tape_bytes() == 0) == (limit == 0)
         out.append((loss.tobytes(), m.backward().tobytes()))
-    assert out[0] == out[1] == out[2]
+    assert out[0] == out[1] == out[2] == out[3]
 
 
 def test_batch_equals_single_specimens(cal, spm):
@@ -183,13 +187,16 @@ def test_autograd_function(cal, spec2k):
     np.testing.assert_array_equal(theta.grad.numpy(), g)
 
 
-def test_queries_after_adjoint_and_digest_opt_in(cal, spm):
-    """The adjoint sweep recomputes earlier states in the model's arrays; the
-    queries after it still see the forward run's final state and break steps.
-    Branch digests exist only when tracked, and tracking changes no result."""
+@pytest.mark.parametrize("checkpoints", [False, True])
+def test_queries_after_adjoint_and_digest_opt_in(cal, spm, checkpoints):
+    """The adjoint sweep works on the run's tape or, with checkpoints, recomputes
+    earlier states; the queries after it still see the forward run's final state and
+    break steps.  Branch digests exist only when tracked, and tracking changes no result."""
     spec = spm.dense_bonded_compression(n=1500, seed=9, coh_mean=2.0, coh_sd=0.2, wall_speed=20.0)
     theta = np.array([[1e5, 3e4, 2.0, 0.3]])
     m = model_of(cal, [spec], K=50)
+    if checkpoints:
+        m.set_tape_limit(0)
     target = np.zeros((1, m.nsamples))
     st, loss = m.forward(theta, target)
     brk, pos, q = m.bond_breaks(), m.particle_data("pos"), m.particle_data("quat")
