@@ -1478,8 +1478,10 @@ __global__ void k_cells_sort(int ncell, const int* cell_start, int* items)
 // 32 lanes search for one particle, a cell each (a single lane's chain of 27
 // cells took 57 us for 10,000 particles, all of it latency: 13 us so); the
 // second pass collects a particle's partners in LDS and places each by counting
-// the smaller ones.  Runs longer than PAIRS_CAP (wide size ranges with flagged
-// lists) are placed by a second look at the cells.
+// the smaller ones.  Runs longer than PAIRS_CAP (wide size ranges, flagged lists)
+// are merged from the cells' own orders by binary searches: counting costs the
+// square of the run, which is small up to PAIRS_CAP and was 142 ms a search for a
+// large sphere under 1,000 small ones (15 ms so, most of it sorting their cells).
 #define PAIRS_CAP 192
 template <bool EMIT, bool FLAGGED>
 __global__ __launch_bounds__(BS) void k_pairs(PView p, GridParams g, double alpha, const int* cell,
@@ -1527,11 +1529,10 @@ __global__ __launch_bounds__(BS) void k_pairs(PView p, GridParams g, double alph
     for (int t = cell_start[c2]; t < t1; t++) {
       const int q = cell_items[t];
       if (!taken(q)) continue;
+      count++;
       if (EMIT) {
         const int k = atomicAdd(&num[grp], 1);
         if (k < PAIRS_CAP) list[grp * PAIRS_CAP + k] = q;
-      } else {
-        count++;
       }
     }
   }
@@ -1559,28 +1560,56 @@ __global__ __launch_bounds__(BS) void k_pairs(PView p, GridParams g, double alph
       for (int k = 0; k < m; k++) r += mine[k] < q ? 1 : 0;
       put(q, r);
     }
-  } else if (c2 >= 0) {
-    // each of this lane's partners against those of every cell
-    const int t1 = cell_start[c2 + 1];
-    const int c = cell[pi];
-    const int cx = c / (g.ny * g.nz), cy = (c / g.nz) % g.ny, cz = c % g.nz;
-    for (int t = cell_start[c2]; t < t1; t++) {
-      const int q = cell_items[t];
-      if (!taken(q)) continue;
+  } else if (base + m > cap) {
+    // no room for the run: what of it fits only has to name particles
+    for (int r = l; r < m; r += L) put(pi, r);
+  } else {
+    // The cells list their particles in slot order, so the partners of a cell are a
+    // sorted segment (out_q), and a partner's place is the sum of its places in the
+    // 27 segments; (partner, place) goes through out_key, since out_q is read until
+    // every place is known.  The group's lanes are in one wave: a fence orders them.
+    int* seg = list + grp * PAIRS_CAP;  // the segments' starts
+    int before = count;
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) {
+      const int u = __shfl_up(before, o, L);
+      if (l >= o) before += u;
+    }
+    before -= count;
+    if (l < 28) seg[l] = base + before;  // lanes past the cells: the end
+    if (c2 >= 0) {
+      int w = base + before;
+      const int t1 = cell_start[c2 + 1];
+      for (int t = cell_start[c2]; t < t1; t++)
+        if (taken(cell_items[t])) out_q[w++] = cell_items[t];
+    }
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+    for (int e = base + l; e < base + m; e += L) {
+      const int q = out_q[e];
       int r = 0;
       for (int k = 0; k < 27; k++) {
-        int x = cx + k / 9 - 1;
-        const int y = cy + (k / 3) % 3 - 1, z = cz + k % 3 - 1;
-        if (g.circ_x) x = (x + g.nx) % g.nx;
-        if (x < 0 || x >= g.nx || y < 0 || y >= g.ny || z < 0 || z >= g.nz) continue;
-        const int c3 = g.ny * g.nz * x + g.nz * y + z;
-        for (int u = cell_start[c3]; u < cell_start[c3 + 1]; u++) {
-          const int o = cell_items[u];
-          if (o < q && taken(o)) r++;
+        const int s0 = seg[k];
+        int lo = s0, hi = seg[k + 1];
+        while (lo < hi) {
+          const int mid = (lo + hi) >> 1;
+          if (out_q[mid] < q) lo = mid + 1;
+          else hi = mid;
         }
+        r += lo - s0;
       }
-      put(q, r);
+      out_key[e] = ((long long)q << 32) | (long long)r;
     }
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+    for (int e = base + l; e < base + m; e += L) {
+      const long long v = out_key[e];
+      out_q[base + (int)(v & 0xffffffffll)] = (int)(v >> 32);
+      out_p[e] = pi;
+    }
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+    for (int e = base + l; e < base + m; e += L) out_key[e] = pair_key(pi, out_q[e]);
   }
 }
 

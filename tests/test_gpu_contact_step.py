@@ -8,6 +8,7 @@ Tolerances: events and lists bit-exact; a step's arithmetic is the oracle's up t
 the order of a particle's sum, so positions after the few dozen steps here agree to
 1e-9 of a radius (sums of up to 500 forces at 2^-53 each, grown by the contacts)."""
 import importlib
+import time
 
 import numpy as np
 import pytest
@@ -129,6 +130,25 @@ def test_long_runs(pkg, orc, spm, form):
     entries (320 touching, 512) hold."""
     g, o = follow(pkg, orc, spm, hub(), 20, NAMES[form], extra=add_groups(pkg, form))
     assert len(o.engine.neighbour_pairs()) > 400
+
+
+@pytest.mark.parametrize("n_small", [190, 191, 192, 193, 1000])
+def test_search_around_one_large_particle(pkg, orc, spm, n_small):
+    """The large particle's partners around the 192 that are placed by counting, and
+    far past them.  A search around the 1,000 takes 20 ms, 170 where they are placed
+    by counting, too: the bound lies between."""
+    spec = hub(n_small)
+    spec["vel"][:] = (600.0, 0.0, 0.0)  # past half the skin in every step
+    follow(pkg, orc, spm, spec, 4, ["el"], extra=add_groups(pkg, "nrot"))
+    g = pkg.LsmMpi(stepsPerBatch=32)
+    spm.apply(g, spec)
+    add_groups(pkg, "nrot")(g)
+    g.runTimeSteps(4)
+    before, t = g.getStats()["num_rebuilds"], time.perf_counter()
+    g.runTimeSteps(30)
+    ms = (time.perf_counter() - t) * 1e3 / (g.getStats()["num_rebuilds"] - before)
+    print("case: %d around one, %.2f ms a search" % (n_small, ms), flush=True)
+    assert ms < 60.0
 
 
 @pytest.mark.parametrize("tagged", [False, True])
