@@ -278,8 +278,11 @@ struct esp_engine {
   DBuf<double> wall_part;
   PinBuf<double> batch_out;  // what the end of a batch reports: a BatchOut, then wall forces
   size_t servo_at = 0;       // and the servo's sums (k_servo_sums)
-  // engines without bonded groups (contact_mode): the arrays a step writes, each
-  // particle's interactions, the 64-particle groups with wall candidates
+  // engines without bonded groups: whether a step is one launch (chosen at every host
+  // step, see fused_form), the arrays it writes, each particle's interactions, and the
+  // 64-particle groups with wall candidates
+  bool fused = false;
+  double long_run = 0.0;  // about the most neighbours of mean radius a particle has room for
   DBuf<double4> pos2, vel2, ang2;
   DBuf<int> wall_mark, wall_list;
   bool wall_list_valid = false;  // false once slots moved under it, until the next host step
@@ -332,11 +335,66 @@ struct esp_engine {
 
 namespace {
 
-// Without bonded groups a step is one launch in which every particle evaluates
-// its own pairs (k_contact_step); with them the pair and bond laws run once per
-// interaction and a second launch gathers their shares (a bond's law is too
-// long to be evaluated from both ends).
-bool contact_mode(const esp_engine* e) { return e->bg.empty(); }
+// Without bonded groups a step may be one launch in which every particle evaluates
+// its own pairs (k_contact_step, k_contact_block); with them the pair and bond laws
+// run once per interaction and a second launch gathers their shares (a bond's law
+// is too long to be evaluated from both ends).
+bool unbonded(const esp_engine* e) { return e->bg.empty(); }
+
+// Whether the steps until the next host step are one launch (the sums have the same
+// bits either way).  p: pairs per particle.  Both forms timed for 2,000 to 1,000,000
+// sheared spheres and skins that give p from 2.4 to 20 (us a step, one launch / two):
+// - one elastic NRot group (k_contact_step): one launch, 8.1 / 12.1 at 2,000, 29 / 61 at
+//   300,000 spheres, unless four lanes walk long runs: 2,000 at p 25 14.1 / 15.8, at 59
+//   23.0 / 19.8, 500 at p 20 14.2 / 13.4, 8,000 at p 121 37 / 48; a large sphere under 100
+//   small ones 14.6 / 12.4, under 420 46 / 18.  A sphere can have about 4 (1 + R/r)^2
+//   neighbours of radius r; more of them than the rest of the step covers is two launches.
+// The other laws run in k_contact_block, whose blocks hold 512 entries of 64 particles
+// at a time and are all on the chip up to 49,152 particles (mixed and rigid forms, with
+// more registers: 32,768):
+// - friction, 30,000: 12.6 / 16.1 at p 3.7, 14.9 / 16.2 at 7, 18.8 / 18.8 at 10; 60,000:
+//   19.3 / 20.2 at 3.8, 24.7 / 21.8 at 5.1; 300,000: 57.6 / 58.5 at 3.8, 77.6 / 65.4 at 5.1;
+//   1,000,000, where the slots fit no cache: 239 / 272 at 3.9, 321 / 342 at 7.3, 420 / 376
+//   at 10
+// - friction among other groups or rigid, rigid 2,000: 11.1 / 14.6 at 3.4, 20.5 / 15.4 at
+//   8.6; 30,000: 15.1 / 16.5 at 3.7, 23.6 / 21.1 at 9.7; 300,000: 97 / 60 at 3.8; friction
+//   and RotElastic 5,000: 15.1 / 13.4 at 4.8; 30,000: 17.6 / 20.0 at 6.3, 23.6 / 22.8 at 10
+// - elastic laws alone, RotElastic 2,000: 12.1 / 12.7 at 6.3, 14.6 / 13.1 at 8.6; 30,000:
+//   15.4 / 23.9 at 9.7; 300,000: 78 / 64 at 4.3 (1.3e6 pairs), 88 / 96 at 6.1 (1.8e6);
+//   1,000,000: 244 / 294 at 3.9
+bool fused_form(const esp_engine* e)
+{
+  if (!unbonded(e)) return false;
+  if (e->dg.empty()) return true;
+  long long pairs = 0;
+  bool friction = false, rigid = false;
+  for (const DynGroup& G : e->dg) {
+    pairs += G.n;
+    friction |= G.kind == 3;
+    rigid |= G.kind == 3 && G.rigid;
+  }
+  const int n = e->n;
+  const double p = n > 0 ? (double)pairs / n : 0.0;
+  const bool one = e->dg.size() == 1;
+  if (one && e->dg[0].kind == 1)
+    return e->long_run <= 64.0 + n / 500.0 && (n >= 8192 || p <= 15.0 + n / 100.0);
+  if (!friction) {
+    if (n < 16384) return p <= (n < 4096 ? 7.0 : 11.0);
+    return !(n > 160000 && n < 500000 && pairs < 1600000);
+  }
+  if (one && !rigid) return p <= (n <= 49152 ? 7.0 : n < 800000 ? 3.9 : 8.0);
+  return n <= 32768 && p <= (n < 8192 ? 3.9 : 6.5);
+}
+
+void choose_form(esp_engine* e)
+{
+  e->fused = fused_form(e);
+  if (!e->fused) return;
+  const size_t c = std::max(e->n, 1);
+  e->pos2.reserve(c);
+  e->vel2.reserve(c);
+  if (e->rot) e->ang2.reserve(c);
+}
 
 // wall partials of one step
 int wall_blocks(const esp_engine* e)
@@ -541,7 +599,7 @@ void reserve_group(DynGroup& G, size_t n_main, bool hist)
 // stored pairs are looked up only when bonds break
 void rebuild_presence(esp_engine* e, DynGroup& G)
 {
-  if (G.kind != 3 || contact_mode(e)) return;
+  if (G.kind != 3 || unbonded(e)) return;
   build_hash(e, G.hs, G.hs_mask, (size_t)G.n + ESP_APP_CAP, G.key.p, G.n);
 }
 
@@ -793,10 +851,14 @@ void upload(esp_engine* e)
   e->xcnt.reserve(cap);
   e->flist.reserve(cap);
   zero(e, e->xcnt.p, cap);
-  if (contact_mode(e)) {
-    e->pos2.reserve(cap);
-    e->vel2.reserve(cap);
-    if (e->rot) e->ang2.reserve(cap);
+  if (unbonded(e)) {
+    double most = 0.0, sum = 0.0;
+    for (int i = 0; i < n; i++) {
+      most = std::max(most, e->h_rad[i]);
+      sum += e->h_rad[i];
+    }
+    const double ratio = sum > 0.0 ? most / (sum / n) : 0.0;
+    e->long_run = 4.0 * (1.0 + ratio) * (1.0 + ratio);
     e->wall_mark.reserve((size_t)contact_groups((int)cap));
     e->wall_list.reserve((size_t)contact_groups((int)cap) + 1);
     zero(e, e->wall_list.p, (size_t)contact_groups((int)cap) + 1);
@@ -1396,7 +1458,7 @@ void rebuild_csr(esp_engine* e, bool cleared)
   launch_exclusive_scan(e->stream, e->inc_cnt.p, e->inc_off.p, e->n, e->scan_tmp.p);
   e->inc_ent64.reserve(std::max(total, 1));
   if (!cleared) zero(e, e->inc_fill.p, e->n + 1);
-  const bool cm = contact_mode(e);
+  const bool cm = e->fused;
   if (cm) e->contact_ent.reserve(std::max(total, 1));
   else e->slot_of.reserve((size_t)std::max<long long>(rec, 1));
   // summation order: dynamic groups by name (storage order), then bonded groups
@@ -1639,14 +1701,14 @@ void launch_contacts(esp_engine* e, const StepCtl& ctl, bool flip, bool last)
 // them in registers only
 void launch_step(esp_engine* e, const StepCtl& ctl, long long step, bool flip, bool last)
 {
-  if (contact_mode(e)) {
+  if (e->fused) {
     launch_contacts(e, ctl, flip, last);
     return;
   }
   PView p = e->view();
   const ForceLaunch fl = force_launch(e, step, flip);
   UpdParams up;
-  const bool dev_update = ctl.guarded;
+  const bool dev_update = ctl.guarded && !unbonded(e);
   if (dev_update) {
     // bookkeeping of the previous step's bond breaks, on the device
     memset(&up, 0, sizeof up);
@@ -1769,7 +1831,7 @@ void swap_step_buffers(esp_engine* e)
 {
   for (auto& G : e->dg)
     if (G.kind == 3) G.ff.swap(G.ff2);
-  if (contact_mode(e)) {
+  if (e->fused) {
     e->pos.swap(e->pos2);
     e->vel.swap(e->vel2);
     e->ang.swap(e->ang2);
@@ -1785,7 +1847,7 @@ void launch_end(esp_engine* e, long long step0, int k)
   be.nblocks = wall_blocks(e);
   be.nwg = (int)e->wg.size();
   be.nsteps = k;
-  if (contact_mode(e)) {
+  if (unbonded(e)) {
     be.list = e->wall_list.p + 1;
     be.list_n = e->wall_list.p;
   }
@@ -1809,7 +1871,7 @@ void launch_end(esp_engine* e, long long step0, int k)
 // then searches step by step.
 bool quick_search(esp_engine* e, long long step)
 {
-  if (!contact_mode(e) || e->first_time || e->dg.size() != 1 || e->dg[0].track || e->erased_last)
+  if (!unbonded(e) || e->first_time || e->dg.size() != 1 || e->dg[0].track || e->erased_last)
     return false;
   DynGroup& G = e->dg[0];
   const bool hist = G.kind == 3;
@@ -1908,7 +1970,7 @@ void host_step(esp_engine* e, int reason)
                        e->upd.p, e->flist.p, e->evt.p, step, nout > 0 ? &e->grid : nullptr);
     HIPCHK(hipGetLastError());
   }
-  if (!contact_mode(e)) fold(e);
+  if (!unbonded(e)) fold(e);
   if (search && !found) rebuild_rest(e, step, nout);
   e->first_time = false;
   e->forced_search = false;
@@ -1925,10 +1987,10 @@ void host_step(esp_engine* e, int reason)
     if (!e->wg.empty()) {
       WallParam w[ESP_MAX_WALL_GROUPS];
       wall_params(e, w);
-      const bool cm = contact_mode(e);
+      const bool list = unbonded(e);
       launch_wall_update(e->stream, e->view(), e->grid, (int)e->wg.size(), w,
-                         cm ? e->wall_mark.p : nullptr);
-      if (cm) {
+                         list ? e->wall_mark.p : nullptr);
+      if (list) {
         launch_wall_list(e->stream, contact_groups(e->n), e->wall_mark.p, e->wall_list.p + 1,
                          e->wall_list.p);
         e->wall_list_valid = true;
@@ -1937,6 +1999,7 @@ void host_step(esp_engine* e, int reason)
     }
     e->last_ns = e->timestamp;
   }
+  choose_form(e);
   rebuild_csr(e, found);
   sync_history_buffers(e);
   launch_step(e, make_ctl(e, step, 1, 0), step, false, true);
@@ -3084,7 +3147,7 @@ bool servo_bonded(esp_engine* e, int k, const double Fa[3], long long cap)
   wall_params(e, wp);
   // a checkpoint's search may have erased particles and moved the slots of the
   // others since the list was made: then every group is looked at
-  const bool listed = contact_mode(e) && e->wall_list_valid;
+  const bool listed = unbonded(e) && e->wall_list_valid;
   double* out = e->batch_out.p + e->servo_at;
   launch_servo_sums(e->stream, e->view(), wp[k], k, e->do2d, e->init.p,
                     listed ? e->wall_list.p + 1 : nullptr, listed ? e->wall_list.p : nullptr, out);
@@ -3800,7 +3863,7 @@ std::string check_state(esp_engine* e)
   d2h(e, xcnt.data(), e->xcnt.p, n);
   d2h(e, off.data(), e->inc_off.p, n + 1);
   d2h(e, &st, e->upd.p, 1);
-  const bool cm = contact_mode(e);  // entries instead of record slots
+  const bool cm = e->fused;  // entries instead of record slots
   std::vector<int2> so(std::max(e->nrec, 1));
   if (!cm) d2h(e, so.data(), e->slot_of.p, e->nrec);
   const size_t nent = cm && csr ? (size_t)e->xbase : 0;
@@ -3832,7 +3895,7 @@ std::string check_state(esp_engine* e)
         break;
       }
   }
-  if (cm && e->wall_list_valid) {  // every wall candidate is in a listed group
+  if (unbonded(e) && e->wall_list_valid) {  // every wall candidate is in a listed group
     const int ng = contact_groups(n);
     std::vector<int> wl(ng + 1), listed(std::max(ng, 1), 0);
     std::vector<unsigned> fl(std::max(n, 1));

@@ -1,5 +1,5 @@
 """The launches that take a size or a form of their own: the fused step of engines
-without bonded groups, its two contact kernels, the pair search's and the summation
+without bonded groups, its two contact kernels, the line to the two-launch step, the pair search's and the summation
 runs' group sizes, the queries' order, the servo's two ways to its force sum, and
 the calibration engine's gathers and tapes.  Sizes are the edges of waves, of the
 64-particle groups, of the runs a group of lanes holds and of the dispatch rules.
@@ -122,6 +122,64 @@ def test_contact_block_forms(pkg, orc, spm, form, n):
     if "fr" in NAMES[form] and form != "two":
         np.testing.assert_array_equal(g.engine.friction_state("fr")[1],
                                       o.engine.friction_state("fr")[1])
+
+
+def launches(sim):
+    """(steps in two launches, steps in all) since kernel timing was turned on."""
+    kt = sim.engine.kernel_times()
+    return kt["forces"][1], kt["gather_integrate"][1]
+
+
+def skin(spec, alpha):
+    spec["ptype"], spec["elastic"] = "RotSphere", []
+    spec["alpha"], spec["grid"] = alpha, 1.0 + alpha
+    return spec
+
+
+@pytest.mark.parametrize("form,n,alpha,fused", [
+    ("friction", 300, 0.8, True), ("friction", 300, 1.2, False),
+    ("rigid", 300, 0.8, True), ("rigid", 300, 1.2, False),
+    ("mixed", 300, 0.2, True), ("mixed", 300, 0.8, False),
+    ("rotelastic", 300, 0.8, True), ("rotelastic", 300, 1.2, False),
+    ("two", 300, 0.2, True), ("two", 300, 1.2, False),
+    ("nrot", 300, 1.6, True), ("nrot", 300, 2.0, False), ("nrot", 2000, 2.0, True)])
+def test_one_launch_or_two(pkg, orc, spm, form, n, alpha, fused):
+    """Skins to both sides of the pairs a particle up to which a step is one launch."""
+    g, o = follow(pkg, orc, spm, skin(cloud(spm, n, seed=n), alpha), 40, NAMES[form],
+                  extra=add_groups(pkg, form))
+    g.engine.set_kernel_timing(True)
+    for sim in (g, o):
+        sim.runTimeSteps(10)
+    assert launches(g) == (0 if fused else 10, 10)
+    g.engine.check_state()
+    assert np.max(np.abs(g.getParticleData("pos") - o.getParticleData("pos"))) <= TOL
+
+
+def test_form_changes_during_a_run(pkg, orc, spm):
+    """A cloud that contracts: one launch a step while it is loose, two once it is
+    dense, with the oracle's lists, history and walls throughout."""
+    spec = skin(cloud(spm, 300, seed=300), 0.8)
+    mid = spec["pos"].mean(0)
+    spec["vel"] = -4.0 * (spec["pos"] - mid)
+    g, o = pkg.LsmMpi(stepsPerBatch=32), orc.oracle_lsm_class(pkg)()
+    for sim in (g, o):
+        spm.apply(sim, spec)
+        add_groups(pkg, "friction")(sim)
+    g.engine.set_kernel_timing(True)
+    print("case: contracting cloud", flush=True)
+    for _ in range(4):
+        for sim in (g, o):
+            sim.runTimeSteps(30)
+        g.engine.check_state()
+        assert np.max(np.abs(g.getParticleData("pos") - o.getParticleData("pos"))) <= TOL
+        np.testing.assert_array_equal(g.getInteractionPairs("fr"), o.getInteractionPairs("fr"))
+        np.testing.assert_array_equal(g.engine.friction_state("fr")[1],
+                                      o.engine.friction_state("fr")[1])
+        np.testing.assert_allclose(list(g.getWallForce("bottom")), list(o.getWallForce("bottom")),
+                                   rtol=1e-9, atol=1e-9)
+    assert g.engine.rebuild_steps().tolist() == o.engine.rebuild_steps().tolist()
+    two, every = launches(g)
+    assert 0 < two < every
 
 
 @pytest.mark.parametrize("form", ["nrot", "friction", "mixed"])
