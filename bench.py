@@ -415,7 +415,7 @@ def main():
         dyn_bytes = ntouch * B_FRICTION + (nd - ntouch) * B_FRICTION_IDLE
     per_launch = {"forces": nb * B_BOND + dyn_bytes,
                   "gather_integrate": n * b_part}
-    if kt["forces"][1] == 0:  # no bonded group: laws and integration are one launch
+    if kt["forces"][1] == 0:  # laws and integration in one launch
         per_launch["gather_integrate"] += dyn_bytes
     dom = max((k for k in per_launch if kt[k][1] > 0), key=lambda k: kt[k][0])
     avg_s = kt[dom][0] / kt[dom][1] * 1e-3

@@ -14,8 +14,9 @@
 //       first-order update and the max-displacement reduction; wall-force
 //       partials of every 64 particles
 //   k_contact_step, k_contact_block
-//       instead of these two where no group is bonded: each particle evaluates
-//       its side of its interactions and integrates
+//       instead of these two where no group is bonded and one launch is faster
+//       (the host step's fused_form): each particle evaluates its side of its
+//       interactions and integrates
 //   k_batch_end (once per queued batch)
 //       fixed-order sums of the wall-force partials of every step of the batch,
 //       written with the batch's status to page-locked host memory
@@ -902,7 +903,8 @@ __device__ __forceinline__ int xcd_block(int b, int nb)
 // G lanes share a particle's pairs (row entries k = lane, lane + G, ...), their
 // shares are added in row order, then one lane per particle integrates.  Bound by
 // the chain row -> entry -> neighbour's position while the chip is not full: 10,000
-// settling spheres 14.1 us (4.7 + 9.4 in two launches) -> 4.3.
+// settling spheres 14.9 us (4.8 + 10.1 in two launches) -> 7.6, by HIP events of the
+// steps that completed (a launch queued past a halt returns at once, after 1.0 us).
 template <bool EXTRA, int G>
 __global__ __launch_bounds__(BS) void k_contact_step(StepCtl ctl, PView p, ContactLaunch cl,
                                                      GatherParams gp)
@@ -997,10 +999,11 @@ __global__ __launch_bounds__(BS) void k_contact_step(StepCtl ctl, PView p, Conta
 // law runs on full waves (of the 7.5 entries a particle has in a sheared bed
 // about 60 % touch, and a wave that walks its particles' runs waits for the
 // longest of 64), their shares go to LDS, and the first wave adds them in entry
-// order and integrates.  Bound by the gathers of the touching neighbours (160 bytes
-// each, twice a pair) at the three waves a SIMD its registers allow.  Sheared bed,
-// us a step: 30,000 particles 17.2 (7.1 + 10.0 in two launches) -> 14.2, 1,000,000
-// 266 -> 242; four lanes walking a particle's run took 20 and 252.
+// order and integrates.  Bound by the latency of the gathers of the touching neighbours
+// (160 bytes each, twice a pair) at the three waves a SIMD its registers allow: 616 MB
+// move in a step of 1,000,000 particles, 2.5 TB/s.  Sheared bed, us a step: 30,000
+// particles 17.2 (7.1 + 10.0 in two launches) -> 14.2, 1,000,000 266 -> 242; four lanes
+// walking a particle's run took 20 and 252.
 template <bool EXTRA, int KIND>
 __global__ __launch_bounds__(BS, KIND ? 3 : 2) void k_contact_block(StepCtl ctl, PView p, ContactLaunch cl,
                                                          GatherParams gp)
@@ -1476,8 +1479,8 @@ __global__ void k_cells_sort(int ncell, const int* cell_start, int* items)
 // the second writes each particle's run in the order of the partner's slot.
 //
 // 32 lanes search for one particle, a cell each (a single lane's chain of 27
-// cells took 57 us for 10,000 particles, all of it latency: 13 us so); the
-// second pass collects a particle's partners in LDS and places each by counting
+// cells took 53.5 us a launch for 10,000 particles, all of it latency: 6.5 us so);
+// the second pass collects a particle's partners in LDS and places each by counting
 // the smaller ones.  Runs longer than PAIRS_CAP (wide size ranges, flagged lists)
 // are merged from the cells' own orders by binary searches: counting costs the
 // square of the run, which is small up to PAIRS_CAP and was 142 ms a search for a

@@ -361,8 +361,8 @@ int esp_get_pair_events(esp_engine* e, const char* name, int* step, int* id1, in
 /* Kernel classes timed by esp_get_kernel_times. */
 #define ESP_KCLASS_FORCES 0 /* force laws of every interaction group (+ break test), with a
                               queued step's bond-break bookkeeping in its block 0 */
-#define ESP_KCLASS_GATHER 1 /* force gather + integration, per step; the whole step where no
-                              group is bonded (laws and integration are one launch) */
+#define ESP_KCLASS_GATHER 1 /* force gather + integration, per step; the whole step where it
+                              is one launch (as may be where no group is bonded) */
 #define ESP_KCLASS_COUNT 2
 /* Enable (1) or disable (0) HIP-event timing of every per-step kernel launch on
  * the engine's stream: each launch stamps a (start, stop) event pair at the
