@@ -1060,6 +1060,8 @@ struct esp_diff {
   DevBuf<DRun> run;
   std::vector<double> wo;  // wall origins per step of the run [step][wall][3]
   int run_nw = 0;          // its walls
+  int run_has_g = 0;       // its gravity
+  double run_g[3] = {0, 0, 0};
   // The states of the last forward run, step by step ([step][x, v, w, q][n]), and
   // the histories touching pairs read in each: kept by runs whose tape fits
   // tape_limit, so that the adjoint sweeps them without recomputing its segments.
@@ -1119,8 +1121,8 @@ struct esp_diff {
       s.wall[k] = wall0[k];
       for (int c = 0; c < 3; c++) s.wall[k].o[c] = wo[((size_t)step * run_nw + k) * 3 + c];
     }
-    s.has_g = has_g;
-    for (int c = 0; c < 3; c++) s.g[c] = g[c];
+    s.has_g = run_has_g;
+    for (int c = 0; c < 3; c++) s.g[c] = run_g[c];
     s.dt = cfg.dt;
     s.step = step;
     return s;
@@ -1561,6 +1563,8 @@ void forward(esp_diff* d, const double* theta, const double* target, double* str
   // pre-time-step moveWallBy of the main engine's setWallStepMotion)
   {
     const int nw = d->run_nw = d->nw;
+    d->run_has_g = d->has_g;
+    for (int c = 0; c < 3; c++) d->run_g[c] = d->g[c];
     std::vector<double>& wo = d->wo;
     wo.assign((size_t)(d->nsteps + 2) * nw * 3, 0.0);
     double o[DIFF_MAX_WALLS][3];
@@ -1767,7 +1771,8 @@ void sweep(esp_diff* d, double* grad, hipEvent_t done)
   }
 }
 
-// the last run again, with checkpoints: every step gives the bits it gave
+// the last run again (its walls, gravity and parameters), with checkpoints: every
+// step gives the bits it gave
 void rerun(esp_diff* d)
 {
   d->have_forward = false;

@@ -7,6 +7,7 @@ the calibration engine's gathers and tapes.  Sizes are the edges of waves, of th
 Tolerances: events and lists bit-exact; a step's arithmetic is the oracle's up to
 the order of a particle's sum, so positions after the few dozen steps here agree to
 1e-9 of a radius (sums of up to 500 forces at 2^-53 each, grown by the contacts)."""
+import ctypes
 import importlib
 import time
 
@@ -375,6 +376,8 @@ def test_tape_limit(cal, weak):
     m.forward(THETA, target)
     m.set_tape_limit(states)
     assert m.tape_bytes() == 0
+    # of the next forward run, not of the run whose gradient follows
+    m.lib.esp_diff_set_gravity(m.h, (ctypes.c_double * 3)(0.0, -50.0, 0.0))
     for _ in range(2):
         np.testing.assert_array_equal(m.particle_data("pos"), ref[3])
         np.testing.assert_array_equal(m.backward(), ref[2])
